@@ -88,7 +88,7 @@ def main():
     ap.add_argument("--hm-workers", type=int, default=None,
                     help="HM: worker contexts for the subtrees below the first split (default: the library's)")
     ap.add_argument("--block-jet-n", type=int, default=None,
-                    help="largest level run by the single-workgroup Jet (default: the library's)")
+                    help="HEIPA_OPT_BLOCK_JET, the edge bound of Jet's team form (default: the library's)")
     ap.add_argument("--no-autotune", action="store_true",
                     help="headline: skip the pool's launch-shape autotuner (defaults stay)")
     ap.add_argument("--tune-graphs", type=int, default=64, help="headline: batched graphs the autotuner times")

@@ -424,9 +424,9 @@ int heipa_ctx_set_option(heipa_ctx *ctx, int option, uint64_t value) {
         else if (option == HEIPA_OPT_GRAPHS) c.use_graphs = value != 0;
         else if (option == HEIPA_OPT_PROF_SAMPLE) c.prof_sample = value < 1 ? 1u : (u32) std::min<uint64_t>(value, 1u << 30);
         else if (option == HEIPA_OPT_BUCKET_COPIES) c.bucket_copies = (u32) std::min<uint64_t>(value, 32);
-        else if (option == HEIPA_OPT_BLOCK_LDS) c.block_lds = value != 0;
+        else if (option == HEIPA_OPT_BLOCK_LDS || option == HEIPA_OPT_BLOCK_GROUP_CAP) {}  // accepted, without effect
         else if (option == HEIPA_OPT_GROUP_CAP) c.group_cap = (u32) std::min<uint64_t>(value, 64);
-        else if (option == HEIPA_OPT_BLOCK_GROUP_CAP) c.block_group_cap = (u32) std::min<uint64_t>(value, 64);
+        else if (option == HEIPA_OPT_TEAM_JET) c.team_jet_max_n = (u32) std::min<uint64_t>(value, 0xFFFFFFFFull);
         else if (option == HEIPA_OPT_REGION_EDGES) c.region_edges = (u32) std::min<uint64_t>(value, 0xFFFFFFFFull);
         else if (option == HEIPA_OPT_HM_WORKERS) {
             c.hm_workers = (u32) std::min<uint64_t>(value, 64);

@@ -189,11 +189,11 @@ struct Ctx {
     u32 resolve_cap = ~0u;   // HEIPA_OPT_RESOLVE_CAP
     u32 block_jet_max_n = 2048;  // HEIPA_OPT_BLOCK_JET
     u32 group_cap = 64;         // HEIPA_OPT_GROUP_CAP
-    u32 block_group_cap = 8;    // HEIPA_OPT_BLOCK_GROUP_CAP
     u32 region_edges = 1024;    // HEIPA_OPT_REGION_EDGES
+    u32 team_jet_max_n = 1u << 16;  // HEIPA_OPT_TEAM_JET
+    u32 n_xcc = 0, xcc = 0;  // XCDs of the device (0: unknown), the one this context's teams use
     bool use_graphs = true;  // HEIPA_OPT_GRAPHS
     u32 bucket_copies = 0;   // HEIPA_OPT_BUCKET_COPIES (0: automatic)
-    bool block_lds = true;   // HEIPA_OPT_BLOCK_LDS
     u32 hm_workers = 8;      // HEIPA_OPT_HM_WORKERS
     u64 hm_worker_bytes = 0; // HEIPA_OPT_HM_WORKER_BYTES (0: the estimate)
     bool race = false;       // HEIPA_OPT_RACE: atomic order instead of the deterministic rules
@@ -284,6 +284,7 @@ struct Ctx {
 // arena_bytes (0: a quarter of the free device memory) and pinned staging.
 // On failure everything opened so far is released and the error rethrown.
 inline void ctx_close(Ctx &c);
+void find_xccs(Ctx &c);  // jet.hip
 inline void ctx_open(Ctx &c, int device, uint64_t arena_bytes) {
     try {
         c.device = device;
@@ -305,6 +306,7 @@ inline void ctx_open(Ctx &c, int device, uint64_t arena_bytes) {
         c.arena.init(c.arena_mem, arena_bytes);
         c.pinned_bytes = 1 << 18;
         HIP_CHECK(hipHostMalloc(&c.pinned, c.pinned_bytes, hipHostMallocDefault));
+        find_xccs(c);
     } catch (...) {
         ctx_close(c);
         throw;
@@ -349,10 +351,9 @@ inline void ctx_copy_settings(Ctx &to, const Ctx &from) {
     to.block_jet_max_n = from.block_jet_max_n;
     to.use_graphs = from.use_graphs;
     to.bucket_copies = from.bucket_copies;
-    to.block_lds = from.block_lds;
     to.group_cap = from.group_cap;
-    to.block_group_cap = from.block_group_cap;
     to.region_edges = from.region_edges;
+    to.team_jet_max_n = from.team_jet_max_n;
     to.hm_workers = from.hm_workers;
     to.hm_worker_bytes = from.hm_worker_bytes;
     to.race = from.race;

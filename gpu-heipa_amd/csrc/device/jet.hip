@@ -35,13 +35,17 @@
 // Launches per iteration: sweep (LP best block | rebalance score), buckets
 // (rebalance only: per-block prefix of the minibucket totals), post
 // (afterburner | rebalance classify), resolve (rebalance only), apply, and a
-// one-workgroup control launch (block weights, counters, loop state).  No
-// kernel synchronises across workgroups: every hand-off is a launch boundary.
+// one-workgroup control launch (block weights, counters, loop state); every
+// hand-off between workgroups is a launch boundary.  Levels of up to 65536
+// vertices run the same steps as a team of workgroups on one XCD instead,
+// whole iterations per launch (jet_team.hpp).
 #include "eval.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 namespace heipa {
 namespace {
@@ -84,14 +88,19 @@ __device__ u32 gain_bucket(s64 gx, s64 vwgt) {
     if (gx > 0) return 0;
     if (gx == 0) return 1;
     const float g = (float) (-gx) / (float) vwgt;
+    // the least k with g >= LO[k] (g < 1) or g <= HI[k] is the logarithm x of
+    // g to the base 1.5 rounded up: round(x) is that k or one less, so one
+    // threshold decides (a walk over the table was up to 25 dependent loads)
+    const float x = __log2f(g) * 1.70951129f;  // 1 / log2(1.5)
     if (g < 1.0f) {
-        for (int k = 1; k <= 23; ++k)
-            if (g >= kLo[k]) return (u32) (MID_BUCKETS - k);
-        return 2;
+        int k = (int) fminf(0.5f - x, 24.0f);
+        k = k < 1 ? 1 : k;
+        if (k <= 23 && g < kLo[k]) ++k;
+        return k <= 23 ? (u32) (MID_BUCKETS - k) : 2u;
     }
-    for (int k = 0; k <= 24; ++k)
-        if (g <= kHi[k]) return (u32) (MID_BUCKETS + k);
-    return MAX_BUCKETS - 1;
+    int k = (int) fminf(x + 0.5f, 25.0f);
+    if (k <= 24 && g > kHi[k]) ++k;
+    return k <= 24 ? (u32) (MID_BUCKETS + k) : MAX_BUCKETS - 1;
 }
 
 __device__ __forceinline__ u64 mix64d(u64 z) {
@@ -145,21 +154,58 @@ struct JetCtl {
     u32 iters;        // iterations that changed the partition
     u32 n_trace;
     u32 last_moves;   // length of the last iteration's move list (update_large when > n / 10)
+    u32 launches;     // team launches that ran
+    u32 failed;       // a team member never arrived at a barrier
 };
 static_assert(sizeof(CtlHead) == 32 && offsetof(JetCtl, st) == sizeof(CtlHead), "control block head layout");
 
-struct JetDev {
+// A pointer to device memory that other workgroups of the same launch write:
+// every load is a device-scope one, which reads the L2 and not this compute
+// unit's L1 (88 ns against 52 ns from L1 on an idle chip; the same rate under
+// load).  Stores are plain: L1 writes through.
+template<typename T>
+struct DevRef {
+    T *p;
+    __device__ __forceinline__ operator T() const { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    __device__ __forceinline__ void operator=(T v) const { *p = v; }
+    __device__ __forceinline__ void operator=(const DevRef &o) const { *p = (T) o; }
+    __device__ __forceinline__ void operator&=(T v) const { *p = (T) ((T) *this & v); }
+};
+template<typename T>
+struct DevPtr {
+    T *p;
+    __device__ __forceinline__ DevRef<T> operator[](u64 i) const { return {p + i}; }
+    __device__ __forceinline__ DevPtr operator+(u64 i) const { return {p + i}; }
+    __device__ __forceinline__ explicit operator bool() const { return p != nullptr; }
+};
+template<typename T>
+__device__ __forceinline__ T *raw(T *p) { return p; }
+template<typename T>
+__device__ __forceinline__ T *raw(const DevPtr<T> &p) { return p.p; }
+
+// TEAM: the view of the team form (one launch in which several workgroups run
+// whole iterations), same layout: the arrays that one workgroup writes and
+// another reads are reached through DevPtr.
+template<bool TEAM, bool MAP>
+struct JetDevT {
+    template<typename T>
+    using S = std::conditional_t<TEAM, DevPtr<T>, T *>;  // shared between workgroups
+    static constexpr bool team = TEAM;
+    static constexpr bool map = MAP;  // may hold D
     u32 n, k;
     s64 lmax, opt;  // opt = ceil(W / k)
     const u32 *xadj, *adj;
     const s32 *ew, *vw;
-    u32 *work, *dest, *dcache, *mark, *oldp, *part;
-    s64 *gcache, *gain1;
-    s64 *icache;  // connection to the own block of a vertex whose neighbours all share its block; -1: unknown
-    u8 *lock;
-    u32 *cand, *moves;      // regions of cap / cap_mv entries, one per sweep workgroup
+    S<u32> work, dest, dcache, mark, oldp;
+    u32 *part;
+    S<s64> gcache, gain1;
+    S<s64> icache;  // connection to the own block of a vertex whose neighbours all share its block; -1: unknown
+    S<u8> lock;
+    S<u32> cand;
+    u32 *moves;             // regions of cap / cap_mv entries, one per sweep workgroup
     u32 *cand_n, *moves_n;  // region lengths
-    u32 *cand_x, *moves_x;  // extra lists (lengths in st[ST_CAND], st[ST_MOVES])
+    u32 *cand_x;
+    S<u32> moves_x;         // extra lists (lengths in st[ST_CAND], st[ST_MOVES])
     unsigned long long *pstat;  // PT_COUNT partial statistics per sweep workgroup
     u32 nreg, cap, cap_mv;
     u32 count_bytes;  // hub kernels add their degree statistics (the byte accounting of the profiler)
@@ -172,26 +218,30 @@ struct JetDev {
     // rebalancing
     u32 sections, width, t;
     u32 nshard;         // workgroup w adds into copy w % nshard (spreads same-address atomics)
-    u32 *gid;           // minibucket per vertex
-    s64 *btot;          // nshard copies of the t + 1 minibucket totals, zero between iterations
-    s64 *Q, *R;         // t: exclusive / inclusive prefix of btot inside each block's range
-    s64 *Tseg;          // k: total of each block's range
-    u64 *rlist;         // resolve list: minibucket << 32 | vertex
+    S<u32> gid;         // minibucket per vertex
+    S<s64> btot;          // nshard copies of the t + 1 minibucket totals, zero between iterations
+    S<s64> Q, R;        // t: exclusive / inclusive prefix of btot inside each block's range
+    S<s64> Tseg;        // k: total of each block's range
+    S<u64> rlist;       // resolve list: minibucket << 32 | vertex
     s64 *evict_adjust;  // k
     s64 *evict_start;   // k + 1
     s64 *counter;       // strong-rebalance overflow position
     const s32 *D;       // k x k distances: mapping objective J (ProMap); null: edge cut
     // BlockConn rows of the wide vertices (degree >= k); rflag null when the level has none
-    u8 *rflag;          // n: bit 0 wide, bit 1 a neighbour is in this iteration's move list,
+    S<u8> rflag;        // n: bit 0 wide, bit 1 a neighbour is in this iteration's move list,
                         // bit 2 its neighbour counts are kept (wcnt)
     u32 *wid;           // n: rank among the wide vertices
-    u32 *wsz;           // per wide vertex: the row's size (BlockConn sizes)
-    u32 *wV, *wP;       // per wide vertex, W words each: blocks of its valid entries / of positive ones
+    S<u32> wsz;         // per wide vertex: the row's size (BlockConn sizes)
+    S<u32> wV, wP;      // per wide vertex, W words each: blocks of its valid entries / of positive ones
     u32 *wcnt;          // per wide vertex, k counts of its neighbours per block, kept by the moves for
                         // the counted ones: k <= 64 and ROW_THREAD_DEG < degree <= hub_deg
     u32 W;              // words per block mask, ceil(k / 32)
     u32 race;           // atomic order: minibucket offsets and strong overflow positions from fetch-adds
+    u32 shard;          // team form: this workgroup's copy of the minibucket totals
 };
+using JetDev = JetDevT<false, true>;
+static_assert(sizeof(JetDev) == sizeof(JetDevT<true, true>) && sizeof(JetDev) == sizeof(JetDevT<true, false>),
+              "views of one layout");
 
 // Per-vertex staleness of the caches, the n bytes after the locks: bit 0
 // the decision cache (dcache, gcache), bit 1 the interior cache.  Moving a
@@ -199,8 +249,10 @@ struct JetDev {
 // rewriting both caches (12 bytes): the bytes stay in L2 where the caches
 // (12n) do not, and most moves of a rebalancing iteration touch vertices
 // many times.
-__device__ __forceinline__ u8 *stale_of(const JetDev &d) { return d.lock + d.n; }
-__device__ __forceinline__ s64 vwt(const JetDev &d, u32 u) { return d.vw ? (s64) d.vw[u] : 1; }
+template<typename JD>
+__device__ __forceinline__ auto stale_of(const JD &d) { return d.lock + d.n; }
+template<typename JD>
+__device__ __forceinline__ s64 vwt(const JD &d, u32 u) { return d.vw ? (s64) d.vw[u] : 1; }
 
 // a candidate's weight into minibucket g: rebalancing puts most candidates of
 // an overloaded block into a few dozen minibuckets, so each workgroup adds into
@@ -209,14 +261,17 @@ __device__ __forceinline__ s64 vwt(const JetDev &d, u32 u) { return d.vw ? (s64)
 // vertex's offset in its minibucket (the reference's temp_gain =
 // atomic_fetch_add, jet:439, :684) in gain1, which no rebalancing iteration
 // reads otherwise.
-__device__ __forceinline__ void btot_add(const JetDev &d, u32 u, u32 g, s64 w) {
-    const u64 copy = d.nshard > 1 ? blockIdx.x % d.nshard : 0;
+template<typename JD>
+__device__ __forceinline__ void btot_add(const JD &d, u32 u, u32 g, s64 w) {
+    const u64 copy = JD::team ? d.shard : d.nshard > 1 ? blockIdx.x % d.nshard : 0;
     const unsigned long long old =
-        atomicAdd((unsigned long long *) &d.btot[copy * ((u64) d.t + 1) + g], (unsigned long long) w);
+        atomicAdd((unsigned long long *) raw(d.btot) + (copy * ((u64) d.t + 1) + g), (unsigned long long) w);
     if (d.race) d.gain1[u] = (s64) old;
 }
-__device__ __forceinline__ s64 ewt(const JetDev &d, u32 j) { return d.ew ? (s64) d.ew[j] : 1; }
-__device__ __forceinline__ u32 degree(const JetDev &d, u32 u) { return d.xadj[u + 1] - d.xadj[u]; }
+template<typename JD>
+__device__ __forceinline__ s64 ewt(const JD &d, u32 j) { return d.ew ? (s64) d.ew[j] : 1; }
+template<typename JD>
+__device__ __forceinline__ u32 degree(const JD &d, u32 u) { return d.xadj[u + 1] - d.xadj[u]; }
 __device__ __forceinline__ bool live(const JetCtl *ctl) { return ctl->active && !ctl->stalled; }
 __device__ __forceinline__ CtlHead ctl_head(const JetCtl *ctl) {
     CtlHead h;
@@ -226,7 +281,8 @@ __device__ __forceinline__ CtlHead ctl_head(const JetCtl *ctl) {
 __device__ __forceinline__ bool live(const CtlHead &h) { return h.active && !h.stalled; }
 
 // eviction threshold of rebalance_strong (jet:363) / rebalance_weak (jet:600-604)
-__device__ __forceinline__ s64 max_block_weight(const JetDev &d, bool strong) {
+template<typename JD>
+__device__ __forceinline__ s64 max_block_weight(const JD &d, bool strong) {
     const s64 a = (s64) ((double) d.lmax * 0.99);
     if (strong) return d.opt + 1 > a ? d.opt + 1 : a;
     return a < d.lmax - 100 ? d.lmax - 100 : a;
@@ -244,7 +300,8 @@ constexpr u32 ROW_THREAD_DEG = 32;  // wide vertices up to this degree walk thei
 // f = rflag[v] and wid = wid[v] (read only if v is counted), loaded by the
 // caller together with the neighbour's other state: a load after the stores
 // of the previous neighbour waited for them
-__device__ __forceinline__ void row_touch(const JetDev &d, u32 v, u8 f, u32 wid, u32 ou, u32 nu) {
+template<typename JD>
+__device__ __forceinline__ void row_touch(const JD &d, u32 v, u8 f, u32 wid, u32 ou, u32 nu) {
     if (f & 1u) {
         if (!(f & 2u)) d.rflag[v] = f | 2u;  // most neighbours of a move list are touched many times
         if ((f & 4u) && ou != nu) {
@@ -256,7 +313,8 @@ __device__ __forceinline__ void row_touch(const JetDev &d, u32 v, u8 f, u32 wid,
 }
 
 // the block mask of a counted vertex's positive entries from its counts
-__device__ __forceinline__ u64 row_count_mask(const JetDev &d, u32 v) {
+template<typename JD>
+__device__ __forceinline__ u64 row_count_mask(const JD &d, u32 v) {
     const u64 base = (u64) d.wid[v] * d.k;
     u64 mask = 0;
     for (u32 b = 0; b < d.k; ++b)
@@ -266,7 +324,8 @@ __device__ __forceinline__ u64 row_count_mask(const JetDev &d, u32 v) {
 
 // the wide vertex u's row holds k entries: its valid entries include the
 // blocks whose connection fell to 0 since the row filled up
-__device__ __forceinline__ bool row_full(const JetDev &d, u32 u, u32 &r) {
+template<typename JD>
+__device__ __forceinline__ bool row_full(const JD &d, u32 u, u32 &r) {
     if (!d.rflag || !(d.rflag[u] & 1u)) return false;
     r = d.wid[u];
     return d.wsz[r] == d.k;
@@ -300,7 +359,8 @@ __device__ __forceinline__ void append64(bool pred, u64 val, u64 *list, unsigned
 }
 
 // wave-aggregated append to this workgroup's region (LDS counter)
-__device__ __forceinline__ void append_local(bool pred, u32 val, u32 *region, u32 *s_cnt) {
+template<typename T>
+__device__ __forceinline__ void append_local(bool pred, T val, T *region, u32 *s_cnt) {
     const u64 bal = __ballot(pred);
     if (!bal) return;
     const u32 first = (u32) __builtin_ctzll(bal);
@@ -377,8 +437,8 @@ constexpr u32 ADJ_UNROLL = 4;
 template<int G>
 constexpr u32 group_unroll() { return G >= 32 ? ADJ_UNROLL : 1; }
 
-template<u32 ADJ_UNROLL>
-__device__ __forceinline__ void conn_accumulate_range(const JetDev &d, const GroupConn &gc, u64 b0, u64 e, u32 lane,
+template<u32 ADJ_UNROLL, typename JD>
+__device__ __forceinline__ void conn_accumulate_range(const JD &d, const GroupConn &gc, u64 b0, u64 e, u32 lane,
                                                       u32 G) {
     for (u64 j0 = b0 + lane; j0 < e; j0 += (u64) G * ADJ_UNROLL) {
         u32 v[ADJ_UNROLL], bl[ADJ_UNROLL];
@@ -401,8 +461,8 @@ __device__ __forceinline__ void conn_accumulate_range(const JetDev &d, const Gro
     }
 }
 
-template<u32 ADJ_UNROLL>
-__device__ __forceinline__ void conn_accumulate(const JetDev &d, const GroupConn &gc, u32 u, u32 lane, u32 G) {
+template<u32 ADJ_UNROLL, typename JD>
+__device__ __forceinline__ void conn_accumulate(const JD &d, const GroupConn &gc, u32 u, u32 lane, u32 G) {
     conn_accumulate_range<ADJ_UNROLL>(d, gc, d.xadj[u], d.xadj[u + 1], lane, G);
 }
 
@@ -468,12 +528,12 @@ __device__ __forceinline__ T group_sum(T x, T *red) {
 // ---------------------------------------------------------------- LP evaluation
 // best_block (:200-236) + filter (:247-258) of one rebuilt vertex; lane 0 of
 // the group writes the results; returns whether u is a candidate
-template<int G>
-__device__ __forceinline__ bool lp_eval(const JetDev &d, const GroupConn &gc, u32 u, u32 own_b, bool locked, u32 lane,
+template<int G, typename JD>
+__device__ __forceinline__ bool lp_eval(const JD &d, const GroupConn &gc, u32 u, u32 own_b, bool locked, u32 lane,
                                         double ratio, Best *red, s64 *red2, bool active) {
     const u32 T = active ? *gc.tcount : 0;
     Best best{0, NO_MOVE};
-    if (d.D) {
+    if (JD::map && d.D) {
         // ProMap_jet_lp best_block (promap_jet_label_propagation.h:230-258):
         // gain_delta (:180-204) of a move to b is J(own) - J(b) with
         // J(x) = sum over the touched blocks c of conn(c) * D(x, c); the lanes
@@ -535,7 +595,7 @@ __device__ __forceinline__ bool lp_eval(const JetDev &d, const GroupConn &gc, u3
         s64 gain = 0;
         if (best_id != NO_MOVE) {
             const s64 bc = best.c;
-            if (d.D) {
+            if (JD::map && d.D) {
                 if (bc >= 0) gain = bc;  // promap:232: best_delta starts at -1
                 else best_id = NO_MOVE;
             } else if (bc >= own || ((double) own - (double) bc) < floor(ratio * (double) own)) {
@@ -569,10 +629,11 @@ struct RebShared {
     u32 under[1];  // k entries
 };
 
-// computed by the first wave, 64 blocks per step
-__device__ __forceinline__ void reb_prologue(const JetDev &d, bool strong, s64 mbw, RebShared *rs) {
-    if (threadIdx.x < WAVE) {
-        const u32 lane = threadIdx.x;
+// computed by one wave, 64 blocks per step
+template<typename JD>
+__device__ __forceinline__ void reb_prologue_wave(const JD &d, bool strong, s64 mbw, RebShared *rs) {
+    {
+        const u32 lane = lane_id();
         if (!strong) {
             u32 c = 0;
             for (u32 b0 = 0; b0 < d.k; b0 += WAVE) {
@@ -591,11 +652,16 @@ __device__ __forceinline__ void reb_prologue(const JetDev &d, bool strong, s64 m
             if (lane == 0) rs->max_vwgt = mx;
         }
     }
+}
+template<typename JD>
+__device__ __forceinline__ void reb_prologue(const JD &d, bool strong, s64 mbw, RebShared *rs) {
+    if (threadIdx.x < WAVE) reb_prologue_wave(d, strong, mbw, rs);
     __syncthreads();
 }
 
 // vertices considered for eviction (weak jet:641-646, strong jet:394-398)
-__device__ __forceinline__ bool reb_eligible(const JetDev &d, bool strong, const RebShared *rs, u32 u, u32 ub) {
+template<typename JD>
+__device__ __forceinline__ bool reb_eligible(const JD &d, bool strong, const RebShared *rs, u32 u, u32 ub) {
     const s64 bwu = d.bw[ub];
     const s64 wu = vwt(d, u);
     if (!strong) return bwu > d.lmax && (double) wu < 1.5 * (double) (bwu - d.opt);
@@ -606,8 +672,8 @@ __device__ __forceinline__ bool reb_eligible(const JetDev &d, bool strong, const
 // weak best block (jet:658-694) / strong score (jet:399-435) of one vertex;
 // lane 0 records dest (weak), the minibucket and its weight; returns whether
 // u is a candidate
-template<int G>
-__device__ __forceinline__ bool reb_eval(const JetDev &d, bool strong, s64 mbw, const RebShared *rs,
+template<int G, typename JD>
+__device__ __forceinline__ bool reb_eval(const JD &d, bool strong, s64 mbw, const RebShared *rs,
                                          const GroupConn &gc, u32 u, u32 own_b, u32 lane, Best *red, s64 *red2,
                                          bool active) {
     const u32 T = active ? *gc.tcount : 0;
@@ -691,7 +757,8 @@ __device__ __forceinline__ bool reb_eval(const JetDev &d, bool strong, s64 mbw, 
 // (own connection `own`), without its adjacency: no other block is touched,
 // so weak sends it to underloaded[u % count] with gain -own and strong
 // scores it 0 / 1 - own.  Returns whether u is a candidate.
-__device__ __forceinline__ bool reb_interior(const JetDev &d, bool strong, const RebShared *rs, u32 u, s64 own) {
+template<typename JD>
+__device__ __forceinline__ bool reb_interior(const JD &d, bool strong, const RebShared *rs, u32 u, s64 own) {
     const u32 own_b = d.work[u];
     const s64 wu = vwt(d, u);
     if (!strong) {
@@ -715,7 +782,8 @@ __device__ __forceinline__ bool reb_interior(const JetDev &d, bool strong, const
 // candidates in minibuckets [ub * width, g).  A strong candidate in the last
 // minibucket of its block lands at index (ub + 1) * width (the reference's +1
 // minibucket offset, jet:437), i.e. after its block's whole range.
-__device__ __forceinline__ s64 bucket_prefix(const JetDev &d, u32 g, u32 ub) {
+template<typename JD>
+__device__ __forceinline__ s64 bucket_prefix(const JD &d, u32 g, u32 ub) {
     return g >= (ub + 1) * d.width ? d.Tseg[ub] : d.Q[g];
 }
 
@@ -957,8 +1025,8 @@ __global__ __launch_bounds__(JB) void hub_sweep_kernel(JetDev d, const u32 *hubs
 // ---------------------------------------------------------------- post: afterburner / classify
 // afterburner (jet:269-328): selected candidates are locked, stamped and
 // appended to the move list
-template<u32 ADJ_UNROLL>
-__device__ __forceinline__ s64 afterburner_change_range(const JetDev &d, u32 u, u64 b, u64 e, u32 lane, u32 stride) {
+template<u32 ADJ_UNROLL, typename JD>
+__device__ __forceinline__ s64 afterburner_change_range(const JD &d, u32 u, u64 b, u64 e, u32 lane, u32 stride) {
     const s64 ug = d.gain1[u];
     const u32 o = d.work[u], nn = d.dest[u];
     const s32 *Do = d.D ? d.D + (u64) o * d.k : nullptr, *Dn = d.D ? d.D + (u64) nn * d.k : nullptr;
@@ -984,7 +1052,7 @@ __device__ __forceinline__ s64 afterburner_change_range(const JetDev &d, u32 u, 
             if (j0 + (u64) q * stride >= e) continue;
             const bool first = vg[q] > ug || (vg[q] == ug && v[q] < u);
             if (!first) continue;
-            if (Do)  // promap:297-314: the gain of u once v has moved minus its gain before
+            if (JD::map && Do)  // promap:297-314: the gain of u once v has moved minus its gain before
                 change += w[q] * (((s64) Do[vn[q]] - (s64) Dn[vn[q]]) - ((s64) Do[vo[q]] - (s64) Dn[vo[q]]));
             else
                 change += w[q] * ((s64) (vn[q] == nn) - (s64) (vn[q] == o) + (s64) (vo[q] == o) - (s64) (vo[q] == nn));
@@ -992,9 +1060,27 @@ __device__ __forceinline__ s64 afterburner_change_range(const JetDev &d, u32 u, 
     }
     return change;
 }
-template<u32 ADJ_UNROLL>
-__device__ __forceinline__ s64 afterburner_change(const JetDev &d, u32 u, u32 lane, u32 stride) {
+template<u32 ADJ_UNROLL, typename JD>
+__device__ __forceinline__ s64 afterburner_change(const JD &d, u32 u, u32 lane, u32 stride) {
     return afterburner_change_range<ADJ_UNROLL>(d, u, d.xadj[u], d.xadj[u + 1], lane, stride);
+}
+
+// one candidate, G lanes; on lane 0, whether it is selected (then locked and
+// stamped)
+template<int G, typename JD>
+__device__ __forceinline__ bool afterburner_one(const JD &d, u32 stamp, u32 u, u32 ub, u32 ue, u32 lane, bool active,
+                                                bool do_hash, u64 &degs, u64 &gh) {
+    s64 ch = active ? afterburner_change_range<group_unroll<G>()>(d, u, ub, ue, lane, G) : 0;
+    ch = group_sum<G>(ch, (s64 *) nullptr);
+    if (!active || lane != 0) return false;
+    degs += ue - ub;
+    const s64 ug = d.gain1[u];
+    if (do_hash) gh += mix64d(mix64d(u) + (u64) ug);
+    if (ug + ch < 0) return false;
+    d.lock[u] = 1;
+    d.mark[u] = stamp;
+    d.oldp[u] = d.work[u];
+    return true;
 }
 
 // afterburner over `len` candidates of `region`, G lanes each; selected
@@ -1023,20 +1109,7 @@ __device__ __forceinline__ void afterburner_list(const JetDev &d, u32 stamp, con
             nxe = d.xadj[nxu + 1];
         }
         const bool hub = active && ue - ub > d.hub_deg;
-        s64 ch = (active && !hub) ? afterburner_change_range<group_unroll<G>()>(d, u, ub, ue, lane, G) : 0;
-        ch = group_sum<G>(ch, (s64 *) nullptr);
-        bool sel = false;
-        if (active && !hub && lane == 0) {
-            degs += ue - ub;
-            const s64 ug = d.gain1[u];
-            if (do_hash) gh += mix64d(mix64d(u) + (u64) ug);
-            if (ug + ch >= 0) {
-                d.lock[u] = 1;
-                d.mark[u] = stamp;
-                d.oldp[u] = d.work[u];
-                sel = true;
-            }
-        }
+        const bool sel = afterburner_one<G>(d, stamp, u, ub, ue, lane, active && !hub, do_hash, degs, gh);
         append_local(sel, u, mregion, s_cnt);
     }
 }
@@ -1049,6 +1122,20 @@ __device__ __forceinline__ void afterburner_list(const JetDev &d, u32 stamp, con
 // adjust_scores) goes to the resolve list.  Both tests depend on the
 // minibucket only, so a minibucket is either wholly in the resolve list or not
 // at all, and offsets computed over the list are offsets in the minibucket.
+enum Take : u32 { TAKE_NO = 0, TAKE_SURE, TAKE_BOUNDARY };
+template<typename JD>
+__device__ __forceinline__ Take classify_take(const JD &d, bool strong, u32 stamp, u32 u, u64 &key) {
+    const u32 g = d.gid[u], ub = d.work[u];
+    const s64 limit = d.bw[ub] - d.lmax;
+    if (bucket_prefix(d, g, ub) >= limit) return TAKE_NO;
+    if (!strong && d.R[g] < limit) {
+        d.mark[u] = stamp;
+        d.oldp[u] = ub;
+        return TAKE_SURE;
+    }
+    key = ((u64) g << 32) | u;
+    return TAKE_BOUNDARY;
+}
 __device__ __forceinline__ void classify_one(const JetDev &d, bool strong, u32 stamp, bool valid, u32 u,
                                              u32 *mregion, u32 *s_cnt) {
     JetCtl *ctl = d.ctl;
@@ -1073,18 +1160,9 @@ __device__ __forceinline__ void classify_one(const JetDev &d, bool strong, u32 s
                 }
             }
         } else if (valid) {
-            const u32 g = d.gid[u], ub = d.work[u];
-            const s64 limit = d.bw[ub] - d.lmax;
-            if (bucket_prefix(d, g, ub) < limit) {
-                if (!strong && d.R[g] < limit) {
-                    sure = true;
-                    d.mark[u] = stamp;
-                    d.oldp[u] = ub;
-                } else {
-                    boundary = true;
-                    key = ((u64) g << 32) | u;
-                }
-            }
+            const Take take = classify_take(d, strong, stamp, u, key);
+            sure = take == TAKE_SURE;
+            boundary = take == TAKE_BOUNDARY;
         }
         append_local(sure, u, mregion, s_cnt);
         append64(boundary, key, d.rlist, &ctl->st[ST_RLIST]);
@@ -1121,16 +1199,17 @@ __device__ __forceinline__ void classify_body(const JetDev &d, bool strong, u32 
 // on its highest-degree vertex, and held few vertices in flight when the
 // lists are long (rebalancing on skewed graphs moves a large share of all
 // vertices per iteration).
-constexpr u32 FLAT_CHUNK = JB;
+template<int NT>
 struct FlatLds {
-    u32 u[FLAT_CHUNK];
-    u32 start[FLAT_CHUNK];  // xadj[u]
-    u32 off[FLAT_CHUNK + 1];
-    u32 a[FLAT_CHUNK], b[FLAT_CHUNK];
-    s64 g[FLAT_CHUNK];
-    unsigned long long acc[FLAT_CHUNK];
-    u32 red[JB / WAVE];
+    u32 u[NT];
+    u32 start[NT];  // xadj[u]
+    u32 off[NT + 1];
+    u32 a[NT], b[NT];
+    s64 g[NT];
+    unsigned long long acc[NT];
+    u32 red[NT / WAVE];
 };
+constexpr u32 FLAT_CHUNK = JB;
 
 // last i in [0, cnt) with off[i] <= x (off non-decreasing, off[0] = 0)
 __device__ __forceinline__ u32 flat_find(const u32 *off, u32 cnt, u32 x) {
@@ -1144,89 +1223,88 @@ __device__ __forceinline__ u32 flat_find(const u32 *off, u32 cnt, u32 x) {
 }
 
 // degrees of the staged vertices -> L.off; returns the chunk's edge count
-__device__ __forceinline__ u32 flat_prefix(FlatLds &L, u32 cnt, u32 deg) {
+template<int NT>
+__device__ __forceinline__ u32 flat_prefix(FlatLds<NT> &L, u32 cnt, u32 deg) {
     u32 tot;
-    const u32 ex = block_exclusive_scan<JB>(threadIdx.x < cnt ? deg : 0u, L.red, tot);
+    const u32 ex = block_exclusive_scan<NT>(threadIdx.x < cnt ? deg : 0u, L.red, tot);
     if (threadIdx.x < cnt) L.off[threadIdx.x] = ex;
     if (threadIdx.x == 0) L.off[cnt] = tot;
     __syncthreads();
     return tot;
 }
 
-// afterburner (promap:284-322 / jet:269-328) over `len` candidates of
-// `region`, edge-balanced; selected vertices go to `mregion`
-__device__ void afterburner_flat(const JetDev &d, u32 stamp, const u32 *region, u32 len, u32 *mregion, u32 *s_cnt,
-                                 FlatLds &L, u64 &degs, u64 &gh) {
-    const bool do_hash = d.trace != nullptr;
-    for (u32 c0 = 0; c0 < len; c0 += FLAT_CHUNK) {
-        const u32 cnt = len - c0 < FLAT_CHUNK ? len - c0 : FLAT_CHUNK;
-        const u32 t = threadIdx.x;
-        u32 u = 0, deg = 0;
-        bool hub = true;
-        if (t < cnt) {
-            u = region[c0 + t];
-            const u32 b = d.xadj[u], e = d.xadj[u + 1];
-            hub = e - b > d.hub_deg;
-            deg = hub ? 0u : e - b;
-            L.u[t] = u;
-            L.start[t] = b;
-            L.g[t] = d.gain1[u];
-            L.a[t] = d.work[u];
-            L.b[t] = d.dest[u];
-            L.acc[t] = 0;
-        }
-        const u32 E = flat_prefix(L, cnt, deg);
-        for (u32 x0 = t; x0 < E; x0 += JB * ADJ_UNROLL) {
-            u32 iv[ADJ_UNROLL], v[ADJ_UNROLL], vn[ADJ_UNROLL], vo[ADJ_UNROLL];
-            s64 vg[ADJ_UNROLL], w[ADJ_UNROLL];
-#pragma unroll
-            for (u32 q = 0; q < ADJ_UNROLL; ++q) {
-                const u32 x = x0 + q * JB;
-                const bool ok = x < E;
-                iv[q] = ok ? flat_find(L.off, cnt, x) : 0u;
-                const u32 j = L.start[iv[q]] + (x - L.off[iv[q]]);
-                v[q] = ok ? d.adj[j] : 0u;
-                w[q] = ok ? ewt(d, j) : 0;
-            }
-#pragma unroll
-            for (u32 q = 0; q < ADJ_UNROLL; ++q) {
-                const bool ok = x0 + q * JB < E;
-                vg[q] = ok ? d.gain1[v[q]] : GAIN_MIN;
-                vn[q] = ok ? d.dest[v[q]] : 0u;
-                vo[q] = ok ? d.work[v[q]] : 0u;
-            }
-#pragma unroll
-            for (u32 q = 0; q < ADJ_UNROLL; ++q) {
-                if (x0 + q * JB >= E) continue;
-                const u32 i = iv[q], cu = L.u[i];
-                const s64 ug = L.g[i];
-                if (!(vg[q] > ug || (vg[q] == ug && v[q] < cu))) continue;
-                const u32 o = L.a[i], nn = L.b[i];
-                s64 c;
-                if (d.D)  // promap:297-314
-                    c = w[q] * (((s64) d.D[(u64) o * d.k + vn[q]] - (s64) d.D[(u64) nn * d.k + vn[q]]) -
-                                ((s64) d.D[(u64) o * d.k + vo[q]] - (s64) d.D[(u64) nn * d.k + vo[q]]));
-                else
-                    c = w[q] * ((s64) (vn[q] == nn) - (s64) (vn[q] == o) + (s64) (vo[q] == o) - (s64) (vo[q] == nn));
-                if (c) atomicAdd(&L.acc[i], (unsigned long long) c);
-            }
-        }
-        __syncthreads();
-        bool sel = false;
-        if (t < cnt && !hub) {
-            degs += deg;
-            const s64 ug = L.g[t];
-            if (do_hash) gh += mix64d(mix64d(u) + (u64) ug);
-            if (ug + (s64) L.acc[t] >= 0) {
-                d.lock[u] = 1;
-                d.mark[u] = stamp;
-                d.oldp[u] = L.a[t];
-                sel = true;
-            }
-        }
-        append_local(sel, u, mregion, s_cnt);
-        __syncthreads();  // the next chunk restages the LDS
+// afterburner (promap:284-322 / jet:269-328) over the `cnt` <= NT candidates
+// of list[c0, c0 + cnt), edge-balanced over a workgroup of NT threads;
+// selected vertices go to `mregion`
+template<int NT, typename JD, typename List>
+__device__ __forceinline__ void afterburner_flat(const JD &d, u32 stamp, List list, u32 c0, u32 cnt, u32 *mregion,
+                                                 u32 *s_cnt, FlatLds<NT> &L, bool do_hash, u64 &degs, u64 &gh) {
+    const u32 t = threadIdx.x;
+    u32 u = 0, deg = 0;
+    bool hub = true;
+    if (t < cnt) {
+        u = list[c0 + t];
+        const u32 b = d.xadj[u], e = d.xadj[u + 1];
+        hub = e - b > d.hub_deg;
+        deg = hub ? 0u : e - b;
+        L.u[t] = u;
+        L.start[t] = b;
+        L.g[t] = d.gain1[u];
+        L.a[t] = d.work[u];
+        L.b[t] = d.dest[u];
+        L.acc[t] = 0;
     }
+    const u32 E = flat_prefix<NT>(L, cnt, deg);
+    for (u32 x0 = t; x0 < E; x0 += NT * ADJ_UNROLL) {
+        u32 iv[ADJ_UNROLL], v[ADJ_UNROLL], vn[ADJ_UNROLL], vo[ADJ_UNROLL];
+        s64 vg[ADJ_UNROLL], w[ADJ_UNROLL];
+#pragma unroll
+        for (u32 q = 0; q < ADJ_UNROLL; ++q) {
+            const u32 x = x0 + q * NT;
+            const bool ok = x < E;
+            iv[q] = ok ? flat_find(L.off, cnt, x) : 0u;
+            const u32 j = L.start[iv[q]] + (x - L.off[iv[q]]);
+            v[q] = ok ? d.adj[j] : 0u;
+            w[q] = ok ? ewt(d, j) : 0;
+        }
+#pragma unroll
+        for (u32 q = 0; q < ADJ_UNROLL; ++q) {
+            const bool ok = x0 + q * NT < E;
+            vg[q] = ok ? (s64) d.gain1[v[q]] : GAIN_MIN;
+            vn[q] = ok ? (u32) d.dest[v[q]] : 0u;
+            vo[q] = ok ? (u32) d.work[v[q]] : 0u;
+        }
+#pragma unroll
+        for (u32 q = 0; q < ADJ_UNROLL; ++q) {
+            if (x0 + q * NT >= E) continue;
+            const u32 i = iv[q], cu = L.u[i];
+            const s64 ug = L.g[i];
+            if (!(vg[q] > ug || (vg[q] == ug && v[q] < cu))) continue;
+            const u32 o = L.a[i], nn = L.b[i];
+            s64 c;
+            if (JD::map && d.D)  // promap:297-314
+                c = w[q] * (((s64) d.D[(u64) o * d.k + vn[q]] - (s64) d.D[(u64) nn * d.k + vn[q]]) -
+                            ((s64) d.D[(u64) o * d.k + vo[q]] - (s64) d.D[(u64) nn * d.k + vo[q]]));
+            else
+                c = w[q] * ((s64) (vn[q] == nn) - (s64) (vn[q] == o) + (s64) (vo[q] == o) - (s64) (vo[q] == nn));
+            if (c) atomicAdd(&L.acc[i], (unsigned long long) c);
+        }
+    }
+    __syncthreads();
+    bool sel = false;
+    if (t < cnt && !hub) {
+        degs += deg;
+        const s64 ug = L.g[t];
+        if (do_hash) gh += mix64d(mix64d(u) + (u64) ug);
+        if (ug + (s64) L.acc[t] >= 0) {
+            d.lock[u] = 1;
+            d.mark[u] = stamp;
+            d.oldp[u] = L.a[t];
+            sel = true;
+        }
+    }
+    append_local(sel, u, mregion, s_cnt);
+    __syncthreads();  // the next chunk restages the LDS
 }
 
 template<int G, bool FLAT>
@@ -1244,8 +1322,11 @@ __global__ __launch_bounds__(JB) void post_kernel(JetDev d) {
     if (mode == 0) {
         u64 gh = 0, degs = 0;
         if constexpr (FLAT) {
-            __shared__ FlatLds L;
-            afterburner_flat(d, stamp, d.cand + (u64) blockIdx.x * d.cap, len, mregion, &s_cnt, L, degs, gh);
+            __shared__ FlatLds<JB> L;
+            for (u32 c0 = 0; c0 < len; c0 += FLAT_CHUNK)
+                afterburner_flat<JB>(d, stamp, d.cand + (u64) blockIdx.x * d.cap, c0,
+                                     len - c0 < FLAT_CHUNK ? len - c0 : FLAT_CHUNK, mregion, &s_cnt, L,
+                                     d.trace != nullptr, degs, gh);
         } else {
             afterburner_list<G>(d, stamp, d.cand + (u64) blockIdx.x * d.cap, len, mregion, &s_cnt, degs, gh);
         }
@@ -1365,7 +1446,8 @@ __device__ __forceinline__ lds_s64 *les_of(const s64 *p) { return (lds_s64 *) p;
 // each block's first candidate, so that position = score + evict_adjust[block].
 // With les, the chunk bounds also go to that LDS array; with lcnt, the
 // overflow counter's start goes there instead of to device memory.
-__device__ void cookie_cutter(const JetDev &d, s64 mbw, s64 *les = nullptr, s64 *lcnt = nullptr) {
+template<typename JD>
+__device__ void cookie_cutter(const JD &d, s64 mbw, s64 *les = nullptr, s64 *lcnt = nullptr) {
     const u32 lane = threadIdx.x;
     s64 carry = 0, carry2 = 0;
     for (u32 b0 = 0; b0 < d.k; b0 += WAVE) {
@@ -1446,8 +1528,8 @@ __device__ inline ResolveLds resolve_lds(char *base, u32 cap) {
 // counting smaller ids, the positions from a scan, and all are checked at
 // once; from the first entry that must take again on, one thread finishes
 // serially.  On exit soff holds each entry's chunk (k: it stays).
-template<int NT, typename P>
-__device__ __forceinline__ void overflow_block(const JetDev &d, P es, const ResolveLds &lds, u32 oc) {
+template<int NT, typename P, typename JD>
+__device__ __forceinline__ void overflow_block(const JD &d, P es, const ResolveLds &lds, u32 oc) {
     static_assert(NT >= (int) OVF_CAP, "one thread per overflow entry");
     u64 *skey = lds.skey;
     s64 *soff = lds.soff;
@@ -1520,9 +1602,10 @@ __device__ __forceinline__ void overflow_block(const JetDev &d, P es, const Reso
 // without a barrier, only stages across waves go through LDS.  For longer
 // lists the LDS form is faster: a shuffle costs about as much as an LDS
 // access, and the LDS form skips the idle threads' work.
-__device__ __forceinline__ void sort_keys_one_per_thread(const u64 *src, u32 L, u32 P2, u64 *skey) {
+template<typename Src>
+__device__ __forceinline__ void sort_keys_one_per_thread(Src src, u32 L, u32 P2, u64 *skey) {
     const u32 i = threadIdx.x;
-    u64 r = i < L ? src[i] : ~0ull;
+    u64 r = i < L ? (u64) src[i] : ~0ull;
     for (u32 kk = 2; kk <= P2; kk <<= 1) {
         for (u32 j = kk >> 1; j > 0; j >>= 1) {
             u64 b;
@@ -1546,8 +1629,8 @@ __device__ __forceinline__ void sort_keys_one_per_thread(const u64 *src, u32 L, 
 // Resolves a list of L entries with NT threads; false: the list (or the
 // strong overflow) does not fit and nothing was appended.  Moves go to the
 // extra move list, counted in LDS (`local_cnt`) or in st[ST_MOVES].
-template<u32 CAP, int NT = RB>
-__device__ __forceinline__ bool resolve_body(const JetDev &d, bool strong, u32 stamp, u32 L, const ResolveLds &lds, u32 *local_cnt) {
+template<u32 CAP, int NT = RB, typename JD>
+__device__ __forceinline__ bool resolve_body(const JD &d, bool strong, u32 stamp, u32 L, const ResolveLds &lds, u32 *local_cnt) {
     u64 *skey = lds.skey;
     s64 *soff = lds.soff;
     u8 *ssel = lds.ssel;
@@ -1565,7 +1648,7 @@ __device__ __forceinline__ bool resolve_body(const JetDev &d, bool strong, u32 s
     if (P2 <= NT) {
         sort_keys_one_per_thread(d.rlist, L, P2, skey);
     } else {
-    for (u32 i = threadIdx.x; i < P2; i += NT) skey[i] = i < L ? d.rlist[i] : ~0ull;
+    for (u32 i = threadIdx.x; i < P2; i += NT) skey[i] = i < L ? (u64) d.rlist[i] : ~0ull;
     __syncthreads();
     // bitonic sort, ascending
     for (u32 kk = 2; kk <= P2; kk <<= 1) {
@@ -1677,8 +1760,8 @@ __device__ __forceinline__ bool resolve_body(const JetDev &d, bool strong, u32 s
     for (u32 i0 = 0; i0 < L; i0 += NT) {
         const u32 i = i0 + threadIdx.x;
         const bool take = i < L && ssel[i] != 0;
-        if (local_cnt) append_local(take, take ? (u32) skey[i] : 0u, d.moves_x, local_cnt);
-        else append(take, take ? (u32) skey[i] : 0u, d.moves_x, &d.ctl->st[ST_MOVES]);
+        if (local_cnt) append_local(take, take ? (u32) skey[i] : 0u, raw(d.moves_x), local_cnt);
+        else append(take, take ? (u32) skey[i] : 0u, raw(d.moves_x), &d.ctl->st[ST_MOVES]);
     }
     return true;
 }
@@ -1744,10 +1827,9 @@ __global__ __launch_bounds__(RB) void resolve_kernel(JetDev d) {
 // neighbours' old block comes from oldp, so concurrent writes to work[] are safe.
 // the change of the objective over edges [b, e) of moved vertex u (lanes
 // `lane`, `lane + stride`, ...), invalidating the caches of the neighbours
-template<u32 ADJ_UNROLL>
-__device__ __forceinline__ s64 move_delta_range(const JetDev &d, u32 u, u64 b, u64 e, u32 lane, u32 stride,
-                                                u32 stamp) {
-    const u32 ou = d.oldp[u], nu = d.dest[u];
+template<u32 ADJ_UNROLL, typename JD>
+__device__ __forceinline__ s64 move_delta_pre(const JD &d, u32 ou, u32 nu, u64 b, u64 e, u32 lane, u32 stride,
+                                              u32 stamp) {
     const s32 *Dn = d.D ? d.D + (u64) nu * d.k : nullptr, *Do = d.D ? d.D + (u64) ou * d.k : nullptr;
     s64 delta = 0;
     for (u64 j0 = b + lane; j0 < e; j0 += (u64) stride * ADJ_UNROLL) {
@@ -1776,7 +1858,7 @@ __device__ __forceinline__ s64 move_delta_range(const JetDev &d, u32 u, u64 b, u
             const bool mv = mk[q] == stamp;
             const u32 ov = mv ? op[q] : wk[q];
             const u32 nv = mv ? ds[q] : ov;
-            if (Dn) {
+            if (JD::map && Dn) {
                 // comm cost change (promap:1174-1207): moves that keep their
                 // block contribute nothing; an edge to a vertex that did not
                 // change block counts twice (its other direction is not visited)
@@ -1795,14 +1877,20 @@ __device__ __forceinline__ s64 move_delta_range(const JetDev &d, u32 u, u64 b, u
     return delta;
 }
 
-template<u32 U>
-__device__ __forceinline__ s64 move_delta(const JetDev &d, u32 u, u32 lane, u32 stride, u32 stamp) {
+template<u32 ADJ_UNROLL, typename JD>
+__device__ __forceinline__ s64 move_delta_range(const JD &d, u32 u, u64 b, u64 e, u32 lane, u32 stride, u32 stamp) {
+    return move_delta_pre<ADJ_UNROLL>(d, d.oldp[u], d.dest[u], b, e, lane, stride, stamp);
+}
+
+template<u32 U, typename JD>
+__device__ __forceinline__ s64 move_delta(const JD &d, u32 u, u32 lane, u32 stride, u32 stamp) {
     return move_delta_range<U>(d, u, d.xadj[u], d.xadj[u + 1], lane, stride, stamp);
 }
 
 // commits a move; the block weight changes go to `bw` (the global array, or a
 // workgroup's LDS copy that is added to it once per block at the end)
-__device__ __forceinline__ void move_commit(const JetDev &d, u32 u, s64 *bw) {
+template<typename JD>
+__device__ __forceinline__ void move_commit(const JD &d, u32 u, s64 *bw) {
     const u32 ou = d.oldp[u], nu = d.dest[u];
     const s64 w = vwt(d, u);
     stale_of(d)[u] = 3;
@@ -1810,7 +1898,8 @@ __device__ __forceinline__ void move_commit(const JetDev &d, u32 u, s64 *bw) {
     atomicAdd((unsigned long long *) &bw[ou], (unsigned long long) (-w));
     atomicAdd((unsigned long long *) &bw[nu], (unsigned long long) w);
 }
-__device__ __forceinline__ void move_commit(const JetDev &d, u32 u) { move_commit(d, u, d.bw); }
+template<typename JD>
+__device__ __forceinline__ void move_commit(const JD &d, u32 u) { move_commit(d, u, d.bw); }
 
 // algorithmic bytes of one iteration's launches (w = 2 when edge weights are
 // stored, else 1; E(X) = summed degree of the vertex set X):
@@ -1824,7 +1913,8 @@ __device__ __forceinline__ void move_commit(const JetDev &d, u32 u) { move_commi
 //   resolve: 32 per resolve-list entry;
 //   apply: 16|M| + 4w E(M) + min(16 E(M), 16n);
 //   a pending best-partition copy adds 8n to the sweep.
-__device__ void account(const JetDev &d, JetCtl *ctl, const unsigned long long *rep, u32 mode, bool saved) {
+template<typename JD>
+__device__ void account(const JD &d, JetCtl *ctl, const unsigned long long *rep, u32 mode, bool saved) {
     const double w = d.ew ? 2.0 : 1.0, n = (double) d.n, wv = d.vw ? 4.0 : 0.0;
     const double nm = (double) rep[ST_MISS], em = (double) rep[ST_MISS_DEG];
     const double nc = (double) rep[ST_CAND], ec = (double) rep[ST_CAND_DEG];
@@ -1846,7 +1936,8 @@ __device__ void account(const JetDev &d, JetCtl *ctl, const unsigned long long *
     ctl->bytes[4] += 16.0 * nmv + 4.0 * w * emv + fmin(16.0 * emv, 16.0 * n);
 }
 
-__device__ void trace_record(const JetDev &d, JetCtl *ctl, const unsigned long long *rep, u32 mode, s64 cur,
+template<typename JD>
+__device__ void trace_record(const JD &d, JetCtl *ctl, const unsigned long long *rep, u32 mode, s64 cur,
                              s64 cur_maxw) {
     heipa_jet_trace &t = d.trace[ctl->n_trace % TRACE_RING];
     t.ratio_idx = ctl->ri;
@@ -1871,7 +1962,8 @@ __device__ void trace_record(const JetDev &d, JetCtl *ctl, const unsigned long l
 // changed) or after two LP iterations in a row without moves (the first
 // clears every lock, so the second and all later ones see the same state);
 // the remaining iterations of the reference change nothing.
-__device__ void map_control(const JetDev &d, JetCtl *ctl, const unsigned long long *rep, s64 maxw) {
+template<typename JD>
+__device__ void map_control(const JD &d, JetCtl *ctl, const unsigned long long *rep, s64 maxw) {
     const u32 mode = ctl->mode;
     const u32 n_moves = (u32) rep[ST_MOVES];
     u32 bal = ctl->bal, it = ctl->it;
@@ -1922,7 +2014,8 @@ __device__ void map_control(const JetDev &d, JetCtl *ctl, const unsigned long lo
 // One step of jet_refine's loop (jet:960-1030) after an iteration: counters,
 // cut and block weight, best-partition tracking, ratio and mode of the next
 // iteration.  Runs on one thread of the control launch.
-__device__ __forceinline__ void control_step(const JetDev &d, s64 maxw, const u64 *tot, const JetCtl &in) {
+template<typename JD>
+__device__ __forceinline__ void control_step(const JD &d, s64 maxw, const u64 *tot, const JetCtl &in) {
     JetCtl cl = in;  // the control block as loaded by the caller; written back at the end
     JetCtl *ctl = &cl;
     unsigned long long rep[ST_COUNT];
@@ -1943,8 +2036,8 @@ __device__ __forceinline__ void control_step(const JetDev &d, s64 maxw, const u6
     const u32 mode = ctl->mode;
     const u32 n_moves = (u32) rep[ST_MOVES];
     ctl->last_moves = n_moves;
-    account(d, ctl, rep, mode, ctl->save != 0);
-    if (d.D) {
+    if (d.count_bytes) account(d, ctl, rep, mode, ctl->save != 0);  // read by the profiler only
+    if (JD::map && d.D) {
         map_control(d, ctl, rep, maxw);
         *d.ctl = cl;
         return;
@@ -2050,8 +2143,8 @@ __global__ void hub_chunk_fill_kernel(const u32 *cnt, const u32 *off, u32 n_hubs
 
 // G lanes per move: this workgroup's move region, then its share of the
 // extra list
-template<int G>
-__device__ __forceinline__ void apply_one(const JetDev &d, u32 u, bool active, u32 lane, u32 stamp, bool do_hash,
+template<int G, typename JD>
+__device__ __forceinline__ void apply_one(const JD &d, u32 u, bool active, u32 lane, u32 stamp, bool do_hash,
                                           s64 &acc, u64 &degs, u64 &mh, s64 *bw) {
     const bool hub = active && degree(d, u) > d.hub_deg;
     if (active && !hub) {
@@ -2062,6 +2155,78 @@ __device__ __forceinline__ void apply_one(const JetDev &d, u32 u, bool active, u
             if (do_hash) mh += mix64d(((u64) u << 32) | d.dest[u]);
         }
     }
+}
+
+// apply of the `cnt` <= NT moves that `entry(i)` names, edge-balanced
+// (perform_moves, jet:753-924 / promap:1104-1216); block weight changes go to
+// `bwt`
+template<int NT, typename JD, typename Entry>
+__device__ __forceinline__ void apply_flat(const JD &d, u32 stamp, Entry entry, u32 cnt, FlatLds<NT> &L, bool do_hash,
+                                           s64 &acc, u64 &degs, u64 &mh, s64 *bwt) {
+    const u32 t = threadIdx.x;
+    u32 u = 0, deg = 0;
+    bool hub = true;
+    if (t < cnt) {
+        u = entry(t);
+        const u32 b = d.xadj[u], e = d.xadj[u + 1];
+        hub = e - b > d.hub_deg;
+        deg = hub ? 0u : e - b;
+        L.u[t] = u;
+        L.start[t] = b;
+        L.a[t] = d.oldp[u];
+        L.b[t] = d.dest[u];
+    }
+    const u32 E = flat_prefix<NT>(L, cnt, deg);
+    for (u32 y0 = t; y0 < E; y0 += NT * ADJ_UNROLL) {
+        u32 iv[ADJ_UNROLL], v[ADJ_UNROLL], mk[ADJ_UNROLL], op[ADJ_UNROLL], ds[ADJ_UNROLL], wk[ADJ_UNROLL];
+        u32 wi[ADJ_UNROLL];
+        u8 rf[ADJ_UNROLL];
+        s64 w[ADJ_UNROLL];
+#pragma unroll
+        for (u32 q = 0; q < ADJ_UNROLL; ++q) {
+            const u32 y = y0 + q * NT;
+            const bool ok = y < E;
+            iv[q] = ok ? flat_find(L.off, cnt, y) : 0u;
+            const u32 j = L.start[iv[q]] + (y - L.off[iv[q]]);
+            v[q] = ok ? d.adj[j] : 0u;
+            w[q] = ok ? ewt(d, j) : 0;
+        }
+#pragma unroll
+        for (u32 q = 0; q < ADJ_UNROLL; ++q) {
+            const bool ok = y0 + q * NT < E;
+            mk[q] = ok ? (u32) d.mark[v[q]] : 0u;
+            op[q] = ok ? (u32) d.oldp[v[q]] : 0u;
+            ds[q] = ok ? (u32) d.dest[v[q]] : 0u;
+            wk[q] = ok ? (u32) d.work[v[q]] : 0u;
+            rf[q] = ok && d.rflag ? (u8) d.rflag[v[q]] : (u8) 0;
+            wi[q] = ok && d.wcnt ? d.wid[v[q]] : 0u;
+        }
+#pragma unroll
+        for (u32 q = 0; q < ADJ_UNROLL; ++q) {
+            if (y0 + q * NT >= E) continue;
+            const u32 ou = L.a[iv[q]], nu = L.b[iv[q]];
+            const bool mv = mk[q] == stamp;
+            const u32 ov = mv ? op[q] : wk[q];
+            const u32 nv = mv ? ds[q] : ov;
+            if (JD::map && d.D) {  // promap:1174-1207
+                if (ou != nu) {
+                    const s64 x = w[q] * ((s64) d.D[(u64) nu * d.k + nv] - (s64) d.D[(u64) ou * d.k + ov]);
+                    acc += nv != ov ? x : 2 * x;
+                }
+            } else {
+                const s64 x = w[q] * ((s64) (nu != nv) - (s64) (ou != ov));
+                acc += mv ? x : 2 * x;
+            }
+            stale_of(d)[v[q]] = 3;
+            row_touch(d, v[q], rf[q], wi[q], ou, nu);
+        }
+    }
+    if (t < cnt && !hub) {
+        degs += deg;
+        move_commit(d, u, bwt);
+        if (do_hash) mh += mix64d(((u64) u << 32) | L.b[t]);
+    }
+    __syncthreads();  // the next chunk restages the LDS
 }
 
 // apply (perform_moves, jet:753-924 / promap:1104-1216): this workgroup's
@@ -2111,7 +2276,7 @@ __global__ __launch_bounds__(JB) void apply_groups_kernel(JetDev d) {
 
 __global__ __launch_bounds__(JB) void apply_kernel(JetDev d) {
     __shared__ u64 s_red[JB / WAVE];
-    __shared__ FlatLds L;
+    __shared__ FlatLds<JB> L;
     __shared__ s64 s_bw[BW_LDS];
     JetCtl *ctl = d.ctl;
     const u32 *region = d.moves + (u64) blockIdx.x * d.cap_mv;
@@ -2136,74 +2301,10 @@ __global__ __launch_bounds__(JB) void apply_kernel(JetDev d) {
     s64 *bwt = lds_bw ? s_bw : d.bw;
     s64 acc = 0;
     u64 mh = 0, degs = 0;
-    for (u32 c0 = 0; c0 < total; c0 += FLAT_CHUNK) {
-        const u32 cnt = total - c0 < FLAT_CHUNK ? total - c0 : FLAT_CHUNK;
-        const u32 t = threadIdx.x;
-        u32 u = 0, deg = 0;
-        bool hub = true;
-        if (t < cnt) {
-            const u32 i = c0 + t;
-            u = i < len ? region[i] : d.moves_x[x0 + (i - len)];
-            const u32 b = d.xadj[u], e = d.xadj[u + 1];
-            hub = e - b > d.hub_deg;
-            deg = hub ? 0u : e - b;
-            L.u[t] = u;
-            L.start[t] = b;
-            L.a[t] = d.oldp[u];
-            L.b[t] = d.dest[u];
-        }
-        const u32 E = flat_prefix(L, cnt, deg);
-        for (u32 y0 = t; y0 < E; y0 += JB * ADJ_UNROLL) {
-            u32 iv[ADJ_UNROLL], v[ADJ_UNROLL], mk[ADJ_UNROLL], op[ADJ_UNROLL], ds[ADJ_UNROLL], wk[ADJ_UNROLL];
-            u32 wi[ADJ_UNROLL];
-            u8 rf[ADJ_UNROLL];
-            s64 w[ADJ_UNROLL];
-#pragma unroll
-            for (u32 q = 0; q < ADJ_UNROLL; ++q) {
-                const u32 y = y0 + q * JB;
-                const bool ok = y < E;
-                iv[q] = ok ? flat_find(L.off, cnt, y) : 0u;
-                const u32 j = L.start[iv[q]] + (y - L.off[iv[q]]);
-                v[q] = ok ? d.adj[j] : 0u;
-                w[q] = ok ? ewt(d, j) : 0;
-            }
-#pragma unroll
-            for (u32 q = 0; q < ADJ_UNROLL; ++q) {
-                const bool ok = y0 + q * JB < E;
-                mk[q] = ok ? d.mark[v[q]] : 0u;
-                op[q] = ok ? d.oldp[v[q]] : 0u;
-                ds[q] = ok ? d.dest[v[q]] : 0u;
-                wk[q] = ok ? d.work[v[q]] : 0u;
-                rf[q] = ok && d.rflag ? d.rflag[v[q]] : (u8) 0;
-                wi[q] = ok && d.wcnt ? d.wid[v[q]] : 0u;
-            }
-#pragma unroll
-            for (u32 q = 0; q < ADJ_UNROLL; ++q) {
-                if (y0 + q * JB >= E) continue;
-                const u32 ou = L.a[iv[q]], nu = L.b[iv[q]];
-                const bool mv = mk[q] == stamp;
-                const u32 ov = mv ? op[q] : wk[q];
-                const u32 nv = mv ? ds[q] : ov;
-                if (d.D) {  // promap:1174-1207
-                    if (ou != nu) {
-                        const s64 x = w[q] * ((s64) d.D[(u64) nu * d.k + nv] - (s64) d.D[(u64) ou * d.k + ov]);
-                        acc += nv != ov ? x : 2 * x;
-                    }
-                } else {
-                    const s64 x = w[q] * ((s64) (nu != nv) - (s64) (ou != ov));
-                    acc += mv ? x : 2 * x;
-                }
-                stale_of(d)[v[q]] = 3;
-                row_touch(d, v[q], rf[q], wi[q], ou, nu);
-            }
-        }
-        if (t < cnt && !hub) {
-            degs += deg;
-            move_commit(d, u, bwt);
-            if (do_hash) mh += mix64d(((u64) u << 32) | L.b[t]);
-        }
-        __syncthreads();  // the next chunk restages the LDS
-    }
+    for (u32 c0 = 0; c0 < total; c0 += FLAT_CHUNK)
+        apply_flat<JB>(
+            d, stamp, [&](u32 t) { return c0 + t < len ? region[c0 + t] : d.moves_x[x0 + (c0 + t - len)]; },
+            total - c0 < FLAT_CHUNK ? total - c0 : FLAT_CHUNK, L, do_hash, acc, degs, mh, bwt);
     if (lds_bw)
         for (u32 b = threadIdx.x; b < d.k; b += JB)
             if (s_bw[b]) atomicAdd((unsigned long long *) &d.bw[b], (unsigned long long) s_bw[b]);
@@ -2289,8 +2390,8 @@ __device__ __forceinline__ void group_sync() {
 // counted vertex's counts.  A walk that needs no counts ends once every
 // block has been seen (P is then all k blocks): a hub of an HM split
 // (k <= 8) sees them all in its first rounds.
-template<int G>
-__device__ __forceinline__ void row_update(const JetDev &d, u32 *wm, u32 u, u32 lane, u32 rmode, bool active,
+template<int G, typename JD>
+__device__ __forceinline__ void row_update(const JD &d, u32 *wm, u32 u, u32 lane, u32 rmode, bool active,
                                            u32 *red, u32 *cl = nullptr) {
     const bool counted = active && (d.rflag[u] & 4u);
     // the same branch for every group of a launch: at init all walk, after
@@ -2370,6 +2471,51 @@ __device__ __forceinline__ void row_update(const JetDev &d, u32 *wm, u32 u, u32 
     group_sync<G>();
 }
 
+// one flagged wide vertex of k <= 64 that is not a hub, by one thread, the
+// block mask in a register
+template<typename JD>
+__device__ __forceinline__ void row_thread(const JD &d, u32 v, u32 rmode) {
+    const u8 f = d.rflag[v];
+    if ((f & 3u) != 3u) return;
+    u64 mask = 0;
+    if (f & 4u) {
+        if (rmode == ROW_INIT) return;  // the row kernel counts them
+        mask = row_count_mask(d, v);
+    } else {
+        const u32 xb = d.xadj[v], xe = d.xadj[v + 1];
+        if (xe - xb > ROW_THREAD_DEG) return;  // a hub
+        for (u32 j = xb; j < xe; j += 4) {
+            u32 nb[4];
+#pragma unroll
+            for (u32 q = 0; q < 4; ++q) nb[q] = j + q < xe ? d.adj[j + q] : 0u;
+#pragma unroll
+            for (u32 q = 0; q < 4; ++q)
+                if (j + q < xe) mask |= 1ull << (u32) d.work[nb[q]];
+        }
+    }
+    const u32 pc = (u32) __popcll(mask);
+    const u32 r = d.wid[v];
+    const u32 sz = d.wsz[r];
+    const bool keep = rmode == ROW_SMALL && sz == d.k;
+    for (u32 i = 0; i < d.W; ++i) {
+        const u64 o = (u64) r * d.W + i;
+        const u32 P = (u32) (mask >> (32 * i));
+        d.wV[o] = keep ? (d.wV[o] | P) : P;
+        d.wP[o] = P;
+    }
+    u32 ns;
+    if (rmode == ROW_INIT) {
+        ns = pc;
+    } else if (rmode == ROW_LARGE) {
+        ns = pc + (pc / 4 < 3 ? 3 : pc / 4);
+        if (ns >= d.k) ns = d.k;
+    } else {
+        ns = sz > pc ? sz : pc;
+    }
+    d.wsz[r] = ns;
+    d.rflag[v] = f & (u8) ~2u;
+}
+
 // Wide vertices of k <= 64 that are not hubs, one thread each, the block
 // mask in a register: those of degree <= ROW_THREAD_DEG walk their adjacency,
 // the counted ones read their counts (at init the row kernel counts them).
@@ -2383,47 +2529,7 @@ __global__ __launch_bounds__(JB) void row_thread_kernel(JetDev d, u32 init) {
         if (!live(hd)) return;
         rmode = d.ctl->last_moves > d.n / 10 ? ROW_LARGE : ROW_SMALL;
     }
-    for (u64 v = (u64) blockIdx.x * JB + threadIdx.x; v < d.n; v += (u64) gridDim.x * JB) {
-        const u8 f = d.rflag[v];
-        if ((f & 3u) != 3u) continue;
-        u64 mask = 0;
-        if (f & 4u) {
-            if (init) continue;  // the row kernel counts them
-            mask = row_count_mask(d, (u32) v);
-        } else {
-            const u32 xb = d.xadj[v], xe = d.xadj[v + 1];
-            if (xe - xb > ROW_THREAD_DEG) continue;  // a hub
-            for (u32 j = xb; j < xe; j += 4) {
-                u32 nb[4];
-#pragma unroll
-                for (u32 q = 0; q < 4; ++q) nb[q] = j + q < xe ? d.adj[j + q] : 0u;
-#pragma unroll
-                for (u32 q = 0; q < 4; ++q)
-                    if (j + q < xe) mask |= 1ull << d.work[nb[q]];
-            }
-        }
-        const u32 pc = (u32) __popcll(mask);
-        const u32 r = d.wid[v];
-        const u32 sz = d.wsz[r];
-        const bool keep = rmode == ROW_SMALL && sz == d.k;
-        for (u32 i = 0; i < d.W; ++i) {
-            const u64 o = (u64) r * d.W + i;
-            const u32 P = (u32) (mask >> (32 * i));
-            d.wV[o] = keep ? (d.wV[o] | P) : P;
-            d.wP[o] = P;
-        }
-        u32 ns;
-        if (rmode == ROW_INIT) {
-            ns = pc;
-        } else if (rmode == ROW_LARGE) {
-            ns = pc + (pc / 4 < 3 ? 3 : pc / 4);
-            if (ns >= d.k) ns = d.k;
-        } else {
-            ns = sz > pc ? sz : pc;
-        }
-        d.wsz[r] = ns;
-        d.rflag[v] = f & (u8) ~2u;
-    }
+    for (u64 v = (u64) blockIdx.x * JB + threadIdx.x; v < d.n; v += (u64) gridDim.x * JB) row_thread(d, (u32) v, rmode);
 }
 
 // the flagged wide vertices that are not hubs, G lanes each; init: every
@@ -2482,430 +2588,8 @@ __global__ __launch_bounds__(JB) void row_hub_kernel(JetDev d, const u32 *hubs, 
     row_update<JB>(d, rsm, u, threadIdx.x, rmode, true, red);
 }
 
-// ---------------------------------------------------------------- single-workgroup form
-// Small levels: one workgroup of BM threads runs whole iterations (sweep,
-// minibucket prefixes, afterburner or classify, resolve, apply, control)
-// with barriers where the multi-launch form has launch boundaries, up to
-// max_iters iterations per launch.  Same device functions, same results.
-// Lists: candidates in d.cand, moves in the extra move list, resolve entries
-// in d.rlist, all counted in LDS.  A resolve list that does not fit stalls
-// the loop: the iteration's lengths and statistics are published in st[] and
-// region counts are zero, so the host's global path and the multi-launch
-// apply and control finish that iteration.
-constexpr int BM = 512;  // 256 registers per lane (1024 threads cap them at 128 and spill)
-constexpr u32 BM_PIECE = 2048;
-constexpr u32 BM_RCAP = 2048;
-constexpr size_t BM_CONN_LDS = 40 * 1024;
-
-__host__ __device__ inline size_t bm_sweep_lds_bytes(u32 k, u32 groups) {
-    return conn_group_bytes(k) * groups + 4ull * BM_PIECE + 16 + 4ull * k;
-}
-
-// LDS copy of the per-vertex state of the single-workgroup form: s64
-// gcache, gain1, icache (n each) and the k block weights, then u32 work,
-// dest, dcache, mark, oldp, gid (n each), then the u8 locks and stale bytes
-__host__ __device__ constexpr size_t bm_state_bytes(u32 n, u32 k) { return 50ull * n + 8ull * k; }
-// the u32 row ids, then the u8 row flags
-__host__ __device__ constexpr size_t bm_rows_bytes(u32 n) { return 5ull * n; }
-
-// LS: the per-vertex state lives in LDS (from byte state_off of the dynamic
-// LDS) for the whole launch: copied in at the start and back to device
-// memory before the kernel returns (the host's global resolve path and the
-// next launch read it there).  The device functions reach it through the
-// same pointers in a local copy of the Jet state, as generic addresses.
-// The control block is kept in LDS the same way in both forms.  With
-// rows_off (LS only, 0: off) the BlockConn row ids and flags of the level's
-// vertices follow at that byte: the apply and row steps read them for every
-// neighbour of a move; the flags go back to device memory at the end.
-template<int G, bool LS>
-__global__ __launch_bounds__(BM) void jet_block_kernel(JetDev dg, u32 max_iters, u32 groups, u32 state_off,
-                                                       u32 rows_off) {
-    extern __shared__ __align__(16) char smem[];
-    constexpr u32 CW = (sizeof(JetCtl) + 7) / 8;
-    static_assert(CW <= BM && sizeof(JetCtl) % 8 == 0, "control block copy");
-    __shared__ u64 s_ctl[CW];
-    JetDev d = dg;
-    if (threadIdx.x < CW) s_ctl[threadIdx.x] = ((const u64 *) dg.ctl)[threadIdx.x];
-    d.ctl = (JetCtl *) s_ctl;
-    if constexpr (LS) {
-        const u32 n = dg.n, k = dg.k;
-        s64 *gc8 = (s64 *) (smem + state_off);
-        d.gcache = gc8;
-        d.gain1 = gc8 + n;
-        d.icache = gc8 + 2ull * n;
-        d.bw = gc8 + 3ull * n;
-        u32 *w4 = (u32 *) (gc8 + 3ull * n + k);
-        d.work = w4;
-        d.dest = w4 + n;
-        d.dcache = w4 + 2ull * n;
-        d.mark = w4 + 3ull * n;
-        d.oldp = w4 + 4ull * n;
-        d.gid = w4 + 5ull * n;
-        d.lock = (u8 *) (w4 + 6ull * n);
-        for (u32 v = threadIdx.x; v < n; v += BM) {
-            d.gcache[v] = dg.gcache[v];
-            d.gain1[v] = dg.gain1[v];
-            d.icache[v] = dg.icache[v];
-            d.work[v] = dg.work[v];
-            d.dest[v] = dg.dest[v];
-            d.dcache[v] = dg.dcache[v];
-            d.mark[v] = dg.mark[v];
-            d.oldp[v] = dg.oldp[v];
-            d.gid[v] = dg.gid[v];
-            d.lock[v] = dg.lock[v];
-            d.lock[n + v] = dg.lock[n + v];  // stale bytes
-        }
-        for (u32 b = threadIdx.x; b < k; b += BM) d.bw[b] = dg.bw[b];
-        if (rows_off) {
-            u32 *wid = (u32 *) (smem + rows_off);
-            u8 *rf = (u8 *) (wid + n);
-            for (u32 v = threadIdx.x; v < n; v += BM) {
-                wid[v] = dg.wid[v];
-                rf[v] = dg.rflag[v];
-            }
-            d.wid = wid;
-            d.rflag = rf;
-        }
-    }
-    __syncthreads();
-    __shared__ u32 s_live, s_mode, s_stamp, s_save;
-    __shared__ double s_ratio;
-    __shared__ u32 s_ncand, s_nlist, s_nmoves, s_nrl;
-    __shared__ u64 s_acc[PT_COUNT];
-    __shared__ u64 s_red[BM / WAVE];
-    JetCtl *ctl = d.ctl;
-    const u32 tid = threadIdx.x, lane = tid % G, gi = tid / G;
-    const bool ingroup = gi < groups;
-    const size_t cgb = conn_group_bytes(d.k);
-    GroupConn gc = group_conn(smem, d.k, ingroup ? gi : 0);
-    u32 *list = (u32 *) (smem + cgb * groups);
-    RebShared *rs = (RebShared *) (smem + cgb * groups + 4ull * BM_PIECE);
-    const ResolveLds rl = resolve_lds(smem, BM_RCAP);
-    for (u32 r = tid; r < d.nreg; r += BM) {
-        d.cand_n[r] = 0;
-        d.moves_n[r] = 0;
-    }
-    for (u64 j = tid; j < (u64) d.nreg * PT_COUNT; j += BM) d.pstat[j] = 0;
-    for (u32 iter = 0; iter < max_iters; ++iter) {
-        if (tid == 0) {
-            const CtlHead hd = ctl_head(ctl);
-            s_live = live(hd);
-            s_mode = hd.mode;
-            s_stamp = hd.stamp;
-            s_save = hd.save;
-            s_ratio = hd.ratio;
-            s_ncand = s_nmoves = s_nrl = 0;
-            for (u32 j = 0; j < PT_COUNT; ++j) s_acc[j] = 0;
-        }
-        __syncthreads();
-        if (!s_live) break;
-        const u32 mode = s_mode, stamp = s_stamp;
-        const bool save = s_save != 0, strong = mode == 2;
-        const double ratio = s_ratio;
-        const s64 mbw = mode ? max_block_weight(d, strong) : 0;
-        // ---- sweep
-        if (ingroup) {
-            for (u32 i = lane; i < d.k; i += G) gc.cnt[i] = 0;
-            if (lane == 0) *gc.tcount = 0;
-        }
-        if (mode) reb_prologue(d, strong, mbw, rs);
-        __syncthreads();
-        u64 nev = 0, degs = 0;
-        for (u64 p0 = 0; p0 < d.n; p0 += BM_PIECE) {
-            const u64 p1 = p0 + BM_PIECE < d.n ? p0 + BM_PIECE : d.n;
-            if (tid == 0) s_nlist = 0;
-            __syncthreads();
-            for (u64 v0 = p0; v0 < p1; v0 += BM) {
-                const u64 vv = v0 + tid;
-                const u32 v = (u32) vv;
-                bool heavy = false, cand = false;
-                if (vv < p1) {
-                    if (save) d.part[v] = d.work[v];
-                    if (mode == 0) {
-                        const u32 dc0 = d.dcache[v];
-                        const u32 dc = (stale_of(d)[v] & 1u) ? NULL_PART : dc0;
-                        if (dc == NULL_PART) {
-                            heavy = true;
-                        } else {
-                            d.dest[v] = dc;
-                            if (dc != NO_MOVE && d.lock[v] == 0) {
-                                cand = true;
-                                d.gain1[v] = d.gcache[v];
-                            } else {
-                                d.gain1[v] = GAIN_MIN;
-                                d.lock[v] = 0;
-                            }
-                        }
-                    } else if (reb_eligible(d, strong, rs, v, d.work[v])) {
-                        const s64 ic0 = d.icache[v];
-                        const s64 ic = (stale_of(d)[v] & 2u) ? -1 : ic0;
-                        if (ic >= 0) cand = reb_interior(d, strong, rs, v, ic);
-                        else heavy = true;
-                    }
-                }
-                append_local(cand, v, d.cand, &s_ncand);
-                append_local(heavy, v, list, &s_nlist);
-            }
-            __syncthreads();
-            const u32 nl = s_nlist;
-            // each round loads the adjacency offsets of the group's vertex of
-            // the next round, so that they arrive with this round's edges
-            u32 nxu = 0, nxb = 0, nxe = 0;
-            if (ingroup && gi < nl) {
-                nxu = list[gi];
-                nxb = d.xadj[nxu];
-                nxe = d.xadj[nxu + 1];
-            }
-            for (u32 r0 = 0; r0 < nl; r0 += groups) {
-                const u32 idx = r0 + gi;
-                const bool active = ingroup && idx < nl;
-                const u32 u = active ? nxu : 0, ub = nxb, ue = nxe;
-                if (ingroup && idx + groups < nl) {
-                    nxu = list[idx + groups];
-                    nxb = d.xadj[nxu];
-                    nxe = d.xadj[nxu + 1];
-                }
-                if (active) {
-                    if (lane == 0) {
-                        nev++;
-                        degs += ue - ub;
-                    }
-                    conn_accumulate_range<group_unroll<G>()>(d, gc, ub, ue, lane, G);
-                }
-                wave_sync();
-                const u32 own = active ? d.work[u] : 0;
-                const bool locked = active && d.lock[u] != 0;
-                const bool listed = mode == 0
-                                        ? lp_eval<G>(d, gc, u, own, locked, lane, ratio, nullptr, nullptr, active)
-                                        : reb_eval<G>(d, strong, mbw, rs, gc, u, own, lane, nullptr, nullptr, active);
-                wave_sync();
-                if (active) conn_reset(gc, *gc.tcount, lane, G);
-                wave_sync();
-                if (active && lane == 0) *gc.tcount = 0;
-                wave_sync();
-                append_local(listed, u, d.cand, &s_ncand);
-            }
-            __syncthreads();
-        }
-        nev = block_total(nev, s_red);
-        degs = block_total(degs, s_red);
-        if (tid == 0) {
-            s_acc[PT_MISS] = nev;
-            s_acc[PT_MISS_DEG] = degs;
-        }
-        // ---- minibucket prefixes, one wave per block range
-        if (mode && d.width <= WAVE) {
-            // one chunk per block: a wave loads PU blocks' totals before
-            // scanning any, so the loads overlap
-            constexpr u32 NW = BM / WAVE, PU = 8;
-            const u32 i = lane_id();
-            for (u32 p0 = tid / WAVE; p0 < d.k; p0 += PU * NW) {
-                s64 v[PU];
-#pragma unroll
-                for (u32 j = 0; j < PU; ++j) {
-                    const u32 p = p0 + j * NW;
-                    v[j] = p < d.k && i < d.width ? d.btot[(u64) p * d.width + i] : 0;
-                }
-#pragma unroll
-                for (u32 j = 0; j < PU; ++j) {
-                    const u32 p = p0 + j * NW;
-                    if (p >= d.k) break;  // uniform in the wave
-                    const s64 inc = wave_inclusive_scan(v[j]);
-                    const u64 base = (u64) p * d.width;
-                    if (i < d.width) {
-                        d.Q[base + i] = inc - v[j];
-                        d.R[base + i] = inc;
-                        d.btot[base + i] = 0;
-                    }
-                    if (i == WAVE - 1) d.Tseg[p] = inc;  // lanes past the width add 0
-                    if (i == 0 && p == d.k - 1) d.btot[(u64) d.k * d.width] = 0;
-                }
-            }
-        } else if (mode) {
-            for (u32 p = tid / WAVE; p < d.k; p += BM / WAVE) {
-                const u64 base = (u64) p * d.width;
-                s64 carry = 0;
-                for (u32 c0 = 0; c0 < d.width; c0 += WAVE) {
-                    const u32 i = c0 + lane_id();
-                    const s64 v = i < d.width ? d.btot[base + i] : 0;
-                    const s64 inc = wave_inclusive_scan(v);
-                    if (i < d.width) {
-                        d.Q[base + i] = carry + inc - v;
-                        d.R[base + i] = carry + inc;
-                        d.btot[base + i] = 0;
-                    }
-                    carry += __shfl(inc, WAVE - 1, WAVE);
-                }
-                if (lane_id() == 0) {
-                    d.Tseg[p] = carry;
-                    if (p == d.k - 1) d.btot[(u64) d.k * d.width] = 0;
-                }
-            }
-        }
-        __syncthreads();
-        // ---- afterburner / classify
-        const u32 nc = s_ncand;
-        if (mode == 0) {
-            u64 cdeg = 0, gh = 0;
-            afterburner_list<G>(d, stamp, d.cand, nc, d.moves_x, &s_nmoves, cdeg, gh);
-            cdeg = block_total(cdeg, s_red);
-            gh = block_total(gh, s_red);
-            if (tid == 0) {
-                s_acc[PT_CAND_DEG] = cdeg;
-                s_acc[PT_GHASH] = gh;
-            }
-        } else {
-            for (u32 i0 = 0; i0 < nc; i0 += BM) {
-                const u32 i = i0 + tid;
-                const bool valid = i < nc;
-                const u32 u = valid ? d.cand[i] : 0u;
-                bool sure = false, boundary = false;
-                u64 key = 0;
-                if (valid) {
-                    const u32 g = d.gid[u], ub = d.work[u];
-                    const s64 limit = d.bw[ub] - d.lmax;
-                    if (bucket_prefix(d, g, ub) < limit) {
-                        if (!strong && d.R[g] < limit) {
-                            sure = true;
-                            d.mark[u] = stamp;
-                            d.oldp[u] = ub;
-                        } else {
-                            boundary = true;
-                            key = ((u64) g << 32) | u;
-                        }
-                    }
-                }
-                append_local(sure, u, d.moves_x, &s_nmoves);
-                // rlist through a 32-bit LDS counter: entries are written by position
-                const u64 bal = __ballot(boundary);
-                if (bal) {
-                    const u32 first = (u32) __builtin_ctzll(bal);
-                    u32 base = 0;
-                    if (lane_id() == first) base = atomicAdd(&s_nrl, (u32) __popcll(bal));
-                    base = __shfl(base, (int) first, WAVE);
-                    if (boundary) d.rlist[base + (u32) __popcll(bal & lanemask_lt())] = key;
-                }
-            }
-        }
-        __syncthreads();
-        // ---- resolve
-        const u32 L = s_nrl;
-        if (mode) {
-            const bool ok = resolve_body<BM_RCAP, BM>(d, strong, stamp, L, rl, &s_nmoves);
-            if (!ok) {
-                if (tid == 0) {
-                    ctl->st[ST_MISS] = s_acc[PT_MISS];
-                    ctl->st[ST_MISS_DEG] = s_acc[PT_MISS_DEG];
-                    ctl->st[ST_CAND] = nc;
-                    ctl->st[ST_MOVES] = s_nmoves;
-                    ctl->st[ST_RLIST] = L;
-                    ctl->stalled = 1;
-                }
-                break;
-            }
-        }
-        __syncthreads();
-        // ---- apply
-        const u32 nm = s_nmoves;
-        s64 acc = 0;
-        u64 mdeg = 0, mh = 0;
-        for (u32 i0 = 0; i0 < nm; i0 += BM / G) {
-            const u32 i = i0 + gi;
-            apply_one<G>(d, i < nm ? d.moves_x[i] : 0u, i < nm, lane, stamp, d.trace != nullptr, acc, mdeg, mh, d.bw);
-        }
-        const u64 a = block_total((u64) acc, s_red);
-        mdeg = block_total(mdeg, s_red);
-        mh = block_total(mh, s_red);
-        __syncthreads();
-        // ---- control (the barrier above completes the block weight updates)
-        s64 mx = INT64_MIN;
-        for (u32 b = tid; b < d.k; b += BM) mx = d.bw[b] > mx ? d.bw[b] : mx;
-        mx = wave_max(mx);
-        if (lane_id() == 0) ((s64 *) s_red)[tid / WAVE] = mx;
-        __syncthreads();
-        if (tid == 0) {
-            s64 m = INT64_MIN;
-            for (u32 w = 0; w < BM / WAVE; ++w) m = ((s64 *) s_red)[w] > m ? ((s64 *) s_red)[w] : m;
-            u64 t[PT_COUNT + 2];
-            for (u32 j = 0; j < PT_COUNT; ++j) t[j] = s_acc[j];
-            t[PT_DELTA] = a;
-            t[PT_MOVE_DEG] = mdeg;
-            t[PT_MHASH] = mh;
-            t[PT_COUNT] = nc;
-            t[PT_COUNT + 1] = nm;
-            ctl->st[ST_RLIST] = L;
-            control_step(d, m, t, *d.ctl);
-        }
-        __syncthreads();
-        // ---- rows of the wide vertices next to the moves (the group's
-        // connectivity counters, all zero between sweeps, hold its mask words)
-        if (d.rflag && nm) {
-            const u32 rmode = nm > d.n / 10 ? ROW_LARGE : ROW_SMALL;
-            u32 *wm = (u32 *) gc.cnt;
-            for (u32 p0 = 0; p0 < d.n; p0 += BM_PIECE) {
-                const u32 p1 = p0 + BM_PIECE < d.n ? p0 + BM_PIECE : d.n;
-                if (tid == 0) s_nlist = 0;
-                __syncthreads();
-                for (u32 v0 = p0; v0 < p1; v0 += BM) {
-                    const u32 v = v0 + tid;
-                    append_local(v < p1 && (d.rflag[v] & 3u) == 3u, v, list, &s_nlist);
-                }
-                __syncthreads();
-                const u32 nl = s_nlist;
-                for (u32 r0 = 0; r0 < nl; r0 += groups) {
-                    const u32 idx = r0 + gi;
-                    const bool act = ingroup && idx < nl;
-                    row_update<G>(d, wm, act ? list[idx] : 0u, lane, rmode, act, nullptr);
-                }
-                __syncthreads();
-            }
-            if (ingroup)
-                for (u32 i = lane; i < d.W; i += G) wm[i] = 0;
-            __syncthreads();
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x < CW) ((u64 *) dg.ctl)[threadIdx.x] = s_ctl[threadIdx.x];
-    if constexpr (LS) {
-        for (u32 v = threadIdx.x; v < dg.n; v += BM) {
-            dg.gcache[v] = d.gcache[v];
-            dg.gain1[v] = d.gain1[v];
-            dg.icache[v] = d.icache[v];
-            dg.work[v] = d.work[v];
-            dg.dest[v] = d.dest[v];
-            dg.dcache[v] = d.dcache[v];
-            dg.mark[v] = d.mark[v];
-            dg.oldp[v] = d.oldp[v];
-            dg.gid[v] = d.gid[v];
-            dg.lock[v] = d.lock[v];
-            dg.lock[dg.n + v] = d.lock[dg.n + v];
-            if (rows_off) dg.rflag[v] = d.rflag[v];
-        }
-        for (u32 b = threadIdx.x; b < dg.k; b += BM) dg.bw[b] = d.bw[b];
-    }
-}
-
-// LDS the single-workgroup kernel declares itself (its __shared__
-// variables), which the hardware adds to the dynamic size of a launch
-template<int G, bool LS>
-size_t jet_block_static_lds() {
-    hipFuncAttributes fa{};
-    HIP_CHECK(hipFuncGetAttributes(&fa, (const void *) jet_block_kernel<G, LS>));
-    return fa.sharedSizeBytes;
-}
-inline size_t jet_block_static_lds_of(u32 G, bool ls);
-inline size_t jet_block_static_lds(u32 G, bool ls) {
-    return std::max<size_t>(1024, jet_block_static_lds_of(G, ls));  // at least 1 KiB of headroom
-}
-inline size_t jet_block_static_lds_of(u32 G, bool ls) {
-    switch (G) {
-        case 4: return ls ? jet_block_static_lds<4, true>() : jet_block_static_lds<4, false>();
-        case 8: return ls ? jet_block_static_lds<8, true>() : jet_block_static_lds<8, false>();
-        case 16: return ls ? jet_block_static_lds<16, true>() : jet_block_static_lds<16, false>();
-        case 32: return ls ? jet_block_static_lds<32, true>() : jet_block_static_lds<32, false>();
-        default: return ls ? jet_block_static_lds<64, true>() : jet_block_static_lds<64, false>();
-    }
-}
+// ---------------------------------------------------------------- team form
+#include "jet_team.hpp"
 
 struct RatioTable {
     double r[MAX_RATIOS];
@@ -2933,6 +2617,8 @@ __global__ void ctl_init_kernel(JetDev d, RatioTable rt, s64 cut, s64 maxw) {
     ctl->save = 0;
     ctl->iters = 0;
     ctl->n_trace = 0;
+    ctl->launches = 0;
+    ctl->failed = 0;
     ctl->stamp = 1;
     double *ratios = (double *) d.ratios;
 #pragma unroll
@@ -3068,14 +2754,8 @@ struct JetHost {
     const DGraph &g;
     const GraphMeta &meta;
     JetDev d{};
-    u32 G = 16, Gs = 16, Gb = 8, sweep_threads = JB;
+    u32 G = 16, Gs = 16, sweep_threads = JB;
     bool big_resolve = false;
-    bool block_mode = false;
-    u32 bm_groups = 1;
-    size_t bm_lds = 0;
-    bool bm_ls = false;  // single-workgroup form with the per-vertex state in LDS
-    u32 bm_state_off = 0;
-    u32 bm_rows_off = 0;  // and the row ids and flags after it (0: in device memory)
     size_t sweep_smem = 0, hub_smem = 0;
     s64 *H = nullptr, *roff = nullptr;
     u32 *over_flag = nullptr, *olist = nullptr, *olen = nullptr;
@@ -3132,15 +2812,29 @@ struct JetHost {
         launch(c, "jet_apply", 0.0, dim3(d.nreg), dim3(JB), 0, apply_groups_kernel<GG>, d);
     }
 
-    template<int GG>
-    void launch_block(u32 max_iters) {
-        if (bm_ls)
-            launch(c, "jet_block", 0.0, dim3(1), dim3(BM),
-                   bm_rows_off ? bm_rows_off + bm_rows_bytes(d.n) : bm_state_off + bm_state_bytes(d.n, d.k),
-                   jet_block_kernel<GG, true>, d, max_iters, bm_groups, bm_state_off, bm_rows_off);
-        else
-            launch(c, "jet_block", 0.0, dim3(1), dim3(BM), bm_lds, jet_block_kernel<GG, false>, d, max_iters, bm_groups,
-                   0u, 0u);
+    bool team_mode = false;
+    TeamArgs ta{};
+    u32 team_next = 0;
+    size_t team_lds = 0;
+
+    void launch_team() {
+        if (team_next == TEAM_SLOTS) {
+            fill<u64>(c, (u64 *) ta.tc, TEAM_SLOTS * sizeof(TeamCtl) / 8, 0);
+            team_next = 0;
+        }
+        TeamArgs a = ta;
+        a.tc += team_next++;
+        a.max_iters = TEAM_ITERS;
+        if (d.D) launch_team_as<true>(a);
+        else launch_team_as<false>(a);
+    }
+    template<bool MAP>
+    void launch_team_as(const TeamArgs &a) {
+        JetDevT<true, MAP> dt;
+        std::memcpy((void *) &dt, &d, sizeof(dt));
+        const dim3 grid(a.want * c.n_xcc);  // dispatched to the XCDs in turn: `want` on each
+        if (flat) launch(c, "jet_team", 0.0, grid, dim3(TM), team_lds, jet_team_kernel<true, MAP>, dt, a);
+        else launch(c, "jet_team", 0.0, grid, dim3(TM), team_lds, jet_team_kernel<false, MAP>, dt, a);
     }
 
     void iteration() {
@@ -3196,6 +2890,28 @@ struct JetHost {
 };
 
 } // namespace
+
+__global__ void xcc_id_kernel(u32 *out) {
+    if (threadIdx.x == 0) out[blockIdx.x] = xcc_id();
+}
+
+// The XCDs that workgroups of this device run on, and the one this context's
+// Jet teams use: contexts take them in turn, so that the teams of a pool's
+// workers spread over the chip.
+void find_xccs(Ctx &c) {
+    constexpr u32 N = 64;
+    if (c.arena.capacity() < 4 * N) return;
+    launch(c, "xcc_id", 0.0, dim3(N), dim3(64), 0, xcc_id_kernel, (u32 *) c.arena_mem);
+    u32 ids[N];
+    readback(c, ids, (const u32 *) c.arena_mem, N);
+    u32 mask = 0;
+    for (u32 x: ids) mask |= 1u << (x & 15u);
+    static std::atomic<u32> turn{0};
+    c.n_xcc = (u32) __builtin_popcount(mask);
+    u32 i = turn++ % c.n_xcc;
+    for (c.xcc = 0;; ++c.xcc)
+        if ((mask >> c.xcc & 1u) && i-- == 0) break;
+}
 
 JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, u32 k, s64 lmax, bool ultra,
                      u32 level, s64 cut, s64 maxw, std::vector<heipa_jet_trace> *trace, const s32 *D) {
@@ -3280,27 +2996,28 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         d.n_ratios = rt.n;
     }
     h.big_resolve = c.max_lds >= 160 * 1024;
-    // single-workgroup form for small levels without hubs
+    // Team form: levels whose iterations are chains of latency.  Measured per
+    // iteration (RGG, k = 64) against the multi-launch form: 15 against 33 us
+    // at 3000 vertices, 21 against 34 at 30000, 42 against 37 at 100000 (one
+    // XCD's 32 compute units and 4 MB of L2 no longer suffice).  Dense levels
+    // do more work per vertex: R-MAT with 116 K edges takes 87 against 114 us,
+    // with 460 K edges 270 against 160.
     {
         const size_t cgb = conn_group_bytes(k);
-        h.Gb = cap_group(meta.G, c.block_group_cap);
-        h.bm_groups = (u32) std::max<size_t>(1, std::min<size_t>(BM / h.Gb, BM_CONN_LDS / cgb));
-        h.bm_lds = std::max(bm_sweep_lds_bytes(k, h.bm_groups), resolve_lds_bytes(BM_RCAP));
-        // one workgroup walks every edge each iteration: dense small levels
-        // (coarse levels of skewed graphs) stay on the multi-launch form
-        h.block_mode = !c.race && n <= c.block_jet_max_n && (u64) g.m <= 32ull * c.block_jet_max_n &&
-                       meta.n_hubs == 0 && h.bm_lds <= std::min<size_t>(c.max_lds, 65536);
-        if (h.block_mode) {
-            // a launch's LDS is its dynamic size plus the kernel's own __shared__ variables
-            h.bm_state_off = (u32) ((h.bm_lds + 15) & ~(size_t) 15);
-            h.bm_ls = c.block_lds &&
-                      h.bm_state_off + bm_state_bytes(n, k) + jet_block_static_lds(h.Gb, true) <= c.max_lds;
-            require(h.bm_ls || h.bm_lds + jet_block_static_lds(h.Gb, false) <= c.max_lds,
-                    "single-workgroup Jet does not fit the LDS");
+        h.ta.wgroups = (u32) std::min<size_t>(WAVE / ROW, std::max<size_t>(1, TEAM_CONN_LDS / (cgb * TW)));
+        h.team_lds = team_lds_bytes(k, h.ta.wgroups);
+        h.team_mode = !c.race && c.n_xcc && c.block_jet_max_n && h.team_lds + 2048 <= c.max_lds &&
+                      ((n <= c.team_jet_max_n && (u64) g.m <= 16ull * n) ||
+                       (n <= std::max(c.team_jet_max_n, c.block_jet_max_n) && (u64) g.m <= 32ull * c.block_jet_max_n));
+        if (h.team_mode) {
+            h.ta.xcc = c.xcc;
+            h.ta.want = std::min<u32>(TEAM_WANT, div_up(n, 64));
+            h.ta.tc = bs.get<TeamCtl>(TEAM_SLOTS);
+            fill<u64>(c, (u64 *) h.ta.tc, TEAM_SLOTS * sizeof(TeamCtl) / 8, 0);
         }
     }
     // copies of the minibucket totals: about one per 64 sweep workgroups, at
-    // most 32 and 8 MiB; the single-workgroup form keeps one
+    // most 32 and 8 MiB; a team, whose additions meet in one L2, one per 8192 vertices up to 8
     {
         const u64 per_copy = 8ull * ((u64) d.t + 1);
         const u64 wgs = (u64) div_up(n, 256);
@@ -3308,9 +3025,11 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         if (c.race)  // one copy: the fetch-add results are offsets in the minibucket
             s = 1;
         else if (c.bucket_copies)
-            while (!h.block_mode && s * 2 <= c.bucket_copies) s *= 2;
+            while (s * 2 <= c.bucket_copies) s *= 2;
+        else if (h.team_mode)
+            while (s < 8 && (u64) s * 8192 < n) s *= 2;
         else
-            while (!h.block_mode && s < 32 && (u64) s * 2 * 64 <= wgs && (u64) s * 2 * per_copy <= (8ull << 20)) s *= 2;
+            while (s < 32 && (u64) s * 2 * 64 <= wgs && (u64) s * 2 * per_copy <= (8ull << 20)) s *= 2;
         d.nshard = s;
         d.btot = bs.get<s64>((u64) s * ((u64) d.t + 1));
     }
@@ -3391,12 +3110,6 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
             d.wcnt = bs.get<u32>((u64) (nw ? nw : 1) * k);
             fill<u32>(c, d.wcnt, (u64) (nw ? nw : 1) * k, 0u);
         }
-        // the single-workgroup form keeps the row ids and flags in LDS too if
-        // they fit beside its state
-        if (h.block_mode && h.bm_ls) {
-            const size_t off = (h.bm_state_off + bm_state_bytes(n, k) + 15) & ~(size_t) 15;
-            if (off + bm_rows_bytes(n) + jet_block_static_lds(h.Gb, true) <= c.max_lds) h.bm_rows_off = (u32) off;
-        }
     }
     copy_d2d(c, d.work, part, 4ull * n);
     fill<u32>(c, d.dcache, n, NULL_PART);
@@ -3421,7 +3134,14 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
             if (e) (void) hipGraphExecDestroy(e);
         }
     } gx;
-    if (!h.block_mode && c.use_graphs && !c.prof_on) {
+    if (h.team_mode) {
+        h.ta.hubs = meta.hubs;
+        h.ta.n_hubs = meta.n_hubs;
+        h.ta.n_chunks = h.n_chunks;
+        h.ta.chunk_hub = h.chunk_hub;
+        h.ta.chunk_idx = h.chunk_idx;
+    }
+    if (!h.team_mode && c.use_graphs && !c.prof_on) {
         hipGraph_t graph = nullptr;
         HIP_CHECK(hipStreamBeginCapture(c.stream, hipStreamCaptureModeRelaxed));
         try {
@@ -3440,10 +3160,9 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
     hipEvent_t ev[2] = {c.get_event(), c.get_event()};
     u32 B = 2, consumed = 0;
     u64 submits = 0;
-    const u32 bm_iters = tracing ? TRACE_RING / 2 : (1u << 20);
     auto submit = [&](int sidx) {
-        if (h.block_mode) {
-            HEIPA_DISPATCH_G(h.Gb, h.template launch_block, bm_iters);
+        if (h.team_mode) {
+            h.launch_team();
         } else if (gx.e) {
             HIP_CHECK(hipGraphLaunch(gx.e, c.stream));
         } else {
@@ -3454,6 +3173,7 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         HIP_CHECK(hipEventRecord(ev[sidx], c.stream));
     };
     JetCtl s{};
+    u32 team_seen = 0;
     int pend = 0;
     submit(0);
     for (;;) {
@@ -3465,7 +3185,10 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
             for (u32 i = consumed; i < s.n_trace; ++i) trace->push_back(ring[i % TRACE_RING]);
             consumed = s.n_trace;
         }
+        if (s.failed) throw Error(HEIPA_ERR_DEVICE, "jet_refine: a team workgroup never arrived at a barrier");
         if (!s.active) break;
+        if (h.team_mode && s.launches == team_seen) h.team_mode = false;  // no workgroup reached the XCD
+        team_seen = s.launches;
         if (s.stalled) {
             HIP_CHECK(hipEventSynchronize(ev[pend ^ 1]));
             h.fallback(s);
@@ -3479,8 +3202,8 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
     c.event_pool.push_back(ev[0]);
     c.event_pool.push_back(ev[1]);
     if (s.save) copy_d2d(c, part, d.work, 4ull * n);
-    if (h.block_mode) {
-        prof_bytes(c, "jet_block", s.bytes[0] + s.bytes[1] + s.bytes[2] + s.bytes[3] + s.bytes[4]);
+    if (h.ta.tc) {
+        prof_bytes(c, "jet_team", s.bytes[0] + s.bytes[1] + s.bytes[2] + s.bytes[3] + s.bytes[4]);
     } else {
         prof_bytes(c, "jet_sweep", s.bytes[0]);
         prof_bytes(c, "jet_buckets", s.bytes[1]);

@@ -15,32 +15,89 @@ constexpr int WAVE = 64;
 __device__ __forceinline__ u32 lane_id() { return threadIdx.x & (WAVE - 1); }
 __device__ __forceinline__ u64 lanemask_lt() { return (1ull << lane_id()) - 1ull; }
 
+// Cross-lane moves inside a row of 16 lanes (DPP): register reads, where a
+// shuffle is an LDS round trip.  All lanes of the wave must be active.
+// ror16<N>: lane i of a row gets lane (i - N) mod 16's value.
+template<int CTRL, int ROWS, bool ZERO>
+__device__ __forceinline__ u32 dpp(u32 x) {
+    return (u32) __builtin_amdgcn_update_dpp(ZERO ? 0 : (int) x, (int) x, CTRL, ROWS, 0xf, ZERO);
+}
+template<int CTRL, int ROWS, bool ZERO, typename T>
+__device__ __forceinline__ T dpp_move(T x) {
+    static_assert(sizeof(T) == 4 || sizeof(T) == 8, "one or two registers");
+    if constexpr (sizeof(T) == 4) {
+        return __builtin_bit_cast(T, dpp<CTRL, ROWS, ZERO>(__builtin_bit_cast(u32, x)));
+    } else {
+        const u64 v = __builtin_bit_cast(u64, x);
+        return __builtin_bit_cast(T, (u64) dpp<CTRL, ROWS, ZERO>((u32) v) |
+                                         (u64) dpp<CTRL, ROWS, ZERO>((u32) (v >> 32)) << 32);
+    }
+}
+template<int N, typename T>
+__device__ __forceinline__ T ror16(T x) { return dpp_move<0x120 + N, 0xf, false>(x); }
+// the value of lane l, in every lane
+template<typename T>
+__device__ __forceinline__ T lane_value(T x, int l) {
+    if constexpr (sizeof(T) == 4) {
+        return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l));
+    } else {
+        const u64 v = __builtin_bit_cast(u64, x);
+        const u32 lo = (u32) __builtin_amdgcn_readlane((int) (u32) v, l);
+        const u32 hi = (u32) __builtin_amdgcn_readlane((int) (u32) (v >> 32), l);
+        return __builtin_bit_cast(T, (u64) lo | (u64) hi << 32);
+    }
+}
+// reductions over a row; every lane of it gets the result
+template<typename T>
+__device__ __forceinline__ T row_sum(T x) {
+    x += ror16<8>(x);
+    x += ror16<4>(x);
+    x += ror16<2>(x);
+    x += ror16<1>(x);
+    return x;
+}
+template<typename T>
+__device__ __forceinline__ T row_max(T x) {
+    T y;
+    y = ror16<8>(x), x = y > x ? y : x;
+    y = ror16<4>(x), x = y > x ? y : x;
+    y = ror16<2>(x), x = y > x ? y : x;
+    y = ror16<1>(x), x = y > x ? y : x;
+    return x;
+}
+template<typename T>
+__device__ __forceinline__ T row_min(T x) {
+    T y;
+    y = ror16<8>(x), x = y < x ? y : x;
+    y = ror16<4>(x), x = y < x ? y : x;
+    y = ror16<2>(x), x = y < x ? y : x;
+    y = ror16<1>(x), x = y < x ? y : x;
+    return x;
+}
+
 template<typename T>
 __device__ __forceinline__ T wave_inclusive_scan(T x) {
-    const u32 lane = lane_id();
-#pragma unroll
-    for (int o = 1; o < WAVE; o <<= 1) {
-        T y = __shfl_up(x, o, WAVE);
-        if (lane >= (u32) o) x += y;
-    }
+    x += dpp_move<0x111, 0xf, true>(x);  // row_shr:1, zeros shifted in
+    x += dpp_move<0x112, 0xf, true>(x);
+    x += dpp_move<0x114, 0xf, true>(x);
+    x += dpp_move<0x118, 0xf, true>(x);
+    x += dpp_move<0x142, 0xa, true>(x);  // row_bcast:15 into rows 1 and 3
+    x += dpp_move<0x143, 0xc, true>(x);  // row_bcast:31 into rows 2 and 3
     return x;
 }
 
 template<typename T>
 __device__ __forceinline__ T wave_sum(T x) {
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) x += __shfl_xor(x, o, WAVE);
-    return x;
+    x = row_sum(x);
+    return lane_value(x, 0) + lane_value(x, 16) + lane_value(x, 32) + lane_value(x, 48);
 }
 
 template<typename T>
 __device__ __forceinline__ T wave_max(T x) {
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) {
-        T y = __shfl_xor(x, o, WAVE);
-        x = y > x ? y : x;
-    }
-    return x;
+    x = row_max(x);
+    const T a = lane_value(x, 0), b = lane_value(x, 16), c = lane_value(x, 32), d = lane_value(x, 48);
+    const T e = a > b ? a : b, f = c > d ? c : d;
+    return e > f ? e : f;
 }
 
 // Block-wide exclusive scan; `lds` needs BLOCK/64 entries.  Returns the

@@ -257,9 +257,9 @@ int heipa_pool_hier_cache_stats(const heipa_pool *pool, uint64_t *entries, uint6
  * allows; 0 forces the device-wide path).  Results do not depend on it; tests use it to cover
  * both paths. */
 #define HEIPA_OPT_RESOLVE_CAP 1
-/* HEIPA_OPT_BLOCK_JET: the largest level (vertices) whose Jet runs in one workgroup when it has no
- * hubs and at most 32 edges per vertex on average (default 2048; 0 forces the multi-launch form
- * everywhere).  Results do not depend on it. */
+/* HEIPA_OPT_BLOCK_JET: levels of up to 32 * value edges (and max(value, HEIPA_OPT_TEAM_JET) vertices) run
+ * whole Jet iterations in one launch, by a team of workgroups on one XCD, however dense they are
+ * (default 2048; 0 forces the multi-launch form everywhere).  Results do not depend on it. */
 #define HEIPA_OPT_BLOCK_JET 2
 /* HEIPA_OPT_GRAPHS: 1 (default) replays each level's batch of Jet iterations as a captured HIP graph;
  * 0 launches every kernel.  Results do not depend on it. */
@@ -272,9 +272,8 @@ int heipa_pool_hier_cache_stats(const heipa_pool *pool, uint64_t *entries, uint6
  * spreads its atomic additions over (0 = automatic, default: about one per 64 sweep workgroups, at
  * most 32; otherwise rounded down to a power of two, at most 32).  Results do not depend on it. */
 #define HEIPA_OPT_BUCKET_COPIES 5
-/* HEIPA_OPT_BLOCK_LDS: 1 (default) keeps the per-vertex Jet state of a single-workgroup level in LDS
- * for the whole launch when it fits (copied in at the start, back at the end); 0 keeps it in device
- * memory.  Results do not depend on it. */
+/* HEIPA_OPT_BLOCK_LDS: accepted, without effect (it placed the state of the former single-workgroup
+ * form of Jet; a team keeps a level's state in its XCD's L2). */
 #define HEIPA_OPT_BLOCK_LDS 6
 /* HEIPA_OPT_HM_WORKERS: worker contexts (each its own stream, arena and host thread, kept by the
  * context between calls) on which heipa_hm_partition solves the subtrees below its first split at
@@ -307,8 +306,8 @@ int heipa_pool_hier_cache_stats(const heipa_pool *pool, uint64_t *entries, uint6
 /* HEIPA_OPT_GROUP_CAP: the widest lane group (lanes per vertex) of the multi-launch Jet's afterburner,
  * apply and row launches (default 64, i.e. the power of two at or above the level's average degree,
  * at most 64; a smaller value rounds down to a power of two, at least 4).  Results do not depend on it.
- * HEIPA_OPT_BLOCK_GROUP_CAP: the same for the single-workgroup Jet (default 8: more vertices in flight
- * in the one workgroup).  heipa_pool_autotune picks both for a pool. */
+ * HEIPA_OPT_BLOCK_GROUP_CAP: accepted, without effect (it was the same cap of the former
+ * single-workgroup form; a team's rows are 16 lanes wide).  heipa_pool_autotune picks both for a pool. */
 #define HEIPA_OPT_GROUP_CAP 12
 #define HEIPA_OPT_BLOCK_GROUP_CAP 13
 /* HEIPA_OPT_REGION_EDGES: the multi-launch Jet gives each sweep workgroup a region of the level's
@@ -318,6 +317,10 @@ int heipa_pool_hier_cache_stats(const heipa_pool *pool, uint64_t *entries, uint6
  * vertex per thread).  The row updates of wide vertices and the matching's repick passes size their
  * pieces the same way (the repick only while that adds workgroups).  Results do not depend on it. */
 #define HEIPA_OPT_REGION_EDGES 14
+/* HEIPA_OPT_TEAM_JET: the largest level (vertices) of at most 16 edges per vertex whose Jet runs as a team
+ * of workgroups on one XCD, whole iterations per launch (default 65536; denser levels follow
+ * HEIPA_OPT_BLOCK_JET, and HEIPA_OPT_BLOCK_JET 0 turns teams off).  Results do not depend on it. */
+#define HEIPA_OPT_TEAM_JET 15
 int heipa_ctx_set_option(heipa_ctx *ctx, int option, uint64_t value);
 /* dst uses src's hierarchy cache (HEIPA_OPT_HIER_CACHE) from now on: one cache for several contexts */
 int heipa_ctx_share_hier_cache(heipa_ctx *dst, const heipa_ctx *src);

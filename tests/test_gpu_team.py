@@ -1,0 +1,124 @@
+"""GPU parity of the team form of Jet (one launch of several workgroups on one
+XCD runs whole iterations) at the sizes where its work split changes: levels
+smaller than a wave, than the team, exactly one vertex per lane and just
+beyond; degrees around the 32 that a rebuild keeps in registers; more than 64
+blocks for the rows of wide vertices; hubs; resolve lists of up to 64 entries
+(one wave) and longer.  Every traced iteration and the result must equal the
+oracle's, bit for bit (integers: no tolerance)."""
+import math
+
+import numpy as np
+import pytest
+
+import heipa
+import heipa_oracle as orc
+from graphs import block_weights, csr_from_arrays, random_partition
+from test_gpu_im import _D
+from test_gpu_parity import GRAPHS, _dev, _trace_tuple
+
+pytestmark = pytest.mark.gpu
+
+
+def _regular(n, deg, wmod=9):
+    """Every vertex has exactly `deg` neighbours (its nearest on a ring, and
+    the opposite one if deg is odd; n even then)."""
+    i = np.arange(n)
+    us, vs = [], []
+    for s in range(1, deg // 2 + 1):
+        us.append(i)
+        vs.append((i + s) % n)
+    if deg % 2:
+        us.append(i[:n // 2])
+        vs.append(i[:n // 2] + n // 2)
+    u, v = np.concatenate(us), np.concatenate(vs)
+    return csr_from_arrays(n, u, v, 1 + (u * 7 + v * 13) % wmod)
+
+
+CASES = {
+    # name: (graph, k, skew of the starting partition, ultra)
+    "one": (lambda: heipa.HostGraph(np.zeros(2, np.uint32), np.zeros(0, np.uint32)), 2, 0.0, False),
+    "n17": (lambda: heipa.gen_rgg(17, 4.0, 3, 9), 3, 1.0, False),
+    "n64": (lambda: heipa.gen_rgg(64, 6.0, 3, 9), 4, 2.0, True),
+    "n4095": (lambda: heipa.gen_rgg(4095, 8.0, 3, 9), 64, 0.9, True),  # 16 vertices per wave
+    "n16384": (lambda: heipa.gen_rgg(16384, 8.0, 3, 0), 23, 0.5, False),  # one vertex per lane of 256 waves
+    "n16385": (lambda: heipa.gen_rgg(16385, 8.0, 3, 0), 7, 0.8, False),
+    "n32769": (lambda: heipa.gen_rgg(32769, 8.0, 3, 100), 64, 0.3, False),  # a second sweep step
+    "n50001": (lambda: heipa.gen_rgg(50001, 10.0, 3, 100), 100, 0.0, True),
+    "deg31": (lambda: _regular(600, 31), 40, 0.7, True),
+    "deg32": (lambda: _regular(600, 32), 40, 0.7, True),
+    "deg33": (lambda: _regular(600, 33), 40, 0.7, True),
+    "wide_k70": (lambda: heipa.gen_rmat(11, 0, 16.0, 0.57, 0.19, 0.19, 5, 10, False), 70, 0.8, True),
+    "wide_k5": (lambda: _regular(900, 12), 5, 1.5, True),
+    "hubs": (lambda: GRAPHS["hubs100"], 16, 0.6, False),
+    "skewed": (lambda: heipa.gen_rmat(13, 0, 8.0, 0.57, 0.19, 0.19, 5, 10, False), 16, 1.0, False),
+}
+
+
+def _start(g, k, skew):
+    part = (np.arange(g.n, dtype=np.int64) * k // max(g.n, 1)).astype(np.uint32)
+    flip = np.random.default_rng(5).random(g.n) < 0.2
+    return np.where(flip, random_partition(g.n, k, 11, skew), part).astype(np.uint32)
+
+
+@pytest.fixture
+def team(ctx):
+    ctx.set_option(heipa.OPT_BLOCK_JET, 1 << 20)  # whole iterations per launch, however dense the level
+    try:
+        yield ctx
+    finally:
+        ctx.set_option(heipa.OPT_BLOCK_JET, 2048)
+
+
+def _compare(gtr, otr, name):
+    assert len(gtr) == len(otr), (name, len(gtr), len(otr))
+    for i, (a, b) in enumerate(zip(gtr, otr)):
+        assert _trace_tuple(a) == _trace_tuple(b), (name, i, _trace_tuple(a), _trace_tuple(b))
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_team_jet(team, name):
+    make, k, skew, ultra = CASES[name]
+    g = make()
+    part0 = _start(g, k, skew)
+    lmax = math.ceil(1.03 * g.g_weight / k)
+    cut0, maxw0 = orc.edge_cut(g, part0), int(block_weights(g, part0, k).max())
+    print(f"team jet {name} n={g.n} m={g.m} k={k}", flush=True)
+    op, ocut, omaxw, otr = orc.jet_refine(g, part0, k, lmax, ultra, 1, cut0, maxw0, trace_cap=4096)
+    pd = heipa.from_numpy_u32(part0)
+    gcut, gmaxw, gtr = team.jet_refine(_dev(g), pd, k, lmax, ultra, 1, cut0, maxw0, trace_cap=4096)
+    _compare(gtr, otr, name)
+    assert (gcut, gmaxw) == (ocut, omaxw)
+    assert np.array_equal(heipa.to_numpy_u32(pd), op)
+
+
+@pytest.mark.parametrize("hier", ["4:8:6", "2:3"])
+@pytest.mark.parametrize("name", ["n64", "n16385", "deg31", "deg33", "wide_k5", "hubs"])
+def test_team_map_refine(team, name, hier):
+    """The mapping objective; with 2:3 most vertices have at least k neighbours
+    and take the block-counter path."""
+    g = CASES[name][0]()
+    D, Dd = _D(*{"4:8:6": ([4, 8, 6], [1, 10, 100]), "2:3": ([2, 3], [7, 1])}[hier])
+    k = D.shape[0]
+    part0 = _start(g, k, 0.5)
+    lmax = math.ceil(1.05 * g.g_weight / k)
+    J0, maxw0 = orc.comm_cost(g, part0, D), int(block_weights(g, part0, k).max())
+    print(f"team map {name} n={g.n} m={g.m} k={k}", flush=True)
+    op, oJ, omaxw, otr = orc.map_refine(g, part0, D, lmax, J0, maxw0, trace_cap=4096)
+    pd = heipa.from_numpy_u32(part0)
+    gJ, gmaxw, gtr = team.map_refine(_dev(g), pd, Dd, k, lmax, 0, J0, maxw0, trace_cap=4096)
+    _compare(gtr, otr, name)
+    assert (gJ, gmaxw) == (oJ, omaxw)
+    assert np.array_equal(heipa.to_numpy_u32(pd), op)
+
+
+def test_team_on_every_xcd():
+    """Contexts use the device's XCDs in turn: nine of them, each its own team."""
+    g = heipa.gen_rgg(3000, 8.0, 3, 9)
+    want = orc.partition(g, 16, 0.03, 1, False)[0]
+    dg = _dev(g)
+    for _ in range(9):
+        c = heipa.Context(0, 64 << 20)
+        try:
+            assert np.array_equal(heipa.to_numpy_u32(c.partition(dg, 16, 0.03, 1, False)[0]), want)
+        finally:
+            c.close()
