@@ -140,10 +140,7 @@ int heipa_edge_cut(heipa_ctx *ctx, const heipa_graph *g, const uint32_t *part, i
         check_graph(g);
         require(cut && (part || g->n == 0), "null argument");
         DGraph d = to_dgraph(g);
-        validate_graph(c, d);
-        BackScope bs(c.arena);
-        GraphMeta meta = make_meta(c, d, true);
-        *cut = edge_cut(c, d, meta, part);
+        *cut = edge_cut_checked(c, d, part);
     });
 }
 
@@ -153,11 +150,7 @@ int heipa_comm_cost(heipa_ctx *ctx, const heipa_graph *g, const uint32_t *part, 
         check_graph(g);
         require(J && D && k > 0 && (part || g->n == 0), "null argument");
         DGraph d = to_dgraph(g);
-        validate_graph(c, d);
-        validate_part(c, part, d.n, k);
-        BackScope bs(c.arena);
-        GraphMeta meta = make_meta(c, d, true);
-        *J = comm_cost(c, d, meta, part, D, k);
+        *J = comm_cost_checked(c, d, part, D, k);
     });
 }
 
@@ -193,12 +186,7 @@ int heipa_block_weights(heipa_ctx *ctx, const heipa_graph *g, const uint32_t *pa
         check_graph(g);
         require(k > 0 && bw_host, "bad argument");
         DGraph d = to_dgraph(g);
-        validate_graph(c, d);
-        validate_part(c, part, d.n, k);
-        BackScope bs(c.arena);
-        s64 *bw = bs.get<s64>(k);
-        block_weights_dev(c, d, part, k, bw);
-        readback(c, (s64 *) bw_host, bw, k);
+        block_weights_checked(c, d, part, k, (s64 *) bw_host);
         if (maxw) {
             s64 m = 0;
             for (u32 i = 0; i < k; ++i) m = std::max<s64>(m, bw_host[i]);
@@ -213,9 +201,8 @@ int heipa_match(heipa_ctx *ctx, const heipa_graph *g, uint32_t seed, uint32_t *m
         check_graph(g);
         require(nc && (mapping || g->n == 0), "null argument");
         DGraph d = to_dgraph(g);
-        validate_graph(c, d);
         BackScope bs(c.arena);
-        GraphMeta meta = make_meta(c, d, true);
+        const GraphMeta meta = validate(c, d);
         *nc = match(c, d, meta, seed, mapping, stats);
     });
 }
@@ -227,8 +214,10 @@ int heipa_contract(heipa_ctx *ctx, const heipa_graph *fine, const uint32_t *mapp
         require(coarse && (mapping || fine->n == 0), "null argument");
         require(nc <= fine->n, "nc exceeds n");
         DGraph d = to_dgraph(fine);
-        validate_graph(c, d);
-        validate_part(c, mapping, d.n, nc);
+        {
+            BackScope bs(c.arena);
+            validate(c, d, mapping, nc);
+        }
         GraphMeta meta;  // unused by contraction
         CoarseGraph cg = contract(c, d, meta, mapping, nc);
         c.sync();
@@ -260,10 +249,8 @@ static int jet_common(heipa_ctx *ctx, const heipa_graph *g, uint32_t *part, int6
         check_graph(g);
         require(cut && maxw && k > 0 && (part || g->n == 0), "null argument");
         DGraph d = to_dgraph(g);
-        validate_graph(c, d);
-        validate_part(c, part, d.n, k);
         BackScope bs(c.arena);
-        GraphMeta meta = make_meta(c, d, true);
+        const GraphMeta meta = validate(c, d, part, k);
         std::vector<heipa_jet_trace> tr;
         JetResult r =
             jet_refine(c, d, meta, part, k, lmax, ultra != 0, level, *cut, *maxw, trace ? &tr : nullptr, D);
@@ -338,7 +325,8 @@ int heipa_im_partition(heipa_ctx *ctx, const heipa_graph *g, const uint32_t *hie
         // the mapping Jet runs on every level above the coarsest, which exists once n > 8k
         require(g->n <= 8 * k || k <= JET_MAX_K, "hierarchy product too large for the mapping refinement");
         DGraph d = to_dgraph(g);
-        validate_graph(c, d);
+        BackScope bs(c.arena);
+        const GraphMeta meta = validate(c, d);
         std::vector<s32> Dh(k * k);
         require(heipa_distance_matrix(hier, dist, l, Dh.data()) == HEIPA_OK, "bad hierarchy");
         const size_t depth0 = c.arena.front_depth();
@@ -346,7 +334,7 @@ int heipa_im_partition(heipa_ctx *ctx, const heipa_graph *g, const uint32_t *hie
         copy_h2d(c, Dd, Dh.data(), 4ull * k * k);
         ms.D = Dd;
         std::vector<heipa_level_trace> lv;
-        SolveResult r = solve(c, d, (u32) k, imbalance, seed, false, part, levels ? &lv : nullptr, &ms);
+        SolveResult r = solve(c, d, (u32) k, imbalance, seed, false, part, levels ? &lv : nullptr, &ms, &meta);
         c.sync();
         c.arena.release_front(depth0);
         fill_stats(stats, r);
@@ -363,9 +351,10 @@ int heipa_partition(heipa_ctx *ctx, const heipa_graph *g, uint32_t k, double imb
         require(k > 0 && (part || g->n == 0), "bad argument");
         require(imbalance >= 0.0, "imbalance must be non-negative");
         DGraph d = to_dgraph(g);
-        validate_graph(c, d);
+        BackScope bs(c.arena);
+        const GraphMeta meta = validate(c, d);
         std::vector<heipa_level_trace> lv;
-        SolveResult r = solve(c, d, k, imbalance, seed, ultra != 0, part, levels ? &lv : nullptr);
+        SolveResult r = solve(c, d, k, imbalance, seed, ultra != 0, part, levels ? &lv : nullptr, nullptr, &meta);
         if (stats) {
             stats->cut = r.cut;
             stats->maxw = r.maxw;
@@ -399,8 +388,9 @@ int heipa_hm_partition(heipa_ctx *ctx, const heipa_graph *g, const uint32_t *hie
             require(prod <= (1u << 16), "hierarchy product too large");
         }
         DGraph d = to_dgraph(g);
-        validate_graph(c, d);
-        hm_partition(c, d, h, imbalance, seed, ultra != 0, part);
+        BackScope bs(c.arena);
+        const GraphMeta meta = validate(c, d);
+        hm_partition(c, d, h, imbalance, seed, ultra != 0, part, &meta);
     });
 }
 

@@ -7,14 +7,19 @@
 
 namespace heipa {
 
-// ---- input validation (eval.hip); throw Error(HEIPA_ERR_INVALID)
-void validate_graph(Ctx &c, const DGraph &g);
-void validate_part(Ctx &c, const u32 *part, u32 n, u32 k);
+// ---- input validation (eval.hip): the checks of a graph and, if part is
+// given, of its block ids (< k); throws Error(HEIPA_ERR_INVALID).  Returns the
+// graph's launch metadata, the hub list on the arena's back stack.
+GraphMeta validate(Ctx &c, const DGraph &g, const u32 *part = nullptr, u32 k = 0);
 
-// ---- evaluators (eval.hip)
-s64 edge_cut(Ctx &c, const DGraph &g, const GraphMeta &meta, const u32 *part);
-s64 comm_cost(Ctx &c, const DGraph &g, const GraphMeta &meta, const u32 *part, const s32 *D, u32 k);
-void block_weights_dev(Ctx &c, const DGraph &g, const u32 *part, u32 k, s64 *bw_dev);
+// ---- evaluators (eval.hip); the checked forms validate their input first
+s64 edge_cut(Ctx &c, const DGraph &g, const u32 *part);
+s64 comm_cost(Ctx &c, const DGraph &g, const u32 *part, const s32 *D, u32 k);
+s64 edge_cut_checked(Ctx &c, const DGraph &g, const u32 *part);
+s64 comm_cost_checked(Ctx &c, const DGraph &g, const u32 *part, const s32 *D, u32 k);
+void block_weights_checked(Ctx &c, const DGraph &g, const u32 *part, u32 k, s64 *bw_host);
+// bad: a checked caller's flags on the device (null: the input is sound)
+void block_weights_dev(Ctx &c, const DGraph &g, const u32 *part, u32 k, s64 *bw_dev, const u32 *bad = nullptr);
 
 // ---- matching (match.hip): mapping is a device array of n entries; returns nc
 u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping, heipa_match_stats *stats);
@@ -54,10 +59,12 @@ struct MapSpec {
     std::vector<u32> hier;
     const s32 *D = nullptr;
 };
-// map != null: ProMapSolver::solve (IM); cut / initial_cut / level cuts hold J
+// map != null: ProMapSolver::solve (IM); cut / initial_cut / level cuts hold J.
+// meta: g's metadata where the caller has it (from validate)
 SolveResult solve(Ctx &c, const DGraph &g, u32 k, double imbalance, u64 seed, bool ultra, u32 *part,
-                  std::vector<heipa_level_trace> *levels, const MapSpec *map = nullptr);
+                  std::vector<heipa_level_trace> *levels, const MapSpec *map = nullptr,
+                  const GraphMeta *meta = nullptr);
 void hm_partition(Ctx &c, const DGraph &g, const std::vector<u32> &hier, double imbalance, u64 seed, bool ultra,
-                  u32 *part);
+                  u32 *part, const GraphMeta *meta = nullptr);
 
 } // namespace heipa

@@ -28,9 +28,6 @@ inline u32 group_for_avg(double avg) {
     return g;
 }
 
-__global__ void max_degree_kernel(const u32 *xadj, u32 n, u32 *out);
-__global__ void hub_count_kernel(const u32 *xadj, u32 n, u32 hub_deg, u32 *count, u32 *list);
-
 // Computes metadata; the hub list is pushed on the arena's BACK stack when
 // `back` is true (temporary) or the FRONT stack otherwise.
 GraphMeta make_meta(Ctx &c, const DGraph &g, bool back);

@@ -184,6 +184,7 @@ struct HMParams {
     u32 gk;
     u64 seed;
     bool ultra;
+    const GraphMeta *meta = nullptr;  // of the input graph
 };
 
 // Builds child `id` of g (the vertices with tmp == id, their internal edges
@@ -395,7 +396,7 @@ void hm_rec(Ctx &c, const DGraph &g, const u32 *n_to_o, u32 level, std::vector<u
     u32 *tmp = (u32 *) c.arena.push_front(4ull * (g.n ? g.n : 1));
     const double imb = adaptive_imbalance(p.eps, p.gW, p.gk, g.gw, p.k_rem[l - 1 - ident.size()], l - ident.size());
     if (k == 1) fill<u32>(c, tmp, g.n, 0u);
-    else solve(c, g, k, imb, p.seed, p.ultra, tmp, nullptr);
+    else solve(c, g, k, imb, p.seed, p.ultra, tmp, nullptr, nullptr, ident.empty() ? p.meta : nullptr);
     c.hkey = 0;  // the caller's graph key names the input graph only, not the children
     if (ident.size() == l - 1) {
         u32 offset = 0;
@@ -521,7 +522,7 @@ void hier_append(Ctx &c, HierEntry &e, size_t l, u32 fine_n, const u32 *map, con
 } // namespace
 
 SolveResult solve(Ctx &c, const DGraph &g0, u32 k, double imbalance, u64 seed, bool ultra, u32 *part,
-                  std::vector<heipa_level_trace> *levels, const MapSpec *map) {
+                  std::vector<heipa_level_trace> *levels, const MapSpec *map, const GraphMeta *meta) {
     SolveResult res;
     require(k >= 1, "k must be >= 1");
     c.prof_l0 = false;
@@ -532,7 +533,7 @@ SolveResult solve(Ctx &c, const DGraph &g0, u32 k, double imbalance, u64 seed, b
     u32 *pa = (u32 *) c.arena.push_front(4ull * (n0 ? n0 : 1));
     u32 *pb = (u32 *) c.arena.push_front(4ull * (n0 ? n0 : 1));
     std::vector<DGraph> graphs{g0};
-    std::vector<GraphMeta> metas{make_meta(c, g0, false)};
+    std::vector<GraphMeta> metas{meta ? *meta : make_meta(c, g0, false)};
     std::vector<u32 *> maps;
     const u32 max_n = 8 * k;
     double t0 = now_ms();
@@ -592,7 +593,7 @@ SolveResult solve(Ctx &c, const DGraph &g0, u32 k, double imbalance, u64 seed, b
         copy_h2d(c, pa, hp.data(), 4ull * cg.n);
         c.sync();
     }
-    s64 cut = map ? comm_cost(c, cg, metas.back(), pa, map->D, k) : edge_cut(c, cg, metas.back(), pa);
+    s64 cut = map ? comm_cost(c, cg, pa, map->D, k) : edge_cut(c, cg, pa);
     s64 maxw = max_block_weight(c, cg, pa, k);
     res.initial_cut = cut;
     res.ms[2] += now_ms() - ti;
@@ -639,7 +640,7 @@ SolveResult solve(Ctx &c, const DGraph &g0, u32 k, double imbalance, u64 seed, b
 }
 
 void hm_partition(Ctx &c, const DGraph &g, const std::vector<u32> &hier, double imbalance, u64 seed, bool ultra,
-                  u32 *part) {
+                  u32 *part, const GraphMeta *meta) {
     require(!hier.empty(), "empty hierarchy");
     HMParams p;
     p.hier = hier;
@@ -667,6 +668,7 @@ void hm_partition(Ctx &c, const DGraph &g, const std::vector<u32> &hier, double 
         u64 key;
         ~KeyRestore() { c.hkey = key; }
     } kr{c, c.hkey};
+    p.meta = meta;
     hm_rec(c, g, n_to_o, l - 1, ident, p, part);
     c.sync();
     c.arena.release_front(depth0);
