@@ -39,7 +39,7 @@
 // hand-off between workgroups is a launch boundary.  Levels of up to 65536
 // vertices run the same steps as a team of workgroups on one XCD instead,
 // whole iterations per launch (jet_team.hpp).
-#include "eval.hpp"
+#include "team.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -158,30 +158,6 @@ struct JetCtl {
     u32 failed;       // a team member never arrived at a barrier
 };
 static_assert(sizeof(CtlHead) == 32 && offsetof(JetCtl, st) == sizeof(CtlHead), "control block head layout");
-
-// A pointer to device memory that other workgroups of the same launch write:
-// every load is a device-scope one, which reads the L2 and not this compute
-// unit's L1 (88 ns against 52 ns from L1 on an idle chip; the same rate under
-// load).  Stores are plain: L1 writes through.
-template<typename T>
-struct DevRef {
-    T *p;
-    __device__ __forceinline__ operator T() const { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-    __device__ __forceinline__ void operator=(T v) const { *p = v; }
-    __device__ __forceinline__ void operator=(const DevRef &o) const { *p = (T) o; }
-    __device__ __forceinline__ void operator&=(T v) const { *p = (T) ((T) *this & v); }
-};
-template<typename T>
-struct DevPtr {
-    T *p;
-    __device__ __forceinline__ DevRef<T> operator[](u64 i) const { return {p + i}; }
-    __device__ __forceinline__ DevPtr operator+(u64 i) const { return {p + i}; }
-    __device__ __forceinline__ explicit operator bool() const { return p != nullptr; }
-};
-template<typename T>
-__device__ __forceinline__ T *raw(T *p) { return p; }
-template<typename T>
-__device__ __forceinline__ T *raw(const DevPtr<T> &p) { return p.p; }
 
 // TEAM: the view of the team form (one launch in which several workgroups run
 // whole iterations), same layout: the arrays that one workgroup writes and
@@ -329,13 +305,6 @@ __device__ __forceinline__ bool row_full(const JD &d, u32 u, u32 &r) {
     if (!d.rflag || !(d.rflag[u] & 1u)) return false;
     r = d.wid[u];
     return d.wsz[r] == d.k;
-}
-
-// orders the LDS traffic of one wave (lane groups never span waves)
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
 // wave-aggregated appends to device lists

@@ -13,36 +13,17 @@
 // iteration; levels that outgrow one XCD's L2 and 32 compute units stay on
 // the multi-launch form.
 //
-// Hand-offs between workgroups: stores write through L1 to the shared L2 and
-// are complete there after s_waitcnt vmcnt(0); readers use device-scope loads
-// (DevPtr), which do not read L1.  No L2 write-back or invalidate is needed
-// inside one XCD (each costs 50-60 ns and they serialise: with one
-// invalidate per workgroup the barrier of 32 took 2.1 us).
-//
-// No assumption on co-residency: the workgroups that have started on the XCD
-// register, the first one closes the registration after a bounded wait, and
-// the team is whoever has registered: every member is running, so every
-// barrier ends.  A launch runs max_iters iterations, so a team that formed
-// small on a busy chip does not last a whole level.
+// The team itself (formation, barrier, hand-offs) is team.hpp.
 #pragma once
 
-constexpr int TM = 512;                       // threads of a team workgroup
-constexpr u32 TW = TM / WAVE;                 // its waves
-constexpr u32 TEAM_MAX = 64;                  // members: one wave polls all flags
-constexpr u32 TEAM_WANT = 32;                 // workgroups wanted: the compute units of an XCD
 constexpr u32 TEAM_ITERS = 64;                // iterations per launch
 constexpr u32 TEAM_RCAP = 4096;               // resolve entries sorted in LDS
 constexpr u32 TEAM_U = 2;                     // sweep tiles a wave has in flight
 constexpr u32 TILE = WAVE * TEAM_U;           // vertices of one sweep step of a wave
-constexpr u32 WBUF = 256;                     // list entries a wave collects before it appends them
 constexpr u32 TEAM_BUF = 2048;                // list entries a workgroup collects (edge-balanced form)
-constexpr u32 ROW = 16;                       // lanes of a DPP row: one vertex each
 constexpr u32 ROW_DEG = 2 * ROW;              // largest degree of the register form of a rebuild
 constexpr size_t TEAM_CONN_LDS = 64 * 1024;   // block counters of the others, per workgroup
 constexpr u32 TEAM_BW = 1024;                 // blocks whose weight changes a workgroup sums in LDS
-constexpr u32 TEAM_FROZEN = 0x80000000u;
-constexpr u64 TEAM_FORM_TICKS = 1000;         // 10 us of the 100 MHz counter
-constexpr u64 TEAM_WAIT_TICKS = 1000000000;   // 10 s: a wait that long is a fault (reported, not hung)
 
 struct TeamAcc {  // totals of the iteration in flight
     unsigned long long delta, mhash, ghash, miss, miss_deg, cand_deg, move_deg;
@@ -51,9 +32,7 @@ struct TeamAcc {  // totals of the iteration in flight
 };
 static_assert(sizeof(TeamAcc) == 128, "one line each");
 struct TeamCtl {  // zero before the launch
-    u32 reg, pad0[31];   // registrations, then TEAM_FROZEN
-    u32 size, pad1[31];  // members, set once
-    u32 flag[TEAM_MAX];  // barrier round of each member
+    TeamHead head;
     TeamAcc acc[2];      // iteration i uses acc[i & 1] and clears the other
 };
 constexpr u32 TEAM_SLOTS = 16;  // launches between two clears
@@ -63,80 +42,6 @@ struct TeamArgs {
     const u32 *hubs, *chunk_hub, *chunk_idx;
     u32 n_hubs, n_chunks, xcc, want, max_iters;
     u32 wgroups;  // lane groups with block counters per wave
-};
-
-template<typename T>
-__device__ __forceinline__ T dev_load(const T *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// the XCD this wave runs on (hardware register 20, bits 0-3)
-__device__ __forceinline__ u32 xcc_id() { return __builtin_amdgcn_s_getreg((3 << 11) | 20) & 15u; }
-
-struct TeamBar {
-    u32 *flag;
-    u32 rank, size, round;
-    u32 *ok;  // LDS
-};
-
-// every member has stored everything before it and sees what the others
-// stored; false: a member never arrived (10 s).  The first wave runs `then`
-// between the last arrival and the workgroup's release.
-template<typename F>
-__device__ __forceinline__ bool team_barrier(TeamBar &b, F &&then) {
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // this wave's stores are in the L2
-    __syncthreads();
-    ++b.round;
-    if (threadIdx.x < WAVE) {
-        if (threadIdx.x == 0)
-            __hip_atomic_store(&b.flag[b.rank], b.round, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        const u32 *p = &b.flag[threadIdx.x < b.size ? threadIdx.x : b.rank];
-        bool ok = true;
-        u64 t0 = 0;
-        for (u32 spin = 1; !__all((s32) (dev_load(p) - b.round) >= 0); ++spin) {
-            if ((spin & 1023u) == 0) {
-                if (t0 == 0) t0 = wall_clock64();
-                if (wall_clock64() - t0 > TEAM_WAIT_TICKS) {
-                    ok = false;
-                    break;
-                }
-            }
-        }
-        if (threadIdx.x == 0) *b.ok = ok;
-        if (ok) then();
-    }
-    __syncthreads();
-    return *b.ok != 0;
-}
-__device__ __forceinline__ bool team_barrier(TeamBar &b) {
-    return team_barrier(b, [] {});
-}
-
-// a list that one wave collects in LDS; the count is a wave-uniform register
-template<typename T>
-struct WaveList {
-    T *buf;
-    u32 cnt;
-    __device__ __forceinline__ void add(bool pred, T val) {
-        const u64 bal = __ballot(pred);
-        if (pred) buf[cnt + (u32) __popcll(bal & lanemask_lt())] = val;
-        cnt += (u32) __popcll(bal);
-    }
-    // appends the entries to a shared list with one counter update
-    __device__ __forceinline__ void flush(T *list, u32 *counter) {
-        if (cnt == 0) return;
-        u32 base = 0;
-        if (lane_id() == 0) base = atomicAdd(counter, cnt);
-        base = (u32) __builtin_amdgcn_readfirstlane((int) base);
-        wave_sync();
-        for (u32 i = lane_id(); i < cnt; i += WAVE) list[base + i] = buf[i];
-        wave_sync();
-        cnt = 0;
-    }
-    // room for the entries of one more step (at most one per vertex of a TILE)
-    __device__ __forceinline__ void reserve(T *list, u32 *counter) {
-        if (cnt + TILE > WBUF) flush(list, counter);
-    }
 };
 
 // the same for a workgroup (edge-balanced form; uniform over the workgroup)
@@ -435,7 +340,7 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
     __shared__ u64 s_ctl[CW];
     __shared__ u64 s_red[TM / WAVE];
     __shared__ Best s_best[TM / WAVE];
-    __shared__ u32 s_rank, s_size, s_ok, s_nmv, s_base;
+    __shared__ u32 s_join[2], s_ok, s_nmv, s_base;
     if (xcc_id() != ta.xcc) return;
     u32 tid = threadIdx.x;
     TeamCtl *tc = ta.tc;
@@ -443,29 +348,9 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
     JetCtl *ctl = (JetCtl *) s_ctl;
     __syncthreads();
     if (!live(ctl)) return;
-    // ---- the team: the workgroups registered when the first one closes the list
-    if (tid == 0) {
-        u32 size = 0;
-        const u32 r = __hip_atomic_fetch_add(&tc->reg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (r == 0) {
-            const u64 t0 = wall_clock64();
-            while (dev_load(&tc->reg) < ta.want && wall_clock64() - t0 < TEAM_FORM_TICKS) __builtin_amdgcn_s_sleep(1);
-            size = __hip_atomic_fetch_or(&tc->reg, TEAM_FROZEN, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            size = size < TEAM_MAX ? size : TEAM_MAX;
-            __hip_atomic_store(&tc->size, size, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else if (r < TEAM_MAX) {  // not closed yet; the first member closes in bounded time
-            const u64 t0 = wall_clock64();
-            while ((size = dev_load(&tc->size)) == 0 && wall_clock64() - t0 < TEAM_WAIT_TICKS)
-                __builtin_amdgcn_s_sleep(1);
-        }
-        s_rank = r;
-        s_size = size;
-    }
-    __syncthreads();
-    const u32 rank = (u32) __builtin_amdgcn_readfirstlane((int) s_rank);
-    const u32 T = (u32) __builtin_amdgcn_readfirstlane((int) s_size);
-    if (rank >= T) return;
-    TeamBar bar{tc->flag, rank, T, 0, &s_ok};
+    u32 rank, T;
+    if (!team_join(&tc->head, ta.want, s_join, rank, T)) return;
+    TeamBar bar{tc->head.flag, rank, T, 0, &s_ok};
     JetDevT<true, MAP> d = dg;
     const bool do_hash = dg.trace != nullptr;
     if (rank) d.trace = nullptr;  // one member writes the trace
@@ -651,7 +536,7 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                         wc.add(listed, u);
                     }
                 }
-                wc.reserve(raw(d.cand), &acc->ncand);  // this step added at most TILE
+                wc.reserve(TILE, raw(d.cand), &acc->ncand);  // this step added at most TILE
                 wave_sync();
             }
             wc.flush(raw(d.cand), &acc->ncand);
@@ -788,7 +673,7 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                         }
                     }
                     wv.add(sel, u);
-                    wv.reserve(raw(d.moves_x), &acc->nmoves);
+                    wv.reserve(TILE, raw(d.moves_x), &acc->nmoves);
                 }
                 wv.flush(raw(d.moves_x), &acc->nmoves);
             }
@@ -821,8 +706,8 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                 const Take take = i < nc ? classify_take(d, strong, stamp, u, key) : TAKE_NO;
                 wv.add(take == TAKE_SURE, u);
                 wr.add(take == TAKE_BOUNDARY, key);
-                wv.reserve(raw(d.moves_x), &acc->nmoves);
-                wr.reserve(raw(d.rlist), &acc->nrl);
+                wv.reserve(TILE, raw(d.moves_x), &acc->nmoves);
+                wr.reserve(TILE, raw(d.rlist), &acc->nrl);
             }
             wv.flush(raw(d.moves_x), &acc->nmoves);
             wr.flush(raw(d.rlist), &acc->nrl);

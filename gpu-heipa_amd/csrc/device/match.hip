@@ -15,12 +15,14 @@
 // wins — the serial order of the reference's CAS loop) and `resolve`.  The
 // repick and the compaction are one launch; the active list lives in device
 // memory, its length too, and the host enqueues rounds without waiting,
-// checking the length every few rounds.  Picks run G lanes per vertex with a
+// checking the length every few rounds.  Once the list is short, one launch of
+// a team of workgroups on one XCD runs all remaining rounds and the mapping.
+// Picks run G lanes per vertex with a
 // lexicographic argmax reduction over shuffles; hubs get a workgroup.  The
 // leaf/twin/relative passes group vertices by exact key with a stable radix
 // sort (key, id) and pair consecutive entries, which is the reference's serial
 // pairing order.
-#include "eval.hpp"
+#include "team.hpp"
 
 namespace heipa {
 namespace {
@@ -318,6 +320,246 @@ __global__ __launch_bounds__(256) void count_unmapped_kernel(const u32 *vcmap, u
     if (threadIdx.x == 0 && c) atomicAdd(out, c);
 }
 
+// ---- all remaining rounds in one launch
+// A round is eight sub-round phases and a repick over a list that shrinks fast:
+// as launches they cost 1.6 us of gap and a cold L2 each, about 32 us a round
+// however short the list.  A team of workgroups on one XCD (team.hpp) runs
+// them with barriers of 0.6 us, about 12 us a round at 16384 vertices, and
+// then counts the unmatched vertices and builds the mapping (unless more than
+// a quarter stay unmatched: the pairing passes are the host's).
+struct MatchTeam {  // zero before the launch, but len0
+    TeamHead head;
+    u32 len[4], pad0[28];  // list lengths, a ring: round r reads len[r & 3]
+    u32 unmapped, pad1[31];
+    u32 nreps[TEAM_MAX];
+    // the result
+    u32 ran, rounds, failed, mapped, nc, un, pad2[26];
+};
+constexpr u32 MT_LIST = 1u << 16;   // longest list a team takes over
+constexpr u32 MT_EDGES = 1u << 20;  // most edges of a graph whose first round it takes
+constexpr u32 MT_MAP = 1u << 18;    // most vertices whose mapping it builds
+constexpr u32 MT_WAVE_DEG = 128;    // longer adjacencies are walked by a whole wave
+struct MatchTeamArgs {
+    MatchTeam *mt;
+    const u32 *list, *len_ptr;  // input of the first round (null: all vertices)
+    u32 *lists[2];
+    u32 *mapping;               // null: the host builds it
+    u32 seed, first_round, xcc, want;
+};
+
+// the best unmatched neighbour over edges b + lane, b + lane + stride, ...
+template<bool UEW>
+__device__ __forceinline__ Cand team_pick(const DGraph &g, const DevPtr<u32> &vcmap, u32 b, u32 e, u32 lane, u32 stride,
+                                          u32 r) {
+    Cand best{0, 0, SENT};
+    for (u32 j = b + lane; j < e; j += 2 * stride) {
+        const bool two = e - j > stride;
+        const u32 v0 = g.adj[j], v1 = two ? g.adj[j + stride] : 0u;
+        const s32 w0 = UEW ? 1 : g.ew[j], w1 = UEW ? 1 : two ? g.ew[j + stride] : 0;
+        const u32 m0 = vcmap[v0], m1 = two ? (u32) vcmap[v1] : 0u;
+        const Cand c0{w0, xorshift32(v0 + r), v0}, c1{w1, xorshift32(v1 + r), v1};
+        if (m0 == SENT && cand_better(c0, best)) best = c0;
+        if (two && m1 == SENT && cand_better(c1, best)) best = c1;
+    }
+    return best;
+}
+template<int N>
+__device__ __forceinline__ void cand_ror(Cand &c) {
+    const Cand d{ror16<N>(c.w), ror16<N>(c.t), ror16<N>(c.v)};
+    if (cand_better(d, c)) c = d;
+}
+__device__ __forceinline__ Cand cand_row(Cand c) {
+    cand_ror<8>(c);
+    cand_ror<4>(c);
+    cand_ror<2>(c);
+    cand_ror<1>(c);
+    return c;
+}
+
+template<bool UEW, bool RACE>
+__global__ __launch_bounds__(TM) void match_team_kernel(DGraph g, DevPtr<u32> vcmap, DevPtr<u32> hn, DevPtr<u32> claim,
+                                                        MatchTeamArgs ta) {
+    __shared__ u32 s_join[2], s_ok, s_sum;
+    __shared__ u32 s_keep[TW][WBUF], s_work[TW][WAVE];
+    __shared__ u32 s_red[TM / WAVE];
+    if (xcc_id() != ta.xcc) return;
+    MatchTeam *mt = ta.mt;
+    u32 rank, T;
+    if (!team_join(&mt->head, ta.want, s_join, rank, T)) return;
+    TeamBar bar{mt->head.flag, rank, T, 0, &s_ok};
+    const u32 tid = threadIdx.x, wl = tid % WAVE;
+    const u32 wid = (u32) __builtin_amdgcn_readfirstlane((int) (tid / WAVE));
+    const u32 gw = rank * TW + wid, NWV = T * TW;
+    const u32 rl = wl % ROW, rg = wl / ROW;
+    bool failed = false;
+    u32 len = ta.list ? *ta.len_ptr : g.n;
+    const u32 *in_list = ta.list;  // the launch's input: plain loads would do, but one path serves all rounds
+    u32 round = ta.first_round;
+#define MT_SYNC()               \
+    if (!team_barrier(bar)) {   \
+        failed = true;          \
+        break;                  \
+    }
+    for (;; ++round) {
+        const DevPtr<u32> list{(u32 *) in_list};
+        const bool all = in_list == nullptr;
+        // entries per wave and step: a whole wave's, fewer on lists that do not fill the team
+        const u32 tile = len >= NWV * WAVE ? WAVE : ((len + NWV - 1) / NWV + 15u) & ~15u;
+        for (u32 r = 0; r < 4; ++r) {
+            for (u64 i0 = (u64) gw * tile; i0 < len; i0 += (u64) NWV * tile) {
+                const u64 i = i0 + wl;
+                if (wl >= tile || i >= len) continue;
+                const u32 u = all ? (u32) i : (u32) list[i];
+                const u32 v = hn[u], mu = vcmap[u];
+                if (v == SENT || mu != SENT || !proposes(u, v, r)) continue;
+                const u32 mv = vcmap[v], hv = hn[v];
+                if (mv != SENT || hv == SENT || proposes(v, hv, r)) continue;
+                if (RACE) atomicCAS(claim.p + v, SENT, u);
+                else atomicMin(claim.p + v, u);
+            }
+            MT_SYNC();
+            for (u64 i0 = (u64) gw * tile; i0 < len; i0 += (u64) NWV * tile) {
+                const u64 i = i0 + wl;
+                if (wl >= tile || i >= len) continue;
+                const u32 u = all ? (u32) i : (u32) list[i];
+                const u32 c = claim[u];
+                if (c == SENT) continue;
+                const u32 cv = u < c ? u : c;
+                vcmap[u] = cv;
+                vcmap[c] = cv;
+                claim[u] = SENT;
+            }
+            MT_SYNC();
+        }
+        if (failed) break;
+        if (rank == 0 && tid == 0) mt->len[(round + 2) & 3] = 0;
+        // repick and compaction, each wave on its own
+        const u32 rs = ta.seed ^ (round * 0x9e3779b1u);
+        u32 *next = ta.lists[round & 1], *next_len = &mt->len[(round + 1) & 3];
+        WaveList<u32> wk{s_keep[wid], 0};
+        for (u64 i0 = (u64) gw * tile; i0 < len; i0 += (u64) NWV * tile) {
+            const u64 i = i0 + wl;
+            u32 u = 0, h = SENT, b = 0, e = 0;
+            bool unmatched = false, need = false;
+            if (wl < tile && i < len) {
+                u = all ? (u32) i : (u32) list[i];
+                unmatched = vcmap[u] == SENT;
+                h = hn[u];
+                if (unmatched && h != SENT && vcmap[h] != SENT) {
+                    need = true;
+                    b = g.xadj[u];
+                    e = g.xadj[u + 1];
+                }
+            }
+            const bool wide = need && e - b > MT_WAVE_DEG;
+            const u64 bs = __ballot(need && !wide);
+            u64 bl = __ballot(wide);
+            const u32 pos = (u32) __popcll(bs & lanemask_lt());
+            if (need && !wide) s_work[wid][pos] = wl;  // the lane that holds the vertex
+            wave_sync();
+            const u32 ns = (u32) __popcll(bs);
+            for (u32 r0 = 0; r0 < ns; r0 += WAVE / ROW) {
+                const bool act = r0 + rg < ns;
+                const int l = act ? (int) s_work[wid][r0 + rg] : 0;
+                const u32 w = (u32) __shfl((int) u, l, WAVE), wb = (u32) __shfl((int) b, l, WAVE);
+                const u32 we = (u32) __shfl((int) e, l, WAVE);
+                Cand c{0, 0, SENT};
+                if (act) c = team_pick<UEW>(g, vcmap, wb, we, rl, ROW, xorshift32(w ^ rs));
+                c = cand_row(c);
+                wave_sync();
+                if (act && rl == 0) s_work[wid][r0 + rg] = c.v;
+            }
+            wave_sync();
+            if (need && !wide) h = s_work[wid][pos];
+            while (bl) {
+                const int l = __builtin_ctzll(bl);
+                bl &= bl - 1;
+                const u32 w = lane_value(u, l), wb = lane_value(b, l), we = lane_value(e, l);
+                const Cand c = cand_reduce<WAVE>(team_pick<UEW>(g, vcmap, wb, we, wl, WAVE, xorshift32(w ^ rs)));
+                if ((int) wl == l) h = c.v;
+            }
+            if (need) hn[u] = h;
+            wave_sync();
+            wk.add(unmatched && h != SENT, u);
+            wk.reserve(WAVE, next, next_len);
+        }
+        wk.flush(next, next_len);
+        MT_SYNC();
+        len = dev_load(next_len);
+        in_list = next;
+        if (len == 0 || round >= 20000) break;
+    }
+    u32 un = 0, mapped = 0, nc = 0;
+    if (!failed && len == 0 && ta.mapping) {
+        // ---- build_mapping: representatives in id order, a contiguous share each
+        const u32 n = g.n, share = (n + T - 1) / T;
+        const u32 v0 = rank * share < n ? rank * share : n, v1 = n - v0 < share ? n : v0 + share;
+        u32 reps = 0, unm = 0;
+        for (u32 v = v0 + tid; v < v1; v += TM) {
+            const u32 x = vcmap[v];
+            unm += x == SENT;
+            reps += x == SENT || x == v;
+        }
+        reps = block_sum<TM>(reps, s_red);
+        unm = block_sum<TM>(unm, s_red);
+        if (tid == 0) {
+            mt->nreps[rank] = reps;
+            if (unm) atomicAdd(&mt->unmapped, unm);
+        }
+        failed = !team_barrier(bar, [&] {
+            const u32 x = wl < T ? dev_load(&mt->nreps[wl]) : 0u;
+            const u32 before = wave_sum(wl < rank ? x : 0u);
+            if (wl == 0) s_sum = before;
+            nc = wave_sum(x);
+        });
+        un = dev_load(&mt->unmapped);
+        if (!failed && !((double) un / (double) n > 0.25)) {
+            const DevPtr<u32> map{ta.mapping};
+            u32 base = s_sum;
+            for (u32 t0 = v0; t0 < v1; t0 += TM) {
+                const u32 v = t0 + tid;
+                const u32 x = v < v1 ? (u32) vcmap[v] : 0u;
+                const bool is_rep = v < v1 && (x == SENT || x == v);
+                u32 tot;
+                const u32 ex = block_exclusive_scan<TM>(is_rep ? 1u : 0u, s_red, tot);
+                if (is_rep) {
+                    vcmap[v] = v;
+                    map[v] = base + ex;
+                }
+                base += tot;
+            }
+            failed = !team_barrier(bar);
+            if (!failed)
+                for (u32 v = v0 + tid; v < v1; v += TM) {
+                    const u32 x = vcmap[v];
+                    if (x != v) map[v] = map[x];
+                }
+            mapped = 1;
+        }
+    }
+#undef MT_SYNC
+    if (failed && tid == 0) mt->failed = 1;
+    if (rank == 0 && tid == 0) {
+        mt->rounds = round + 1;
+        mt->un = un;
+        mt->nc = nc;
+        mt->mapped = mapped;
+        mt->ran = 1;
+    }
+}
+
+// vcmap, hn and claim to "none", the list lengths and the team's block to zero
+__global__ void match_init_kernel(u32 n, u32 *vcmap, u32 *hn, u32 *claim, u32 *lens, u32 *mt, u32 mt_words) {
+    const u64 stride = (u64) gridDim.x * blockDim.x, t = (u64) blockIdx.x * blockDim.x + threadIdx.x;
+    for (u64 i = t; i < n; i += stride) {
+        vcmap[i] = SENT;
+        hn[i] = SENT;
+        claim[i] = SENT;
+    }
+    for (u64 i = t; i < 64; i += stride) lens[i] = 0;
+    for (u64 i = t; i < mt_words; i += stride) mt[i] = 0;
+}
+
 // ---- keyed pairing (leaf / twin / relative)
 struct LeafPred {
     const u32 *vcmap, *xadj;
@@ -565,11 +807,10 @@ u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping
     u32 *claim = bs.get<u32>(n);
     u32 *lists[2] = {bs.get<u32>(n), bs.get<u32>(n)};
     u32 *lens = bs.get<u32>(64);  // ring of list lengths, one per round
-    fill<u32>(c, vcmap, n, SENT);
-    fill<u32>(c, hn, n, SENT);
-    fill<u32>(c, claim, n, SENT);
-    fill<u32>(c, lens, 64, 0u);
+    MatchTeam *mt = bs.get<MatchTeam>(1);
     const dim3 blk(256);
+    launch(c, "match_init", 12.0 * n, dim3(grid_for(c, n, 256 * 4)), blk, 0, match_init_kernel, n, vcmap, hn, claim, lens,
+           (u32 *) mt, (u32) (sizeof(MatchTeam) / 4));
 
     // initial pick
     // profiling: summed degree of the repicked vertices, for the byte model
@@ -600,7 +841,29 @@ u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping
     u32 batch = 2;
     u32 *pinned = c.pinned_as<u32>();
     u32 exact_rounds = 0;
+    MatchTeam res{};
+    bool team = c.n_xcc != 0 && c.block_jet_max_n != 0;  // HEIPA_OPT_BLOCK_JET 0: one launch per step
     while (true) {
+        // the first rounds of a large graph need the whole chip; the team takes
+        // over with the first list that fits one XCD
+        if (team && len_bound <= MT_LIST && (round > 0 || g.m <= MT_EDGES)) {
+            team = false;  // once per call
+            MatchTeamArgs a{mt, cur_list, cur_len, {lists[0], lists[1]}, n <= MT_MAP ? mapping : nullptr, seed, round, c.xcc,
+                            std::min<u32>(TEAM_WANT, div_up(len_bound, 64))};
+            const dim3 grid(a.want * c.n_xcc);
+            const DevPtr<u32> pv{vcmap}, ph{hn}, pc{claim};
+            launch(c, "match_team", 0.0, grid, dim3(TM), 0,
+                   c.race ? (g.ew ? match_team_kernel<false, true> : match_team_kernel<true, true>)
+                          : (g.ew ? match_team_kernel<false, false> : match_team_kernel<true, false>),
+                   g, pv, ph, pc, a);
+            readback(c, &res, (const MatchTeam *) mt, 1);
+            if (res.failed) throw Error(HEIPA_ERR_DEVICE, "matching: a team workgroup never arrived at a barrier");
+            if (res.ran) {
+                require(res.rounds < 20000, "matching did not converge (is the graph symmetric?)");
+                exact_rounds = res.rounds;
+                break;
+            }
+        }
         const u32 first_round = round;
         for (u32 bi = 0; bi < batch; ++bi, ++round) {
             const u32 round_seed = seed ^ (round * 0x9e3779b1u);
@@ -658,8 +921,13 @@ u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping
         prof_bytes(c, "match_repick", 4.0 * wb * (double) dsum + 4.0 * std::min<double>((double) dsum, n));
     }
 
+    if (res.mapped) {
+        st.after_hem = st.after_leaf = st.after_twin = st.after_relative = res.un;
+        if (stats) *stats = st;
+        return res.nc;
+    }
     u32 *scr = bs.get<u32>(4);
-    u32 unmapped = count_unmapped(c, vcmap, n, scr);
+    u32 unmapped = res.ran && n <= MT_MAP ? res.un : count_unmapped(c, vcmap, n, scr);
     st.after_hem = st.after_leaf = st.after_twin = st.after_relative = unmapped;
     u32 *plist = lists[0];
     u32 *plen = scr + 1;

@@ -122,3 +122,30 @@ def test_team_on_every_xcd():
             assert np.array_equal(heipa.to_numpy_u32(c.partition(dg, 16, 0.03, 1, False)[0]), want)
         finally:
             c.close()
+
+
+MATCH = {
+    "n1": lambda: heipa.HostGraph(np.zeros(2, np.uint32), np.zeros(0, np.uint32)),
+    "n2": lambda: _regular(2, 1),
+    "tile": lambda: _regular(16384, 4),  # one list entry per lane of 256 waves
+    "tile_and_one": lambda: _regular(16385, 4),
+    "list_limit": lambda: heipa.gen_rgg(65536, 6.0, 3, 0),  # the longest list a team takes over
+    "beyond_list": lambda: heipa.gen_rgg(65537, 6.0, 3, 10),  # launches first, then a team
+    "beyond_map": lambda: heipa.gen_rgg((1 << 18) + 1, 5.0, 3, 10),  # the mapping is the host's
+    "wide": lambda: _regular(700, 130),  # adjacencies walked by a whole wave
+    "dense": lambda: heipa.gen_rmat(15, 0, 24.0, 0.57, 0.19, 0.19, 5, 10, False),  # over 2^20 edges
+    "hubs": lambda: GRAPHS["hubs100"],
+}
+
+
+@pytest.mark.parametrize("name", sorted(MATCH))
+def test_team_match(ctx, name):
+    """Matching where the rounds move from launches to a team, and within it."""
+    g = MATCH[name]()
+    print(f"team match {name} n={g.n} m={g.m}", flush=True)
+    omp, onc, ost = orc.match(g, 12345)
+    gmp, gnc, gst = ctx.match(_dev(g))
+    assert gnc == onc
+    assert np.array_equal(heipa.to_numpy_u32(gmp), omp)
+    for f in ("rounds", "after_hem", "ran_leaf", "ran_twin", "ran_relative", "after_relative"):
+        assert getattr(gst, f) == getattr(ost, f), f
