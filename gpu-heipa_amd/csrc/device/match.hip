@@ -679,6 +679,161 @@ __global__ void pair_kernel(const u32 *head, const u32 *gid_excl, const u32 *gst
     }
 }
 
+// ---- pairing of equal keys in one launch
+// Stable radix sort of (key, id) and the pairing of the sorted list.  Sorting
+// 64-bit digests takes 8 passes of three launches and the pairing four more,
+// about 16 us a pass however short the list; a team (team.hpp) takes about 4 us
+// a pass: member r counts and moves a contiguous share of the list, and every
+// member sums the counts of all for its own offsets.
+constexpr u32 PT_LIST = 1u << 16;  // longest list (a member's share is then 2048 entries)
+struct PairTeam {  // zero before the launch
+    TeamHead head;
+    u32 ran, failed, pad[30];
+    u32 last[TEAM_MAX];          // 1 + the last group head of each member's share (0: none)
+    u32 counts[2][256 * TEAM_MAX];  // entries of each digit per member (digit-major), passes in turn
+};
+template<typename K>
+struct PairTeamArgs {
+    PairTeam *pt;
+    DevPtr<K> keys[2];  // the list, and the buffer of the same size
+    DevPtr<u32> vals[2];
+    u32 len, bits, xcc, want;
+    u32 *vcmap;
+};
+
+template<typename K>
+__global__ __launch_bounds__(TM) void pair_team_kernel(PairTeamArgs<K> ta) {
+    __shared__ u32 s_join[2], s_ok, s_carry;
+    __shared__ u32 s_run[256], s_wcnt[TW][256], s_goff[256];
+    __shared__ u32 s_red[TM / WAVE];
+    if (xcc_id() != ta.xcc) return;
+    PairTeam *pt = ta.pt;
+    u32 rank, T;
+    if (!team_join(&pt->head, ta.want, s_join, rank, T)) return;
+    TeamBar bar{pt->head.flag, rank, T, 0, &s_ok};
+    const u32 tid = threadIdx.x, wl = tid % WAVE, wid = tid / WAVE;
+    const u32 share = (ta.len + T - 1) / T;
+    const u32 i0 = rank * share < ta.len ? rank * share : ta.len, i1 = ta.len - i0 < share ? ta.len : i0 + share;
+    bool failed = false, flip = false;
+    for (u32 shift = 0; shift < ta.bits && !failed; shift += 8) {
+        const DevPtr<K> ik = ta.keys[flip], ok = ta.keys[!flip];
+        const DevPtr<u32> iv = ta.vals[flip], ov = ta.vals[!flip];
+        if (tid < 256) s_run[tid] = 0;
+        __syncthreads();
+        for (u32 i = i0 + tid; i < i1; i += TM) atomicAdd(&s_run[(u32) ((K) ik[i] >> shift) & 255u], 1u);
+        __syncthreads();
+        u32 *counts = pt->counts[(shift >> 3) & 1];
+        if (tid < 256) counts[tid * TEAM_MAX + rank] = s_run[tid];
+        failed = !team_barrier(bar);
+        if (failed) break;
+        // this member's first position of each digit
+        u32 tot = 0, before = 0;
+        if (tid < 256)
+            for (u32 m = 0; m < T; ++m) {
+                const u32 x = dev_load(&counts[tid * TEAM_MAX + m]);
+                before += m < rank ? x : 0u;
+                tot += x;
+            }
+        u32 all;
+        const u32 ex = block_exclusive_scan<TM>(tot, s_red, all);
+        const bool one_digit = __syncthreads_or(tot == ta.len);  // nothing to move in this pass
+        if (tid < 256) {
+            s_goff[tid] = ex + before;
+            s_run[tid] = 0;
+        }
+        for (u32 d = tid; d < TW * 256; d += TM) ((u32 *) s_wcnt)[d] = 0;
+        __syncthreads();
+        if (one_digit) continue;  // the same in every member
+        for (u32 r0 = i0; r0 < i1; r0 += TM) {
+            const u32 i = r0 + tid;
+            const bool valid = i < i1;
+            const K key = valid ? (K) ik[i] : K(0);
+            const u32 val = valid ? (u32) iv[i] : 0u;
+            const u32 d = (u32) (key >> shift) & 255u;
+            u64 mask = __ballot(valid);  // the wave's lanes with the same digit
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const bool bit = (d >> b) & 1u;
+                const u64 bal = __ballot(bit);
+                mask &= bit ? bal : ~bal;
+            }
+            const u32 lower = (u32) __popcll(mask & lanemask_lt());
+            if (valid && lower == 0) s_wcnt[wid][d] = (u32) __popcll(mask);
+            __syncthreads();
+            if (valid) {
+                u32 pos = s_goff[d] + s_run[d] + lower;
+                for (u32 w = 0; w < wid; ++w) pos += s_wcnt[w][d];
+                ok[pos] = key;
+                ov[pos] = val;
+            }
+            __syncthreads();
+            if (tid < 256) {
+                u32 t = 0;
+#pragma unroll
+                for (u32 w = 0; w < TW; ++w) {
+                    t += s_wcnt[w][tid];
+                    s_wcnt[w][tid] = 0;
+                }
+                s_run[tid] += t;
+            }
+            __syncthreads();
+        }
+        failed = !team_barrier(bar);
+        flip = !flip;
+    }
+    // pair entries 2j and 2j + 1 of every group of equal keys
+    const DevPtr<K> sk = ta.keys[flip];
+    const DevPtr<u32> sv = ta.vals[flip];
+    if (!failed) {
+        u32 last = 0;
+        for (u32 i = i0 + tid; i < i1; i += TM)
+            if (i == 0 || (K) sk[i] != (K) sk[i - 1]) last = i + 1;
+        last = wave_max(last);
+        if (wl == 0) s_red[wid] = last;
+        __syncthreads();
+        if (tid == 0) {
+            for (u32 w = 1; w < TW; ++w) last = s_red[w] > last ? s_red[w] : last;
+            pt->last[rank] = last;
+        }
+        failed = !team_barrier(bar, [&] {
+            const u32 x = wl < rank ? dev_load(&pt->last[wl]) : 0u;
+            const u32 mx = wave_max(x);
+            if (wl == 0) s_carry = mx;
+        });
+    }
+    if (!failed) {
+        u32 carry = s_carry;  // 1 + the head of the group that runs into this share
+        for (u32 r0 = i0; r0 < i1; r0 += TM) {
+            const u32 i = r0 + tid;
+            const bool in = i < i1;
+            const K key = in ? (K) sk[i] : K(0);
+            const bool head = in && (i == 0 || (K) sk[i - 1] != key);
+            // the last head at or before i: within the wave, then of the waves before
+            const u64 hb = __ballot(head);
+            const u64 mine = hb & (lanemask_lt() | 1ull << wl);
+            u32 h = mine ? r0 + wid * WAVE + (63u - (u32) __builtin_clzll(mine)) + 1 : 0u;
+            __syncthreads();
+            if (wl == 0) s_red[wid] = hb ? r0 + wid * WAVE + (63u - (u32) __builtin_clzll(hb)) + 1 : 0u;
+            __syncthreads();
+            u32 best = carry;
+            for (u32 w = 0; w < TW; ++w) {
+                const u32 x = s_red[w];
+                if (w < wid && x > best) best = x;
+            }
+            if (!h) h = best;
+            for (u32 w = 0; w < TW; ++w) carry = s_red[w] > carry ? s_red[w] : carry;
+            if (in && i + 1 < ta.len && ((i + 1 - h) & 1u) == 0 && (K) sk[i + 1] == key) {
+                const u32 a = sv[i], b = sv[i + 1];
+                const u32 cv = a < b ? a : b;
+                ta.vcmap[a] = cv;
+                ta.vcmap[b] = cv;
+            }
+        }
+    }
+    if (failed && tid == 0) pt->failed = 1;
+    if (rank == 0 && tid == 0) pt->ran = 1;
+}
+
 // ---- build_mapping (two_hop_matching.h:613-641)
 struct RepSrc {
     u32 *vcmap;
@@ -777,6 +932,17 @@ void pair_by_key(Ctx &c, K *keys, u32 *vals, u32 len, u32 bits, u32 *vcmap) {
     BackScope bs(c.arena);
     K *ktmp = bs.get<K>(len);
     u32 *vtmp = bs.get<u32>(len);
+    if (c.n_xcc && c.block_jet_max_n && len <= PT_LIST) {
+        PairTeam *pt = bs.get<PairTeam>(1);
+        fill<u32>(c, (u32 *) pt, sizeof(TeamHead) / 4 + 32, 0u);
+        PairTeamArgs<K> a{pt, {{keys}, {ktmp}}, {{vals}, {vtmp}}, len, bits, c.xcc, std::min<u32>(TEAM_WANT, div_up(len, 256)),
+                          vcmap};
+        launch(c, "match_pair", 0.0, dim3(a.want * c.n_xcc), dim3(TM), 0, pair_team_kernel<K>, a);
+        u32 res[2];
+        readback(c, res, &pt->ran, 2);
+        if (res[1]) throw Error(HEIPA_ERR_DEVICE, "matching: a team workgroup never arrived at a barrier");
+        if (res[0]) return;
+    }
     const bool flip = radix_sort_pairs<K>(c, keys, vals, ktmp, vtmp, len, bits);
     const K *sk = flip ? ktmp : keys;
     const u32 *sv = flip ? vtmp : vals;

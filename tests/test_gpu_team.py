@@ -124,7 +124,18 @@ def test_team_on_every_xcd():
             c.close()
 
 
+def _twins(leaves, groups):
+    """`leaves` vertices of degree 2 in `groups` interleaved groups of twins."""
+    i = np.arange(leaves)
+    a, b = i % groups, groups + (i % groups) * 7 % groups
+    return csr_from_arrays(leaves + 2 * groups, np.concatenate([i + 2 * groups] * 2), np.concatenate([a, b]))
+
+
 MATCH = {
+    "twins": lambda: _twins(20000, 6),  # groups that span the members' shares
+    "twins_many": lambda: _twins(5000, 1500),  # groups of 3 and 4
+    "isolated": lambda: csr_from_arrays(40000, [0, 1], [1, 2]),  # one group of all but three
+    "isolated_many": lambda: csr_from_arrays(70001, [0, 1], [1, 2]),  # longer than a team sorts
     "n1": lambda: heipa.HostGraph(np.zeros(2, np.uint32), np.zeros(0, np.uint32)),
     "n2": lambda: _regular(2, 1),
     "tile": lambda: _regular(16384, 4),  # one list entry per lane of 256 waves
