@@ -218,8 +218,7 @@ int heipa_contract(heipa_ctx *ctx, const heipa_graph *fine, const uint32_t *mapp
             BackScope bs(c.arena);
             validate(c, d, mapping, nc);
         }
-        GraphMeta meta;  // unused by contraction
-        CoarseGraph cg = contract(c, d, meta, mapping, nc);
+        CoarseGraph cg = contract(c, d, mapping, nc, ~0u);
         c.sync();
         coarse->n = cg.g.n;
         coarse->m = cg.g.m;

@@ -30,17 +30,31 @@ constexpr u32 PAD = 0xFFFFFFFFu;
 constexpr u32 BLK_ROW_MAX = 4096;
 constexpr int CB = 256;
 
-// members of coarse vertices (counting sort by M(u)) + coarse weights + ub
+// members of coarse vertices (counting sort by M(u)) + coarse weights; one
+// 64-bit word per coarse vertex counts its members (low half) and the sum of
+// their degrees (high half, the upper bound ub of its row's length): one
+// update per member, and one scan gives both offsets
 template<bool UVW>
-__global__ void member_count_kernel(DGraph g, const u32 *__restrict__ map, u32 *__restrict__ mcnt,
-                                    unsigned long long *__restrict__ cw, u32 *__restrict__ ub) {
+__global__ void member_count_kernel(DGraph g, const u32 *__restrict__ map, unsigned long long *__restrict__ cnt64,
+                                    unsigned long long *__restrict__ cw) {
     for (u64 u = (u64) blockIdx.x * blockDim.x + threadIdx.x; u < g.n; u += (u64) gridDim.x * blockDim.x) {
         const u32 c = map[u];
-        atomicAdd(&mcnt[c], 1u);
+        atomicAdd(&cnt64[c], (u64) (g.xadj[u + 1] - g.xadj[u]) << 32 | 1u);
         atomicAdd(&cw[c], (unsigned long long) (UVW ? 1 : g.vw[u]));
-        atomicAdd(&ub[c], g.xadj[u + 1] - g.xadj[u]);
     }
 }
+struct MemberSrc {
+    const unsigned long long *cnt64;
+    u64 nc;
+    __device__ u64 operator()(u64 c) const { return c < nc ? cnt64[c] : 0; }
+};
+struct MemberDst {
+    u32 *moff, *uboff;
+    __device__ void operator()(u64 c, u64 v) const {
+        moff[c] = (u32) v;
+        uboff[c] = (u32) (v >> 32);
+    }
+};
 
 __global__ void member_scatter_kernel(u32 n, const u32 *__restrict__ map, const u32 *__restrict__ moff,
                                       u32 *__restrict__ mfill, u32 *__restrict__ mem) {
@@ -50,13 +64,13 @@ __global__ void member_scatter_kernel(u32 n, const u32 *__restrict__ map, const 
     }
 }
 
-__global__ void cw_finish_kernel(u32 nc, const unsigned long long *__restrict__ cw, s32 *__restrict__ cvw,
-                                 u32 *__restrict__ overflow) {
+__global__ void contract_init_kernel(u32 nc, unsigned long long *cnt64, unsigned long long *cw, u32 *mfill, u32 *scal) {
     for (u64 c = (u64) blockIdx.x * blockDim.x + threadIdx.x; c < nc; c += (u64) gridDim.x * blockDim.x) {
-        const unsigned long long w = cw[c];
-        if (w > (unsigned long long) INT32_MAX) *overflow = 1;
-        cvw[c] = (s32) w;
+        cnt64[c] = 0;
+        cw[c] = 0;
+        mfill[c] = 0;
     }
+    if (blockIdx.x == 0 && threadIdx.x < 16) scal[threadIdx.x] = 0;
 }
 
 // tiers: 0..3 -> W = 8,16,32,64; 4 -> workgroup; 5 -> global sort
@@ -69,10 +83,13 @@ __device__ __forceinline__ u32 tier_of(u32 ub) {
     return 5;
 }
 
-// Each workgroup takes a contiguous chunk of coarse vertices: it counts them
+// The coarse weights, and the coarse vertices listed by tier: each workgroup
+// takes a contiguous chunk of coarse vertices, counts them
 // per tier in LDS, reserves each tier's space with one counter update, then
 // writes its entries (per-wave updates of the six counters serialised).
-__global__ __launch_bounds__(256) void classify_kernel(u32 nc, const u32 *__restrict__ ub, u32 *__restrict__ tier_cnt,
+__global__ __launch_bounds__(256) void classify_kernel(u32 nc, const u32 *__restrict__ uboff,
+                                                       const unsigned long long *__restrict__ cw, s32 *__restrict__ cvw,
+                                                       u32 *__restrict__ overflow, u32 *__restrict__ tier_cnt,
                                                        u32 *__restrict__ tier_lists, u32 stride) {
     __shared__ u32 s_cnt[6], s_base[6];
     const u64 chunk = ((u64) nc + gridDim.x - 1) / gridDim.x;
@@ -82,7 +99,12 @@ __global__ __launch_bounds__(256) void classify_kernel(u32 nc, const u32 *__rest
     __syncthreads();
     for (u64 i0 = c0; i0 < c1; i0 += blockDim.x) {
         const u64 c = i0 + threadIdx.x;
-        const u32 t = c < c1 ? tier_of(ub[c]) : 99u;
+        const u32 t = c < c1 ? tier_of(uboff[c + 1] - uboff[c]) : 99u;
+        if (c < c1) {
+            const unsigned long long w = cw[c];
+            if (w > (unsigned long long) INT32_MAX) *overflow = 1;
+            cvw[c] = (s32) w;
+        }
         for (u32 tt = 0; tt < 6; ++tt) {
             const u64 bal = __ballot(t == tt);
             if (bal && lane_id() == 0) atomicAdd(&s_cnt[tt], (u32) __popcll(bal));
@@ -97,7 +119,7 @@ __global__ __launch_bounds__(256) void classify_kernel(u32 nc, const u32 *__rest
     __syncthreads();
     for (u64 i0 = c0; i0 < c1; i0 += blockDim.x) {
         const u64 c = i0 + threadIdx.x;
-        const u32 t = c < c1 ? tier_of(ub[c]) : 99u;
+        const u32 t = c < c1 ? tier_of(uboff[c + 1] - uboff[c]) : 99u;
         for (u32 tt = 0; tt < 6; ++tt) {
             const bool mine = t == tt;
             const u64 bal = __ballot(mine);
@@ -129,8 +151,10 @@ template<int W, bool UEW>
 __global__ __launch_bounds__(CB) void row_small_kernel(DGraph g, const u32 *__restrict__ map,
                                                        const u32 *__restrict__ moff, const u32 *__restrict__ mem,
                                                        const u32 *__restrict__ uboff, const u32 *__restrict__ list,
-                                                       u32 len, u32 *__restrict__ tkey, s32 *__restrict__ tw,
-                                                       u32 *__restrict__ cnt, u32 *__restrict__ overflow) {
+                                                       const u32 *__restrict__ len_ptr, u32 *__restrict__ tkey,
+                                                       s32 *__restrict__ tw, u32 *__restrict__ cnt,
+                                                       u32 *__restrict__ overflow) {
+    const u32 len = *len_ptr;
     const u32 l = threadIdx.x % W;
     const u64 groups = (u64) gridDim.x * (CB / W);
     const u32 sub_base = (lane_id() / W) * W;  // first wave lane of this group
@@ -200,15 +224,17 @@ __global__ __launch_bounds__(CB) void row_small_kernel(DGraph g, const u32 *__re
 template<bool UEW>
 __global__ __launch_bounds__(CB) void row_block_kernel(DGraph g, const u32 *__restrict__ map,
                                                        const u32 *__restrict__ moff, const u32 *__restrict__ mem,
-                                                       const u32 *__restrict__ uboff, const u32 *__restrict__ ub,
-                                                       const u32 *__restrict__ list, u32 *__restrict__ tkey,
+                                                       const u32 *__restrict__ uboff, const u32 *__restrict__ list,
+                                                       const u32 *__restrict__ len_ptr, u32 *__restrict__ tkey,
                                                        s32 *__restrict__ tw, u32 *__restrict__ cnt,
                                                        u32 *__restrict__ overflow) {
     __shared__ u32 skey[BLK_ROW_MAX];
     __shared__ s32 sw[BLK_ROW_MAX];
     __shared__ u32 red[CB / WAVE];
-    const u32 c = list[blockIdx.x];
-    const u32 len = ub[c];
+    const u32 rows = *len_ptr;
+    for (u32 row = blockIdx.x; row < rows; row += gridDim.x) {
+    const u32 c = list[row];
+    const u32 len = uboff[c + 1] - uboff[c];
     // P is a power of two and a multiple of the block size, so every thread's
     // slot in the dedupe loop below holds a sorted key or PAD
     u32 P = CB;
@@ -269,6 +295,8 @@ __global__ __launch_bounds__(CB) void row_block_kernel(DGraph g, const u32 *__re
         carry += tot;
     }
     if (threadIdx.x == 0) cnt[c] = carry;
+    __syncthreads();  // the next row restages the LDS
+    }
 }
 
 // ---- hub rows through a global sort of (row index << 32 | coarse id)
@@ -322,10 +350,10 @@ __global__ void hub_merge_kernel(const u64 *__restrict__ keys, const u32 *__rest
     if (threadIdx.x == 0) cnt[c] = carry;
 }
 
-__global__ void hub_offsets_kernel(const u32 *__restrict__ list, u32 nh, const u32 *__restrict__ ub,
+__global__ void hub_offsets_kernel(const u32 *__restrict__ list, u32 nh, const u32 *__restrict__ uboff,
                                    u32 *__restrict__ hub_ub) {
     for (u64 t = (u64) blockIdx.x * blockDim.x + threadIdx.x; t < nh; t += (u64) gridDim.x * blockDim.x)
-        hub_ub[t] = ub[list[t]];
+        hub_ub[t] = uboff[list[t] + 1] - uboff[list[t]];
 }
 
 // compact copy of the staged rows, W lanes per row
@@ -359,21 +387,16 @@ __global__ void project_kernel(const u32 *__restrict__ map, u32 n, const u32 *__
 
 template<int W>
 void launch_row_small(Ctx &c, const DGraph &g, const u32 *map, const u32 *moff, const u32 *mem, const u32 *uboff,
-                      const u32 *list, u32 len, u32 *tkey, s32 *tw, u32 *cnt, u32 *overflow) {
-    if (!len) return;
-    const dim3 grid(grid_for(c, len, CB / W, 8)), block(CB);
-    if (g.ew)
-        launch(c, "contract_rows", 0.0, grid, block, 0, row_small_kernel<W, false>, g, map, moff, mem, uboff,
-               list, len, tkey, tw, cnt, overflow);
-    else
-        launch(c, "contract_rows", 0.0, grid, block, 0, row_small_kernel<W, true>, g, map, moff, mem, uboff,
-               list, len, tkey, tw, cnt, overflow);
+                      const u32 *list, const u32 *len_ptr, u32 bound, u32 *tkey, s32 *tw, u32 *cnt, u32 *overflow) {
+    if (!bound) return;
+    const dim3 grid(grid_for(c, bound, CB / W, 8)), block(CB);
+    launch(c, "contract_rows", 0.0, grid, block, 0, g.ew ? row_small_kernel<W, false> : row_small_kernel<W, true>, g, map,
+           moff, mem, uboff, list, len_ptr, tkey, tw, cnt, overflow);
 }
 
 } // namespace
 
-CoarseGraph contract(Ctx &c, const DGraph &fine, const GraphMeta &meta, const u32 *map, u32 nc) {
-    (void) meta;
+CoarseGraph contract(Ctx &c, const DGraph &fine, const u32 *map, u32 nc, u32 max_row) {
     CoarseGraph out;
     out.front_depth_before = c.arena.front_depth();
     const u32 n = fine.n;
@@ -381,64 +404,50 @@ CoarseGraph contract(Ctx &c, const DGraph &fine, const GraphMeta &meta, const u3
     s32 *cvw = (s32 *) c.arena.push_front(4ull * (nc ? nc : 1));
     u32 *cxadj = (u32 *) c.arena.push_front(4ull * (nc + 1));
     BackScope bs(c.arena);
-    u32 *mcnt = bs.get<u32>(nc + 1);
     u32 *moff = bs.get<u32>(nc + 1);
     u32 *mfill = bs.get<u32>(nc + 1);
     u32 *mem = bs.get<u32>(n);
+    auto *cnt64 = bs.get<unsigned long long>(nc + 1);
     auto *cw = bs.get<unsigned long long>(nc + 1);
-    u32 *ub = bs.get<u32>(nc + 1);
     u32 *uboff = bs.get<u32>(nc + 1);
     u32 *cnt = bs.get<u32>(nc + 1);
-    u32 *scal = bs.get<u32>(16);  // [0..5] tier counts, [8] overflow
-    fill<u32>(c, mcnt, nc + 1, 0u);
-    fill<u32>(c, mfill, nc + 1, 0u);
-    fill<unsigned long long>(c, cw, nc + 1, 0ull);
-    fill<u32>(c, ub, nc + 1, 0u);
-    fill<u32>(c, scal, 16, 0u);
+    // [0..5] tier counts, [8] overflow, [9] inconsistent rows, [10] largest degree, [11] hubs
+    u32 *scal = bs.get<u32>(16);
     const dim3 blk(256);
     const dim3 gn(grid_for(c, n, 256)), gc(grid_for(c, nc, 256));
-    const double read_bytes = 4.0 * (n + 1) + 4.0 * fine.m * (fine.ew ? 2 : 1) + 4.0 * n + (fine.vw ? 4.0 * n : 0.0);
-    if (fine.vw)
-        launch(c, "contract_members", 0.0, gn, blk, 0, member_count_kernel<false>, fine, map, mcnt, cw, ub);
-    else
-        launch(c, "contract_members", 0.0, gn, blk, 0, member_count_kernel<true>, fine, map, mcnt, cw, ub);
-    exclusive_sum<u32>(c, "contract_members", mcnt, moff, nc);
+    launch(c, "contract_init", 20.0 * nc, gc, blk, 0, contract_init_kernel, nc, cnt64, cw, mfill, scal);
+    launch(c, "contract_members", 0.0, gn, blk, 0, fine.vw ? member_count_kernel<false> : member_count_kernel<true>, fine, map,
+           cnt64, cw);
+    scan<u64>(c, "contract_members", MemberSrc{cnt64, nc}, MemberDst{moff, uboff}, (u64) nc + 1, (u64 *) nullptr);
     launch(c, "contract_members", 0.0, gn, blk, 0, member_scatter_kernel, n, map, (const u32 *) moff, mfill, mem);
-    launch(c, "contract_members", 0.0, gc, blk, 0, cw_finish_kernel, nc, (const unsigned long long *) cw, cvw,
-           scal + 8);
-    exclusive_sum<u32>(c, "contract_offsets", ub, uboff, nc);
     // staging rows
     const u32 mtot = fine.m;
     u32 *tkey = bs.get<u32>(mtot);
     s32 *tw = bs.get<s32>(mtot);
     const u32 stride = nc;
     u32 *tier_lists = bs.get<u32>((u64) 6 * stride);
-    launch(c, "contract_classify", 0.0, dim3(grid_for(c, nc, 256, 2)), blk, 0, classify_kernel, nc, (const u32 *) ub,
-           scal, tier_lists, stride);
-    u32 tc[6];
-    readback(c, tc, scal, 6);
-    launch_row_small<8>(c, fine, map, moff, mem, uboff, tier_lists + 0ull * stride, tc[0], tkey, tw, cnt, scal + 8);
-    launch_row_small<16>(c, fine, map, moff, mem, uboff, tier_lists + 1ull * stride, tc[1], tkey, tw, cnt, scal + 8);
-    launch_row_small<32>(c, fine, map, moff, mem, uboff, tier_lists + 2ull * stride, tc[2], tkey, tw, cnt, scal + 8);
-    launch_row_small<64>(c, fine, map, moff, mem, uboff, tier_lists + 3ull * stride, tc[3], tkey, tw, cnt, scal + 8);
-    if (tc[4]) {
-        if (fine.ew)
-            launch(c, "contract_rows", 0.0, dim3(tc[4]), dim3(CB), 0, row_block_kernel<false>, fine, map,
-                   (const u32 *) moff, (const u32 *) mem, (const u32 *) uboff, (const u32 *) ub,
-                   (const u32 *) (tier_lists + 4ull * stride), tkey, tw, cnt, scal + 8);
-        else
-            launch(c, "contract_rows", 0.0, dim3(tc[4]), dim3(CB), 0, row_block_kernel<true>, fine, map,
-                   (const u32 *) moff, (const u32 *) mem, (const u32 *) uboff, (const u32 *) ub,
-                   (const u32 *) (tier_lists + 4ull * stride), tkey, tw, cnt, scal + 8);
-    }
-    if (tc[5]) {
-        const u32 nh = tc[5];
-        const u32 *hl = tier_lists + 5ull * stride;
+    launch(c, "contract_classify", 0.0, dim3(grid_for(c, nc, 256, 2)), blk, 0, classify_kernel, nc, (const u32 *) uboff,
+           (const unsigned long long *) cw, cvw, scal + 8, scal, tier_lists, stride);
+    // the tiers that rows of at most max_row entries can fill; the kernels read
+    // the tiers' lengths on the device
+    auto tier = [&](u32 t) { return (const u32 *) (tier_lists + (u64) t * stride); };
+    launch_row_small<8>(c, fine, map, moff, mem, uboff, tier(0), scal + 0, nc, tkey, tw, cnt, scal + 8);
+    if (max_row > 8) launch_row_small<16>(c, fine, map, moff, mem, uboff, tier(1), scal + 1, nc, tkey, tw, cnt, scal + 8);
+    if (max_row > 16) launch_row_small<32>(c, fine, map, moff, mem, uboff, tier(2), scal + 2, nc, tkey, tw, cnt, scal + 8);
+    if (max_row > 32) launch_row_small<64>(c, fine, map, moff, mem, uboff, tier(3), scal + 3, nc, tkey, tw, cnt, scal + 8);
+    if (max_row > 64 && nc)
+        launch(c, "contract_rows", 0.0, dim3(std::min<u32>(nc, (u32) c.num_cus * 8)), dim3(CB), 0,
+               fine.ew ? row_block_kernel<false> : row_block_kernel<true>, fine, map, (const u32 *) moff, (const u32 *) mem,
+               (const u32 *) uboff, tier(4), (const u32 *) (scal + 4), tkey, tw, cnt, scal + 8);
+    u32 nh = 0;
+    if (max_row > BLK_ROW_MAX) readback(c, &nh, scal + 5, 1);
+    if (nh) {
+        const u32 *hl = tier(5);
         BackScope hs(c.arena);
         u32 *hub_ub = hs.get<u32>(nh + 1);
         u32 *hoff = hs.get<u32>(nh + 1);
         launch(c, "contract_hubs", 0.0, dim3(grid_for(c, nh, 256)), blk, 0, hub_offsets_kernel, hl, nh,
-               (const u32 *) ub, hub_ub);
+               (const u32 *) uboff, hub_ub);
         exclusive_sum<u32>(c, "contract_hubs", hub_ub, hoff, nh);
         u32 tot;
         readback(c, &tot, hoff + nh, 1);
@@ -469,13 +478,9 @@ CoarseGraph contract(Ctx &c, const DGraph &fine, const GraphMeta &meta, const u3
     if (hm[1]) throw Error(HEIPA_ERR_OVERFLOW, "coarse weight exceeds the s32 range of the graph format");
     u32 *cadj = (u32 *) c.arena.push_front(4ull * (mc ? mc : 1));
     s32 *cew = (s32 *) c.arena.push_front(4ull * (mc ? mc : 1));
-    (void) read_bytes;
     launch(c, "contract_copy", 16.0 * mc + 8.0 * (nc + 1), dim3(grid_for(c, nc, CB / 16, 8)), dim3(CB), 0,
            copy_rows_kernel, nc, (const u32 *) uboff, (const u32 *) cxadj, (const u32 *) tkey, (const s32 *) tw, cadj,
            cew, scal + 9);
-    u32 bad;
-    readback(c, &bad, scal + 9, 1);
-    if (bad) throw Error(HEIPA_ERR_DEVICE, "contraction produced an inconsistent coarse graph");
     out.g.n = nc;
     out.g.m = mc;
     out.g.gw = fine.gw;
@@ -483,6 +488,14 @@ CoarseGraph contract(Ctx &c, const DGraph &fine, const GraphMeta &meta, const u3
     out.g.adj = cadj;
     out.g.ew = cew;
     out.g.vw = cvw;
+    // the coarse graph's metadata with the copy's check: one wait
+    out.meta = meta_of(out.g);
+    if (nc) meta_launch(c, out.g, out.meta, scal + 10);
+    u32 fin[3];
+    readback(c, fin, scal + 9, 3);
+    if (fin[0]) throw Error(HEIPA_ERR_DEVICE, "contraction produced an inconsistent coarse graph");
+    out.meta.max_deg = fin[1];
+    out.meta.n_hubs = fin[2];
     return out;
 }
 

@@ -309,6 +309,8 @@ void check_throw(u32 f) {
     if (f & 16u) throw Error(HEIPA_ERR_INVALID, "invalid graph: self loops are not allowed");
     if (f & 32u) throw Error(HEIPA_ERR_INVALID, "partition holds a block id >= k");
 }
+} // namespace
+
 GraphMeta meta_of(const DGraph &g) {
     GraphMeta meta;
     meta.G = group_for_avg(g.n ? (double) g.m / (double) g.n : 0.0);
@@ -323,7 +325,10 @@ void hub_list(Ctx &c, const DGraph &g, GraphMeta &meta, bool back) {
     launch(c, "graph_meta", 4.0 * (g.n + 1), dim3(grid_for(c, g.n, 256)), dim3(256), 0, hub_list_kernel, g.xadj, g.n,
            meta.hub_deg, cnt, meta.hubs);
 }
-} // namespace
+void meta_launch(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *out) {
+    launch(c, "graph_meta", 4.0 * (g.n + 1), dim3(grid_for(c, g.n, 256 * 4, 2)), dim3(256), 0, degrees_kernel, g.xadj, g.n,
+           meta.hub_deg, out);
+}
 
 GraphMeta validate(Ctx &c, const DGraph &g, const u32 *part, u32 k) {
     GraphMeta meta = meta_of(g);
@@ -353,8 +358,7 @@ GraphMeta make_meta(Ctx &c, const DGraph &g, bool back) {
         BackScope bs(c.arena);
         u32 *scr = bs.get<u32>(2);
         fill<u32>(c, scr, 2, 0u);
-        launch(c, "graph_meta", 4.0 * (g.n + 1), dim3(grid_for(c, g.n, 256 * 4, 2)), dim3(256), 0, degrees_kernel, g.xadj,
-               g.n, meta.hub_deg, scr);
+        meta_launch(c, g, meta, scr);
         u32 h[2];
         readback(c, h, scr, 2);
         meta.max_deg = h[0];
@@ -423,6 +427,9 @@ s64 comm_cost(Ctx &c, const DGraph &g, const u32 *part, const s32 *D, u32 k) { r
 
 void block_weights_dev(Ctx &c, const DGraph &g, const u32 *part, u32 k, s64 *bw_dev, const u32 *bad) {
     fill<s64>(c, bw_dev, k, 0);
+    block_weights_add(c, g, part, k, bw_dev, bad);
+}
+void block_weights_add(Ctx &c, const DGraph &g, const u32 *part, u32 k, s64 *bw_dev, const u32 *bad) {
     const double bytes = 4.0 * g.n * (g.vw ? 2 : 1);
     const size_t shmem = sizeof(unsigned long long) * k;
     if (shmem > 64 * 1024) {  // no LDS histogram: one global atomic per vertex

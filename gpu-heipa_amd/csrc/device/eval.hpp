@@ -20,6 +20,7 @@ s64 comm_cost_checked(Ctx &c, const DGraph &g, const u32 *part, const s32 *D, u3
 void block_weights_checked(Ctx &c, const DGraph &g, const u32 *part, u32 k, s64 *bw_host);
 // bad: a checked caller's flags on the device (null: the input is sound)
 void block_weights_dev(Ctx &c, const DGraph &g, const u32 *part, u32 k, s64 *bw_dev, const u32 *bad = nullptr);
+void block_weights_add(Ctx &c, const DGraph &g, const u32 *part, u32 k, s64 *bw_dev, const u32 *bad = nullptr);
 
 // ---- matching (match.hip): mapping is a device array of n entries; returns nc
 u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping, heipa_match_stats *stats);
@@ -28,9 +29,12 @@ u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping
 // front stack in the order vwgt, xadj, adjncy, adjwgt.
 struct CoarseGraph {
     DGraph g;
+    GraphMeta meta;  // without the hub list (hub_list makes it)
     size_t front_depth_before = 0;  // release_front(front_depth_before) frees it
 };
-CoarseGraph contract(Ctx &c, const DGraph &fine, const GraphMeta &meta, const u32 *mapping, u32 nc);
+// max_row: no coarse vertex's members have more than this many edges together
+// (a matching joins two: twice the largest degree; ~0u if unknown)
+CoarseGraph contract(Ctx &c, const DGraph &fine, const u32 *mapping, u32 nc, u32 max_row);
 void project(Ctx &c, const u32 *mapping, u32 fine_n, const u32 *coarse_part, u32 *fine_part);
 
 // ---- Jet refinement (jet.hip)

@@ -31,6 +31,12 @@ inline u32 group_for_avg(double avg) {
 // Computes metadata; the hub list is pushed on the arena's BACK stack when
 // `back` is true (temporary) or the FRONT stack otherwise.
 GraphMeta make_meta(Ctx &c, const DGraph &g, bool back);
+// its steps: the lane-group width and hub threshold from the sizes; the launch
+// that adds the largest degree and the hub count to out[0..1] (zero before);
+// the hub list once meta.n_hubs is known
+GraphMeta meta_of(const DGraph &g);
+void meta_launch(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *out);
+void hub_list(Ctx &c, const DGraph &g, GraphMeta &meta, bool back);
 
 // Dispatch a templated kernel launcher on the group width.
 #define HEIPA_DISPATCH_G(Gval, FN, ...)            \

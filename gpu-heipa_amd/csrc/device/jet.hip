@@ -2565,7 +2565,24 @@ struct RatioTable {
     u32 n;
 };
 
-__global__ void ctl_init_kernel(JetDev d, RatioTable rt, s64 cut, s64 maxw) {
+// a level's state before its first iteration: one launch instead of a fill per
+// array (about 3 us of host time each, ten of them on levels whose iterations
+// take 12 us)
+__global__ __launch_bounds__(256) void jet_init_kernel(JetDev d, RatioTable rt, s64 cut, s64 maxw, u32 *team, u32 team_words,
+                                                       u64 wcnt_words) {
+    const u64 stride = (u64) gridDim.x * blockDim.x, t0 = (u64) blockIdx.x * blockDim.x + threadIdx.x;
+    for (u64 v = t0; v < d.n; v += stride) {
+        d.work[v] = d.part[v];
+        d.dcache[v] = NULL_PART;
+        d.icache[v] = -1;
+        d.mark[v] = 0;
+        d.lock[v] = 0;
+        d.lock[d.n + v] = 0;  // stale bytes
+    }
+    for (u64 i = t0; i < (u64) d.nshard * ((u64) d.t + 1); i += stride) d.btot[i] = 0;
+    for (u64 i = t0; i < d.k; i += stride) d.bw[i] = 0;
+    for (u64 i = t0; i < team_words; i += stride) team[i] = 0;
+    for (u64 i = t0; i < wcnt_words; i += stride) d.wcnt[i] = 0;
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     JetCtl *ctl = d.ctl;
 #pragma unroll
@@ -2732,6 +2749,7 @@ struct JetHost {
     u32 n_chunks = 0;  // hub chunks of the apply step
     u32 *chunk_hub = nullptr, *chunk_idx = nullptr;
     bool rows = false;  // the level has wide vertices (degree >= k)
+    bool over_clear = false;
 
     JetHost(Ctx &cc, const DGraph &gg, const GraphMeta &mm) : c(cc), g(gg), meta(mm) {}
 
@@ -2829,6 +2847,8 @@ struct JetHost {
     // the stalled iteration's resolve on the global path, then its apply
     void fallback(const JetCtl &s) {
         BackScope bs(c.arena);
+        if (!over_clear) fill<u32>(c, over_flag, g.n, 0u);  // the overflow kernel leaves it clear
+        over_clear = true;
         const bool strong = s.mode == 2;
         const u32 L = (u32) s.st[ST_RLIST];
         u64 *k2 = bs.get<u64>(L);
@@ -2981,8 +3001,7 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         if (h.team_mode) {
             h.ta.xcc = c.xcc;
             h.ta.want = std::min<u32>(TEAM_WANT, div_up(n, 64));
-            h.ta.tc = bs.get<TeamCtl>(TEAM_SLOTS);
-            fill<u64>(c, (u64 *) h.ta.tc, TEAM_SLOTS * sizeof(TeamCtl) / 8, 0);
+            h.ta.tc = bs.get<TeamCtl>(TEAM_SLOTS);  // cleared by the init launch
         }
     }
     // copies of the minibucket totals: about one per 64 sweep workgroups, at
@@ -3063,6 +3082,7 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
                meta.n_hubs, h.chunk_hub, h.chunk_idx);
     }
     // BlockConn rows of the wide vertices (block_conn.h)
+    u64 wcnt_words = 0;
     if (meta.max_deg >= k) {
         h.rows = true;
         d.W = (k + 31) / 32;
@@ -3070,25 +3090,26 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         d.wid = bs.get<u32>(n);
         u32 *cnt = bs.get<u32>(1);
         scan<u32>(c, "jet_init", WideSrc{g.xadj, k}, WideDst{g.xadj, k, d.wid, d.rflag, meta.hub_deg}, n, cnt);
-        u32 nw = 0;
-        readback(c, &nw, cnt, 1);
-        d.wsz = bs.get<u32>(nw ? nw : 1);
-        d.wV = bs.get<u32>((u64) (nw ? nw : 1) * d.W);
-        d.wP = bs.get<u32>((u64) (nw ? nw : 1) * d.W);
-        if (d.W <= 2) {  // counts of the counted vertices; nw * k <= m (a wide vertex has k edges)
-            d.wcnt = bs.get<u32>((u64) (nw ? nw : 1) * k);
-            fill<u32>(c, d.wcnt, (u64) (nw ? nw : 1) * k, 0u);
+        // rows for the most wide vertices there can be (each has k edges): that
+        // saves a wait of 12-15 us per level; where they would take more than an
+        // eighth of the free scratch, the vertices are counted instead
+        u64 nw = std::min<u64>(n, g.m / k);
+        if (nw * (8ull * d.W + 4ull * k + 4) > (c.arena.capacity() - c.arena.in_use()) / 8) {
+            u32 exact = 0;
+            readback(c, &exact, cnt, 1);
+            nw = std::max(exact, 1u);
+        }
+        d.wsz = bs.get<u32>(nw);
+        d.wV = bs.get<u32>(nw * d.W);
+        d.wP = bs.get<u32>(nw * d.W);
+        if (d.W <= 2 && meta.max_deg > ROW_THREAD_DEG) {  // counts of the counted vertices
+            wcnt_words = nw * k;
+            d.wcnt = bs.get<u32>(wcnt_words);
         }
     }
-    copy_d2d(c, d.work, part, 4ull * n);
-    fill<u32>(c, d.dcache, n, NULL_PART);
-    fill<s64>(c, d.icache, n, -1);
-    fill<u8>(c, d.lock, 2ull * n, (u8) 0);
-    fill<u32>(c, d.mark, n, 0u);
-    fill<u32>(c, h.over_flag, n, 0u);
-    fill<s64>(c, d.btot, (u64) d.nshard * ((u64) d.t + 1), 0);
-    block_weights_dev(c, g, d.work, k, d.bw);
-    launch(c, "jet_init", 0.0, dim3(1), dim3(64), 0, ctl_init_kernel, d, rt, cut, maxw);
+    launch(c, "jet_init", 0.0, dim3(grid_for(c, std::max<u64>(n, wcnt_words / 4), 256, 8)), dim3(256), 0, jet_init_kernel, d, rt,
+           cut, maxw, (u32 *) h.ta.tc, h.ta.tc ? (u32) (TEAM_SLOTS * sizeof(TeamCtl) / 4) : 0u, wcnt_words);
+    block_weights_add(c, g, part, k, d.bw);
     h.row_update_launches(1);  // init_BlockConn (jet:951)
 
     // Batches of iterations; the host reads the control block (and the trace
@@ -3146,7 +3167,9 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
     int pend = 0;
     submit(0);
     for (;;) {
-        submit(pend ^ 1);
+        // a batch ahead; a team's launch is most often a level's last
+        const bool ahead = !h.team_mode;
+        if (ahead) submit(pend ^ 1);
         HIP_CHECK(hipEventSynchronize(ev[pend]));
         std::memcpy(&s, slot[pend], sizeof(JetCtl));
         if (tracing) {
@@ -3159,15 +3182,16 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         if (h.team_mode && s.launches == team_seen) h.team_mode = false;  // no workgroup reached the XCD
         team_seen = s.launches;
         if (s.stalled) {
-            HIP_CHECK(hipEventSynchronize(ev[pend ^ 1]));
+            if (ahead) HIP_CHECK(hipEventSynchronize(ev[pend ^ 1]));
             h.fallback(s);
             submit(pend);
             continue;
         }
-        pend ^= 1;
+        if (ahead) pend ^= 1;
+        else submit(pend);
         B = std::min<u32>(B * 2, BATCH_MAX);
     }
-    c.sync();
+    if (gx.e || c.prof_on) c.sync();  // the graph's last replay ends before it is destroyed
     c.event_pool.push_back(ev[0]);
     c.event_pool.push_back(ev[1]);
     if (s.save) copy_d2d(c, part, d.work, 4ull * n);
@@ -3180,7 +3204,7 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         prof_bytes(c, "jet_resolve", s.bytes[3]);
         prof_bytes(c, "jet_apply", s.bytes[4]);
     }
-    c.sync();
+    if (c.prof_on) c.sync();
     res.cut = s.best_cut;
     res.maxw = s.best_maxw;
     res.iterations = s.iters;

@@ -16,7 +16,7 @@
 // The team itself (formation, barrier, hand-offs) is team.hpp.
 #pragma once
 
-constexpr u32 TEAM_ITERS = 64;                // iterations per launch
+constexpr u32 TEAM_ITERS = 128;               // iterations per launch
 constexpr u32 TEAM_RCAP = 4096;               // resolve entries sorted in LDS
 constexpr u32 TEAM_U = 2;                     // sweep tiles a wave has in flight
 constexpr u32 TILE = WAVE * TEAM_U;           // vertices of one sweep step of a wave

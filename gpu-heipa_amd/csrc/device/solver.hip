@@ -554,16 +554,16 @@ SolveResult solve(Ctx &c, const DGraph &g0, u32 k, double imbalance, u64 seed, b
         double ta = now_ms();
         c.prof_l0 = c.prof_on && graphs.size() == 1;
         const u32 nc = match(c, g, metas.back(), 12345u, map, nullptr);
-        c.sync();
         double tb = now_ms();
         res.ms[0] += tb - ta;
-        CoarseGraph cg = contract(c, g, metas.back(), map, nc);
+        const u32 max_row = metas.back().max_deg <= 0x7FFFFFFFu ? 2 * metas.back().max_deg : ~0u;  // at most two members
+        CoarseGraph cg = contract(c, g, map, nc, max_row);
         c.prof_l0 = false;
         const u32 fine_n = g.n;
         maps.push_back(map);
         graphs.push_back(cg.g);
-        metas.push_back(make_meta(c, cg.g, false));
-        c.sync();
+        hub_list(c, cg.g, cg.meta, false);
+        metas.push_back(cg.meta);
         res.ms[1] += now_ms() - tb;
         if (ent) hier_append(c, *ent, l, fine_n, map, cg.g);
     }
@@ -614,7 +614,6 @@ SolveResult solve(Ctx &c, const DGraph &g0, u32 k, double imbalance, u64 seed, b
         double ta = now_ms();
         project(c, maps[l], graphs[l].n, cur, other);
         std::swap(cur, other);
-        c.sync();
         double tb = now_ms();
         res.ms[3] += tb - ta;
         c.prof_l0 = c.prof_on && l == 0;
