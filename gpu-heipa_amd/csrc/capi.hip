@@ -415,6 +415,7 @@ int heipa_ctx_set_option(heipa_ctx *ctx, int option, uint64_t value) {
         else if (option == HEIPA_OPT_BUCKET_COPIES) c.bucket_copies = (u32) std::min<uint64_t>(value, 32);
         else if (option == HEIPA_OPT_BLOCK_LDS || option == HEIPA_OPT_BLOCK_GROUP_CAP) {}  // accepted, without effect
         else if (option == HEIPA_OPT_GROUP_CAP) c.group_cap = (u32) std::min<uint64_t>(value, 64);
+        else if (option == HEIPA_OPT_WIDE_JET) c.wide_jet_max_n = (u32) std::min<uint64_t>(value, 0xFFFFFFFFull);
         else if (option == HEIPA_OPT_TEAM_JET) c.team_jet_max_n = (u32) std::min<uint64_t>(value, 0xFFFFFFFFull);
         else if (option == HEIPA_OPT_REGION_EDGES) c.region_edges = (u32) std::min<uint64_t>(value, 0xFFFFFFFFull);
         else if (option == HEIPA_OPT_HM_WORKERS) {

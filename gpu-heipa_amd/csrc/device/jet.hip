@@ -2800,18 +2800,20 @@ struct JetHost {
         launch(c, "jet_apply", 0.0, dim3(d.nreg), dim3(JB), 0, apply_groups_kernel<GG>, d);
     }
 
-    bool team_mode = false;
+    bool team_mode = false, wide = false;  // wide: the team spans all XCDs
     TeamArgs ta{};
     u32 team_next = 0;
     size_t team_lds = 0;
 
     void launch_team() {
-        if (team_next == TEAM_SLOTS) {
-            fill<u64>(c, (u64 *) ta.tc, TEAM_SLOTS * sizeof(TeamCtl) / 8, 0);
+        if (team_next == (wide ? WIDE_SLOTS : TEAM_SLOTS)) {
+            if (wide) fill<u64>(c, (u64 *) ta.wc, WIDE_SLOTS * sizeof(WideCtl) / 8, 0);
+            else fill<u64>(c, (u64 *) ta.tc, TEAM_SLOTS * sizeof(TeamCtl) / 8, 0);
             team_next = 0;
         }
         TeamArgs a = ta;
-        a.tc += team_next++;
+        if (wide) a.wc += team_next++;
+        else a.tc += team_next++;
         a.max_iters = TEAM_ITERS;
         if (d.D) launch_team_as<true>(a);
         else launch_team_as<false>(a);
@@ -2820,9 +2822,15 @@ struct JetHost {
     void launch_team_as(const TeamArgs &a) {
         JetDevT<true, MAP> dt;
         std::memcpy((void *) &dt, &d, sizeof(dt));
+        if (wide) {
+            const dim3 grid(a.want);
+            if (flat) launch(c, "jet_team", 0.0, grid, dim3(TM), team_lds, jet_team_kernel<true, MAP, true>, dt, a);
+            else launch(c, "jet_team", 0.0, grid, dim3(TM), team_lds, jet_team_kernel<false, MAP, true>, dt, a);
+            return;
+        }
         const dim3 grid(a.want * c.n_xcc);  // dispatched to the XCDs in turn: `want` on each
-        if (flat) launch(c, "jet_team", 0.0, grid, dim3(TM), team_lds, jet_team_kernel<true, MAP>, dt, a);
-        else launch(c, "jet_team", 0.0, grid, dim3(TM), team_lds, jet_team_kernel<false, MAP>, dt, a);
+        if (flat) launch(c, "jet_team", 0.0, grid, dim3(TM), team_lds, jet_team_kernel<true, MAP, false>, dt, a);
+        else launch(c, "jet_team", 0.0, grid, dim3(TM), team_lds, jet_team_kernel<false, MAP, false>, dt, a);
     }
 
     void iteration() {
@@ -2986,23 +2994,35 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         d.n_ratios = rt.n;
     }
     h.big_resolve = c.max_lds >= 160 * 1024;
-    // Team form: levels whose iterations are chains of latency.  Measured per
-    // iteration (RGG, k = 64) against the multi-launch form: 15 against 33 us
-    // at 3000 vertices, 21 against 34 at 30000, 42 against 37 at 100000 (one
-    // XCD's 32 compute units and 4 MB of L2 no longer suffice).  Dense levels
-    // do more work per vertex: R-MAT with 116 K edges takes 87 against 114 us,
-    // with 460 K edges 270 against 160.
+    // Team form on one XCD: levels whose iterations are chains of latency; on
+    // all XCDs: larger ones.  Measured, us per iteration (one XCD / all XCDs /
+    // multi-launch): RGG, k = 64, 8000 vertices 16.5 / 21.8 / 33, 16000 18.9 /
+    // 21.1 / 34, 30000 22.3 / 22.4 / 34, 60000 29.5 / 23.0 / 33, 500000 - / 38 /
+    // 45, 1000000 - / 57 / 55 (a wave per SIMD pair no longer hides the latency of
+    // a sweep that streams the level).  Skewed levels, k = 16: R-MAT of 400
+    // vertices and 3200 edges 42 / 46 / 61, 1000 and 8000 55 / 48 / 68, 16000 and
+    // 256000 274 / 104 / 132, 1000000 and 12 million - / 1150 / 1840.
     {
         const size_t cgb = conn_group_bytes(k);
         h.ta.wgroups = (u32) std::min<size_t>(WAVE / ROW, std::max<size_t>(1, TEAM_CONN_LDS / (cgb * TW)));
         h.team_lds = team_lds_bytes(k, h.ta.wgroups);
-        h.team_mode = !c.race && c.n_xcc && c.block_jet_max_n && h.team_lds + 2048 <= c.max_lds &&
-                      ((n <= c.team_jet_max_n && (u64) g.m <= 16ull * n) ||
-                       (n <= std::max(c.team_jet_max_n, c.block_jet_max_n) && (u64) g.m <= 32ull * c.block_jet_max_n));
-        if (h.team_mode) {
+        const bool teams = !c.race && c.n_xcc && c.block_jet_max_n && h.team_lds + 2048 <= c.max_lds;
+        h.flat = meta.max_deg > 8u * meta.G;  // skewed: a lane group per vertex would wait on the heaviest ones
+        const u64 dense = (h.flat ? 4ull : 32ull) * c.block_jet_max_n;
+        const bool narrow = (!h.flat && n <= c.team_jet_max_n && (u64) g.m <= 16ull * n) ||
+                            (n <= std::max(c.team_jet_max_n, c.block_jet_max_n) && (u64) g.m <= dense);
+        const u32 want = std::min<u32>({WIDE_MAX, (u32) c.num_cus, std::max<u32>(div_up(n, 64), div_up(g.m, 512u))});
+        if (teams && narrow) {
+            h.team_mode = true;
             h.ta.xcc = c.xcc;
             h.ta.want = std::min<u32>(TEAM_WANT, div_up(n, 64));
             h.ta.tc = bs.get<TeamCtl>(TEAM_SLOTS);  // cleared by the init launch
+        } else if (teams && c.n_xcc > 1 && c.wide_jet_max_n && (h.flat || n <= c.wide_jet_max_n) &&
+                   // its list regions; scratch that is short of eight times that keeps to the lists of the launches
+                   8 * (n + want * 2ull * TW * WAVE * TEAM_U) <= (c.arena.capacity() - c.arena.in_use()) / 8) {
+            h.team_mode = h.wide = true;
+            h.ta.want = want;
+            h.ta.wc = bs.get<WideCtl>(WIDE_SLOTS);
         }
     }
     // copies of the minibucket totals: about one per 64 sweep workgroups, at
@@ -3015,6 +3035,8 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
             s = 1;
         else if (c.bucket_copies)
             while (s * 2 <= c.bucket_copies) s *= 2;
+        else if (h.wide)
+            s = 8;  // an XCD's additions go to one copy
         else if (h.team_mode)
             while (s < 8 && (u64) s * 8192 < n) s *= 2;
         else
@@ -3027,7 +3049,6 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
     // k-counter array per group, so wide k shrinks the groups per workgroup and,
     // if one wave's groups do not fit, widens the groups
     h.G = cap_group(meta.G, c.group_cap);
-    h.flat = meta.max_deg > 8u * meta.G;  // skewed: a lane group per vertex would wait on the heaviest ones
     {
         const size_t cgb = conn_group_bytes(k);
         require(cgb <= SWEEP_LDS, "k too large for the LDS block-connectivity counters");
@@ -3062,8 +3083,10 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         d.cap = (u32) (div_up(n, (u64) d.nreg * per_block) * per_block);
         d.nreg = div_up(n, d.cap);
         d.cap_mv = d.cap + div_up(meta.n_hubs, d.nreg);
-        d.cand = bs.get<u32>((u64) d.nreg * d.cap);
-        d.moves = bs.get<u32>((u64) d.nreg * d.cap_mv);
+        u64 ent = 0;  // of a wide team's regions, however many members it has
+        if (h.wide) ent = (u64) n + (u64) h.ta.want * (TW * WAVE * TEAM_U + 1) + meta.n_hubs;
+        d.cand = bs.get<u32>(std::max((u64) d.nreg * d.cap, ent));
+        d.moves = bs.get<u32>(std::max((u64) d.nreg * d.cap_mv, ent));
         d.cand_n = bs.get<u32>(d.nreg);
         d.moves_n = bs.get<u32>(d.nreg);
         d.pstat = bs.get<unsigned long long>((u64) d.nreg * PT_COUNT);
@@ -3109,7 +3132,9 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         }
     }
     launch(c, "jet_init", 0.0, dim3(grid_for(c, std::max<u64>(n, wcnt_words / 4), 256, 8)), dim3(256), 0, jet_init_kernel, d, rt,
-           cut, maxw, (u32 *) h.ta.tc, h.ta.tc ? (u32) (TEAM_SLOTS * sizeof(TeamCtl) / 4) : 0u, wcnt_words);
+           cut, maxw, h.wide ? (u32 *) h.ta.wc : (u32 *) h.ta.tc,
+           h.wide ? (u32) (WIDE_SLOTS * sizeof(WideCtl) / 4) : h.team_mode ? (u32) (TEAM_SLOTS * sizeof(TeamCtl) / 4) : 0u,
+           wcnt_words);
     block_weights_add(c, g, part, k, d.bw);
     h.row_update_launches(1);  // init_BlockConn (jet:951)
 
@@ -3203,7 +3228,7 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
     c.event_pool.push_back(ev[0]);
     c.event_pool.push_back(ev[1]);
     if (s.save) copy_d2d(c, part, d.work, 4ull * n);
-    if (h.ta.tc) {
+    if (h.ta.tc || h.ta.wc) {
         prof_bytes(c, "jet_team", s.bytes[0] + s.bytes[1] + s.bytes[2] + s.bytes[3] + s.bytes[4]);
     } else {
         prof_bytes(c, "jet_sweep", s.bytes[0]);

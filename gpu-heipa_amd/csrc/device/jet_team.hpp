@@ -22,13 +22,14 @@ constexpr u32 TEAM_U = 2;                     // sweep tiles a wave has in fligh
 constexpr u32 TILE = WAVE * TEAM_U;           // vertices of one sweep step of a wave
 constexpr u32 TEAM_BUF = 2048;                // list entries a workgroup collects (edge-balanced form)
 constexpr u32 ROW_DEG = 2 * ROW;              // largest degree of the register form of a rebuild
+constexpr u32 LONG_DEG = 128;                 // degree from which a rebuild takes a whole wave
 constexpr size_t TEAM_CONN_LDS = 64 * 1024;   // block counters of the others, per workgroup
 constexpr u32 TEAM_BW = 1024;                 // blocks whose weight changes a workgroup sums in LDS
 
 struct TeamAcc {  // totals of the iteration in flight
     unsigned long long delta, mhash, ghash, miss, miss_deg, cand_deg, move_deg;
-    u32 ncand, nmoves, nrl, stall;
-    u32 pad[14];
+    u32 ncand, nmoves, nrl, stall, nextra;
+    u32 pad[13];
 };
 static_assert(sizeof(TeamAcc) == 128, "one line each");
 struct TeamCtl {  // zero before the launch
@@ -36,9 +37,16 @@ struct TeamCtl {  // zero before the launch
     TeamAcc acc[2];      // iteration i uses acc[i & 1] and clears the other
 };
 constexpr u32 TEAM_SLOTS = 16;  // launches between two clears
+struct WideCtl {  // zero before the launch
+    WideHead head;
+    TeamAcc acc[2][XCC_MAX];  // a copy per XCD; the resolve list's and its moves' lengths are in the first
+};
+constexpr u32 WIDE_SLOTS = 4;
+constexpr u32 WIDE_SHORT = 8;  // iterations of a launch whose team formed at less than half its size
 
 struct TeamArgs {
     TeamCtl *tc;
+    WideCtl *wc;
     const u32 *hubs, *chunk_hub, *chunk_idx;
     u32 n_hubs, n_chunks, xcc, want, max_iters;
     u32 wgroups;  // lane groups with block counters per wave
@@ -332,7 +340,17 @@ __device__ __forceinline__ u32 resolve_wave(const JD &d, bool strong, u32 stamp,
     return nmoves + (u32) __popcll(bal);
 }
 
-template<bool FLAT, bool MAP>
+// entries a wide team's member has room for in its list regions
+__host__ __device__ inline u32 wide_cap(u32 n, u32 members, u32 n_hubs) {
+    const u64 step = (u64) members * TW * WAVE * TEAM_U;
+    return (u32) ((((u64) n + step - 1) / step) * TW * WAVE * TEAM_U + (n_hubs + members - 1) / members);
+}
+
+// WIDE: a team over all XCDs, for levels that outgrow one.  Its lists stay with
+// the member that made them (regions of cand and moves, counted in LDS): one
+// list for all would cost an update of one address per wave (15 ns each, 2048
+// waves).  Totals have a copy per XCD.
+template<bool FLAT, bool MAP, bool WIDE>
 __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, TeamArgs ta) {
     extern __shared__ __align__(16) char smem[];
     constexpr u32 CW = (sizeof(JetCtl) + 7) / 8;
@@ -340,22 +358,41 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
     __shared__ u64 s_ctl[CW];
     __shared__ u64 s_red[TM / WAVE];
     __shared__ Best s_best[TM / WAVE];
-    __shared__ u32 s_join[2], s_ok, s_nmv, s_base;
-    if (xcc_id() != ta.xcc) return;
+    __shared__ u32 s_join[3], s_ok, s_nmv, s_base, s_cc, s_mc, s_rc, s_nm;
+    __shared__ unsigned long long s_delta;
+    if (!WIDE && xcc_id() != ta.xcc) return;
     u32 tid = threadIdx.x;
     TeamCtl *tc = ta.tc;
+    WideCtl *wc = ta.wc;
     if (tid < CW) s_ctl[tid] = ((const u64 *) dg.ctl)[tid];
     JetCtl *ctl = (JetCtl *) s_ctl;
     __syncthreads();
     if (!live(ctl)) return;
     u32 rank, T;
-    if (!team_join(&tc->head, ta.want, s_join, rank, T)) return;
-    TeamBar bar{tc->head.flag, rank, T, 0, &s_ok};
+    std::conditional_t<WIDE, WideBar, TeamBar> bar;
+    bool failed = false;
+    if constexpr (WIDE) {
+        if (!team_join<WIDE_MAX>(&wc->head, ta.want, s_join, rank, T)) return;
+        bar.h = &wc->head;
+        bar.ok = &s_ok;
+        __syncthreads();
+        failed = !wide_place(bar, T, s_join);
+        if (2 * T < ta.want && ta.max_iters > WIDE_SHORT) ta.max_iters = WIDE_SHORT;
+    } else {
+        if (!team_join(&tc->head, ta.want, s_join, rank, T)) return;
+        bar = TeamBar{tc->head.flag, rank, T, 0, &s_ok};
+    }
     JetDevT<true, MAP> d = dg;
     const bool do_hash = dg.trace != nullptr;
     if (rank) d.trace = nullptr;  // one member writes the trace
     d.ctl = ctl;
-    d.shard = rank % dg.nshard;
+    u32 xcd = 0;
+    if constexpr (WIDE) xcd = bar.x;
+    d.shard = (WIDE ? xcd : rank) % dg.nshard;
+    // this member's list regions
+    const u32 rcap = WIDE ? wide_cap(dg.n, T, ta.n_hubs) : 0u;
+    u32 *const cand_l = raw(dg.cand) + (u64) rank * rcap;
+    u32 *const move_l = WIDE ? dg.moves + (u64) rank * rcap : raw(dg.moves_x);
     s64 *s_bw = (s64 *) smem;
     d.bw = s_bw;
     RebShared *rs = (RebShared *) (smem + 8ull * d.k);
@@ -366,15 +403,15 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
     const size_t cgb = conn_group_bytes(d.k);
     const u32 NWV = T * TW;  // waves of the team
     // vertices per sweep tile: a whole wave's, fewer on levels that do not fill the team
-    const u32 tile = d.n >= NWV * WAVE ? WAVE : ((d.n + NWV - 1) / NWV + 15u) & ~15u;
-    bool failed = false;
+    const u32 tile = d.n >= NWV * WAVE ? WAVE : WIDE ? (d.n + NWV - 1) / NWV : ((d.n + NWV - 1) / NWV + 15u) & ~15u;
 #define TEAM_SYNC()             \
     if (!team_barrier(bar)) {   \
         failed = true;          \
         break;                  \
     }
-    for (u32 iter = 0; iter < ta.max_iters; ++iter) {
+    for (u32 iter = 0; iter < ta.max_iters && !failed; ++iter) {
         __syncthreads();  // the control step's block is complete
+        if (WIDE && tid == 0) s_cc = s_mc = s_rc = 0, s_delta = 0;
         const CtlHead hd = ctl_head(ctl);
         if (!live(hd)) break;
         // opaque per iteration: hoisting every per-thread address out of this
@@ -388,15 +425,22 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
         const bool save = __builtin_amdgcn_readfirstlane((int) hd.save) != 0, strong = mode == 2;
         const double ratio = hd.ratio;
         const s64 mbw = mode ? max_block_weight(d, strong) : 0;
-        TeamAcc *acc = &tc->acc[iter & 1];
+        TeamAcc *acc = WIDE ? &wc->acc[iter & 1][xcd] : &tc->acc[iter & 1];
+        TeamAcc *acc0 = WIDE ? &wc->acc[iter & 1][0] : acc;
+        u32 *const ncand = WIDE ? &s_cc : &acc->ncand, *const nmoves = WIDE ? &s_mc : &acc->nmoves;
+        if (WIDE) __syncthreads();
         const u32 rl = wl % ROW, rg = wl / ROW;
         // ---- sweep, each wave on its own
         {
             char *wm = um + cgb * ta.wgroups * TW + TEAM_WAVE_SWEEP * wid;
             u32 *list = (u32 *) wm, *lbeg = list + TILE, *linfo = lbeg + TILE;
-            WaveList<u32> wc{linfo + TILE, 0};
+            WaveList<u32> wl_c{linfo + TILE, 0};
             u64 nev = 0, degs = 0;
-            for (u64 t0 = (u64) gw * tile; t0 < d.n; t0 += (u64) NWV * tile * TEAM_U) {
+            // skewed levels keep their heavy vertices together (low numbers, and
+            // numbers with few bits set): there a wave's vertices lie far apart
+            u32 off = gw * tile + wl;
+            if (FLAT && WIDE) off = wl * NWV + (gw + wl * 37) % NWV;
+            for (u64 t0 = 0; t0 < d.n; t0 += (u64) NWV * tile * TEAM_U) {
                 // phase A, one vertex per lane, TEAM_U tiles in flight: cached
                 // decisions are taken (LP) or eligibility is tested
                 // (rebalancing); the vertices to rebuild go to the list, from
@@ -407,7 +451,7 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                 u8 lk[TEAM_U];
 #pragma unroll
                 for (u32 q = 0; q < TEAM_U; ++q) {
-                    const u64 v = t0 + (u64) q * NWV * tile + wl;
+                    const u64 v = t0 + (u64) q * NWV * tile + off;
                     in[q] = wl < tile && v < d.n;
                     vv[q] = (u32) v;
                     own[q] = in[q] ? (u32) d.work[v] : 0u;
@@ -470,7 +514,7 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
 #pragma unroll
                 for (u32 q = 0; q < TEAM_U; ++q) {
                     if (save && in[q]) d.part[vv[q]] = own[q];
-                    wc.add(cand[q], vv[q]);
+                    wl_c.add(cand[q], vv[q]);
                     const u32 deg = he[q] - hb[q];
                     const bool small = deg <= ROW_DEG && !(MAP && deg >= d.k);
                     const u32 info = own[q] << 16 | (lk[q] ? 1u << 15 : 0u) | deg;
@@ -499,9 +543,10 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                     }
                     const bool listed = row_eval(d, mode, mbw, rs, ratio, u, ub, info & 0x7FFFu, info >> 16,
                                                  (info >> 15) & 1u, rl, active);
-                    wc.add(listed, u);
+                    wl_c.add(listed, u);
                 }
-                // the others through LDS block counters, a row each
+                // the others through LDS block counters, a row each, then a wave
+                // each for the longest
                 if (nw) {
                     const u32 gi = rg;
                     const bool ingroup = gi < ta.wgroups;
@@ -511,18 +556,22 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                         if (rl == 0) *gc.tcount = 0;
                     }
                     wave_sync();
+                    bool longer = false;
                     for (u32 r0 = 0; r0 < nw; r0 += ta.wgroups) {
-                        const bool active = ingroup && r0 + gi < nw;
+                        const bool here = ingroup && r0 + gi < nw;
                         const u32 idx = TILE - 1 - (r0 + gi);
-                        const u32 u = active ? list[idx] : 0;
-                        const u32 ub = active ? lbeg[idx] : 0, info = active ? linfo[idx] : 0;
+                        const u32 u = here ? list[idx] : 0;
+                        const u32 ub = here ? lbeg[idx] : 0, info = here ? linfo[idx] : 0;
                         const u32 ow = info >> 16, deg = info & 0x7FFFu;
+                        const bool active = here && deg <= LONG_DEG;
+                        longer |= here && deg > LONG_DEG;
+                        if (!__any(active)) continue;
                         if (active) {
                             if (rl == 0) {
                                 nev++;
                                 degs += deg;
                             }
-                            conn_accumulate_range<2>(d, gc, ub, (u64) ub + deg, rl, ROW);
+                            conn_accumulate_range<4>(d, gc, ub, (u64) ub + deg, rl, ROW);
                         }
                         wave_sync();
                         const bool listed =
@@ -533,13 +582,34 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                         wave_sync();
                         if (active && rl == 0) *gc.tcount = 0;
                         wave_sync();
-                        wc.add(listed, u);
+                        wl_c.add(listed, u);
+                    }
+                    const GroupConn g0 = group_conn(um, d.k, wid * ta.wgroups);
+                    for (u32 r0 = 0; __any(longer) && r0 < nw; ++r0) {
+                        const u32 idx = TILE - 1 - r0, info = linfo[idx], deg = info & 0x7FFFu;
+                        if (deg <= LONG_DEG) continue;
+                        const u32 u = list[idx], ub = lbeg[idx], ow = info >> 16;
+                        if (wl == 0) {
+                            nev++;
+                            degs += deg;
+                        }
+                        conn_accumulate_range<8>(d, g0, ub, (u64) ub + deg, wl, WAVE);
+                        wave_sync();
+                        const bool listed =
+                            mode == 0 ? lp_eval<(int) WAVE>(d, g0, u, ow, (info >> 15) & 1u, wl, ratio, nullptr, nullptr, true)
+                                      : reb_eval<(int) WAVE>(d, strong, mbw, rs, g0, u, ow, wl, nullptr, nullptr, true);
+                        wave_sync();
+                        conn_reset(g0, *g0.tcount, wl, WAVE);
+                        wave_sync();
+                        if (wl == 0) *g0.tcount = 0;
+                        wave_sync();
+                        wl_c.add(listed, u);
                     }
                 }
-                wc.reserve(TILE, raw(d.cand), &acc->ncand);  // this step added at most TILE
+                wl_c.reserve(TILE, cand_l, ncand);  // this step added at most TILE
                 wave_sync();
             }
-            wc.flush(raw(d.cand), &acc->ncand);
+            wl_c.flush(cand_l, ncand);
             if (FLAT && ta.n_hubs) {  // hubs come with skewed degrees only
                 // the members' sweeps have read the hubs' caches: one member
                 // per hub now rebuilds or scores it
@@ -565,7 +635,7 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                         mode == 0
                             ? lp_eval<TM>(d, hc, u, own, locked, tid, ratio, s_best, (s64 *) s_red, true)
                             : reb_eval<TM>(d, strong, mbw, rs, hc, u, own, tid, s_best, (s64 *) s_red, true);
-                    if (listed) raw(d.cand)[atomicAdd(&acc->ncand, 1u)] = u;
+                    if (listed) cand_l[atomicAdd(ncand, 1u)] = u;
                     if (tid == 0) {
                         nev++;
                         degs += degree(d, u);
@@ -578,7 +648,12 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
             }
         }
         TEAM_SYNC();
-        if (rank == 0 && tid < sizeof(TeamAcc) / 8) ((u64 *) &tc->acc[(iter + 1) & 1])[tid] = 0;
+        if constexpr (WIDE) {
+            if (rank == 0 && tid < XCC_MAX * sizeof(TeamAcc) / 8) ((u64 *) &wc->acc[(iter + 1) & 1][0])[tid] = 0;
+            static_assert(XCC_MAX * sizeof(TeamAcc) / 8 <= TM, "one word per thread");
+        } else {
+            if (rank == 0 && tid < sizeof(TeamAcc) / 8) ((u64 *) &tc->acc[(iter + 1) & 1])[tid] = 0;
+        }
         // ---- minibucket prefixes, one wave per block range
         if (mode) {
             const u64 stride = (u64) d.t + 1;
@@ -619,7 +694,13 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
             TEAM_SYNC();
         }
         // ---- afterburner / classify
-        const u32 nc = (u32) __builtin_amdgcn_readfirstlane((int) dev_load(&acc->ncand));
+        // (the candidates of all members, or of this one)
+        u32 nc = (u32) __builtin_amdgcn_readfirstlane((int) (WIDE ? s_cc : dev_load(&acc->ncand)));
+        const DevPtr<u32> cl{cand_l};
+        if (WIDE && tid == 0 && nc) atomicAdd(&acc->ncand, nc);
+        // list i of the members' (one-XCD form) or of this member's own
+        const u32 lrank = WIDE ? 0u : rank, lsize = WIDE ? 1u : T;
+        const u32 lw = WIDE ? wid : gw, lwaves = WIDE ? TW : NWV;
         if (mode == 0) {
             u64 cdeg = 0, gh = 0;
             if constexpr (FLAT) {
@@ -627,25 +708,29 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                 u32 *s_mv = (u32 *) (um + 8ull * TEAM_BW + sizeof(FlatLds<TM>));
                 if (tid == 0) s_nmv = 0;
                 __syncthreads();
-                u32 cs = (nc + T - 1) / T;
+                u32 cs = (nc + lsize - 1) / lsize;
                 cs = cs < TM ? (cs ? cs : 1u) : (u32) TM;
-                for (u32 c0 = rank * cs; c0 < nc; c0 += T * cs) {
-                    afterburner_flat<TM>(d, stamp, d.cand, c0, nc - c0 < cs ? nc - c0 : cs, s_mv, &s_nmv, L, do_hash,
-                                         cdeg, gh);
-                    if (s_nmv + TM > TEAM_BUF) team_flush(s_mv, &s_nmv, &s_base, raw(d.moves_x), &acc->nmoves);
+                for (u32 c0 = lrank * cs; c0 < nc; c0 += lsize * cs) {
+                    const u32 cnt = nc - c0 < cs ? nc - c0 : cs;
+                    if constexpr (WIDE) {
+                        afterburner_flat<TM>(d, stamp, cl, c0, cnt, move_l, &s_mc, L, do_hash, cdeg, gh);
+                    } else {
+                        afterburner_flat<TM>(d, stamp, cl, c0, cnt, s_mv, &s_nmv, L, do_hash, cdeg, gh);
+                        if (s_nmv + TM > TEAM_BUF) team_flush(s_mv, &s_nmv, &s_base, move_l, nmoves);
+                    }
                 }
-                team_flush(s_mv, &s_nmv, &s_base, raw(d.moves_x), &acc->nmoves);
+                if constexpr (!WIDE) team_flush(s_mv, &s_nmv, &s_base, move_l, nmoves);
             } else {
                 WaveList<u32> wv{(u32 *) um + wid * WBUF, 0};
-                const u32 step = NWV * (WAVE / ROW);
-                u32 i = gw * (WAVE / ROW) + rg;
+                const u32 step = lwaves * (WAVE / ROW);
+                u32 i = lw * (WAVE / ROW) + rg;
                 u32 nxu = 0, nxb = 0, nxe = 0;
                 if (i < nc) {
-                    nxu = d.cand[i];
+                    nxu = cl[i];
                     nxb = d.xadj[nxu];
                     nxe = d.xadj[nxu + 1];
                 }
-                for (u32 i0 = gw * (WAVE / ROW); i0 < nc; i0 += step, i += step) {
+                for (u32 i0 = lw * (WAVE / ROW); i0 < nc; i0 += step, i += step) {
                     const bool active = i < nc && nxe - nxb <= d.hub_deg;
                     const u32 u = nxu, ub = nxb, ue = active ? nxe : nxb;
                     s64 ug = 0;
@@ -656,7 +741,7 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                         nn = d.dest[u];
                     }
                     if (i + step < nc) {
-                        nxu = d.cand[i + step];
+                        nxu = cl[i + step];
                         nxb = d.xadj[nxu];
                         nxe = d.xadj[nxu + 1];
                     }
@@ -673,9 +758,9 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                         }
                     }
                     wv.add(sel, u);
-                    wv.reserve(TILE, raw(d.moves_x), &acc->nmoves);
+                    wv.reserve(TILE, move_l, nmoves);
                 }
-                wv.flush(raw(d.moves_x), &acc->nmoves);
+                wv.flush(move_l, nmoves);
             }
             for (u32 h = rank; FLAT && h < ta.n_hubs; h += T) {
                 const u32 u = ta.hubs[h];
@@ -690,7 +775,7 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                         d.lock[u] = 1;
                         d.mark[u] = stamp;
                         d.oldp[u] = d.work[u];
-                        raw(d.moves_x)[atomicAdd(&acc->nmoves, 1u)] = u;
+                        move_l[atomicAdd(nmoves, 1u)] = u;
                     }
                 }
             }
@@ -699,45 +784,69 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
         } else {
             WaveList<u64> wr{(u64 *) um + wid * WBUF, 0};
             WaveList<u32> wv{(u32 *) (um + 8ull * WBUF * TW) + wid * WBUF, 0};
-            for (u32 i0 = gw * WAVE; i0 < nc; i0 += NWV * WAVE) {
+            for (u32 i0 = lw * WAVE; i0 < nc; i0 += lwaves * WAVE) {
                 const u32 i = i0 + wl;
-                const u32 u = i < nc ? (u32) d.cand[i] : 0u;
+                const u32 u = i < nc ? (u32) cl[i] : 0u;
                 u64 key = 0;
                 const Take take = i < nc ? classify_take(d, strong, stamp, u, key) : TAKE_NO;
                 wv.add(take == TAKE_SURE, u);
                 wr.add(take == TAKE_BOUNDARY, key);
-                wv.reserve(TILE, raw(d.moves_x), &acc->nmoves);
-                wr.reserve(TILE, raw(d.rlist), &acc->nrl);
+                wv.reserve(TILE, move_l, nmoves);
+                wr.reserve(TILE, raw(d.rlist), &acc0->nrl);
             }
-            wv.flush(raw(d.moves_x), &acc->nmoves);
-            wr.flush(raw(d.rlist), &acc->nrl);
+            wv.flush(move_l, nmoves);
+            if constexpr (WIDE) {  // one update of the shared counter per member
+                u32 base = 0;
+                if (wl == 0 && wr.cnt) base = atomicAdd(&s_rc, wr.cnt);
+                base = (u32) __builtin_amdgcn_readfirstlane((int) base);
+                __syncthreads();
+                if (tid == 0 && s_rc) s_base = atomicAdd(&acc0->nrl, s_rc);
+                __syncthreads();
+                if (s_rc)
+                    for (u32 i = wl; i < wr.cnt; i += WAVE) raw(d.rlist)[s_base + base + i] = wr.buf[i];
+            } else {
+                wr.flush(raw(d.rlist), &acc->nrl);
+            }
+        }
+        if constexpr (WIDE) {
+            __syncthreads();
+            if (tid == 0 && s_mc) atomicAdd(&acc->nmoves, s_mc);
         }
         TEAM_SYNC();
         // ---- resolve, by one member
         u32 L = 0;
         if (mode) {
-            L = (u32) __builtin_amdgcn_readfirstlane((int) dev_load(&acc->nrl));
+            L = (u32) __builtin_amdgcn_readfirstlane((int) dev_load(&acc0->nrl));
             if (L) {
                 if (rank == 0 && L <= WAVE && L <= d.rcap) {
                     if (wid == 0) {
-                        const u32 n2 = resolve_wave(d, strong, stamp, L, (s64 *) um, dev_load(&acc->nmoves));
-                        if (tid == 0) acc->nmoves = n2;
+                        const u32 n2 = resolve_wave(d, strong, stamp, L, (s64 *) um, WIDE ? 0u : dev_load(&acc->nmoves));
+                        if (tid == 0) (WIDE ? acc0->nextra : acc->nmoves) = n2;
                     }
                 } else if (rank == 0) {
-                    if (tid == 0) s_nmv = dev_load(&acc->nmoves);
+                    if (tid == 0) s_nmv = WIDE ? 0u : dev_load(&acc->nmoves);
                     __syncthreads();
                     const bool ok = resolve_body<TEAM_RCAP, TM>(d, strong, stamp, L, resolve_lds(um, TEAM_RCAP), &s_nmv);
                     __syncthreads();
                     if (tid == 0) {
-                        if (ok) acc->nmoves = s_nmv;
-                        else acc->stall = 1;
+                        if (ok) (WIDE ? acc0->nextra : acc->nmoves) = s_nmv;
+                        else acc0->stall = 1;
                     }
                 }
                 TEAM_SYNC();
-                if (dev_load(&acc->stall)) {
+                if (dev_load(&acc0->stall)) {
                     // the list does not fit: the host's global path and the
                     // multi-launch apply finish this iteration (the region
                     // lists are empty, the moves so far in the extra list)
+                    if constexpr (WIDE) {
+                        if (tid == 0 && s_mc) s_base = atomicAdd(&acc0->nextra, s_mc);
+                        __syncthreads();
+                        if (s_mc)
+                            for (u32 i = tid; i < s_mc; i += TM) raw(d.moves_x)[s_base + i] = dev_load(&move_l[i]);
+                        TEAM_SYNC();
+                        nc = 0;
+                        for (u32 x = 0; x < XCC_MAX; ++x) nc += dev_load(&wc->acc[iter & 1][x].ncand);
+                    }
                     if (rank == 0) {
                         for (u32 r = tid; r < d.nreg; r += TM) {
                             d.cand_n[r] = 0;
@@ -745,10 +854,15 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                         }
                         for (u64 j = tid; j < (u64) d.nreg * PT_COUNT; j += TM) d.pstat[j] = 0;
                         if (tid == 0) {
-                            ctl->st[ST_MISS] = dev_load(&acc->miss);
-                            ctl->st[ST_MISS_DEG] = dev_load(&acc->miss_deg);
+                            u64 miss = 0, miss_deg = 0;
+                            for (u32 x = 0; x < (WIDE ? XCC_MAX : 1u); ++x) {
+                                miss += dev_load(&acc0[x].miss);
+                                miss_deg += dev_load(&acc0[x].miss_deg);
+                            }
+                            ctl->st[ST_MISS] = miss;
+                            ctl->st[ST_MISS_DEG] = miss_deg;
                             ctl->st[ST_CAND] = nc;
-                            ctl->st[ST_MOVES] = dev_load(&acc->nmoves);
+                            ctl->st[ST_MOVES] = dev_load(WIDE ? &acc0->nextra : &acc->nmoves);
                             ctl->st[ST_RLIST] = L;
                             ctl->stalled = 1;
                         }
@@ -758,13 +872,16 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
             }
         }
         // ---- apply
-        const u32 nm = (u32) __builtin_amdgcn_readfirstlane((int) dev_load(&acc->nmoves));
+        // (the moves of all members, or of this one and then the resolve step's)
+        u32 nm = (u32) __builtin_amdgcn_readfirstlane((int) (WIDE ? s_mc : dev_load(&acc->nmoves)));
+        const u32 nx = WIDE && L ? (u32) __builtin_amdgcn_readfirstlane((int) dev_load(&acc0->nextra)) : 0u;
+        const DevPtr<u32> ml{move_l};
         {
             s64 delta = 0;
             u64 mdeg = 0, mh = 0;
             // block weight changes: summed per workgroup in LDS where a
             // workgroup has many moves, else added directly
-            const bool lds_bw = d.k <= TEAM_BW && (FLAT || nm >= 8 * T * TW);
+            const bool lds_bw = d.k <= TEAM_BW && (FLAT || nm >= 8 * lsize * TW);
             s64 *s_bwa = (s64 *) um;
             if (lds_bw)
                 for (u32 b = tid; b < d.k; b += TM) s_bwa[b] = 0;
@@ -772,25 +889,46 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
             s64 *bwt = lds_bw ? s_bwa : dg.bw;
             if constexpr (FLAT) {
                 FlatLds<TM> &L2 = *(FlatLds<TM> *) (um + 8ull * TEAM_BW);
-                u32 cs = (nm + T - 1) / T;
-                cs = cs < TM ? (cs ? cs : 1u) : (u32) TM;
-                for (u32 c0 = rank * cs; c0 < nm; c0 += T * cs)
-                    apply_flat<TM>(d, stamp, [&](u32 t) { return (u32) d.moves_x[c0 + t]; }, nm - c0 < cs ? nm - c0 : cs,
-                                   L2, do_hash, delta, mdeg, mh, bwt);
+                if constexpr (WIDE) {  // the own moves and a share of the others in one list
+                    const u32 xc = (nx + T - 1) / T, x0 = rank * xc < nx ? rank * xc : nx;
+                    const u32 all = nm + (x0 + xc < nx ? xc : nx - x0);
+                    for (u32 c0 = 0; c0 < all; c0 += TM)
+                        apply_flat<TM>(
+                            d, stamp,
+                            [&](u32 t) { return c0 + t < nm ? (u32) ml[c0 + t] : (u32) d.moves_x[x0 + (c0 + t - nm)]; },
+                            all - c0 < TM ? all - c0 : (u32) TM, L2, do_hash, delta, mdeg, mh, bwt);
+                } else {
+                    u32 cs = (nm + T - 1) / T;
+                    cs = cs < TM ? (cs ? cs : 1u) : (u32) TM;
+                    for (u32 c0 = rank * cs; c0 < nm; c0 += T * cs)
+                        apply_flat<TM>(d, stamp, [&](u32 t) { return (u32) ml[c0 + t]; }, nm - c0 < cs ? nm - c0 : cs, L2,
+                                       do_hash, delta, mdeg, mh, bwt);
+                }
             } else {
-                for (u32 i0 = gw * (WAVE / ROW); i0 < nm; i0 += NWV * (WAVE / ROW)) {
-                    const u32 i = i0 + rg;
+                // own moves first, then the others' by waves of the whole team
+                const u32 o4 = ((nm + 3) / 4 + lwaves - 1) / lwaves * lwaves;  // rounds of four, whole passes
+                const u32 x4 = WIDE ? (nx + 3) / 4 : 0u;
+                for (u32 r = lw;; r += lwaves) {
+                    if (!WIDE && r * (WAVE / ROW) >= nm) break;
+                    u32 i = r * (WAVE / ROW) + rg;
+                    bool has = i < nm;
+                    if (r >= o4) {
+                        const u32 xr = ((r - o4) / TW) * NWV + gw;
+                        if (xr >= x4) break;
+                        i = xr * (WAVE / ROW) + rg;
+                        has = i < nx;
+                    }
                     u32 u = 0, xb = 0, xe = 0, ou = 0, nu = 0;
                     s64 wu = 0;
-                    if (i < nm) {
-                        u = d.moves_x[i];
+                    if (has) {
+                        u = WIDE && r >= o4 ? (u32) d.moves_x[i] : (u32) ml[i];
                         xb = d.xadj[u];
                         xe = d.xadj[u + 1];
                         ou = d.oldp[u];
                         nu = d.dest[u];
                         wu = vwt(d, u);
                     }
-                    const bool mine = i < nm && xe - xb <= d.hub_deg;
+                    const bool mine = has && xe - xb <= d.hub_deg;
                     if (mine) delta += move_delta_pre<1>(d, ou, nu, xb, xe, rl, ROW, stamp);
                     if (mine && rl == 0) {
                         mdeg += xe - xb;
@@ -815,7 +953,7 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                 }
             }
             delta = wave_sum(delta);
-            if (wl == 0 && delta) atomicAdd(&acc->delta, (unsigned long long) delta);
+            if (wl == 0 && delta) atomicAdd(WIDE ? &s_delta : &acc->delta, (unsigned long long) delta);
             if (d.count_bytes) wave_add(&acc->move_deg, mdeg);
             if (do_hash) wave_add(&acc->mhash, mh);
             if (lds_bw) {
@@ -823,11 +961,25 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                 for (u32 b = tid; b < d.k; b += TM)
                     if (s_bwa[b]) atomicAdd((unsigned long long *) &dg.bw[b], (unsigned long long) s_bwa[b]);
             }
+            if constexpr (WIDE) {
+                __syncthreads();
+                if (tid == 0 && s_delta) atomicAdd(&acc->delta, s_delta);
+            }
         }
         // ---- control, the same step in every member, and the next
         // iteration's rebalance prologue, by the wave that saw the barrier end
         const bool ok = team_barrier(bar, [&] {
-            const s64 delta = (s64) dev_load(&acc->delta);
+            s64 delta;
+            if constexpr (WIDE) {  // the XCDs' totals, one per lane
+                const bool in = wl < XCC_MAX;
+                const TeamAcc *a = &wc->acc[iter & 1][in ? wl : 0];
+                delta = wave_sum(in ? (s64) dev_load(&a->delta) : 0);
+                nc = wave_sum(in ? dev_load(&a->ncand) : 0u);
+                nm = wave_sum(in ? dev_load(&a->nmoves) : 0u) + nx;
+                if (wl == 0) s_nm = nm;
+            } else {
+                delta = (s64) dev_load(&acc->delta);
+            }
             s64 mx = INT64_MIN;
             for (u32 b = wl; b < d.k; b += WAVE) {
                 const s64 w = dev_load(&dg.bw[b]);
@@ -841,12 +993,15 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                 for (u32 j = 0; j < PT_COUNT; ++j) t[j] = 0;
                 t[PT_DELTA] = (u64) delta;
                 if (d.count_bytes || do_hash) {
-                    t[PT_MISS] = dev_load(&acc->miss);
-                    t[PT_MISS_DEG] = dev_load(&acc->miss_deg);
-                    t[PT_CAND_DEG] = dev_load(&acc->cand_deg);
-                    t[PT_GHASH] = dev_load(&acc->ghash);
-                    t[PT_MOVE_DEG] = dev_load(&acc->move_deg);
-                    t[PT_MHASH] = dev_load(&acc->mhash);
+#pragma unroll 1
+                    for (u32 x = 0; x < (WIDE ? XCC_MAX : 1u); ++x) {
+                        t[PT_MISS] += dev_load(&acc0[x].miss);
+                        t[PT_MISS_DEG] += dev_load(&acc0[x].miss_deg);
+                        t[PT_CAND_DEG] += dev_load(&acc0[x].cand_deg);
+                        t[PT_GHASH] += dev_load(&acc0[x].ghash);
+                        t[PT_MOVE_DEG] += dev_load(&acc0[x].move_deg);
+                        t[PT_MHASH] += dev_load(&acc0[x].mhash);
+                    }
                 }
                 t[PT_COUNT] = nc;
                 t[PT_COUNT + 1] = nm;
@@ -861,6 +1016,7 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
             failed = true;
             break;
         }
+        if constexpr (WIDE) nm = (u32) __builtin_amdgcn_readfirstlane((int) s_nm);
         // ---- rows of the wide vertices next to the moves
         if (d.rflag && nm) {
             const u32 rmode = nm > d.n / 10 ? ROW_LARGE : ROW_SMALL;

@@ -25,6 +25,8 @@ constexpr int TM = 512;                       // threads of a team workgroup
 constexpr u32 TW = TM / WAVE;                 // its waves
 constexpr u32 TEAM_MAX = 64;                  // members: one wave polls all flags
 constexpr u32 TEAM_WANT = 32;                 // workgroups wanted: the compute units of an XCD
+constexpr u32 WIDE_MAX = 512;                 // members of a team over all XCDs
+constexpr u32 XCC_MAX = 16;
 constexpr u32 ROW = 16;                       // lanes of a DPP row
 constexpr u32 WBUF = 256;                     // list entries a wave collects before it appends them
 constexpr u32 TEAM_FROZEN = 0x80000000u;
@@ -35,6 +37,16 @@ struct TeamHead {  // zero before the launch
     u32 reg, pad0[31];   // registrations, then TEAM_FROZEN
     u32 size, pad1[31];  // members, set once
     u32 flag[TEAM_MAX];  // barrier round of each member
+};
+
+struct WideHead {  // of a team over all XCDs; zero before the launch
+    u32 reg, pad0[31];
+    u32 size, pad1[31];
+    u32 here, pad2[31];          // members that know their place on their XCD
+    u32 xreg[XCC_MAX][32];       // members of each XCD
+    u32 xdone[XCC_MAX][32];      // barrier round that all members of the XCD have reached
+    u32 xgo[XCC_MAX][32];        // barrier round that the XCD's members may leave
+    u32 flag[XCC_MAX][WIDE_MAX]; // barrier round of each member
 };
 
 // A pointer to device memory that other workgroups of the same launch write:
@@ -79,7 +91,8 @@ __device__ __forceinline__ void wave_sync() {
 // Registers this workgroup (all threads call it); false: it is not a member
 // (another XCD's turn is the caller's test).  The first to register closes the
 // list once `want` are there or 10 us have passed.  s: two LDS words.
-__device__ __forceinline__ bool team_join(TeamHead *h, u32 want, u32 *s, u32 &rank, u32 &size) {
+template<u32 MAX = TEAM_MAX, typename Head>
+__device__ __forceinline__ bool team_join(Head *h, u32 want, u32 *s, u32 &rank, u32 &size) {
     if (threadIdx.x == 0) {
         u32 sz = 0;
         const u32 r = __hip_atomic_fetch_add(&h->reg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -87,9 +100,9 @@ __device__ __forceinline__ bool team_join(TeamHead *h, u32 want, u32 *s, u32 &ra
             const u64 t0 = wall_clock64();
             while (dev_load(&h->reg) < want && wall_clock64() - t0 < TEAM_FORM_TICKS) __builtin_amdgcn_s_sleep(1);
             sz = __hip_atomic_fetch_or(&h->reg, TEAM_FROZEN, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            sz = sz < TEAM_MAX ? sz : TEAM_MAX;
+            sz = sz < MAX ? sz : MAX;
             __hip_atomic_store(&h->size, sz, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else if (r < TEAM_MAX) {  // not closed yet; the first member closes in bounded time
+        } else if (r < MAX) {  // not closed yet; the first member closes in bounded time
             const u64 t0 = wall_clock64();
             while ((sz = dev_load(&h->size)) == 0 && wall_clock64() - t0 < TEAM_WAIT_TICKS) __builtin_amdgcn_s_sleep(1);
         }
@@ -138,6 +151,99 @@ __device__ __forceinline__ bool team_barrier(TeamBar &b, F &&then) {
     return *b.ok != 0;
 }
 __device__ __forceinline__ bool team_barrier(TeamBar &b) {
+    return team_barrier(b, [] {});
+}
+
+// The barrier of a team over all XCDs.  Each XCD has an L2 of its own, so what
+// crosses XCDs goes past L2: the members of an XCD meet there first, its
+// leader (local rank 0) writes the L2 back (one fence for all of them: their
+// stores are in it), the leaders meet, each invalidates its L2, and the members
+// go on.  2.0 us for 256 workgroups on 8 XCDs, of which a launch boundary
+// (3.6 us from the last wave to the first of the next kernel) also pays the
+// write-back and the invalidate.  The loads that follow are device-scope ones
+// (DevPtr), as in the one-XCD form.
+struct WideBar {
+    WideHead *h;
+    u32 x, lr, xs;  // XCD, rank and members there
+    u32 xmask;      // XCDs with members
+    u32 round;
+    u32 *ok;  // LDS
+};
+
+template<typename P>
+__device__ __forceinline__ bool team_poll(P &&arrived) {
+    u64 t0 = 0;
+    for (u32 spin = 1; !__all(arrived()); ++spin) {
+        if ((spin & 1023u) == 0) {
+            if (t0 == 0) t0 = wall_clock64();
+            if (wall_clock64() - t0 > TEAM_WAIT_TICKS) return false;
+        }
+    }
+    return true;
+}
+
+// the member's place on its XCD, once the team is closed (all threads call it)
+__device__ __forceinline__ bool wide_place(WideBar &b, u32 size, u32 *s) {
+    b.x = xcc_id() % XCC_MAX;
+    b.round = 0;
+    if (threadIdx.x < WAVE) {
+        u32 lr = 0;
+        if (threadIdx.x == 0) {
+            lr = __hip_atomic_fetch_add(&b.h->xreg[b.x][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" : "+v"(lr)::"memory");
+            __hip_atomic_fetch_add(&b.h->here, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        const bool ok = team_poll([&] { return dev_load(&b.h->here) >= size; });
+        const u32 cnt = threadIdx.x < XCC_MAX ? dev_load(&b.h->xreg[threadIdx.x][0]) : 0u;
+        const u64 mask = __ballot(cnt != 0);
+        if (threadIdx.x == b.x) s[1] = cnt;
+        if (threadIdx.x == 0) {
+            s[0] = lr;
+            s[2] = (u32) mask;
+            *b.ok = ok;
+        }
+    }
+    __syncthreads();
+    b.lr = (u32) __builtin_amdgcn_readfirstlane((int) s[0]);
+    b.xs = (u32) __builtin_amdgcn_readfirstlane((int) s[1]);
+    b.xmask = (u32) __builtin_amdgcn_readfirstlane((int) s[2]);
+    return *b.ok != 0;
+}
+
+template<typename F>
+__device__ __forceinline__ bool team_barrier(WideBar &b, F &&then) {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // this wave's stores are in its XCD's L2
+    __syncthreads();
+    ++b.round;
+    if (threadIdx.x < WAVE) {
+        const u32 l = threadIdx.x;
+        bool ok = true;
+        if (l == 0)
+            __hip_atomic_store(&b.h->flag[b.x][b.lr], b.round, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (b.lr == 0) {
+            for (u32 m0 = 0; m0 < b.xs && ok; m0 += WAVE) {
+                const u32 *p = &b.h->flag[b.x][m0 + l < b.xs ? m0 + l : 0];
+                ok = team_poll([&] { return (s32) (dev_load(p) - b.round) >= 0; });
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            if (l == 0) __hip_atomic_store(&b.h->xdone[b.x][0], b.round, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const u32 *q = &b.h->xdone[l < XCC_MAX && (b.xmask >> l & 1u) ? l : b.x][0];
+            ok = ok && team_poll([&] { return (s32) (dev_load(q) - b.round) >= 0; });
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (l == 0 && ok)
+                __hip_atomic_store(&b.h->xgo[b.x][0], b.round, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        } else {
+            const u32 *q = &b.h->xgo[b.x][0];
+            ok = team_poll([&] { return (s32) (dev_load(q) - b.round) >= 0; });
+        }
+        if (l == 0) *b.ok = ok;
+        if (ok) then();
+    }
+    __syncthreads();
+    return *b.ok != 0;
+}
+__device__ __forceinline__ bool team_barrier(WideBar &b) {
     return team_barrier(b, [] {});
 }
 

@@ -35,6 +35,7 @@ OPT_GROUP_CAP = 12
 OPT_BLOCK_GROUP_CAP = 13
 OPT_REGION_EDGES = 14
 OPT_TEAM_JET = 15
+OPT_WIDE_JET = 16
 UNIFORM_VW, UNIFORM_EW = 1, 2
 
 u32p = ctypes.POINTER(ctypes.c_uint32)

@@ -257,9 +257,10 @@ int heipa_pool_hier_cache_stats(const heipa_pool *pool, uint64_t *entries, uint6
  * allows; 0 forces the device-wide path).  Results do not depend on it; tests use it to cover
  * both paths. */
 #define HEIPA_OPT_RESOLVE_CAP 1
-/* HEIPA_OPT_BLOCK_JET: levels of up to 32 * value edges (and max(value, HEIPA_OPT_TEAM_JET) vertices) run
- * whole Jet iterations in one launch, by a team of workgroups on one XCD, however dense they are
- * (default 2048; 0 forces the multi-launch form everywhere).  Results do not depend on it. */
+/* HEIPA_OPT_BLOCK_JET: levels of up to 32 * value edges (4 * value if the degrees are skewed) and
+ * max(value, HEIPA_OPT_TEAM_JET) vertices run whole Jet iterations in one launch, by a team of workgroups
+ * on one XCD, however dense they are (default 2048; 0 forces the multi-launch form everywhere).  Results
+ * do not depend on it. */
 #define HEIPA_OPT_BLOCK_JET 2
 /* HEIPA_OPT_GRAPHS: 1 (default) replays each level's batch of Jet iterations as a captured HIP graph;
  * 0 launches every kernel.  Results do not depend on it. */
@@ -317,10 +318,15 @@ int heipa_pool_hier_cache_stats(const heipa_pool *pool, uint64_t *entries, uint6
  * vertex per thread).  The row updates of wide vertices and the matching's repick passes size their
  * pieces the same way (the repick only while that adds workgroups).  Results do not depend on it. */
 #define HEIPA_OPT_REGION_EDGES 14
-/* HEIPA_OPT_TEAM_JET: the largest level (vertices) of at most 16 edges per vertex whose Jet runs as a team
- * of workgroups on one XCD, whole iterations per launch (default 65536; denser levels follow
- * HEIPA_OPT_BLOCK_JET, and HEIPA_OPT_BLOCK_JET 0 turns teams off).  Results do not depend on it. */
+/* HEIPA_OPT_TEAM_JET: the largest level (vertices) of at most 16 edges per vertex, without a skewed degree
+ * distribution, whose Jet runs as a team of workgroups on one XCD, whole iterations per launch (default
+ * 32768; denser levels follow HEIPA_OPT_BLOCK_JET, and HEIPA_OPT_BLOCK_JET 0 turns teams off).  Results do
+ * not depend on it. */
 #define HEIPA_OPT_TEAM_JET 15
+/* HEIPA_OPT_WIDE_JET: the largest level (vertices) beyond those that runs as a team over all XCDs, whole
+ * iterations per launch (default 1000000; levels with a skewed degree distribution of any size do; 0 and
+ * HEIPA_OPT_BLOCK_JET 0 turn it off).  Results do not depend on it. */
+#define HEIPA_OPT_WIDE_JET 16
 int heipa_ctx_set_option(heipa_ctx *ctx, int option, uint64_t value);
 /* dst uses src's hierarchy cache (HEIPA_OPT_HIER_CACHE) from now on: one cache for several contexts */
 int heipa_ctx_share_hier_cache(heipa_ctx *dst, const heipa_ctx *src);

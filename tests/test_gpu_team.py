@@ -111,6 +111,58 @@ def test_team_map_refine(team, name, hier):
     assert np.array_equal(heipa.to_numpy_u32(pd), op)
 
 
+@pytest.fixture
+def wide(ctx):
+    """Every level runs as a team over all XCDs."""
+    for opt, v in ((heipa.OPT_TEAM_JET, 0), (heipa.OPT_BLOCK_JET, 1), (heipa.OPT_WIDE_JET, 1 << 31)):
+        ctx.set_option(opt, v)
+    try:
+        yield ctx
+    finally:
+        for opt, v in WIDE_DEFAULTS:
+            ctx.set_option(opt, v)
+
+
+WIDE_DEFAULTS = ((heipa.OPT_TEAM_JET, 1 << 15), (heipa.OPT_BLOCK_JET, 2048), (heipa.OPT_WIDE_JET, 1000000))
+WIDE_CASES = dict(CASES,
+                  n131072=(lambda: heipa.gen_rgg(131072, 6.0, 3, 0), 12, 0.6, False),  # a vertex per lane of 2048 waves
+                  n131073=(lambda: heipa.gen_rgg(131073, 6.0, 3, 9), 65, 0.6, False),
+                  n270001=(lambda: heipa.gen_rgg(270001, 4.0, 3, 9), 5, 0.6, False))  # a second sweep step
+
+
+@pytest.mark.parametrize("name", sorted(WIDE_CASES))
+def test_wide_jet(wide, name):
+    make, k, skew, ultra = WIDE_CASES[name]
+    g = make()
+    part0 = _start(g, k, skew)
+    lmax = math.ceil(1.03 * g.g_weight / k)
+    cut0, maxw0 = orc.edge_cut(g, part0), int(block_weights(g, part0, k).max())
+    print(f"wide jet {name} n={g.n} m={g.m} k={k}", flush=True)
+    op, ocut, omaxw, otr = orc.jet_refine(g, part0, k, lmax, ultra, 1, cut0, maxw0, trace_cap=4096)
+    pd = heipa.from_numpy_u32(part0)
+    gcut, gmaxw, gtr = wide.jet_refine(_dev(g), pd, k, lmax, ultra, 1, cut0, maxw0, trace_cap=4096)
+    _compare(gtr, otr, name)
+    assert (gcut, gmaxw) == (ocut, omaxw)
+    assert np.array_equal(heipa.to_numpy_u32(pd), op)
+
+
+@pytest.mark.parametrize("cap", [0, 16])
+@pytest.mark.parametrize("name", ["n4095", "hubs", "skewed"])
+def test_wide_stall(wide, name, cap):
+    """Resolve lists beyond the LDS: the iteration ends on the device-wide path."""
+    wide.set_option(heipa.OPT_RESOLVE_CAP, cap)
+    try:
+        test_wide_jet(wide, name)
+    finally:
+        wide.set_option(heipa.OPT_RESOLVE_CAP, 1 << 32)
+
+
+@pytest.mark.parametrize("hier", ["4:8:6", "2:3"])
+@pytest.mark.parametrize("name", ["n64", "n16385", "deg33", "wide_k5", "hubs"])
+def test_wide_map_refine(wide, name, hier):
+    test_team_map_refine(wide, name, hier)
+
+
 def test_team_on_every_xcd():
     """Contexts use the device's XCDs in turn: nine of them, each its own team."""
     g = heipa.gen_rgg(3000, 8.0, 3, 9)
