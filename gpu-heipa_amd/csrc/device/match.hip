@@ -320,20 +320,170 @@ __global__ __launch_bounds__(256) void count_unmapped_kernel(const u32 *vcmap, u
     if (threadIdx.x == 0 && c) atomicAdd(out, c);
 }
 
+// ---- pairing of equal keys in one launch
+// Stable radix sort of (key, id) and the pairing of the sorted list.  Sorting
+// 64-bit digests takes 8 passes of three launches and the pairing four more,
+// about 16 us a pass however short the list; a team (team.hpp) takes about 4 us
+// a pass: member r counts and moves a contiguous share of the list, and every
+// member sums the counts of all for its own offsets.
+constexpr u32 PT_LIST = 1u << 16;  // longest list (a member's share is then 2048 entries)
+struct PairScratch {
+    u32 last[TEAM_MAX];          // 1 + the last group head of each member's share (0: none)
+    u32 counts[2][256 * TEAM_MAX];  // entries of each digit per member (digit-major), passes in turn
+};
+struct PairTeam {  // head, ran and failed zero before the launch
+    TeamHead head;
+    u32 ran, failed, pad[30];
+    PairScratch s;
+};
+struct PairLds {
+    u32 run[256], wcnt[TW][256], goff[256], red[TM / WAVE], carry;
+};
+// the members' part; keys[0] / vals[0] hold the list.  False: a member never
+// arrived at a barrier.
+template<typename K>
+__device__ __forceinline__ bool pair_team_body(TeamBar &bar, PairScratch *ps, PairLds &L, const DevPtr<K> (&keys)[2],
+                                               const DevPtr<u32> (&vals)[2], u32 len, u32 bits, DevPtr<u32> vcmap) {
+    const u32 rank = bar.rank, T = bar.size;
+    const u32 tid = threadIdx.x, wl = tid % WAVE, wid = tid / WAVE;
+    const u32 share = (len + T - 1) / T;
+    const u32 i0 = rank * share < len ? rank * share : len, i1 = len - i0 < share ? len : i0 + share;
+    bool failed = false, flip = false;
+    for (u32 shift = 0; shift < bits && !failed; shift += 8) {
+        const DevPtr<K> ik = keys[flip], ok = keys[!flip];
+        const DevPtr<u32> iv = vals[flip], ov = vals[!flip];
+        if (tid < 256) L.run[tid] = 0;
+        __syncthreads();
+        for (u32 i = i0 + tid; i < i1; i += TM) atomicAdd(&L.run[(u32) ((K) ik[i] >> shift) & 255u], 1u);
+        __syncthreads();
+        u32 *counts = ps->counts[(shift >> 3) & 1];
+        if (tid < 256) counts[tid * TEAM_MAX + rank] = L.run[tid];
+        failed = !team_barrier(bar);
+        if (failed) break;
+        // this member's first position of each digit
+        u32 tot = 0, before = 0;
+        if (tid < 256)
+            for (u32 m = 0; m < T; ++m) {
+                const u32 x = dev_load(&counts[tid * TEAM_MAX + m]);
+                before += m < rank ? x : 0u;
+                tot += x;
+            }
+        u32 all;
+        const u32 ex = block_exclusive_scan<TM>(tot, L.red, all);
+        const bool one_digit = __syncthreads_or(tot == len);  // nothing to move in this pass
+        if (tid < 256) {
+            L.goff[tid] = ex + before;
+            L.run[tid] = 0;
+        }
+        for (u32 d = tid; d < TW * 256; d += TM) ((u32 *) L.wcnt)[d] = 0;
+        __syncthreads();
+        if (one_digit) continue;  // the same in every member
+        for (u32 r0 = i0; r0 < i1; r0 += TM) {
+            const u32 i = r0 + tid;
+            const bool valid = i < i1;
+            const K key = valid ? (K) ik[i] : K(0);
+            const u32 val = valid ? (u32) iv[i] : 0u;
+            const u32 d = (u32) (key >> shift) & 255u;
+            u64 mask = __ballot(valid);  // the wave's lanes with the same digit
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const bool bit = (d >> b) & 1u;
+                const u64 bal = __ballot(bit);
+                mask &= bit ? bal : ~bal;
+            }
+            const u32 lower = (u32) __popcll(mask & lanemask_lt());
+            if (valid && lower == 0) L.wcnt[wid][d] = (u32) __popcll(mask);
+            __syncthreads();
+            if (valid) {
+                u32 pos = L.goff[d] + L.run[d] + lower;
+                for (u32 w = 0; w < wid; ++w) pos += L.wcnt[w][d];
+                ok[pos] = key;
+                ov[pos] = val;
+            }
+            __syncthreads();
+            if (tid < 256) {
+                u32 t = 0;
+#pragma unroll
+                for (u32 w = 0; w < TW; ++w) {
+                    t += L.wcnt[w][tid];
+                    L.wcnt[w][tid] = 0;
+                }
+                L.run[tid] += t;
+            }
+            __syncthreads();
+        }
+        failed = !team_barrier(bar);
+        flip = !flip;
+    }
+    // pair entries 2j and 2j + 1 of every group of equal keys
+    const DevPtr<K> sk = keys[flip];
+    const DevPtr<u32> sv = vals[flip];
+    if (!failed) {
+        u32 last = 0;
+        for (u32 i = i0 + tid; i < i1; i += TM)
+            if (i == 0 || (K) sk[i] != (K) sk[i - 1]) last = i + 1;
+        last = wave_max(last);
+        if (wl == 0) L.red[wid] = last;
+        __syncthreads();
+        if (tid == 0) {
+            for (u32 w = 1; w < TW; ++w) last = L.red[w] > last ? L.red[w] : last;
+            ps->last[rank] = last;
+        }
+        failed = !team_barrier(bar, [&] {
+            const u32 x = wl < rank ? dev_load(&ps->last[wl]) : 0u;
+            const u32 mx = wave_max(x);
+            if (wl == 0) L.carry = mx;
+        });
+    }
+    if (!failed) {
+        u32 carry = L.carry;  // 1 + the head of the group that runs into this share
+        for (u32 r0 = i0; r0 < i1; r0 += TM) {
+            const u32 i = r0 + tid;
+            const bool in = i < i1;
+            const K key = in ? (K) sk[i] : K(0);
+            const bool head = in && (i == 0 || (K) sk[i - 1] != key);
+            // the last head at or before i: within the wave, then of the waves before
+            const u64 hb = __ballot(head);
+            const u64 mine = hb & (lanemask_lt() | 1ull << wl);
+            u32 h = mine ? r0 + wid * WAVE + (63u - (u32) __builtin_clzll(mine)) + 1 : 0u;
+            __syncthreads();
+            if (wl == 0) L.red[wid] = hb ? r0 + wid * WAVE + (63u - (u32) __builtin_clzll(hb)) + 1 : 0u;
+            __syncthreads();
+            u32 best = carry;
+            for (u32 w = 0; w < TW; ++w) {
+                const u32 x = L.red[w];
+                if (w < wid && x > best) best = x;
+            }
+            if (!h) h = best;
+            for (u32 w = 0; w < TW; ++w) carry = L.red[w] > carry ? L.red[w] : carry;
+            if (in && i + 1 < len && ((i + 1 - h) & 1u) == 0 && (K) sk[i + 1] == key) {
+                const u32 a = sv[i], b = sv[i + 1];
+                const u32 cv = a < b ? a : b;
+                vcmap[a] = cv;
+                vcmap[b] = cv;
+            }
+        }
+    }
+    return !failed;
+}
+
 // ---- all remaining rounds in one launch
 // A round is eight sub-round phases and a repick over a list that shrinks fast:
 // as launches they cost 1.6 us of gap and a cold L2 each, about 32 us a round
 // however short the list.  A team of workgroups on one XCD (team.hpp) runs
 // them with barriers of 0.6 us, about 12 us a round at 16384 vertices, and
-// then counts the unmatched vertices and builds the mapping (unless more than
-// a quarter stay unmatched: the pairing passes are the host's).
-struct MatchTeam {  // zero before the launch, but len0
+// then the leaf, twin and relative passes while more than a quarter stay
+// unmatched, and builds the mapping.  As launches and waits of the host those
+// passes took 14 launches and 7 waits (12-15 us each) on every level of a
+// skewed graph, most of the time of a level of a few hundred vertices.
+struct MatchTeam {  // zero before the launch
     TeamHead head;
     u32 len[4], pad0[28];  // list lengths, a ring: round r reads len[r & 3]
-    u32 unmapped, pad1[31];
-    u32 nreps[TEAM_MAX];
+    u32 share[2][3][TEAM_MAX];  // representatives, unmatched vertices and leaves of each member's share
     // the result
-    u32 ran, rounds, failed, mapped, nc, un, pad2[26];
+    u32 ran, rounds, failed, mapped, nc;
+    u32 counted;  // un holds the unmatched after the rounds and after each of `passes` passes
+    u32 passes, un[4], pad2[21];
 };
 constexpr u32 MT_LIST = 1u << 16;   // longest list a team takes over
 constexpr u32 MT_EDGES = 1u << 20;  // most edges of a graph whose first round it takes
@@ -344,8 +494,99 @@ struct MatchTeamArgs {
     const u32 *list, *len_ptr;  // input of the first round (null: all vertices)
     u32 *lists[2];
     u32 *mapping;               // null: the host builds it
-    u32 seed, first_round, xcc, want;
+    u64 *keys[2];               // PT_LIST or n entries each; null: the passes are the host's
+    PairScratch *ps;
+    u32 seed, first_round, xcc, want, leaf_bits;
 };
+
+// relative key of an edge: neighbour of minimum degree, ties -> larger edge
+// weight, then first in adjacency order
+struct Rel {
+    u32 d;
+    s32 w;
+    u32 j, v;
+};
+__device__ __forceinline__ bool rel_better(const Rel &a, const Rel &b) {
+    if (a.j == SENT) return false;
+    if (b.j == SENT) return true;
+    if (a.d != b.d) return a.d < b.d;
+    if (a.w != b.w) return a.w > b.w;
+    return a.j < b.j;
+}
+template<int N>
+__device__ __forceinline__ void rel_ror(Rel &c) {
+    const Rel d{ror16<N>(c.d), ror16<N>(c.w), ror16<N>(c.j), ror16<N>(c.v)};
+    if (rel_better(d, c)) c = d;
+}
+__device__ __forceinline__ Rel rel_row(Rel c) {
+    rel_ror<8>(c);
+    rel_ror<4>(c);
+    rel_ror<2>(c);
+    rel_ror<1>(c);
+    return c;
+}
+template<bool UEW>
+__device__ __forceinline__ Rel rel_range(const DGraph &g, u32 b, u32 e, u32 lane, u32 stride) {
+    Rel best{SENT, 0, SENT, SENT};
+    for (u32 j = b + lane; j < e; j += stride) {
+        const u32 v = g.adj[j];
+        const Rel x{g.xadj[v + 1] - g.xadj[v], UEW ? 1 : g.ew[j], j, v};
+        if (rel_better(x, best)) best = x;
+    }
+    return best;
+}
+__device__ __forceinline__ u64 twin_range(const DGraph &g, u32 b, u32 e, u32 lane, u32 stride) {
+    u64 h = 0;
+    for (u32 j = b + lane; j < e; j += stride) {
+        const u64 y = pod_hash(g.adj[j]);
+        h += y * y + y;
+    }
+    return h;
+}
+
+// keys of the listed vertices, a row of lanes each, the longest a wave each
+template<bool UEW>
+__device__ __forceinline__ void team_keys(const DGraph &g, u32 pass, DevPtr<u32> list, u32 len, u64 *keys, u32 gw, u32 NWV) {
+    const u32 wl = lane_id(), rl = wl % ROW, rg = wl / ROW;
+    for (u32 i0 = gw * (WAVE / ROW); i0 < len; i0 += NWV * (WAVE / ROW)) {
+        const u32 i = i0 + rg;
+        u32 b = 0, e = 0;
+        if (i < len) {
+            const u32 u = list[i];
+            b = g.xadj[u];
+            e = g.xadj[u + 1];
+        }
+        if (pass == 0) {
+            if (i < len && rl == 0) ((u32 *) keys)[i] = g.adj[b];
+            continue;
+        }
+        const bool wide = e - b > MT_WAVE_DEG;
+        const u32 re = wide ? b : e;
+        if (pass == 1) {
+            const u64 h = row_sum(twin_range(g, b, re, rl, ROW));
+            if (i < len && !wide && rl == 0) keys[i] = h;
+        } else {
+            const Rel r = rel_row(rel_range<UEW>(g, b, re, rl, ROW));
+            if (i < len && !wide && rl == 0) ((u32 *) keys)[i] = r.v;
+        }
+        for (u64 left = __ballot(wide && rl == 0); left; left &= left - 1) {
+            const int l = __builtin_ctzll(left);
+            const u32 wb = lane_value(b, l), we = lane_value(e, l), wi = lane_value(i, l);
+            if (pass == 1) {
+                const u64 h = wave_sum(twin_range(g, wb, we, wl, WAVE));
+                if (wl == 0) keys[wi] = h;
+            } else {
+                Rel r = rel_row(rel_range<UEW>(g, wb, we, wl, WAVE));
+#pragma unroll
+                for (int q = 16; q < 64; q += 16) {
+                    const Rel o{lane_value(r.d, q), (s32) lane_value((u32) r.w, q), lane_value(r.j, q), lane_value(r.v, q)};
+                    if (rel_better(o, r)) r = o;  // of use in lane 0
+                }
+                if (wl == 0) ((u32 *) keys)[wi] = r.v;
+            }
+        }
+    }
+}
 
 // the best unmatched neighbour over edges b + lane, b + lane + stride, ...
 template<bool UEW>
@@ -379,7 +620,8 @@ __device__ __forceinline__ Cand cand_row(Cand c) {
 template<bool UEW, bool RACE>
 __global__ __launch_bounds__(TM) void match_team_kernel(DGraph g, DevPtr<u32> vcmap, DevPtr<u32> hn, DevPtr<u32> claim,
                                                         MatchTeamArgs ta) {
-    __shared__ u32 s_join[2], s_ok, s_sum;
+    __shared__ u32 s_join[2], s_ok, s_tot[3], s_before[3];
+    __shared__ PairLds s_pair;
     __shared__ u32 s_keep[TW][WBUF], s_work[TW][WAVE];
     __shared__ u32 s_red[TM / WAVE];
     if (xcc_id() != ta.xcc) return;
@@ -489,59 +731,101 @@ __global__ __launch_bounds__(TM) void match_team_kernel(DGraph g, DevPtr<u32> vc
         in_list = next;
         if (len == 0 || round >= 20000) break;
     }
-    u32 un = 0, mapped = 0, nc = 0;
+    u32 mapped = 0, nc = 0, pass = 0, counted = 0;
     if (!failed && len == 0 && ta.mapping) {
-        // ---- build_mapping: representatives in id order, a contiguous share each
         const u32 n = g.n, share = (n + T - 1) / T;
         const u32 v0 = rank * share < n ? rank * share : n, v1 = n - v0 < share ? n : v0 + share;
-        u32 reps = 0, unm = 0;
-        for (u32 v = v0 + tid; v < v1; v += TM) {
-            const u32 x = vcmap[v];
-            unm += x == SENT;
-            reps += x == SENT || x == v;
-        }
-        reps = block_sum<TM>(reps, s_red);
-        unm = block_sum<TM>(unm, s_red);
-        if (tid == 0) {
-            mt->nreps[rank] = reps;
-            if (unm) atomicAdd(&mt->unmapped, unm);
-        }
-        failed = !team_barrier(bar, [&] {
-            const u32 x = wl < T ? dev_load(&mt->nreps[wl]) : 0u;
-            const u32 before = wave_sum(wl < rank ? x : 0u);
-            if (wl == 0) s_sum = before;
-            nc = wave_sum(x);
-        });
-        un = dev_load(&mt->unmapped);
-        if (!failed && !((double) un / (double) n > 0.25)) {
-            const DevPtr<u32> map{ta.mapping};
-            u32 base = s_sum;
-            for (u32 t0 = v0; t0 < v1; t0 += TM) {
-                const u32 v = t0 + tid;
-                const u32 x = v < v1 ? (u32) vcmap[v] : 0u;
-                const bool is_rep = v < v1 && (x == SENT || x == v);
-                u32 tot;
-                const u32 ex = block_exclusive_scan<TM>(is_rep ? 1u : 0u, s_red, tot);
-                if (is_rep) {
-                    vcmap[v] = v;
-                    map[v] = base + ex;
-                }
-                base += tot;
+        for (;; ++pass) {
+            // representatives, unmatched vertices and leaves of this member's
+            // contiguous share, and of the shares before it
+            u32 reps = 0, unm = 0, leaves = 0;
+            for (u32 v = v0 + tid; v < v1; v += TM) {
+                const u32 x = vcmap[v];
+                unm += x == SENT;
+                reps += x == SENT || x == v;
+                if (pass == 0) leaves += x == SENT && g.xadj[v + 1] - g.xadj[v] == 1;
             }
-            failed = !team_barrier(bar);
-            if (!failed)
-                for (u32 v = v0 + tid; v < v1; v += TM) {
-                    const u32 x = vcmap[v];
-                    if (x != v) map[v] = map[x];
+            reps = block_sum<TM>(reps, s_red);
+            unm = block_sum<TM>(unm, s_red);
+            leaves = block_sum<TM>(leaves, s_red);
+            if (tid == 0) {
+                mt->share[pass & 1][0][rank] = reps;
+                mt->share[pass & 1][1][rank] = unm;
+                mt->share[pass & 1][2][rank] = leaves;
+            }
+            failed = !team_barrier(bar, [&] {
+#pragma unroll
+                for (u32 q = 0; q < 3; ++q) {
+                    const u32 x = wl < T ? dev_load(&mt->share[pass & 1][q][wl]) : 0u;
+                    const u32 before = wave_sum(wl < rank ? x : 0u), total = wave_sum(x);
+                    if (wl == 0) s_tot[q] = total, s_before[q] = before;
                 }
-            mapped = 1;
+            });
+            if (failed) break;
+            nc = s_tot[0];
+            const u32 un = s_tot[1];
+            if (rank == 0 && tid == 0) mt->un[pass] = un;
+            counted = 1;
+            const bool last = pass == 3 || !((double) un / (double) n > 0.25);
+            if (last) {
+                // ---- build_mapping: representatives in id order
+                const DevPtr<u32> map{ta.mapping};
+                u32 base = s_before[0];
+                for (u32 t0 = v0; t0 < v1; t0 += TM) {
+                    const u32 v = t0 + tid;
+                    const u32 x = v < v1 ? (u32) vcmap[v] : 0u;
+                    const bool is_rep = v < v1 && (x == SENT || x == v);
+                    u32 tot;
+                    const u32 ex = block_exclusive_scan<TM>(is_rep ? 1u : 0u, s_red, tot);
+                    if (is_rep) {
+                        vcmap[v] = v;
+                        map[v] = base + ex;
+                    }
+                    base += tot;
+                }
+                failed = !team_barrier(bar);
+                if (!failed)
+                    for (u32 v = v0 + tid; v < v1; v += TM) {
+                        const u32 x = vcmap[v];
+                        if (x != v) map[v] = map[x];
+                    }
+                mapped = 1;
+                break;
+            }
+            // ---- the next pass: vertices in id order, their keys, equal keys paired
+            const u32 pl = pass == 0 ? s_tot[2] : un;
+            if (!ta.keys[0] || pl > PT_LIST) break;
+            if (pl > 1) {
+                u32 base = s_before[pass == 0 ? 2 : 1];
+                for (u32 t0 = v0; t0 < v1; t0 += TM) {
+                    const u32 v = t0 + tid;
+                    const bool in = v < v1 && vcmap[v] == SENT && (pass != 0 || g.xadj[v + 1] - g.xadj[v] == 1);
+                    u32 tot;
+                    const u32 ex = block_exclusive_scan<TM>(in ? 1u : 0u, s_red, tot);
+                    if (in) ta.lists[0][base + ex] = v;
+                    base += tot;
+                }
+                if ((failed = !team_barrier(bar))) break;
+                const DevPtr<u32> vals[2] = {{ta.lists[0]}, {ta.lists[1]}};
+                team_keys<UEW>(g, pass, vals[0], pl, ta.keys[0], gw, NWV);
+                if ((failed = !team_barrier(bar))) break;
+                if (pass == 1) {
+                    const DevPtr<u64> keys[2] = {{ta.keys[0]}, {ta.keys[1]}};
+                    failed = !pair_team_body<u64>(bar, ta.ps, s_pair, keys, vals, pl, 64, vcmap);
+                } else {
+                    const DevPtr<u32> keys[2] = {{(u32 *) ta.keys[0]}, {(u32 *) ta.keys[1]}};
+                    failed = !pair_team_body<u32>(bar, ta.ps, s_pair, keys, vals, pl, pass == 0 ? ta.leaf_bits : 32u, vcmap);
+                }
+                if (failed || (failed = !team_barrier(bar))) break;
+            }
         }
     }
 #undef MT_SYNC
     if (failed && tid == 0) mt->failed = 1;
     if (rank == 0 && tid == 0) {
         mt->rounds = round + 1;
-        mt->un = un;
+        mt->counted = counted;
+        mt->passes = pass;
         mt->nc = nc;
         mt->mapped = mapped;
         mt->ran = 1;
@@ -679,19 +963,6 @@ __global__ void pair_kernel(const u32 *head, const u32 *gid_excl, const u32 *gst
     }
 }
 
-// ---- pairing of equal keys in one launch
-// Stable radix sort of (key, id) and the pairing of the sorted list.  Sorting
-// 64-bit digests takes 8 passes of three launches and the pairing four more,
-// about 16 us a pass however short the list; a team (team.hpp) takes about 4 us
-// a pass: member r counts and moves a contiguous share of the list, and every
-// member sums the counts of all for its own offsets.
-constexpr u32 PT_LIST = 1u << 16;  // longest list (a member's share is then 2048 entries)
-struct PairTeam {  // zero before the launch
-    TeamHead head;
-    u32 ran, failed, pad[30];
-    u32 last[TEAM_MAX];          // 1 + the last group head of each member's share (0: none)
-    u32 counts[2][256 * TEAM_MAX];  // entries of each digit per member (digit-major), passes in turn
-};
 template<typename K>
 struct PairTeamArgs {
     PairTeam *pt;
@@ -703,133 +974,15 @@ struct PairTeamArgs {
 
 template<typename K>
 __global__ __launch_bounds__(TM) void pair_team_kernel(PairTeamArgs<K> ta) {
-    __shared__ u32 s_join[2], s_ok, s_carry;
-    __shared__ u32 s_run[256], s_wcnt[TW][256], s_goff[256];
-    __shared__ u32 s_red[TM / WAVE];
+    __shared__ u32 s_join[2], s_ok;
+    __shared__ PairLds s_pair;
     if (xcc_id() != ta.xcc) return;
     PairTeam *pt = ta.pt;
     u32 rank, T;
     if (!team_join(&pt->head, ta.want, s_join, rank, T)) return;
     TeamBar bar{pt->head.flag, rank, T, 0, &s_ok};
-    const u32 tid = threadIdx.x, wl = tid % WAVE, wid = tid / WAVE;
-    const u32 share = (ta.len + T - 1) / T;
-    const u32 i0 = rank * share < ta.len ? rank * share : ta.len, i1 = ta.len - i0 < share ? ta.len : i0 + share;
-    bool failed = false, flip = false;
-    for (u32 shift = 0; shift < ta.bits && !failed; shift += 8) {
-        const DevPtr<K> ik = ta.keys[flip], ok = ta.keys[!flip];
-        const DevPtr<u32> iv = ta.vals[flip], ov = ta.vals[!flip];
-        if (tid < 256) s_run[tid] = 0;
-        __syncthreads();
-        for (u32 i = i0 + tid; i < i1; i += TM) atomicAdd(&s_run[(u32) ((K) ik[i] >> shift) & 255u], 1u);
-        __syncthreads();
-        u32 *counts = pt->counts[(shift >> 3) & 1];
-        if (tid < 256) counts[tid * TEAM_MAX + rank] = s_run[tid];
-        failed = !team_barrier(bar);
-        if (failed) break;
-        // this member's first position of each digit
-        u32 tot = 0, before = 0;
-        if (tid < 256)
-            for (u32 m = 0; m < T; ++m) {
-                const u32 x = dev_load(&counts[tid * TEAM_MAX + m]);
-                before += m < rank ? x : 0u;
-                tot += x;
-            }
-        u32 all;
-        const u32 ex = block_exclusive_scan<TM>(tot, s_red, all);
-        const bool one_digit = __syncthreads_or(tot == ta.len);  // nothing to move in this pass
-        if (tid < 256) {
-            s_goff[tid] = ex + before;
-            s_run[tid] = 0;
-        }
-        for (u32 d = tid; d < TW * 256; d += TM) ((u32 *) s_wcnt)[d] = 0;
-        __syncthreads();
-        if (one_digit) continue;  // the same in every member
-        for (u32 r0 = i0; r0 < i1; r0 += TM) {
-            const u32 i = r0 + tid;
-            const bool valid = i < i1;
-            const K key = valid ? (K) ik[i] : K(0);
-            const u32 val = valid ? (u32) iv[i] : 0u;
-            const u32 d = (u32) (key >> shift) & 255u;
-            u64 mask = __ballot(valid);  // the wave's lanes with the same digit
-#pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                const bool bit = (d >> b) & 1u;
-                const u64 bal = __ballot(bit);
-                mask &= bit ? bal : ~bal;
-            }
-            const u32 lower = (u32) __popcll(mask & lanemask_lt());
-            if (valid && lower == 0) s_wcnt[wid][d] = (u32) __popcll(mask);
-            __syncthreads();
-            if (valid) {
-                u32 pos = s_goff[d] + s_run[d] + lower;
-                for (u32 w = 0; w < wid; ++w) pos += s_wcnt[w][d];
-                ok[pos] = key;
-                ov[pos] = val;
-            }
-            __syncthreads();
-            if (tid < 256) {
-                u32 t = 0;
-#pragma unroll
-                for (u32 w = 0; w < TW; ++w) {
-                    t += s_wcnt[w][tid];
-                    s_wcnt[w][tid] = 0;
-                }
-                s_run[tid] += t;
-            }
-            __syncthreads();
-        }
-        failed = !team_barrier(bar);
-        flip = !flip;
-    }
-    // pair entries 2j and 2j + 1 of every group of equal keys
-    const DevPtr<K> sk = ta.keys[flip];
-    const DevPtr<u32> sv = ta.vals[flip];
-    if (!failed) {
-        u32 last = 0;
-        for (u32 i = i0 + tid; i < i1; i += TM)
-            if (i == 0 || (K) sk[i] != (K) sk[i - 1]) last = i + 1;
-        last = wave_max(last);
-        if (wl == 0) s_red[wid] = last;
-        __syncthreads();
-        if (tid == 0) {
-            for (u32 w = 1; w < TW; ++w) last = s_red[w] > last ? s_red[w] : last;
-            pt->last[rank] = last;
-        }
-        failed = !team_barrier(bar, [&] {
-            const u32 x = wl < rank ? dev_load(&pt->last[wl]) : 0u;
-            const u32 mx = wave_max(x);
-            if (wl == 0) s_carry = mx;
-        });
-    }
-    if (!failed) {
-        u32 carry = s_carry;  // 1 + the head of the group that runs into this share
-        for (u32 r0 = i0; r0 < i1; r0 += TM) {
-            const u32 i = r0 + tid;
-            const bool in = i < i1;
-            const K key = in ? (K) sk[i] : K(0);
-            const bool head = in && (i == 0 || (K) sk[i - 1] != key);
-            // the last head at or before i: within the wave, then of the waves before
-            const u64 hb = __ballot(head);
-            const u64 mine = hb & (lanemask_lt() | 1ull << wl);
-            u32 h = mine ? r0 + wid * WAVE + (63u - (u32) __builtin_clzll(mine)) + 1 : 0u;
-            __syncthreads();
-            if (wl == 0) s_red[wid] = hb ? r0 + wid * WAVE + (63u - (u32) __builtin_clzll(hb)) + 1 : 0u;
-            __syncthreads();
-            u32 best = carry;
-            for (u32 w = 0; w < TW; ++w) {
-                const u32 x = s_red[w];
-                if (w < wid && x > best) best = x;
-            }
-            if (!h) h = best;
-            for (u32 w = 0; w < TW; ++w) carry = s_red[w] > carry ? s_red[w] : carry;
-            if (in && i + 1 < ta.len && ((i + 1 - h) & 1u) == 0 && (K) sk[i + 1] == key) {
-                const u32 a = sv[i], b = sv[i + 1];
-                const u32 cv = a < b ? a : b;
-                ta.vcmap[a] = cv;
-                ta.vcmap[b] = cv;
-            }
-        }
-    }
+    const u32 tid = threadIdx.x;
+    const bool failed = !pair_team_body<K>(bar, &pt->s, s_pair, ta.keys, ta.vals, ta.len, ta.bits, DevPtr<u32>{ta.vcmap});
     if (failed && tid == 0) pt->failed = 1;
     if (rank == 0 && tid == 0) pt->ran = 1;
 }
@@ -974,6 +1127,17 @@ u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping
     u32 *lists[2] = {bs.get<u32>(n), bs.get<u32>(n)};
     u32 *lens = bs.get<u32>(64);  // ring of list lengths, one per round
     MatchTeam *mt = bs.get<MatchTeam>(1);
+    // buffers of the team's pairing passes, where they leave most of the scratch free
+    u64 *pkeys[2] = {nullptr, nullptr};
+    PairScratch *ps = nullptr;
+    {
+        const u64 ent = std::min(n, PT_LIST);
+        if (n <= MT_MAP && c.n_xcc && c.block_jet_max_n &&
+            8 * (16 * ent + sizeof(PairScratch)) <= c.arena.capacity() - c.arena.in_use()) {
+            for (u64 *&k: pkeys) k = bs.get<u64>(ent);
+            ps = bs.get<PairScratch>(1);
+        }
+    }
     const dim3 blk(256);
     launch(c, "match_init", 12.0 * n, dim3(grid_for(c, n, 256 * 4)), blk, 0, match_init_kernel, n, vcmap, hn, claim, lens,
            (u32 *) mt, (u32) (sizeof(MatchTeam) / 4));
@@ -1014,8 +1178,8 @@ u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping
         // over with the first list that fits one XCD
         if (team && len_bound <= MT_LIST && (round > 0 || g.m <= MT_EDGES)) {
             team = false;  // once per call
-            MatchTeamArgs a{mt, cur_list, cur_len, {lists[0], lists[1]}, n <= MT_MAP ? mapping : nullptr, seed, round, c.xcc,
-                            std::min<u32>(TEAM_WANT, div_up(len_bound, 64))};
+            MatchTeamArgs a{mt, cur_list, cur_len, {lists[0], lists[1]}, n <= MT_MAP ? mapping : nullptr, {pkeys[0], pkeys[1]},
+                            ps, seed, round, c.xcc, std::min<u32>(TEAM_WANT, div_up(len_bound, 64)), bits_for(n - 1)};
             const dim3 grid(a.want * c.n_xcc);
             const DevPtr<u32> pv{vcmap}, ph{hn}, pc{claim};
             launch(c, "match_team", 0.0, grid, dim3(TM), 0,
@@ -1087,17 +1251,29 @@ u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping
         prof_bytes(c, "match_repick", 4.0 * wb * (double) dsum + 4.0 * std::min<double>((double) dsum, n));
     }
 
+    u32 *scr = bs.get<u32>(4);
+    u32 unmapped = res.counted ? res.un[0] : count_unmapped(c, vcmap, n, scr);
+    st.after_hem = st.after_leaf = st.after_twin = st.after_relative = unmapped;
+    // the passes that the team has run
+    if (res.passes >= 1) {
+        st.ran_leaf = 1;
+        st.after_leaf = st.after_twin = st.after_relative = unmapped = res.un[1];
+    }
+    if (res.passes >= 2) {
+        st.ran_twin = 1;
+        st.after_twin = st.after_relative = unmapped = res.un[2];
+    }
+    if (res.passes >= 3) {
+        st.ran_relative = 1;
+        st.after_relative = unmapped = res.un[3];
+    }
     if (res.mapped) {
-        st.after_hem = st.after_leaf = st.after_twin = st.after_relative = res.un;
         if (stats) *stats = st;
         return res.nc;
     }
-    u32 *scr = bs.get<u32>(4);
-    u32 unmapped = res.ran && n <= MT_MAP ? res.un : count_unmapped(c, vcmap, n, scr);
-    st.after_hem = st.after_leaf = st.after_twin = st.after_relative = unmapped;
     u32 *plist = lists[0];
     u32 *plen = scr + 1;
-    if ((double) unmapped / (double) n > 0.25) {  // leaf
+    if (res.passes < 1 && (double) unmapped / (double) n > 0.25) {  // leaf
         st.ran_leaf = 1;
         LeafPred pred{vcmap, g.xadj};
         scan<u32>(c, "match_leaf_list", pred, CompactStore<LeafPred>{pred, plist}, n, plen);
@@ -1111,9 +1287,9 @@ u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping
             pair_by_key<u32>(c, keys, plist, len, bits_for(n - 1), vcmap);
         }
         unmapped = count_unmapped(c, vcmap, n, scr);
+        st.after_leaf = st.after_twin = st.after_relative = unmapped;
     }
-    st.after_leaf = st.after_twin = st.after_relative = unmapped;
-    if ((double) unmapped / (double) n > 0.25) {  // twin
+    if (res.passes < 2 && (double) unmapped / (double) n > 0.25) {  // twin
         st.ran_twin = 1;
         UnmappedPred pred{vcmap};
         scan<u32>(c, "match_twin_list", pred, CompactStore<UnmappedPred>{pred, plist}, n, plen);
@@ -1125,9 +1301,9 @@ u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping
             pair_by_key<u64>(c, keys, plist, len, 64, vcmap);
         }
         unmapped = count_unmapped(c, vcmap, n, scr);
+        st.after_twin = st.after_relative = unmapped;
     }
-    st.after_twin = st.after_relative = unmapped;
-    if ((double) unmapped / (double) n > 0.25) {  // relative
+    if (res.passes < 3 && (double) unmapped / (double) n > 0.25) {  // relative
         st.ran_relative = 1;
         UnmappedPred pred{vcmap};
         scan<u32>(c, "match_relative_list", pred, CompactStore<UnmappedPred>{pred, plist}, n, plen);

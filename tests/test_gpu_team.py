@@ -183,7 +183,18 @@ def _twins(leaves, groups):
     return csr_from_arrays(leaves + 2 * groups, np.concatenate([i + 2 * groups] * 2), np.concatenate([a, b]))
 
 
+def _bipartite(leaves, hubs, deg, seed):
+    """Vertices with `deg` random neighbours among `hubs` (of varied degree and edge weight)."""
+    rng = np.random.default_rng(seed)
+    v = np.concatenate([np.sort(rng.choice(hubs, deg, replace=False)) for _ in range(leaves)])
+    u = hubs + np.repeat(np.arange(leaves), deg)
+    return csr_from_arrays(hubs + leaves, u, v, 1 + (u + v) % 5)
+
+
 MATCH = {
+    "leaves": lambda: csr_from_arrays(9007, np.arange(7, 9007), np.arange(7, 9007) ** 2 % 7),  # all passes' first
+    "relatives": lambda: _bipartite(6000, 300, 3, 1),  # few twins, the rest by their smallest neighbour
+    "relatives_long": lambda: _bipartite(600, 140, 130, 2),  # keys by a wave each
     "twins": lambda: _twins(20000, 6),  # groups that span the members' shares
     "twins_many": lambda: _twins(5000, 1500),  # groups of 3 and 4
     "isolated": lambda: csr_from_arrays(40000, [0, 1], [1, 2]),  # one group of all but three
