@@ -19,9 +19,13 @@
 #include "eval.hpp"
 #include "../host/host_graph.hpp"
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <condition_variable>
+#include <deque>
 #include <exception>
+#include <mutex>
 #include <system_error>
 #include <thread>
 
@@ -177,6 +181,7 @@ __global__ void write_leaf_kernel(const u32 *n_to_o, const u32 *tmp, u32 n, u32 
         global[n_to_o[u]] = offset + tmp[u];
 }
 
+struct HMTeam;
 struct HMParams {
     std::vector<u32> hier, index_vec, k_rem;
     double eps;
@@ -185,6 +190,7 @@ struct HMParams {
     u64 seed;
     bool ultra;
     const GraphMeta *meta = nullptr;  // of the input graph
+    HMTeam *team = nullptr;           // the workers share the subtrees below the first split
 };
 
 // Builds child `id` of g (the vertices with tmp == id, their internal edges
@@ -242,6 +248,71 @@ bool build_child(Ctx &c, const DGraph &g, const u32 *tmp, const u32 *n_to_o, u32
 
 void hm_rec(Ctx &c, const DGraph &g, const u32 *n_to_o, u32 level, std::vector<u32> &ident, const HMParams &p,
             u32 *global);
+
+// The subtrees of a multisection that its workers share.  The subtrees of the
+// first split differ widely on skewed graphs (one worker was still busy when
+// the others had been idle for a fifth of the call), so a subtree's own
+// children are put up for every worker once its split is known.
+struct HMOwner {  // a subtree whose children are out
+    size_t left = 0;
+    std::exception_ptr err;
+};
+struct HMSub {
+    DGraph g;
+    const u32 *n_to_o;
+    u32 level;
+    std::vector<u32> ident;
+    HMOwner *owner;
+};
+struct HMTeam {
+    std::mutex m;
+    std::condition_variable cv;
+    std::deque<HMSub> subs;
+    size_t next_kid = 0, kids_open = 0;
+};
+
+// one child, on whatever worker; its owner learns of an error
+void hm_run_sub(Ctx &w, HMTeam &t, HMSub &sub, const HMParams &p, u32 *global) {
+    const size_t fd = w.arena.front_depth(), bd = w.arena.back_depth();
+    std::exception_ptr err;
+    try {
+        hm_rec(w, sub.g, sub.n_to_o, sub.level, sub.ident, p, global);
+        w.sync();
+    } catch (...) {
+        err = std::current_exception();
+        (void) hipStreamSynchronize(w.stream);
+        w.arena.release_back(bd);
+        w.arena.release_front(fd);
+    }
+    std::lock_guard<std::mutex> lk(t.m);
+    if (err && !sub.owner->err) sub.owner->err = err;
+    sub.owner->left--;
+    t.cv.notify_all();
+}
+
+// puts a subtree's children up and works (on them first) until they are done:
+// their graphs are in w's arena
+void hm_run_children(Ctx &w, HMTeam &t, std::vector<HMSub> &mine, HMOwner &o, const HMParams &p, u32 *global) {
+    std::unique_lock<std::mutex> lk(t.m);
+    o.left = mine.size();
+    for (HMSub &x: mine) t.subs.push_back(std::move(x));
+    t.cv.notify_all();
+    while (o.left) {
+        if (t.subs.empty()) {
+            t.cv.wait(lk);
+            continue;
+        }
+        auto it = std::find_if(t.subs.begin(), t.subs.end(), [&](const HMSub &x) { return x.owner == &o; });
+        if (it == t.subs.end()) it = t.subs.begin();
+        HMSub x = std::move(*it);
+        t.subs.erase(it);
+        lk.unlock();
+        hm_run_sub(w, t, x, p, global);
+        lk.lock();
+    }
+    lk.unlock();
+    if (o.err) std::rethrow_exception(o.err);
+}
 
 // Arena bytes of one child subtree's solve (the pool's job estimate for a
 // multisection of what remains of the hierarchy).
@@ -310,7 +381,8 @@ bool hm_split_parallel(Ctx &c, const DGraph &g, const u32 *tmp, const u32 *n_to_
             W.pop_back();
         }
     } else {
-        const size_t nw = std::min<size_t>(kids.size(), c.hm_workers);
+        // below the second split as many children as the hierarchy names
+        const size_t nw = std::min<size_t>(kids.size() * (level > 1 ? p.hier[level - 1] : 1u), c.hm_workers);
         u64 need = 0;
         for (const Kid &kd: kids) need = std::max(need, hm_child_bytes(kd.g, p, level - 1));
         if (c.hm_worker_bytes) need = c.hm_worker_bytes;
@@ -332,27 +404,55 @@ bool hm_split_parallel(Ctx &c, const DGraph &g, const u32 *tmp, const u32 *n_to_
         for (size_t i = 0; i < nw; ++i) W.push_back(c.workers[i].get());
     }
     const size_t nw = W.size();
-    // each worker's children one after another on its own stream
-    std::vector<std::exception_ptr> errors(nw);
-    std::vector<u8> done(kids.size(), 0);
-    auto run = [&](size_t wi) {
-        Ctx &w = *W[wi];
+    // the subtrees go to the workers largest first
+    std::vector<size_t> order(kids.size());
+    for (size_t i = 0; i < order.size(); ++i) order[i] = i;
+    std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return kids[x].g.m > kids[y].g.m; });
+    std::vector<std::exception_ptr> errors(kids.size());
+    std::vector<Ctx *> ran_on(kids.size(), nullptr);
+    HMTeam team;
+    team.kids_open = kids.size();
+    HMParams pt = p;
+    pt.team = nw > 1 ? &team : nullptr;
+    auto run_kid = [&](Ctx &w, size_t i) {
         const size_t fd = w.arena.front_depth(), bd = w.arena.back_depth();
+        ran_on[i] = &w;
         try {
-            HIP_CHECK(hipSetDevice(w.device));
-            if (&w != &c) ctx_copy_settings(w, c);
-            for (size_t i = wi; i < kids.size(); i += nw) {
-                std::vector<u32> ident{kids[i].id};
-                hm_rec(w, kids[i].g, kids[i].n_to_o, level - 1, ident, p, global);
-                w.sync();
-                done[i] = 1;
-            }
+            std::vector<u32> ident{kids[i].id};
+            hm_rec(w, kids[i].g, kids[i].n_to_o, level - 1, ident, pt, global);
+            w.sync();
         } catch (...) {
-            errors[wi] = std::current_exception();
+            errors[i] = std::current_exception();
             // the worker is reused by later calls: leave its arena as it was
             (void) hipStreamSynchronize(w.stream);
             w.arena.release_back(bd);
             w.arena.release_front(fd);
+        }
+    };
+    auto run = [&](size_t wi) {
+        Ctx &w = *W[wi];
+        (void) hipSetDevice(w.device);
+        if (&w != &c) ctx_copy_settings(w, c);
+        std::unique_lock<std::mutex> lk(team.m);
+        for (;;) {
+            if (!team.subs.empty()) {
+                HMSub x = std::move(team.subs.front());
+                team.subs.pop_front();
+                lk.unlock();
+                hm_run_sub(w, team, x, pt, global);
+                lk.lock();
+            } else if (team.next_kid < kids.size()) {
+                const size_t i = order[team.next_kid++];
+                lk.unlock();
+                run_kid(w, i);
+                lk.lock();
+                team.kids_open--;
+                team.cv.notify_all();
+            } else if (team.kids_open) {
+                team.cv.wait(lk);  // their children may still come up
+            } else {
+                break;
+            }
         }
     };
     std::vector<std::thread> threads;
@@ -368,22 +468,22 @@ bool hm_split_parallel(Ctx &c, const DGraph &g, const u32 *tmp, const u32 *n_to_
     for (size_t wi = 0; wi < nw; ++wi)
         if (W[wi] != &c) ctx_merge_prof(c, *W[wi]);
     HIP_CHECK(hipSetDevice(c.device));
-    // A worker whose arena (sized by the estimate) ran out hands its
-    // unfinished children back: they run one after another on c, whose arena
-    // is the caller's.  A child solved again rewrites the same output entries
-    // with the same values.  Any other error is the call's.
-    for (size_t wi = 0; wi < nw; ++wi) {
-        if (!errors[wi]) continue;
+    // A worker whose arena (sized by the estimate) ran out hands its subtree
+    // back: they run one after another on c, whose arena is the caller's.  A
+    // child solved again rewrites the same output entries with the same
+    // values.  Any other error is the call's.
+    for (size_t i = 0; i < kids.size(); ++i) {
+        if (!errors[i]) continue;
         try {
-            std::rethrow_exception(errors[wi]);
+            std::rethrow_exception(errors[i]);
         } catch (const Error &e) {
-            if (e.code != HEIPA_ERR_OOM || W[wi] == &c) throw;
+            if (e.code != HEIPA_ERR_OOM || (ran_on[i] == &c && nw == 1)) throw;
         }
-        for (size_t i = wi; i < kids.size(); i += nw) {
-            if (done[i]) continue;
-            std::vector<u32> ident{kids[i].id};
-            hm_rec(c, kids[i].g, kids[i].n_to_o, level - 1, ident, p, global);
-        }
+    }
+    for (size_t i = 0; i < kids.size(); ++i) {
+        if (!errors[i]) continue;
+        std::vector<u32> ident{kids[i].id};
+        hm_rec(c, kids[i].g, kids[i].n_to_o, level - 1, ident, p, global);
     }
     return true;
 }
@@ -408,6 +508,21 @@ void hm_rec(Ctx &c, const DGraph &g, const u32 *n_to_o, u32 level, std::vector<u
     }
     if (ident.empty() && level > 0 && (c.hm_workers > 1 || c.borrow) &&
         hm_split_parallel(c, g, tmp, n_to_o, level, p, global)) {
+        c.arena.release_front(depth0);
+        return;
+    }
+    if (p.team && ident.size() == 1) {
+        std::vector<HMSub> subs;
+        HMOwner owner;
+        for (u32 id = 0; id < k; ++id) {
+            DGraph child;
+            u32 *c_n_to_o = nullptr;
+            if (!build_child(c, g, tmp, n_to_o, id, child, c_n_to_o)) continue;
+            subs.push_back(HMSub{child, c_n_to_o, level - 1, {ident[0], id}, &owner});
+        }
+        c.sync();  // complete before other streams read them
+        std::stable_sort(subs.begin(), subs.end(), [](const HMSub &x, const HMSub &y) { return x.g.m > y.g.m; });
+        hm_run_children(c, *p.team, subs, owner, p, global);
         c.arena.release_front(depth0);
         return;
     }
