@@ -1596,6 +1596,82 @@ __device__ __forceinline__ void sort_keys_one_per_thread(Src src, u32 L, u32 P2,
     __syncthreads();
 }
 
+// Sort of keys g << 32 | u (u < 2^ubits, g < 2^gbits) in a[0, L) by NT threads:
+// least significant digits of 8 bits first, the buffers a and b in turn, the
+// result in a.  cnt: NT / WAVE * 128 words; the waves take contiguous chunks and
+// count two digits per word (at most 8192 entries).  A pass costs 1.5 us at 1000
+// entries and 3 at 8000, and 20 + 12 bits take five; the bitonic form took 38 us
+// for a list of 900 and 90 for one of 1900.
+template<int NT>
+__device__ __forceinline__ void sort_keys_lds(u64 *a, u64 *b, u32 *cnt, u32 L, u32 ubits, u32 gbits) {
+    constexpr u32 NW = NT / WAVE;
+    const u32 wl = lane_id(), wid = threadIdx.x / WAVE;
+    const u32 chunk = ((L + NW - 1) / NW + WAVE - 1) / WAVE * WAVE;
+    const u32 c0 = wid * chunk < L ? wid * chunk : L, c1 = L - c0 < chunk ? L : c0 + chunk;
+    u32 *wc = cnt + wid * 128;
+    bool odd = false;
+    for (u32 shift = 0; shift < 32 + gbits; shift = shift + 8 < ubits || shift >= 32 ? shift + 8 : 32u) {
+        for (u32 i = wl; i < 128; i += WAVE) wc[i] = 0;
+        wave_sync();
+        for (u32 i = c0 + wl; i < c1; i += WAVE) {
+            const u32 d = (u32) (a[i] >> shift) & 255u;
+            atomicAdd(&wc[d >> 1], 1u << ((d & 1u) * 16));
+        }
+        __syncthreads();
+        if (wid == 0) {  // first position of each digit of each wave
+            u32 tot[2];
+#pragma unroll
+            for (u32 q = 0; q < 2; ++q) {
+                u32 run = 0;
+#pragma unroll
+                for (u32 w = 0; w < NW; ++w) {
+                    const u32 x = cnt[w * 128 + 2 * wl + q];
+                    cnt[w * 128 + 2 * wl + q] = run;
+                    run += x;
+                }
+                tot[q] = run;
+            }
+            const u32 s0 = (tot[0] & 0xFFFFu) + (tot[0] >> 16), s1 = (tot[1] & 0xFFFFu) + (tot[1] >> 16);
+            u32 ex = wave_inclusive_scan(s0 + s1) - (s0 + s1);
+#pragma unroll
+            for (u32 q = 0; q < 2; ++q) {
+                const u32 p = ex | (ex + (tot[q] & 0xFFFFu)) << 16;
+#pragma unroll
+                for (u32 w = 0; w < NW; ++w) cnt[w * 128 + 2 * wl + q] += p;
+                ex += s0;
+            }
+        }
+        __syncthreads();
+        for (u32 i0 = c0; i0 < c1; i0 += WAVE) {
+            const u32 i = i0 + wl;
+            const bool in = i < c1;
+            const u64 key = in ? a[i] : 0;
+            const u32 d = (u32) (key >> shift) & 255u;
+            u64 mask = __ballot(in);  // the lanes with the same digit
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const bool bit = (d >> t) & 1u;
+                const u64 bal = __ballot(bit);
+                mask &= bit ? bal : ~bal;
+            }
+            const u32 lower = (u32) __popcll(mask & lanemask_lt());
+            if (in) b[(wc[d >> 1] >> ((d & 1u) * 16) & 0xFFFFu) + lower] = key;
+            wave_sync();
+            if (in && lower == 0) atomicAdd(&wc[d >> 1], (u32) __popcll(mask) << ((d & 1u) * 16));
+            wave_sync();
+        }
+        __syncthreads();
+        u64 *t = a;
+        a = b;
+        b = t;
+        odd = !odd;
+    }
+    if (odd) {
+        for (u32 i = threadIdx.x; i < L; i += NT) b[i] = a[i];
+        __syncthreads();
+    }
+}
+
 // Resolves a list of L entries with NT threads; false: the list (or the
 // strong overflow) does not fit and nothing was appended.  Moves go to the
 // extra move list, counted in LDS (`local_cnt`) or in st[ST_MOVES].
@@ -1615,7 +1691,11 @@ __device__ __forceinline__ bool resolve_body(const JD &d, bool strong, u32 stamp
     if (threadIdx.x == 0) ocount = 0;
     if (strong)
         for (u32 b = threadIdx.x; b < d.k; b += NT) d.evict_adjust[b] = 0;
-    if (P2 <= NT) {
+    if constexpr (JD::team) {
+        for (u32 i = threadIdx.x; i < L; i += NT) skey[i] = d.rlist[i];
+        __syncthreads();
+        sort_keys_lds<NT>(skey, (u64 *) soff, (u32 *) ssel, L, 32 - (u32) __builtin_clz(d.n), 32 - (u32) __builtin_clz(d.t | 1u));
+    } else if (P2 <= NT) {
         sort_keys_one_per_thread(d.rlist, L, P2, skey);
     } else {
     for (u32 i = threadIdx.x; i < P2; i += NT) skey[i] = i < L ? (u64) d.rlist[i] : ~0ull;
@@ -3005,7 +3085,8 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
     {
         const size_t cgb = conn_group_bytes(k);
         h.ta.wgroups = (u32) std::min<size_t>(WAVE / ROW, std::max<size_t>(1, TEAM_CONN_LDS / (cgb * TW)));
-        h.team_lds = team_lds_bytes(k, h.ta.wgroups);
+        h.team_lds = team_lds_bytes(k, h.ta.wgroups, TEAM_RCAP);
+        h.ta.rcap = TEAM_RCAP;
         const bool teams = !c.race && c.n_xcc && c.block_jet_max_n && h.team_lds + 2048 <= c.max_lds;
         h.flat = meta.max_deg > 8u * meta.G;  // skewed: a lane group per vertex would wait on the heaviest ones
         const u64 dense = (h.flat ? 4ull : 32ull) * c.block_jet_max_n;
@@ -3023,6 +3104,12 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
             h.team_mode = h.wide = true;
             h.ta.want = want;
             h.ta.wc = bs.get<WideCtl>(WIDE_SLOTS);
+            // one member per compute unit: its whole LDS for the resolve list
+            const size_t all = team_lds_bytes(k, h.ta.wgroups, RESOLVE_CAP);
+            if (all + 2048 <= c.max_lds) {
+                h.team_lds = all;
+                h.ta.rcap = RESOLVE_CAP;
+            }
         }
     }
     // copies of the minibucket totals: about one per 64 sweep workgroups, at
@@ -3044,7 +3131,7 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         d.nshard = s;
         d.btot = bs.get<s64>((u64) s * ((u64) d.t + 1));
     }
-    d.rcap = std::min<u32>(c.resolve_cap, h.big_resolve ? RESOLVE_CAP : RESOLVE_CAP_SMALL);
+    d.rcap = std::min<u32>(c.resolve_cap, h.team_mode ? h.ta.rcap : h.big_resolve ? RESOLVE_CAP : RESOLVE_CAP_SMALL);
     // lane-group geometry: G lanes per vertex; the sweep keeps one LDS
     // k-counter array per group, so wide k shrinks the groups per workgroup and,
     // if one wave's groups do not fit, widens the groups

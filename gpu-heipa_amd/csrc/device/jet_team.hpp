@@ -50,6 +50,7 @@ struct TeamArgs {
     const u32 *hubs, *chunk_hub, *chunk_idx;
     u32 n_hubs, n_chunks, xcc, want, max_iters;
     u32 wgroups;  // lane groups with block counters per wave
+    u32 rcap;     // resolve entries that fit the LDS
 };
 
 // the same for a workgroup (edge-balanced form; uniform over the workgroup)
@@ -71,8 +72,8 @@ __device__ __forceinline__ void team_flush(const u32 *buf, u32 *s_cnt, u32 *s_ba
 // rebalance prologue's result
 __host__ __device__ inline size_t team_union_off(u32 k) { return (8ull * k + 16 + 4ull * k + 15) & ~(size_t) 15; }
 constexpr size_t TEAM_WAVE_SWEEP = 12ull * TILE + 4ull * WBUF;
-__host__ inline size_t team_lds_bytes(u32 k, u32 wgroups) {
-    size_t u = std::max<size_t>(conn_group_bytes(k) * wgroups * TW + TEAM_WAVE_SWEEP * TW, resolve_lds_bytes(TEAM_RCAP));
+__host__ inline size_t team_lds_bytes(u32 k, u32 wgroups, u32 rcap) {
+    size_t u = std::max<size_t>(conn_group_bytes(k) * wgroups * TW + TEAM_WAVE_SWEEP * TW, resolve_lds_bytes(rcap));
     u = std::max<size_t>(u, 12ull * WBUF * TW);
     u = std::max<size_t>(u, 16ull * k + 8);
     u = std::max<size_t>(u, 8ull * TEAM_BW + sizeof(FlatLds<TM>) + 4ull * TEAM_BUF);
@@ -826,7 +827,7 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
                 } else if (rank == 0) {
                     if (tid == 0) s_nmv = WIDE ? 0u : dev_load(&acc->nmoves);
                     __syncthreads();
-                    const bool ok = resolve_body<TEAM_RCAP, TM>(d, strong, stamp, L, resolve_lds(um, TEAM_RCAP), &s_nmv);
+                    const bool ok = resolve_body<WIDE ? RESOLVE_CAP : TEAM_RCAP, TM>(d, strong, stamp, L, resolve_lds(um, ta.rcap), &s_nmv);
                     __syncthreads();
                     if (tid == 0) {
                         if (ok) (WIDE ? acc0->nextra : acc->nmoves) = s_nmv;
