@@ -2521,28 +2521,9 @@ __device__ __forceinline__ void row_update(const JD &d, u32 *wm, u32 u, u32 lane
     group_sync<G>();
 }
 
-// one flagged wide vertex of k <= 64 that is not a hub, by one thread, the
-// block mask in a register
+// the row of wide vertex v of k <= 64 from its block mask; f = rflag[v]
 template<typename JD>
-__device__ __forceinline__ void row_thread(const JD &d, u32 v, u32 rmode) {
-    const u8 f = d.rflag[v];
-    if ((f & 3u) != 3u) return;
-    u64 mask = 0;
-    if (f & 4u) {
-        if (rmode == ROW_INIT) return;  // the row kernel counts them
-        mask = row_count_mask(d, v);
-    } else {
-        const u32 xb = d.xadj[v], xe = d.xadj[v + 1];
-        if (xe - xb > ROW_THREAD_DEG) return;  // a hub
-        for (u32 j = xb; j < xe; j += 4) {
-            u32 nb[4];
-#pragma unroll
-            for (u32 q = 0; q < 4; ++q) nb[q] = j + q < xe ? d.adj[j + q] : 0u;
-#pragma unroll
-            for (u32 q = 0; q < 4; ++q)
-                if (j + q < xe) mask |= 1ull << (u32) d.work[nb[q]];
-        }
-    }
+__device__ __forceinline__ void row_finish(const JD &d, u32 v, u8 f, u64 mask, u32 rmode) {
     const u32 pc = (u32) __popcll(mask);
     const u32 r = d.wid[v];
     const u32 sz = d.wsz[r];
@@ -2564,6 +2545,31 @@ __device__ __forceinline__ void row_thread(const JD &d, u32 v, u32 rmode) {
     }
     d.wsz[r] = ns;
     d.rflag[v] = f & (u8) ~2u;
+}
+
+// one flagged wide vertex of k <= 64 that is not a hub, by one thread, the
+// block mask in a register
+template<typename JD>
+__device__ __forceinline__ void row_thread(const JD &d, u32 v, u32 rmode) {
+    const u8 f = d.rflag[v];
+    if ((f & 3u) != 3u) return;
+    u64 mask = 0;
+    if (f & 4u) {
+        if (rmode == ROW_INIT) return;  // the row kernel counts them
+        mask = row_count_mask(d, v);
+    } else {
+        const u32 xb = d.xadj[v], xe = d.xadj[v + 1];
+        if (xe - xb > ROW_THREAD_DEG) return;  // a hub, or not counted: the row kernel's
+        for (u32 j = xb; j < xe; j += 4) {
+            u32 nb[4];
+#pragma unroll
+            for (u32 q = 0; q < 4; ++q) nb[q] = j + q < xe ? d.adj[j + q] : 0u;
+#pragma unroll
+            for (u32 q = 0; q < 4; ++q)
+                if (j + q < xe) mask |= 1ull << (u32) d.work[nb[q]];
+        }
+    }
+    row_finish(d, v, f, mask, rmode);
 }
 
 // Wide vertices of k <= 64 that are not hubs, one thread each, the block
@@ -2606,10 +2612,10 @@ __global__ __launch_bounds__(JB) void row_kernel(JetDev d, u32 init, u32 piece) 
         for (u64 v0 = p0; v0 < p1; v0 += JB) {
             const u64 vv = v0 + threadIdx.x;
             bool take = false;
-            // k <= 64: the thread kernel takes the rest (the counted ones after init)
+            // k <= 64: the thread kernel takes the rest (those with kept counts after init)
             if (vv < p1 && (d.rflag[vv] & 3u) == 3u) {
                 const u32 dg = degree(d, (u32) vv);
-                take = dg <= d.hub_deg && (d.W > 2 || (init && dg > ROW_THREAD_DEG));
+                take = dg <= d.hub_deg && (d.W > 2 || ((init || !d.wcnt) && dg > ROW_THREAD_DEG));
             }
             append_local(take, (u32) vv, list, &s_nlist);
         }
@@ -2806,10 +2812,11 @@ struct WideDst {
     u32 *wid;
     u8 *rflag;
     u32 hub_deg;
+    bool count;  // keep counts (the launches do; a team walks the adjacencies again)
     __device__ void operator()(u64 u, u32 pos) const {
         const u32 deg = xadj[u + 1] - xadj[u];
         const bool w = deg >= k;
-        const bool counted = w && k <= 64 && deg > ROW_THREAD_DEG && deg <= hub_deg;
+        const bool counted = w && count && k <= 64 && deg > ROW_THREAD_DEG && deg <= hub_deg;
         wid[u] = w ? pos : ~0u;
         rflag[u] = w ? (counted ? 7 : 3) : 0;  // the init pass builds every wide row
     }
@@ -2850,7 +2857,7 @@ struct JetHost {
         if (!rows) return;
         if (d.W <= 2)
             launch(c, "jet_rows", 0.0, dim3(grid_for(c, d.n, JB, 8)), dim3(JB), 0, row_thread_kernel, d, init);
-        if (d.W > 2 || (init && meta.max_deg > ROW_THREAD_DEG)) HEIPA_DISPATCH_G(G, launch_rows, init);
+        if (d.W > 2 || ((init || !d.wcnt) && meta.max_deg > ROW_THREAD_DEG)) HEIPA_DISPATCH_G(G, launch_rows, init);
         if (meta.n_hubs)
             launch(c, "jet_rows_hub", 0.0, dim3(meta.n_hubs), dim3(JB), 4ull * d.W, row_hub_kernel, d,
                    (const u32 *) meta.hubs, init);
@@ -3200,7 +3207,7 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         d.rflag = bs.get<u8>(n);
         d.wid = bs.get<u32>(n);
         u32 *cnt = bs.get<u32>(1);
-        scan<u32>(c, "jet_init", WideSrc{g.xadj, k}, WideDst{g.xadj, k, d.wid, d.rflag, meta.hub_deg}, n, cnt);
+        scan<u32>(c, "jet_init", WideSrc{g.xadj, k}, WideDst{g.xadj, k, d.wid, d.rflag, meta.hub_deg, !h.team_mode}, n, cnt);
         // rows for the most wide vertices there can be (each has k edges): that
         // saves a wait of 12-15 us per level; where they would take more than an
         // eighth of the free scratch, the vertices are counted instead
@@ -3213,7 +3220,7 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         d.wsz = bs.get<u32>(nw);
         d.wV = bs.get<u32>(nw * d.W);
         d.wP = bs.get<u32>(nw * d.W);
-        if (d.W <= 2 && meta.max_deg > ROW_THREAD_DEG) {  // counts of the counted vertices
+        if (d.W <= 2 && meta.max_deg > ROW_THREAD_DEG && !h.team_mode) {  // counts of the counted vertices
             wcnt_words = nw * k;
             d.wcnt = bs.get<u32>(wcnt_words);
         }

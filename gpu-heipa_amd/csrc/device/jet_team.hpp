@@ -247,6 +247,37 @@ __device__ __forceinline__ s64 row_burn(const JD &d, u32 u, s64 ug, u32 o, u32 n
     return row_sum(change);
 }
 
+// the blocks (k <= 64) of the neighbours over edges [b, e), by the G = ROW or
+// WAVE lanes of a group
+template<u32 G, typename JD>
+__device__ __forceinline__ u64 row_blocks(const JD &d, u32 b, u32 e, u32 lane) {
+    u64 m = 0;
+    for (u32 j0 = b + lane; j0 < e; j0 += 8 * G) {
+        u32 v[8];
+#pragma unroll
+        for (u32 q = 0; q < 8; ++q) v[q] = e - j0 > q * G ? d.adj[j0 + q * G] : 0u;
+#pragma unroll
+        for (u32 q = 0; q < 8; ++q)
+            if (e - j0 > q * G) m |= 1ull << (u32) d.work[v[q]];
+    }
+    u32 lo = (u32) m, hi = (u32) (m >> 32);
+    lo |= ror16<8>(lo);
+    lo |= ror16<4>(lo);
+    lo |= ror16<2>(lo);
+    lo |= ror16<1>(lo);
+    if (d.k > 32) {
+        hi |= ror16<8>(hi);
+        hi |= ror16<4>(hi);
+        hi |= ror16<2>(hi);
+        hi |= ror16<1>(hi);
+    }
+    if (G == WAVE) {
+        lo = lane_value(lo, 0) | lane_value(lo, 16) | lane_value(lo, 32) | lane_value(lo, 48);
+        hi = lane_value(hi, 0) | lane_value(hi, 16) | lane_value(hi, 32) | lane_value(hi, 48);
+    }
+    return (u64) hi << 32 | lo;
+}
+
 // resolve_body for a list of L <= 64 entries (most lists) by one wave, entry i
 // in lane i: offsets inside a minibucket by comparing all pairs instead of a
 // sort, block tables in LDS (2k + 1 words at `lds`), no barrier.  Returns the
@@ -1022,7 +1053,39 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
         if (d.rflag && nm) {
             const u32 rmode = nm > d.n / 10 ? ROW_LARGE : ROW_SMALL;
             if (d.W <= 2) {
-                for (u64 v = (u64) rank * TM + tid; v < d.n; v += (u64) T * TM) row_thread(d, (u32) v, rmode);
+                // From the adjacencies, a lane, a row or a wave each by their
+                // length.  Counts kept by the moves (two updates of shared
+                // memory per edge of a moved vertex) made the apply step of a
+                // skewed level 50 us where most vertices move; walking the
+                // touched rows again is a gather per edge.
+                u32 *list = (u32 *) um + wid * TILE;
+                u32 off = gw * tile + wl;
+                if (FLAT && WIDE) off = wl * NWV + (gw + wl * 37) % NWV;
+                for (u64 t0 = 0; t0 < d.n; t0 += (u64) NWV * tile) {
+                    const u64 vv = t0 + off;
+                    const u32 v = (u32) vv;
+                    const bool flagged = wl < tile && vv < d.n && (d.rflag[v] & 3u) == 3u;
+                    const u32 deg = flagged ? degree(d, v) : 0u;
+                    const bool mid = deg > ROW_THREAD_DEG && deg <= 2 * LONG_DEG;
+                    const u64 bm = __ballot(mid);
+                    if (mid) list[(u32) __popcll(bm & lanemask_lt())] = v;
+                    if (flagged && deg <= ROW_THREAD_DEG) row_thread(d, v, rmode);
+                    wave_sync();
+                    const u32 nl = (u32) __popcll(bm);
+                    for (u32 r0 = 0; r0 < nl; r0 += WAVE / ROW) {
+                        const bool act = r0 + rg < nl;
+                        const u32 u = act ? list[r0 + rg] : 0u;
+                        const u32 xb = act ? d.xadj[u] : 0u, xe = act ? d.xadj[u + 1] : 0u;
+                        const u64 mask = row_blocks<ROW>(d, xb, xe, rl);
+                        if (act && rl == 0) row_finish(d, u, (u8) 3u, mask, rmode);
+                    }
+                    for (u64 left = __ballot(deg > 2 * LONG_DEG && deg <= d.hub_deg); left; left &= left - 1) {
+                        const u32 u = lane_value(v, __builtin_ctzll(left));
+                        const u64 mask = row_blocks<WAVE>(d, d.xadj[u], d.xadj[u + 1], wl);
+                        if (wl == 0) row_finish(d, u, (u8) 3u, mask, rmode);
+                    }
+                    wave_sync();
+                }
             } else {
                 // a wave per vertex, its block mask in LDS
                 u32 *wm = (u32 *) um + wid * (TILE + d.W), *list = wm + d.W;
