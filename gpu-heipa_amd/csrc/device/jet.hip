@@ -3103,7 +3103,7 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         if (teams && narrow) {
             h.team_mode = true;
             h.ta.xcc = c.xcc;
-            h.ta.want = std::min<u32>(TEAM_WANT, div_up(n, 64));
+            h.ta.want = std::min<u32>(TEAM_WANT, div_up(n, 16));  // a vertex or two per row of lanes
             h.ta.tc = bs.get<TeamCtl>(TEAM_SLOTS);  // cleared by the init launch
         } else if (teams && c.n_xcc > 1 && c.wide_jet_max_n && (h.flat || n <= c.wide_jet_max_n) &&
                    // its list regions; scratch that is short of eight times that keeps to the lists of the launches

@@ -435,7 +435,7 @@ __global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, Tea
     const size_t cgb = conn_group_bytes(d.k);
     const u32 NWV = T * TW;  // waves of the team
     // vertices per sweep tile: a whole wave's, fewer on levels that do not fill the team
-    const u32 tile = d.n >= NWV * WAVE ? WAVE : WIDE ? (d.n + NWV - 1) / NWV : ((d.n + NWV - 1) / NWV + 15u) & ~15u;
+    const u32 tile = d.n >= NWV * WAVE ? WAVE : WIDE ? (d.n + NWV - 1) / NWV : ((d.n + NWV - 1) / NWV + 3u) & ~3u;
 #define TEAM_SYNC()             \
     if (!team_barrier(bar)) {   \
         failed = true;          \
