@@ -191,7 +191,7 @@ struct Ctx {
     u32 group_cap = 64;         // HEIPA_OPT_GROUP_CAP
     u32 region_edges = 1024;    // HEIPA_OPT_REGION_EDGES
     u32 team_jet_max_n = 1u << 15;  // HEIPA_OPT_TEAM_JET
-    u32 wide_jet_max_n = 1000000;   // HEIPA_OPT_WIDE_JET
+    u32 wide_jet_max_n = ~0u;       // HEIPA_OPT_WIDE_JET
     u32 n_xcc = 0, xcc = 0;  // XCDs of the device (0: unknown), the one this context's teams use
     bool use_graphs = true;  // HEIPA_OPT_GRAPHS
     u32 bucket_copies = 0;   // HEIPA_OPT_BUCKET_COPIES (0: automatic)

@@ -2887,7 +2887,7 @@ struct JetHost {
         launch(c, "jet_apply", 0.0, dim3(d.nreg), dim3(JB), 0, apply_groups_kernel<GG>, d);
     }
 
-    bool team_mode = false, wide = false;  // wide: the team spans all XCDs
+    bool team_mode = false, wide = false, twice = false;  // wide: the team spans all XCDs, twice: two members per compute unit
     TeamArgs ta{};
     u32 team_next = 0;
     size_t team_lds = 0;
@@ -2911,7 +2911,8 @@ struct JetHost {
         std::memcpy((void *) &dt, &d, sizeof(dt));
         if (wide) {
             const dim3 grid(a.want);
-            if (flat) launch(c, "jet_team", 0.0, grid, dim3(TM), team_lds, jet_team_kernel<true, MAP, true>, dt, a);
+            if (twice) launch(c, "jet_team", 0.0, grid, dim3(TM), team_lds, jet_team_kernel<false, MAP, true, 2>, dt, a);
+            else if (flat) launch(c, "jet_team", 0.0, grid, dim3(TM), team_lds, jet_team_kernel<true, MAP, true>, dt, a);
             else launch(c, "jet_team", 0.0, grid, dim3(TM), team_lds, jet_team_kernel<false, MAP, true>, dt, a);
             return;
         }
@@ -3084,11 +3085,10 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
     // Team form on one XCD: levels whose iterations are chains of latency; on
     // all XCDs: larger ones.  Measured, us per iteration (one XCD / all XCDs /
     // multi-launch): RGG, k = 64, 8000 vertices 16.5 / 21.8 / 33, 16000 18.9 /
-    // 21.1 / 34, 30000 22.3 / 22.4 / 34, 60000 29.5 / 23.0 / 33, 500000 - / 38 /
-    // 45, 1000000 - / 57 / 55 (a wave per SIMD pair no longer hides the latency of
-    // a sweep that streams the level).  Skewed levels, k = 16: R-MAT of 400
-    // vertices and 3200 edges 42 / 46 / 61, 1000 and 8000 55 / 48 / 68, 16000 and
-    // 256000 274 / 104 / 132, 1000000 and 12 million - / 1150 / 1840.
+    // 21.1 / 34, 30000 22.3 / 22.4 / 34, 60000 29.5 / 23.0 / 33, 500000 - / 37 /
+    // 45, 1000000 - / 47 / 50, 3000000 - / 130 / 135.  Skewed levels, k = 16:
+    // R-MAT of 400 vertices and 3200 edges 42 / 46 / 61, 1000 and 8000 55 / 48 /
+    // 68, 16000 and 256000 274 / 104 / 132, 1000000 and 12 million - / 1150 / 1840.
     {
         const size_t cgb = conn_group_bytes(k);
         h.ta.wgroups = (u32) std::min<size_t>(WAVE / ROW, std::max<size_t>(1, TEAM_CONN_LDS / (cgb * TW)));
@@ -3105,15 +3105,22 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
             h.ta.xcc = c.xcc;
             h.ta.want = std::min<u32>(TEAM_WANT, div_up(n, 16));  // a vertex or two per row of lanes
             h.ta.tc = bs.get<TeamCtl>(TEAM_SLOTS);  // cleared by the init launch
-        } else if (teams && c.n_xcc > 1 && c.wide_jet_max_n && (h.flat || n <= c.wide_jet_max_n) &&
+        } else if (teams && c.n_xcc > 1 && n <= c.wide_jet_max_n &&
                    // its list regions; scratch that is short of eight times that keeps to the lists of the launches
                    8 * (n + want * 2ull * TW * WAVE * TEAM_U) <= (c.arena.capacity() - c.arena.in_use()) / 8) {
             h.team_mode = h.wide = true;
             h.ta.want = want;
             h.ta.wc = bs.get<WideCtl>(WIDE_SLOTS);
-            // one member per compute unit: its whole LDS for the resolve list
-            const size_t all = team_lds_bytes(k, h.ta.wgroups, RESOLVE_CAP);
-            if (all + 2048 <= c.max_lds) {
+            // one member per compute unit: its whole LDS for the resolve list;
+            // two where one per unit would take a second sweep step (regular
+            // levels only: skewed ones have long resolve lists)
+            const size_t all = team_lds_bytes(k, h.ta.wgroups, RESOLVE_CAP), half = team_lds_bytes(k, h.ta.wgroups, 2048);
+            if (!h.flat && n > (u64) c.num_cus * TW * WAVE && 2 * (half + 2048) <= c.max_lds) {
+                h.twice = true;
+                h.team_lds = half;
+                h.ta.rcap = 2048;
+                h.ta.want = std::min<u32>(WIDE_MAX, 2 * (u32) c.num_cus);
+            } else if (all + 2048 <= c.max_lds) {
                 h.team_lds = all;
                 h.ta.rcap = RESOLVE_CAP;
             }

@@ -381,9 +381,12 @@ __host__ __device__ inline u32 wide_cap(u32 n, u32 members, u32 n_hubs) {
 // WIDE: a team over all XCDs, for levels that outgrow one.  Its lists stay with
 // the member that made them (regions of cand and moves, counted in LDS): one
 // list for all would cost an update of one address per wave (15 ns each, 2048
-// waves).  Totals have a copy per XCD.
-template<bool FLAT, bool MAP, bool WIDE>
-__global__ __launch_bounds__(TM) void jet_team_kernel(JetDevT<true, MAP> dg, TeamArgs ta) {
+// waves).  Totals have a copy per XCD.  PER_CU 2: two members per compute unit,
+// 128 registers each (26 spilled), for levels whose sweep takes one member per
+// unit several steps: us per iteration with one / two, RGG, 300000 vertices
+// 31.6 / 29.4, 1000000 51.4 / 47.0, 1500000 48.7 / 41.4, 3000000 151 / 130.
+template<bool FLAT, bool MAP, bool WIDE, int PER_CU = 1>
+__global__ __launch_bounds__(TM, PER_CU == 2 ? 4 : 1) void jet_team_kernel(JetDevT<true, MAP> dg, TeamArgs ta) {
     extern __shared__ __align__(16) char smem[];
     constexpr u32 CW = (sizeof(JetCtl) + 7) / 8;
     static_assert(CW <= TM && sizeof(JetCtl) % 8 == 0, "control block copy");

@@ -324,8 +324,8 @@ int heipa_pool_hier_cache_stats(const heipa_pool *pool, uint64_t *entries, uint6
  * not depend on it. */
 #define HEIPA_OPT_TEAM_JET 15
 /* HEIPA_OPT_WIDE_JET: the largest level (vertices) beyond those that runs as a team over all XCDs, whole
- * iterations per launch (default 1000000; levels with a skewed degree distribution of any size do; 0 and
- * HEIPA_OPT_BLOCK_JET 0 turn it off).  Results do not depend on it. */
+ * iterations per launch (default: any; 0 and HEIPA_OPT_BLOCK_JET 0 turn it off).  Results do not depend
+ * on it. */
 #define HEIPA_OPT_WIDE_JET 16
 int heipa_ctx_set_option(heipa_ctx *ctx, int option, uint64_t value);
 /* dst uses src's hierarchy cache (HEIPA_OPT_HIER_CACHE) from now on: one cache for several contexts */

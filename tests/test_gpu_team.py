@@ -123,11 +123,12 @@ def wide(ctx):
             ctx.set_option(opt, v)
 
 
-WIDE_DEFAULTS = ((heipa.OPT_TEAM_JET, 1 << 15), (heipa.OPT_BLOCK_JET, 2048), (heipa.OPT_WIDE_JET, 1000000))
+WIDE_DEFAULTS = ((heipa.OPT_TEAM_JET, 1 << 15), (heipa.OPT_BLOCK_JET, 2048), (heipa.OPT_WIDE_JET, 0xFFFFFFFF))
 WIDE_CASES = dict(CASES,
                   n131072=(lambda: heipa.gen_rgg(131072, 6.0, 3, 0), 12, 0.6, False),  # a vertex per lane of 2048 waves
                   n131073=(lambda: heipa.gen_rgg(131073, 6.0, 3, 9), 65, 0.6, False),
-                  n270001=(lambda: heipa.gen_rgg(270001, 4.0, 3, 9), 5, 0.6, False))  # a second sweep step
+                  n262145=(lambda: heipa.gen_rgg(262145, 5.0, 3, 9), 33, 0.2, False),  # beyond one step of twice the waves
+                  n270001=(lambda: heipa.gen_rgg(270001, 4.0, 3, 9), 5, 0.6, False))
 
 
 @pytest.mark.parametrize("name", sorted(WIDE_CASES))
