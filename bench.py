@@ -11,7 +11,7 @@ the plain drop-in, with p50/p99 latency at equal cut:
     every graph exactly once (ceil(4096 / K) graphs per step); `value` is
     their undirected input edges / the time of the K steps.  Before the
     warmup, the pool's autotuner picks the lane-group caps and the
-    single-workgroup threshold on a sample of 64 of the graphs (launch shapes
+    edge bound of Jet's teams on a sample of 64 of the graphs (launch shapes
     only: results do not change).  The plain path
     (one context, graphs one after another) is timed on the graphs of the
     first timed step beside it, and every one of those partitions must be
