@@ -381,25 +381,34 @@ bool hm_split_parallel(Ctx &c, const DGraph &g, const u32 *tmp, const u32 *n_to_
             W.pop_back();
         }
     } else {
-        // below the second split as many children as the hierarchy names
-        const size_t nw = std::min<size_t>(kids.size() * (level > 1 ? p.hier[level - 1] : 1u), c.hm_workers);
         u64 need = 0;
         for (const Kid &kd: kids) need = std::max(need, hm_child_bytes(kd.g, p, level - 1));
         if (c.hm_worker_bytes) need = c.hm_worker_bytes;
-        try {
-            if (c.workers.size() < nw) c.workers.resize(nw);
-            for (size_t i = 0; i < nw; ++i) {
-                auto &w = c.workers[i];
-                if (w && w->arena.capacity() >= need) continue;
-                if (w) ctx_close(*w);
-                w = std::make_unique<Ctx>();
-                ctx_open(*w, c.device, need);
+        auto open = [&](size_t nw) {
+            try {
+                if (c.workers.size() < nw) c.workers.resize(nw);
+                for (size_t i = 0; i < nw; ++i) {
+                    auto &w = c.workers[i];
+                    if (w && w->arena.capacity() >= need) continue;
+                    if (w) ctx_close(*w);
+                    w = std::make_unique<Ctx>();
+                    ctx_open(*w, c.device, need);
+                }
+            } catch (const std::exception &) {
+                for (auto &w: c.workers)
+                    if (w) ctx_close(*w);
+                c.workers.clear();
+                return false;
             }
-        } catch (const std::exception &) {  // device or host memory for the workers: one after another here
-            for (auto &w: c.workers)
-                if (w) ctx_close(*w);
-            c.workers.clear();
-            return sequential();
+            return true;
+        };
+        // one per subtree of the second split; where device or host memory does
+        // not allow that, one per subtree of the first, or none
+        size_t nw = std::min<size_t>(kids.size() * (level > 1 ? p.hier[level - 1] : 1u), c.hm_workers);
+        if (!open(nw)) {
+            const size_t first = std::min<size_t>(kids.size(), c.hm_workers);
+            if (first == nw || !open(first)) return sequential();
+            nw = first;
         }
         for (size_t i = 0; i < nw; ++i) W.push_back(c.workers[i].get());
     }
