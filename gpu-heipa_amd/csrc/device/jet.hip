@@ -36,9 +36,9 @@
 // (rebalance only: per-block prefix of the minibucket totals), post
 // (afterburner | rebalance classify), resolve (rebalance only), apply, and a
 // one-workgroup control launch (block weights, counters, loop state); every
-// hand-off between workgroups is a launch boundary.  Levels of up to 65536
-// vertices run the same steps as a team of workgroups on one XCD instead,
-// whole iterations per launch (jet_team.hpp).
+// hand-off between workgroups is a launch boundary.  Most levels run
+// the same steps as a team of workgroups, on one XCD or on all, whole
+// iterations per launch (jet_team.hpp; the rule is in jet_refine).
 #include "team.hpp"
 
 #include <algorithm>

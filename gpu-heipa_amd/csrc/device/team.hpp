@@ -10,6 +10,8 @@
 // inside one XCD (each costs 50-60 ns and they serialise: with one
 // invalidate per workgroup the barrier of 32 took 2.1 us).
 //
+// A team over all XCDs (WideHead) meets XCD by XCD; see its barrier below.
+//
 // No assumption on co-residency: the workgroups that have started on the XCD
 // register, the first one closes the registration after a bounded wait, and
 // the team is whoever has registered: every member is running, so every
