@@ -1453,7 +1453,7 @@ __device__ void cookie_cutter(const JD &d, s64 mbw, s64 *les = nullptr, s64 *lcn
 struct ResolveLds {
     u64 *skey;
     s64 *soff;
-    u8 *ssel;
+    u8 *ssel;    // before the selection: the digit counters of sort_keys_lds
     s64 *red;    // RB / WAVE
     u32 *ocount; // [0] overflow entries, [1] the first that takes the counter twice
     s64 *cnt;    // the overflow counter during one resolve step
@@ -1463,16 +1463,24 @@ struct ResolveLds {
     s64 *s_es;   // ES_CAP
 };
 
+// bytes of sort_keys_lds's digit counters: 256 digits of 16 bits for each wave
+__host__ __device__ constexpr u32 sort_count_bytes(int nt) { return (u32) (nt / WAVE) * 512u; }
+// bytes of ssel: a flag per entry, and room for a team's digit counters, which
+// take more than the flags below 4096 entries
+__host__ __device__ constexpr u32 resolve_sel_bytes(u32 cap) {
+    const u32 flags = (cap + 15) & ~15u;
+    return flags > sort_count_bytes(TM) ? flags : sort_count_bytes(TM);
+}
 // LDS bytes of ResolveLds for CAP entries (16-byte aligned parts)
 __host__ __device__ constexpr size_t resolve_lds_bytes(u32 cap) {
-    return 16ull * cap + ((cap + 15) & ~15u) + 8ull * (RB / WAVE) + 16 + 12ull * OVF_CAP + 8ull * ES_CAP;
+    return 16ull * cap + resolve_sel_bytes(cap) + 8ull * (RB / WAVE) + 16 + 12ull * OVF_CAP + 8ull * ES_CAP;
 }
 __device__ inline ResolveLds resolve_lds(char *base, u32 cap) {
     ResolveLds r;
     r.skey = (u64 *) base;
     r.soff = (s64 *) (base + 8ull * cap);
     r.ssel = (u8 *) (base + 16ull * cap);
-    char *p = base + 16ull * cap + ((cap + 15) & ~15u);
+    char *p = base + 16ull * cap + resolve_sel_bytes(cap);
     r.red = (s64 *) p;
     p += 8ull * (RB / WAVE);
     r.ocount = (u32 *) p;
@@ -1694,6 +1702,7 @@ __device__ __forceinline__ bool resolve_body(const JD &d, bool strong, u32 stamp
     if constexpr (JD::team) {
         for (u32 i = threadIdx.x; i < L; i += NT) skey[i] = d.rlist[i];
         __syncthreads();
+        static_assert(sort_count_bytes(NT) <= resolve_sel_bytes(0), "the counters end where red begins");
         sort_keys_lds<NT>(skey, (u64 *) soff, (u32 *) ssel, L, 32 - (u32) __builtin_clz(d.n), 32 - (u32) __builtin_clz(d.t | 1u));
     } else if (P2 <= NT) {
         sort_keys_one_per_thread(d.rlist, L, P2, skey);

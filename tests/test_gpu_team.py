@@ -12,6 +12,7 @@ import pytest
 
 import heipa
 import heipa_oracle as orc
+from brute import vertex_weighted
 from graphs import block_weights, csr_from_arrays, random_partition
 from test_gpu_im import _D
 from test_gpu_parity import GRAPHS, _dev, _trace_tuple
@@ -224,3 +225,51 @@ def test_team_match(ctx, name):
     assert np.array_equal(heipa.to_numpy_u32(gmp), omp)
     for f in ("rounds", "after_hem", "ran_leaf", "ran_twin", "ran_relative", "after_relative"):
         assert getattr(gst, f) == getattr(ost, f), f
+
+
+def _overloaded(n, k, moved, eps, weighted):
+    """Consecutive blocks, `moved` vertices of them in block 0 instead."""
+    g = heipa.gen_rgg(n, 6.0, 3, 9)
+    if weighted:
+        g = vertex_weighted(g, 4, 40)
+    part = (np.arange(n, dtype=np.int64) * k // n).astype(np.uint32)
+    part[np.random.default_rng(1).choice(n, moved, replace=False)] = 0
+    return g, part, math.ceil((1 + eps) * int(g.g_weight) / k)
+
+
+@pytest.mark.parametrize("k,moved,eps,weighted", [(33, 300, 0.0005, True), (64, 40000, 0.0005, False),
+                                                  (8, 300, 0.0005, False)])
+def test_two_member_resolve(ctx, k, moved, eps, weighted):
+    """Resolve lists of a level with two members per compute unit (more than
+    512 vertices for each of 256): those that fit its 2048 entries are resolved
+    in the launch, by weak and by strong rebalancing; only the longer ones go to
+    the device-wide path, as often as in launches with the same capacity."""
+    g, part0, lmax = _overloaded(140000, k, moved, eps, weighted)
+    dg = _dev(g)
+    cut0, maxw0 = ctx.edge_cut(dg, heipa.from_numpy_u32(part0)), int(block_weights(g, part0, k).max())
+    print(f"two members k={k} moved={moved} eps={eps}", flush=True)
+
+    def run(block_jet, cap):
+        ctx.set_option(heipa.OPT_BLOCK_JET, block_jet)
+        ctx.set_option(heipa.OPT_RESOLVE_CAP, cap)
+        ctx.prof_enable(True)
+        ctx.prof_filter("jet_rebalance_global")
+        ctx.prof_reset()
+        try:
+            pd = heipa.from_numpy_u32(part0)
+            cut, maxw, tr = ctx.jet_refine(dg, pd, k, lmax, False, 1, cut0, maxw0, trace_cap=4096)
+            launches = ctx.prof_stats().get("jet_rebalance_global", {"launches": 0})["launches"]
+        finally:
+            ctx.prof_enable(False)
+            ctx.prof_filter("")
+            ctx.set_option(heipa.OPT_BLOCK_JET, 2048)
+            ctx.set_option(heipa.OPT_RESOLVE_CAP, 1 << 32)
+        return launches, (cut, maxw, heipa.to_numpy_u32(pd).tobytes(), [_trace_tuple(t) for t in tr])
+
+    short, want = run(0, 64)
+    long, same = run(0, 2048)
+    assert same == want
+    assert long < short and any(t[2] == 2 and t[4] > 64 for t in want[3])  # lists of 65 to 2048, strong ones too
+    team, got = run(2048, 1 << 32)
+    assert got == want
+    assert team == long
