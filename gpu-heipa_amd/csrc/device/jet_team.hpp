@@ -1057,6 +1057,8 @@ __global__ __launch_bounds__(TM, PER_CU == 2 ? 4 : 1) void jet_team_kernel(JetDe
         // ---- rows of the wide vertices next to the moves
         if (d.rflag && nm) {
             const u32 rmode = nm > d.n / 10 ? ROW_LARGE : ROW_SMALL;
+            u32 off = gw * tile + wl;
+            if (FLAT && WIDE) off = wl * NWV + (gw + wl * 37) % NWV;
             if (d.W <= 2) {
                 // From the adjacencies, a lane, a row or a wave each by their
                 // length.  Counts kept by the moves (two updates of shared
@@ -1064,8 +1066,6 @@ __global__ __launch_bounds__(TM, PER_CU == 2 ? 4 : 1) void jet_team_kernel(JetDe
                 // skewed level 50 us where most vertices move; walking the
                 // touched rows again is a gather per edge.
                 u32 *list = (u32 *) um + wid * TILE;
-                u32 off = gw * tile + wl;
-                if (FLAT && WIDE) off = wl * NWV + (gw + wl * 37) % NWV;
                 for (u64 t0 = 0; t0 < d.n; t0 += (u64) NWV * tile) {
                     const u64 vv = t0 + off;
                     const u32 v = (u32) vv;
@@ -1092,16 +1092,29 @@ __global__ __launch_bounds__(TM, PER_CU == 2 ? 4 : 1) void jet_team_kernel(JetDe
                     wave_sync();
                 }
             } else {
-                // a wave per vertex, its block mask in LDS
-                u32 *wm = (u32 *) um + wid * (TILE + d.W), *list = wm + d.W;
-                for (u64 p0 = (u64) gw * WAVE; p0 < d.n; p0 += (u64) NWV * WAVE) {
-                    const u64 v = p0 + wl;
-                    const bool take = v < d.n && (d.rflag[v] & 3u) == 3u && degree(d, (u32) v) <= d.hub_deg;
-                    const u64 bal = __ballot(take);
-                    if (take) list[(u32) __popcll(bal & lanemask_lt())] = (u32) v;
+                // The same with the block masks in LDS, W words each: the
+                // vertices have degree >= k > 64, so a row or a wave each.  The
+                // vertices are spread as in the sweep: with 64 consecutive ones
+                // per wave, one after another, the first waves of a skewed level
+                // took 64 long adjacencies in turn while most had none (R-MAT of
+                // 16384 vertices, k = 128: 9.9 ms per refine, 4.5 now).
+                u32 *list = (u32 *) um + wid * (WAVE + WAVE / ROW * d.W), *wm = list + WAVE;
+                for (u64 t0 = 0; t0 < d.n; t0 += (u64) NWV * tile) {
+                    const u64 vv = t0 + off;
+                    const u32 v = (u32) vv;
+                    const bool flagged = wl < tile && vv < d.n && (d.rflag[v] & 3u) == 3u;
+                    const u32 deg = flagged ? degree(d, v) : 0u;
+                    const bool mid = flagged && deg <= 2 * LONG_DEG;
+                    const u64 bm = __ballot(mid);
+                    if (mid) list[(u32) __popcll(bm & lanemask_lt())] = v;
                     wave_sync();
-                    for (u32 i = 0; i < (u32) __popcll(bal); ++i)
-                        row_update<(int) WAVE>(d, wm, list[i], wl, rmode, true, nullptr);
+                    const u32 nl = (u32) __popcll(bm);
+                    for (u32 r0 = 0; r0 < nl; r0 += WAVE / ROW) {
+                        const bool act = r0 + rg < nl;
+                        row_update<(int) ROW>(d, wm + rg * d.W, act ? list[r0 + rg] : 0u, rl, rmode, act, nullptr);
+                    }
+                    for (u64 left = __ballot(deg > 2 * LONG_DEG && deg <= d.hub_deg); left; left &= left - 1)
+                        row_update<(int) WAVE>(d, wm, lane_value(v, __builtin_ctzll(left)), wl, rmode, true, nullptr);
                     wave_sync();
                 }
             }

@@ -273,3 +273,39 @@ def test_two_member_resolve(ctx, k, moved, eps, weighted):
     team, got = run(2048, 1 << 32)
     assert got == want
     assert team == long
+
+
+ROWS = {
+    # rows of wide vertices beyond 64 blocks: degrees around the 256 up to which
+    # 16 lanes take one, lane groups on both sides of it, hubs, three and more words per mask
+    "deg256": (lambda: _regular(1200, 256), 70),
+    "deg257": (lambda: _regular(1200, 257), 70),
+    "rmat_k65": (lambda: heipa.gen_rmat(12, 0, 40.0, 0.57, 0.19, 0.19, 5, 10, False), 65),
+    "rmat_k97": (lambda: heipa.gen_rmat(13, 0, 30.0, 0.57, 0.19, 0.19, 5, 10, False), 97),
+    "rmat_k200": (lambda: heipa.gen_rmat(14, 0, 30.0, 0.57, 0.19, 0.19, 5, 10, False), 200),
+    "rgg_k66": (lambda: heipa.gen_rgg(20000, 90.0, 3, 10), 66),
+}
+
+
+@pytest.mark.parametrize("form", ["one_xcd", "all_xcds"])
+@pytest.mark.parametrize("name", sorted(ROWS))
+def test_team_rows_many_blocks(ctx, name, form):
+    make, k = ROWS[name]
+    g = make()
+    part0 = _start(g, k, 0.8)
+    lmax = math.ceil(1.03 * g.g_weight / k)
+    cut0, maxw0 = orc.edge_cut(g, part0), int(block_weights(g, part0, k).max())
+    print(f"team rows {name} {form} n={g.n} m={g.m} k={k}", flush=True)
+    op, ocut, omaxw, otr = orc.jet_refine(g, part0, k, lmax, False, 1, cut0, maxw0, trace_cap=4096)
+    opts = {"one_xcd": ((heipa.OPT_BLOCK_JET, 1 << 20),), "all_xcds": ((heipa.OPT_TEAM_JET, 0), (heipa.OPT_BLOCK_JET, 1))}
+    for opt, v in opts[form]:
+        ctx.set_option(opt, v)
+    try:
+        pd = heipa.from_numpy_u32(part0)
+        gcut, gmaxw, gtr = ctx.jet_refine(_dev(g), pd, k, lmax, False, 1, cut0, maxw0, trace_cap=4096)
+    finally:
+        for opt, v in WIDE_DEFAULTS:
+            ctx.set_option(opt, v)
+    _compare(gtr, otr, name)
+    assert (gcut, gmaxw) == (ocut, omaxw)
+    assert np.array_equal(heipa.to_numpy_u32(pd), op)
