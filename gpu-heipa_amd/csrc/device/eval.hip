@@ -398,18 +398,20 @@ void block_weights_checked(Ctx &c, const DGraph &g, const u32 *part, u32 k, s64 
     s64 *bw = bs.get<s64>(k);
     const Checks r = check_launch(c, bs, g, part, k, ~0u, false);
     block_weights_dev(c, g, part, k, bw, r.flags());
-    copy_d2h(c, c.pinned, r.flags(), 4);
-    if (8ull * k + 64 <= c.pinned_bytes) {
-        copy_d2h(c, (char *) c.pinned + 64, bw, 8ull * k);
-        c.sync();
-        std::memcpy(bw_host, (char *) c.pinned + 64, 8ull * k);
-    } else {
-        copy_d2h(c, bw_host, bw, 8ull * k);
-        c.sync();
+    // the caller's array is written only once the checks are known to have passed
+    std::vector<s64> h;
+    s64 *got = (s64 *) ((char *) c.pinned + 64);
+    if (8ull * k + 64 > c.pinned_bytes) {
+        h.resize(k);
+        got = h.data();
     }
+    copy_d2h(c, c.pinned, r.flags(), 4);
+    copy_d2h(c, got, bw, 8ull * k);
+    c.sync();
     u32 f;
     std::memcpy(&f, c.pinned, 4);
     check_throw(f);
+    std::memcpy(bw_host, got, 8ull * k);
 }
 
 static s64 evaluate(Ctx &c, const DGraph &g, const u32 *part, const s32 *D, u32 k) {

@@ -3,6 +3,8 @@ workgroups: rows that span several shares, shares whose source vertices do not
 fit the offsets a workgroup holds at a time (2048), isolated vertices, and a
 fault at any place of a share.  Values against numpy in 64 bits (integers: no
 tolerance)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -91,3 +93,17 @@ def test_block_id_out_of_range(ctx):
         with pytest.raises(heipa.HeipaError, match="block id"):
             call()
     assert ctx.edge_cut(dg, pd) > 0  # an edge cut takes any block ids
+
+
+@pytest.mark.parametrize("k", [4, 40000])  # staged in the context's pinned block, or beyond its size
+def test_refused_block_weights_leave_the_output(ctx, k):
+    g = _sparse_ids()
+    dg = _dev(g)
+    part = random_partition(g.n, k, 7)
+    part[17] = k
+    pd = heipa.from_numpy_u32(part)
+    bw, maxw = np.full(k, -7, np.int64), ctypes.c_int64(-9)
+    rc = ctx.L.heipa_block_weights(ctx.h, ctypes.byref(dg.desc), pd.data_ptr(), k,
+                                   bw.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)), ctypes.byref(maxw))
+    assert rc == heipa.ERR_INVALID
+    assert (bw == -7).all() and maxw.value == -9
