@@ -65,6 +65,7 @@ int guarded_host(F &&f) {
 void check_graph(const heipa_graph *g) {
     require(g != nullptr, "null graph");
     require(g->n == 0 || (g->xadj && (g->m == 0 || g->adjncy)), "graph arrays missing");
+    require(g->n != 0 || g->m == 0, "invalid graph: edges without vertices");
     require((g->flags & HEIPA_UNIFORM_EW) || g->m == 0 || g->adjwgt, "edge weights missing");
     require((g->flags & HEIPA_UNIFORM_VW) || g->n == 0 || g->vwgt, "vertex weights missing");
 }
@@ -184,7 +185,7 @@ int heipa_block_weights(heipa_ctx *ctx, const heipa_graph *g, const uint32_t *pa
                         int64_t *maxw) {
     return guarded(ctx, [&](Ctx &c) {
         check_graph(g);
-        require(k > 0 && bw_host, "bad argument");
+        require(k > 0 && bw_host && (part || g->n == 0), "bad argument");
         DGraph d = to_dgraph(g);
         block_weights_checked(c, d, part, k, (s64 *) bw_host);
         if (maxw) {

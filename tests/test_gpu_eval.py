@@ -107,3 +107,17 @@ def test_refused_block_weights_leave_the_output(ctx, k):
                                    bw.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)), ctypes.byref(maxw))
     assert rc == heipa.ERR_INVALID
     assert (bw == -7).all() and maxw.value == -9
+
+
+def test_missing_arrays_are_refused(ctx):
+    """A null partition, and a graph that claims edges without having vertices
+    or arrays: refused before anything reaches the device."""
+    g = _dev(_sparse_ids())
+    bw, out = (ctypes.c_int64 * 4)(), ctypes.c_int64()
+    assert ctx.L.heipa_block_weights(ctx.h, ctypes.byref(g.desc), None, 4, bw, None) == heipa.ERR_INVALID
+    empty = heipa.Graph(0, 5, 0, heipa.UNIFORM_EW | heipa.UNIFORM_VW, 0, None, None, None, None)
+    assert ctx.L.heipa_edge_cut(ctx.h, ctypes.byref(empty), None, ctypes.byref(out)) == heipa.ERR_INVALID
+    assert ctx.L.heipa_block_weights(ctx.h, ctypes.byref(empty), None, 4, bw, None) == heipa.ERR_INVALID
+    none = heipa.Graph(0, 0, 0, heipa.UNIFORM_EW | heipa.UNIFORM_VW, 0, None, None, None, None)
+    assert ctx.L.heipa_edge_cut(ctx.h, ctypes.byref(none), None, ctypes.byref(out)) == heipa.OK and out.value == 0
+    assert ctx.L.heipa_block_weights(ctx.h, ctypes.byref(none), None, 4, bw, None) == heipa.OK and list(bw) == [0] * 4
