@@ -192,21 +192,24 @@ __global__ __launch_bounds__(EVAL_BLOCK) void eval_kernel(DGraph g, const u32 *_
         }
         __syncthreads();
         const u32 end = sx[rows] < c1 ? sx[rows] : c1;
-        for (u32 j0 = c + threadIdx.x; j0 < end; j0 += EVAL_BLOCK * 4) {
+        const u32 cnt = end - c;  // counted from c: offsets up to 2^32 - 1 never wrap
+        const u32 *adj = g.adj + c;
+        const s32 *ew = UEW ? nullptr : g.ew + c;
+        for (u32 x0 = threadIdx.x; x0 < cnt; x0 += EVAL_BLOCK * 4) {
             u32 v[4];
             s32 w[4];
 #pragma unroll
             for (u32 q = 0; q < 4; ++q) {
-                const u32 j = j0 + q * EVAL_BLOCK;
-                v[q] = j < end ? g.adj[j] : 0u;
-                w[q] = UEW ? 1 : j < end ? g.ew[j] : 0;
+                const u32 x = x0 + q * EVAL_BLOCK;
+                v[q] = x < cnt ? adj[x] : 0u;
+                w[q] = UEW ? 1 : x < cnt ? ew[x] : 0;
             }
 #pragma unroll
-            for (u32 q = 0; q < 4; ++q) v[q] = j0 + q * EVAL_BLOCK < end ? part[v[q]] : 0u;
+            for (u32 q = 0; q < 4; ++q) v[q] = x0 + q * EVAL_BLOCK < cnt ? part[v[q]] : 0u;
 #pragma unroll
             for (u32 q = 0; q < 4; ++q) {
-                const u32 j = j0 + q * EVAL_BLOCK;
-                if (j >= end) continue;
+                const u32 x = x0 + q * EVAL_BLOCK, j = c + x;
+                if (x >= cnt) continue;
                 u32 a = 0, b = rows;  // the last row that starts at or before j
                 while (b - a > 1) {
                     const u32 mid = (a + b) >> 1;

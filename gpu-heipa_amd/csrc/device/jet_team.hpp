@@ -219,9 +219,10 @@ __device__ __forceinline__ bool row_eval(const JD &d, u32 mode, s64 mbw, const R
 template<typename JD>
 __device__ __forceinline__ s64 row_burn(const JD &d, u32 u, s64 ug, u32 o, u32 nn, u32 beg, u32 end, u32 lane) {
     s64 change = 0;
-    for (u32 j0 = beg + lane; __any(j0 < end); j0 += 2 * ROW) {
-        const u32 j1 = j0 + ROW;
-        const bool a0 = j0 < end, a1 = j1 < end;
+    const u32 deg = end - beg;
+    for (u32 x0 = lane; __any(x0 < deg); x0 += 2 * ROW) {
+        const u32 j0 = beg + x0, j1 = j0 + ROW;
+        const bool a0 = x0 < deg, a1 = x0 + ROW < deg;
         u32 v[2] = {0, 0};
         s64 w[2] = {0, 0}, vg[2] = {GAIN_MIN, GAIN_MIN};
         u32 vn[2] = {0, 0}, vo[2] = {0, 0};
@@ -254,13 +255,14 @@ __device__ __forceinline__ s64 row_burn(const JD &d, u32 u, s64 ug, u32 o, u32 n
 template<u32 G, typename JD>
 __device__ __forceinline__ u64 row_blocks(const JD &d, u32 b, u32 e, u32 lane) {
     u64 m = 0;
-    for (u32 j0 = b + lane; j0 < e; j0 += 8 * G) {
+    const u32 deg = e - b;
+    for (u32 x = lane; x < deg; x += 8 * G) {
         u32 v[8];
 #pragma unroll
-        for (u32 q = 0; q < 8; ++q) v[q] = e - j0 > q * G ? d.adj[j0 + q * G] : 0u;
+        for (u32 q = 0; q < 8; ++q) v[q] = x + q * G < deg ? d.adj[b + x + q * G] : 0u;
 #pragma unroll
         for (u32 q = 0; q < 8; ++q)
-            if (e - j0 > q * G) m |= 1ull << (u32) d.work[v[q]];
+            if (x + q * G < deg) m |= 1ull << (u32) d.work[v[q]];
     }
     u32 lo = (u32) m, hi = (u32) (m >> 32);
     lo |= ror16<8>(lo);

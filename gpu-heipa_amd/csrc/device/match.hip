@@ -593,8 +593,10 @@ template<bool UEW>
 __device__ __forceinline__ Cand team_pick(const DGraph &g, const DevPtr<u32> &vcmap, u32 b, u32 e, u32 lane, u32 stride,
                                           u32 r) {
     Cand best{0, 0, SENT};
-    for (u32 j = b + lane; j < e; j += 2 * stride) {
-        const bool two = e - j > stride;
+    const u32 deg = e - b;
+    for (u32 x = lane; x < deg; x += 2 * stride) {
+        const bool two = deg - x > stride;
+        const u32 j = b + x;
         const u32 v0 = g.adj[j], v1 = two ? g.adj[j + stride] : 0u;
         const s32 w0 = UEW ? 1 : g.ew[j], w1 = UEW ? 1 : two ? g.ew[j + stride] : 0;
         const u32 m0 = vcmap[v0], m1 = two ? (u32) vcmap[v1] : 0u;

@@ -7,6 +7,7 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 import heipa
 from graphs import csr_from_arrays, random_partition
@@ -121,3 +122,25 @@ def test_missing_arrays_are_refused(ctx):
     none = heipa.Graph(0, 0, 0, heipa.UNIFORM_EW | heipa.UNIFORM_VW, 0, None, None, None, None)
     assert ctx.L.heipa_edge_cut(ctx.h, ctypes.byref(none), None, ctypes.byref(out)) == heipa.OK and out.value == 0
     assert ctx.L.heipa_block_weights(ctx.h, ctypes.byref(none), None, 4, bw, None) == heipa.OK and list(bw) == [0] * 4
+
+
+def test_edge_offsets_near_the_limit(ctx):
+    """4294966296 directed edges, the last offsets within one stride of 2^32:
+    every vertex but vertex 0 has all its edges to vertex 0 (made on the device)."""
+    n, m = 1025, 2 ** 32 - 1000
+    xadj = np.concatenate([[0], np.arange(n, dtype=np.uint64) * m // (n - 1)]).astype(np.uint32)
+    adj = torch.zeros(m, dtype=torch.int32, device="cuda:0")
+    xd = heipa.from_numpy_u32(xadj)
+    g = heipa.Graph(n, m, n, heipa.UNIFORM_EW | heipa.UNIFORM_VW, 0, xd.data_ptr(), adj.data_ptr(), None, None)
+    part = np.arange(n, dtype=np.uint32) % 3
+    pd = heipa.from_numpy_u32(part)
+    D = np.random.default_rng(1).integers(0, 1000, (3, 3)).astype(np.int32)
+    Dd = heipa.from_numpy_u32(D.reshape(-1).view(np.uint32))
+    deg = np.diff(xadj.astype(np.int64))
+    print(f"eval m={m}", flush=True)
+    torch.cuda.synchronize()
+    out = ctypes.c_int64()
+    assert ctx.L.heipa_edge_cut(ctx.h, ctypes.byref(g), pd.data_ptr(), ctypes.byref(out)) == heipa.OK
+    assert out.value == int(deg[part != part[0]].sum()) // 2
+    assert ctx.L.heipa_comm_cost(ctx.h, ctypes.byref(g), pd.data_ptr(), Dd.data_ptr(), 3, ctypes.byref(out)) == heipa.OK
+    assert out.value == int((deg * D[part, part[0]].astype(np.int64)).sum())
