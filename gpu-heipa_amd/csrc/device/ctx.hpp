@@ -119,6 +119,10 @@ public:
     void reset_peak() { peak_ = in_use(); }
     size_t capacity() const { return cap_; }
     size_t in_use() const { return front_ + (cap_ - back_); }
+    size_t free_bytes() const { return back_ - front_; }
+    // `extra` bytes may be taken for speed: what the form without them still
+    // needs, `keep`, fits beside them (8 KiB for the alignment of its parts)
+    bool spare(size_t extra, size_t keep) const { return free_bytes() >= extra + keep + 8192; }
 
 private:
     static size_t align(size_t b) { return (b + 255) & ~(size_t) 255; }

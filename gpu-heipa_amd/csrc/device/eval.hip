@@ -228,12 +228,18 @@ __global__ __launch_bounds__(EVAL_BLOCK) void eval_kernel(DGraph g, const u32 *_
     if (threadIdx.x == 0) out[blockIdx.x] = acc;
 }
 
-u32 eval_grid(const Ctx &c, u64 items) { return grid_for(c, items, EVAL_SHARE, EVAL_PER_CU); }
+// at most as many workgroups as their partial results (8 bytes each of the
+// checks and of the evaluator) fit the free scratch
+u32 eval_grid(const Ctx &c, u64 items) {
+    const u64 room = (c.arena.free_bytes() & ~(size_t) 255) / 16;
+    return (u32) std::min<u64>(grid_for(c, items, EVAL_SHARE, EVAL_PER_CU), room > 1 ? room - 1 : 1);
+}
 
-void eval_launch(Ctx &c, const DGraph &g, const u32 *part, const s32 *D, u32 k, int mode, const u32 *bad, s64 *out) {
+void eval_launch(Ctx &c, const DGraph &g, const u32 *part, const s32 *D, u32 k, int mode, const u32 *bad, u32 groups,
+                 s64 *out) {
     const bool uew = g.ew == nullptr;
     const double bytes = 4.0 * (g.n + 1) + 4.0 * g.m * (uew ? 1 : 2) + 4.0 * g.n;
-    const dim3 grid(eval_grid(c, g.m)), block(EVAL_BLOCK);
+    const dim3 grid(groups), block(EVAL_BLOCK);
     const bool dl = mode == 1 && (u64) k * k <= D_LDS_MAX;
     const size_t shmem = dl ? sizeof(s32) * k * k : 0;
     const char *name = mode == 0 ? "edge_cut" : "comm_cost";
@@ -333,23 +339,26 @@ void meta_launch(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *out) {
            meta.hub_deg, out);
 }
 
+// the checks alone, and their wait; adds up the degrees in meta
+static void check(Ctx &c, const DGraph &g, const u32 *part, u32 k, GraphMeta &meta) {
+    BackScope bs(c.arena);
+    const Checks r = check_launch(c, bs, g, part, k, meta.hub_deg, false);
+    std::vector<char> h(r.bytes);
+    readback(c, h.data(), (const char *) r.dev, r.bytes);
+    u32 f;
+    std::memcpy(&f, h.data(), 4);
+    check_throw(f);
+    for (u32 i = 0; i < r.grid_c; ++i) {
+        CheckPart p;
+        std::memcpy(&p, h.data() + 8 + sizeof(p) * i, sizeof(p));
+        meta.max_deg = std::max(meta.max_deg, p.max_deg);
+        meta.n_hubs += p.n_hubs;
+    }
+}
+
 GraphMeta validate(Ctx &c, const DGraph &g, const u32 *part, u32 k) {
     GraphMeta meta = meta_of(g);
-    {
-        BackScope bs(c.arena);
-        const Checks r = check_launch(c, bs, g, part, k, meta.hub_deg, false);
-        std::vector<char> h(r.bytes);
-        readback(c, h.data(), (const char *) r.dev, r.bytes);
-        u32 f;
-        std::memcpy(&f, h.data(), 4);
-        check_throw(f);
-        for (u32 i = 0; i < r.grid_c; ++i) {
-            CheckPart p;
-            std::memcpy(&p, h.data() + 8 + sizeof(p) * i, sizeof(p));
-            meta.max_deg = std::max(meta.max_deg, p.max_deg);
-            meta.n_hubs += p.n_hubs;
-        }
-    }
+    check(c, g, part, k, meta);
     hub_list(c, g, meta, true);
     return meta;
 }
@@ -376,7 +385,7 @@ GraphMeta make_meta(Ctx &c, const DGraph &g, bool back) {
 static s64 evaluate_checked(Ctx &c, const DGraph &g, const u32 *part, const s32 *D, u32 k) {
     BackScope bs(c.arena);
     const Checks r = check_launch(c, bs, g, D ? part : nullptr, k, ~0u, true);
-    eval_launch(c, g, part, D, k, D ? 1 : 0, r.flags(), r.sums());
+    eval_launch(c, g, part, D, k, D ? 1 : 0, r.flags(), r.grid_e, r.sums());
     std::vector<char> h(r.bytes);
     readback(c, h.data(), (const char *) r.dev, r.bytes);
     u32 f;
@@ -398,6 +407,14 @@ s64 comm_cost_checked(Ctx &c, const DGraph &g, const u32 *part, const s32 *D, u3
 }
 void block_weights_checked(Ctx &c, const DGraph &g, const u32 *part, u32 k, s64 *bw_host) {
     BackScope bs(c.arena);
+    if (!c.arena.spare(8ull * k, 0)) {  // one after the other in the same scratch, a wait each
+        GraphMeta meta = meta_of(g);
+        check(c, g, part, k, meta);
+        s64 *bw = bs.get<s64>(k);
+        block_weights_dev(c, g, part, k, bw);
+        readback(c, bw_host, bw, k);
+        return;
+    }
     s64 *bw = bs.get<s64>(k);
     const Checks r = check_launch(c, bs, g, part, k, ~0u, false);
     block_weights_dev(c, g, part, k, bw, r.flags());
@@ -421,7 +438,7 @@ static s64 evaluate(Ctx &c, const DGraph &g, const u32 *part, const s32 *D, u32 
     BackScope bs(c.arena);
     std::vector<s64> h(eval_grid(c, g.m));
     s64 *sums = bs.get<s64>(h.size());
-    eval_launch(c, g, part, D, k, D ? 1 : 0, nullptr, sums);
+    eval_launch(c, g, part, D, k, D ? 1 : 0, nullptr, (u32) h.size(), sums);
     readback(c, h.data(), (const s64 *) sums, h.size());
     s64 sum = 0;
     for (s64 x: h) sum += x;

@@ -2950,6 +2950,8 @@ struct JetHost {
         apply();
     }
 
+    // scratch of fallback(): its list, and the sort's and the scans' counts
+    u64 fallback_bytes() const { return 24ull * g.n + 1100ull * div_up(g.n, RS_TILE) + 8192; }
     // the stalled iteration's resolve on the global path, then its apply
     void fallback(const JetCtl &s) {
         BackScope bs(c.arena);
@@ -3109,26 +3111,35 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         const bool narrow = (!h.flat && n <= c.team_jet_max_n && (u64) g.m <= 16ull * n) ||
                             (n <= std::max(c.team_jet_max_n, c.block_jet_max_n) && (u64) g.m <= dense);
         const u32 want = std::min<u32>({WIDE_MAX, (u32) c.num_cus, std::max<u32>(div_up(n, 64), div_up(g.m, 512u))});
-        if (teams && narrow) {
+        // two members per compute unit: where one would take a second sweep step
+        // (regular levels only: skewed ones have long resolve lists)
+        const size_t all = team_lds_bytes(k, h.ta.wgroups, RESOLVE_CAP), half = team_lds_bytes(k, h.ta.wgroups, 2048);
+        const bool twice = !h.flat && n > (u64) c.num_cus * TW * WAVE && 2 * (half + 2048) <= c.max_lds;
+        const u32 members = twice ? std::min<u32>(WIDE_MAX, 2 * (u32) c.num_cus) : want;
+        // A team's blocks, its copies of the minibucket totals and its list
+        // regions are scratch that the launches do without: taken where what
+        // they may still need stays free (lists, statistics, rows, and the
+        // device-wide resolve path)
+        const u64 totals = 8ull * ((u64) d.t + 1) * std::max(8u, c.bucket_copies);
+        const u64 rows = meta.max_deg >= k ? std::min<u64>(n, g.m / k) * (8ull * ((k + 31) / 32) + 4) : 0;
+        const u64 keep = 34ull * n + 24ull * meta.n_hubs + 8ull * (g.m / HUB_CHUNK) + rows + h.fallback_bytes();
+        const bool room = c.arena.spare(TEAM_SLOTS * sizeof(TeamCtl) + totals, keep);
+        const bool wide_room = c.arena.spare(
+            WIDE_SLOTS * sizeof(WideCtl) + totals + 8 * (n + members * (TW * WAVE * TEAM_U + 1ull) + meta.n_hubs), keep);
+        if (teams && narrow && room) {
             h.team_mode = true;
             h.ta.xcc = c.xcc;
             h.ta.want = std::min<u32>(TEAM_WANT, div_up(n, 16));  // a vertex or two per row of lanes
             h.ta.tc = bs.get<TeamCtl>(TEAM_SLOTS);  // cleared by the init launch
-        } else if (teams && c.n_xcc > 1 && n <= c.wide_jet_max_n &&
-                   // its list regions; scratch that is short of eight times that keeps to the lists of the launches
-                   8 * (n + want * 2ull * TW * WAVE * TEAM_U) <= (c.arena.capacity() - c.arena.in_use()) / 8) {
+        } else if (teams && !narrow && c.n_xcc > 1 && n <= c.wide_jet_max_n && wide_room) {
             h.team_mode = h.wide = true;
-            h.ta.want = want;
+            h.ta.want = members;
             h.ta.wc = bs.get<WideCtl>(WIDE_SLOTS);
-            // one member per compute unit: its whole LDS for the resolve list;
-            // two where one per unit would take a second sweep step (regular
-            // levels only: skewed ones have long resolve lists)
-            const size_t all = team_lds_bytes(k, h.ta.wgroups, RESOLVE_CAP), half = team_lds_bytes(k, h.ta.wgroups, 2048);
-            if (!h.flat && n > (u64) c.num_cus * TW * WAVE && 2 * (half + 2048) <= c.max_lds) {
+            // one member per compute unit: its whole LDS for the resolve list
+            if (twice) {
                 h.twice = true;
                 h.team_lds = half;
                 h.ta.rcap = 2048;
-                h.ta.want = std::min<u32>(WIDE_MAX, 2 * (u32) c.num_cus);
             } else if (all + 2048 <= c.max_lds) {
                 h.team_lds = all;
                 h.ta.rcap = RESOLVE_CAP;
@@ -3228,7 +3239,8 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         // saves a wait of 12-15 us per level; where they would take more than an
         // eighth of the free scratch, the vertices are counted instead
         u64 nw = std::min<u64>(n, g.m / k);
-        if (nw * (8ull * d.W + 4ull * k + 4) > (c.arena.capacity() - c.arena.in_use()) / 8) {
+        const u64 row = 8ull * d.W + 4ull * k + 4;
+        if (nw * row > c.arena.free_bytes() / 8 || !c.arena.spare(nw * row, h.fallback_bytes())) {
             u32 exact = 0;
             readback(c, &exact, cnt, 1);
             nw = std::max(exact, 1u);

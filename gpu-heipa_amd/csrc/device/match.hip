@@ -1087,7 +1087,8 @@ void pair_by_key(Ctx &c, K *keys, u32 *vals, u32 len, u32 bits, u32 *vcmap) {
     BackScope bs(c.arena);
     K *ktmp = bs.get<K>(len);
     u32 *vtmp = bs.get<u32>(len);
-    if (c.n_xcc && c.block_jet_max_n && len <= PT_LIST) {
+    const u64 tiles = div_up(len, RS_TILE);
+    if (c.n_xcc && c.block_jet_max_n && len <= PT_LIST && c.arena.spare(sizeof(PairTeam), 12ull * len + 1024 * tiles)) {
         PairTeam *pt = bs.get<PairTeam>(1);
         fill<u32>(c, (u32 *) pt, sizeof(TeamHead) / 4 + 32, 0u);
         PairTeamArgs<K> a{pt, {{keys}, {ktmp}}, {{vals}, {vtmp}}, len, bits, c.xcc, std::min<u32>(TEAM_WANT, div_up(len, 256)),
@@ -1128,21 +1129,25 @@ u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping
     u32 *claim = bs.get<u32>(n);
     u32 *lists[2] = {bs.get<u32>(n), bs.get<u32>(n)};
     u32 *lens = bs.get<u32>(64);  // ring of list lengths, one per round
-    MatchTeam *mt = bs.get<MatchTeam>(1);
-    // buffers of the team's pairing passes, where they leave most of the scratch free
+    // the team's block, and the buffers of its pairing passes: taken where the
+    // host's passes keep the scratch they may need (keys, their copies, the
+    // sort's counts, and the groups of up to n entries)
+    MatchTeam *mt = nullptr;
     u64 *pkeys[2] = {nullptr, nullptr};
     PairScratch *ps = nullptr;
     {
-        const u64 ent = std::min(n, PT_LIST);
-        if (n <= MT_MAP && c.n_xcc && c.block_jet_max_n &&
-            8 * (16 * ent + sizeof(PairScratch)) <= c.arena.capacity() - c.arena.in_use()) {
+        const u64 keep = 32ull * n + 1024ull * div_up(n, RS_TILE), ent = std::min(n, PT_LIST);
+        const u64 pair = 16 * ent + sizeof(PairScratch);
+        if (c.n_xcc && c.block_jet_max_n && c.arena.spare(sizeof(MatchTeam), keep))  // HEIPA_OPT_BLOCK_JET 0: one launch per step
+            mt = bs.get<MatchTeam>(1);
+        if (mt && n <= MT_MAP && c.arena.spare(pair, keep)) {
             for (u64 *&k: pkeys) k = bs.get<u64>(ent);
             ps = bs.get<PairScratch>(1);
         }
     }
     const dim3 blk(256);
     launch(c, "match_init", 12.0 * n, dim3(grid_for(c, n, 256 * 4)), blk, 0, match_init_kernel, n, vcmap, hn, claim, lens,
-           (u32 *) mt, (u32) (sizeof(MatchTeam) / 4));
+           (u32 *) mt, mt ? (u32) (sizeof(MatchTeam) / 4) : 0u);
 
     // initial pick
     // profiling: summed degree of the repicked vertices, for the byte model
@@ -1174,7 +1179,7 @@ u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping
     u32 *pinned = c.pinned_as<u32>();
     u32 exact_rounds = 0;
     MatchTeam res{};
-    bool team = c.n_xcc != 0 && c.block_jet_max_n != 0;  // HEIPA_OPT_BLOCK_JET 0: one launch per step
+    bool team = mt != nullptr;
     while (true) {
         // the first rounds of a large graph need the whole chip; the team takes
         // over with the first list that fits one XCD
