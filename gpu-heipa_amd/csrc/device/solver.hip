@@ -326,12 +326,41 @@ u64 hm_child_bytes(const DGraph &g, const HMParams &p, u32 level) {
     return 80 * n + 88 * m + 50ull * k * sections * 32 + (2ull << 20);
 }
 
+// Worker contexts with arenas of at least `need` bytes on the context, at most
+// `want`; returns how many there are.  Those kept from earlier calls stay, unless
+// their arena is too small; an open that fails ends the search and leaves the
+// others.  The ones beyond `first` share in the second split only and are opened
+// while they take no more than an eighth of the free device memory together.
+size_t open_workers(Ctx &c, u64 need, size_t first, size_t want) {
+    auto &ws = c.workers;
+    const auto fits = [&](const std::unique_ptr<Ctx> &w) { return w && w->arena.capacity() >= need; };
+    const size_t kept = (size_t) (std::stable_partition(ws.begin(), ws.end(), fits) - ws.begin());
+    if (kept >= want) return want;
+    ctx_trim_workers(c, kept);
+    try {
+        ws.reserve(want);
+        for (size_t extra = 0; ws.size() < want;) {
+            if (ws.size() >= first) {
+                size_t free_b = 0, total_b = 0;
+                HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+                if (need > (free_b + extra * need) / 8 / (extra + 1)) break;
+                ++extra;
+            }
+            auto w = std::make_unique<Ctx>();
+            ctx_open(*w, c.device, need);
+            ws.push_back(std::move(w));
+        }
+    } catch (const std::exception &) {
+        (void) hipGetLastError();  // no device memory is an answer here
+    }
+    return std::min(ws.size(), want);
+}
+
 // The subtrees below the first split are independent (disjoint vertices,
 // disjoint entries of the output, deterministic solves), so they run at the
 // same time on worker contexts, one host thread each; the result does not
-// depend on their order.  The children are built here first, on c's
-// stream; a worker context that cannot be opened leaves the caller on the
-// sequential path (false, nothing changed but the children built).
+// depend on their order.  The children are built here first, on c's stream;
+// without two worker contexts they are solved one after another there.
 bool hm_split_parallel(Ctx &c, const DGraph &g, const u32 *tmp, const u32 *n_to_o, u32 level, const HMParams &p,
                        u32 *global) {
     struct Kid {
@@ -370,7 +399,7 @@ bool hm_split_parallel(Ctx &c, const DGraph &g, const u32 *tmp, const u32 *n_to_
     };
     if (kids.size() < 2) return sequential();
     c.sync();  // the children are complete before other streams read them
-    // W: the contexts that solve the subtrees, kid i on W[i mod nw]
+    // W: the contexts that solve the subtrees
     std::vector<Ctx *> W;
     if (lending) {
         W.push_back(&c);
@@ -384,31 +413,13 @@ bool hm_split_parallel(Ctx &c, const DGraph &g, const u32 *tmp, const u32 *n_to_
         u64 need = 0;
         for (const Kid &kd: kids) need = std::max(need, hm_child_bytes(kd.g, p, level - 1));
         if (c.hm_worker_bytes) need = c.hm_worker_bytes;
-        auto open = [&](size_t nw) {
-            try {
-                if (c.workers.size() < nw) c.workers.resize(nw);
-                for (size_t i = 0; i < nw; ++i) {
-                    auto &w = c.workers[i];
-                    if (w && w->arena.capacity() >= need) continue;
-                    if (w) ctx_close(*w);
-                    w = std::make_unique<Ctx>();
-                    ctx_open(*w, c.device, need);
-                }
-            } catch (const std::exception &) {
-                for (auto &w: c.workers)
-                    if (w) ctx_close(*w);
-                c.workers.clear();
-                return false;
-            }
-            return true;
-        };
-        // one per subtree of the second split; where device or host memory does
-        // not allow that, one per subtree of the first, or none
-        size_t nw = std::min<size_t>(kids.size() * (level > 1 ? p.hier[level - 1] : 1u), c.hm_workers);
-        if (!open(nw)) {
-            const size_t first = std::min<size_t>(kids.size(), c.hm_workers);
-            if (first == nw || !open(first)) return sequential();
-            nw = first;
+        // one worker per subtree of the second split, as far as the device has
+        // room; one alone would only take turns with this context
+        const size_t nw = open_workers(c, need, std::min<size_t>(kids.size(), c.hm_workers),
+                                       std::min<size_t>(kids.size() * (level > 1 ? p.hier[level - 1] : 1u), c.hm_workers));
+        if (nw < 2) {
+            ctx_trim_workers(c, 0);
+            return sequential();
         }
         for (size_t i = 0; i < nw; ++i) W.push_back(c.workers[i].get());
     }

@@ -278,8 +278,11 @@ int heipa_pool_hier_cache_stats(const heipa_pool *pool, uint64_t *entries, uint6
 #define HEIPA_OPT_BLOCK_LDS 6
 /* HEIPA_OPT_HM_WORKERS: worker contexts (each its own stream, arena and host thread, kept by the
  * context between calls) on which heipa_hm_partition solves the subtrees below its first split at
- * the same time (default 8, at most 64; 0 or 1: one after another on the context's stream).  Setting
- * it closes the cached workers beyond the new count, which frees their arenas.  Results do not
+ * the same time (default 8, at most 64; 0 or 1: one after another on the context's stream).  A call
+ * opens up to one per subtree of its second split, each with an arena for the largest subtree of the
+ * first; those beyond one per subtree of the first split only while they take no more than an eighth
+ * of the free device memory together.  A worker that cannot be opened is done without.  Setting the
+ * option closes the cached workers beyond the new count, which frees their arenas.  Results do not
  * depend on it. */
 #define HEIPA_OPT_HM_WORKERS 7
 /* HEIPA_OPT_HM_WORKER_BYTES: arena bytes of each HM worker context (default 0: an estimate from the

@@ -36,3 +36,28 @@ def test_hm_shared_subtrees(ctx, case, hier, workers, worker_bytes):
     finally:
         ctx.set_option(heipa.OPT_HM_WORKERS, 8)
         ctx.set_option(heipa.OPT_HM_WORKER_BYTES, 0)
+
+
+@pytest.mark.parametrize("share,workers", [(0.4, 2), (0.15, 3), (0.02, 6)])
+def test_hm_worker_memory(ctx, case, share, workers):
+    """Arenas of the given share of the free device memory, three subtrees of
+    the first split and six of the second: workers that cannot be opened
+    leave the others, those beyond the three stay within an eighth of the free
+    memory, and a later call uses the ones that the first call opened."""
+    import torch
+    g, want = case
+    dg = _dev(g)
+    ctx.set_option(heipa.OPT_HM_WORKERS, 0)  # none kept from earlier calls
+    ctx.set_option(heipa.OPT_HM_WORKERS, 8)
+    free = torch.cuda.mem_get_info()[0]
+    ctx.set_option(heipa.OPT_HM_WORKER_BYTES, int(share * free))
+    print(f"hm worker memory {share}", flush=True)
+    try:
+        for _ in range(2):
+            part = ctx.hm_partition(dg, HIERS["2:3:2:3"], 0.03, 1, False)
+            assert np.array_equal(heipa.to_numpy_u32(part), want["2:3:2:3"])
+            held = (free - torch.cuda.mem_get_info()[0]) / free
+            assert abs(held - share * workers) < 0.01
+    finally:
+        ctx.set_option(heipa.OPT_HM_WORKER_BYTES, 0)
+        ctx.set_option(heipa.OPT_HM_WORKERS, 8)
