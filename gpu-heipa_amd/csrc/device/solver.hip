@@ -23,10 +23,9 @@
 #include <chrono>
 #include <cmath>
 #include <condition_variable>
-#include <deque>
 #include <exception>
+#include <list>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 namespace heipa {
@@ -267,7 +266,7 @@ struct HMSub {
 struct HMTeam {
     std::mutex m;
     std::condition_variable cv;
-    std::deque<HMSub> subs;
+    std::list<HMSub> subs;
     size_t next_kid = 0, kids_open = 0;
 };
 
@@ -291,11 +290,12 @@ void hm_run_sub(Ctx &w, HMTeam &t, HMSub &sub, const HMParams &p, u32 *global) {
 }
 
 // puts a subtree's children up and works (on them first) until they are done:
-// their graphs are in w's arena
-void hm_run_children(Ctx &w, HMTeam &t, std::vector<HMSub> &mine, HMOwner &o, const HMParams &p, u32 *global) {
+// their graphs are in w's arena.  From the splice on nothing throws until then
+// (the other workers hold the address of o).
+void hm_run_children(Ctx &w, HMTeam &t, std::list<HMSub> &mine, HMOwner &o, const HMParams &p, u32 *global) {
     std::unique_lock<std::mutex> lk(t.m);
     o.left = mine.size();
-    for (HMSub &x: mine) t.subs.push_back(std::move(x));
+    t.subs.splice(t.subs.end(), mine);
     t.cv.notify_all();
     while (o.left) {
         if (t.subs.empty()) {
@@ -304,10 +304,10 @@ void hm_run_children(Ctx &w, HMTeam &t, std::vector<HMSub> &mine, HMOwner &o, co
         }
         auto it = std::find_if(t.subs.begin(), t.subs.end(), [&](const HMSub &x) { return x.owner == &o; });
         if (it == t.subs.end()) it = t.subs.begin();
-        HMSub x = std::move(*it);
-        t.subs.erase(it);
+        std::list<HMSub> x;
+        x.splice(x.begin(), t.subs, it);
         lk.unlock();
-        hm_run_sub(w, t, x, p, global);
+        hm_run_sub(w, t, x.front(), p, global);
         lk.lock();
     }
     lk.unlock();
@@ -452,14 +452,13 @@ bool hm_split_parallel(Ctx &c, const DGraph &g, const u32 *tmp, const u32 *n_to_
     auto run = [&](size_t wi) {
         Ctx &w = *W[wi];
         (void) hipSetDevice(w.device);
-        if (&w != &c) ctx_copy_settings(w, c);
         std::unique_lock<std::mutex> lk(team.m);
         for (;;) {
             if (!team.subs.empty()) {
-                HMSub x = std::move(team.subs.front());
-                team.subs.pop_front();
+                std::list<HMSub> x;
+                x.splice(x.begin(), team.subs, team.subs.begin());
                 lk.unlock();
-                hm_run_sub(w, team, x, pt, global);
+                hm_run_sub(w, team, x.front(), pt, global);
                 lk.lock();
             } else if (team.next_kid < kids.size()) {
                 const size_t i = order[team.next_kid++];
@@ -475,11 +474,15 @@ bool hm_split_parallel(Ctx &c, const DGraph &g, const u32 *tmp, const u32 *n_to_
             }
         }
     };
+    // what may throw comes before the first thread starts
+    for (Ctx *w: W)
+        if (w != &c) ctx_copy_settings(*w, c);
     std::vector<std::thread> threads;
+    threads.reserve(nw);
     for (size_t wi = lending ? 1 : 0; wi < nw; ++wi) {
         try {
             threads.emplace_back(run, wi);
-        } catch (const std::system_error &) {
+        } catch (const std::exception &) {
             run(wi);  // no thread available: this worker's children run here
         }
     }
@@ -532,7 +535,7 @@ void hm_rec(Ctx &c, const DGraph &g, const u32 *n_to_o, u32 level, std::vector<u
         return;
     }
     if (p.team && ident.size() == 1) {
-        std::vector<HMSub> subs;
+        std::list<HMSub> subs;
         HMOwner owner;
         for (u32 id = 0; id < k; ++id) {
             DGraph child;
@@ -541,7 +544,7 @@ void hm_rec(Ctx &c, const DGraph &g, const u32 *n_to_o, u32 level, std::vector<u
             subs.push_back(HMSub{child, c_n_to_o, level - 1, {ident[0], id}, &owner});
         }
         c.sync();  // complete before other streams read them
-        std::stable_sort(subs.begin(), subs.end(), [](const HMSub &x, const HMSub &y) { return x.g.m > y.g.m; });
+        subs.sort([](const HMSub &x, const HMSub &y) { return x.g.m > y.g.m; });
         hm_run_children(c, *p.team, subs, owner, p, global);
         c.arena.release_front(depth0);
         return;
