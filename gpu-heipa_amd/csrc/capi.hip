@@ -334,7 +334,7 @@ int heipa_im_partition(heipa_ctx *ctx, const heipa_graph *g, const uint32_t *hie
         copy_h2d(c, Dd, Dh.data(), 4ull * k * k);
         ms.D = Dd;
         std::vector<heipa_level_trace> lv;
-        SolveResult r = solve(c, d, (u32) k, imbalance, seed, false, part, levels ? &lv : nullptr, &ms, &meta);
+        SolveResult r = solve(c, d, (u32) k, imbalance, seed, false, part, levels ? &lv : nullptr, &ms, &meta, stats != nullptr);
         c.sync();
         c.arena.release_front(depth0);
         fill_stats(stats, r);
@@ -354,7 +354,7 @@ int heipa_partition(heipa_ctx *ctx, const heipa_graph *g, uint32_t k, double imb
         BackScope bs(c.arena);
         const GraphMeta meta = validate(c, d);
         std::vector<heipa_level_trace> lv;
-        SolveResult r = solve(c, d, k, imbalance, seed, ultra != 0, part, levels ? &lv : nullptr, nullptr, &meta);
+        SolveResult r = solve(c, d, k, imbalance, seed, ultra != 0, part, levels ? &lv : nullptr, nullptr, &meta, stats != nullptr);
         if (stats) {
             stats->cut = r.cut;
             stats->maxw = r.maxw;

@@ -379,10 +379,17 @@ __global__ __launch_bounds__(CB) void copy_rows_kernel(u32 nc, const u32 *__rest
     }
 }
 
+// span (if any): the clock at the start of the first workgroup and at the ends of
+// the first and the last one (the XCDs' clocks agree to a microsecond)
 __global__ void project_kernel(const u32 *__restrict__ map, u32 n, const u32 *__restrict__ cpart,
-                               u32 *__restrict__ fpart) {
+                               u32 *__restrict__ fpart, u64 *span) {
+    if (span && blockIdx.x == 0 && threadIdx.x == 0) span[0] = wall_clock64();
     for (u64 u = (u64) blockIdx.x * blockDim.x + threadIdx.x; u < n; u += (u64) gridDim.x * blockDim.x)
         fpart[u] = cpart[map[u]];
+    if (span && threadIdx.x == 0) {
+        if (blockIdx.x == 0) span[1] = wall_clock64();
+        if (blockIdx.x == gridDim.x - 1) span[2] = wall_clock64();
+    }
 }
 
 template<int W>
@@ -499,9 +506,9 @@ CoarseGraph contract(Ctx &c, const DGraph &fine, const u32 *map, u32 nc, u32 max
     return out;
 }
 
-void project(Ctx &c, const u32 *map, u32 fine_n, const u32 *cpart, u32 *fpart) {
+void project(Ctx &c, const u32 *map, u32 fine_n, const u32 *cpart, u32 *fpart, u64 *span) {
     launch(c, "project", 12.0 * fine_n, dim3(grid_for(c, fine_n, 256 * 4)), dim3(256), 0, project_kernel, map, fine_n,
-           cpart, fpart);
+           cpart, fpart, span);
 }
 
 } // namespace heipa

@@ -210,6 +210,8 @@ struct Ctx {
     // pinned host staging for scalar readbacks
     void *pinned = nullptr;
     size_t pinned_bytes = 0;
+    u64 *spans = nullptr;  // pinned, behind the staging: three clock values for each of SPAN_LEVELS launches
+    static constexpr u32 SPAN_LEVELS = 128;
     std::string last_error;
     // profiling
     bool prof_on = false;
@@ -310,7 +312,8 @@ inline void ctx_open(Ctx &c, int device, uint64_t arena_bytes) {
         HIP_CHECK(hipMalloc(&c.arena_mem, arena_bytes));
         c.arena.init(c.arena_mem, arena_bytes);
         c.pinned_bytes = 1 << 18;
-        HIP_CHECK(hipHostMalloc(&c.pinned, c.pinned_bytes, hipHostMallocDefault));
+        HIP_CHECK(hipHostMalloc(&c.pinned, c.pinned_bytes + 24 * Ctx::SPAN_LEVELS, hipHostMallocDefault));
+        c.spans = (u64 *) ((char *) c.pinned + c.pinned_bytes);
         find_xccs(c);
     } catch (...) {
         ctx_close(c);

@@ -35,7 +35,8 @@ struct CoarseGraph {
 // max_row: no coarse vertex's members have more than this many edges together
 // (a matching joins two: twice the largest degree; ~0u if unknown)
 CoarseGraph contract(Ctx &c, const DGraph &fine, const u32 *mapping, u32 nc, u32 max_row);
-void project(Ctx &c, const u32 *mapping, u32 fine_n, const u32 *coarse_part, u32 *fine_part);
+// span (pinned, 3 words): the kernel's clock at its start and at the ends of two workgroups
+void project(Ctx &c, const u32 *mapping, u32 fine_n, const u32 *coarse_part, u32 *fine_part, u64 *span = nullptr);
 
 // ---- Jet refinement (jet.hip)
 // Largest k one Jet call takes: the sweep keeps one LDS counter per block for
@@ -64,10 +65,11 @@ struct MapSpec {
     const s32 *D = nullptr;
 };
 // map != null: ProMapSolver::solve (IM); cut / initial_cut / level cuts hold J.
-// meta: g's metadata where the caller has it (from validate)
+// meta: g's metadata where the caller has it (from validate); phases: the
+// caller reads ms[3] and ms[4] (projection and refinement are told apart)
 SolveResult solve(Ctx &c, const DGraph &g, u32 k, double imbalance, u64 seed, bool ultra, u32 *part,
                   std::vector<heipa_level_trace> *levels, const MapSpec *map = nullptr,
-                  const GraphMeta *meta = nullptr);
+                  const GraphMeta *meta = nullptr, bool phases = false);
 void hm_partition(Ctx &c, const DGraph &g, const std::vector<u32> &hier, double imbalance, u64 seed, bool ultra,
                   u32 *part, const GraphMeta *meta = nullptr);
 

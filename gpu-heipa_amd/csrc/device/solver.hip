@@ -660,7 +660,7 @@ void hier_append(Ctx &c, HierEntry &e, size_t l, u32 fine_n, const u32 *map, con
 } // namespace
 
 SolveResult solve(Ctx &c, const DGraph &g0, u32 k, double imbalance, u64 seed, bool ultra, u32 *part,
-                  std::vector<heipa_level_trace> *levels, const MapSpec *map, const GraphMeta *meta) {
+                  std::vector<heipa_level_trace> *levels, const MapSpec *map, const GraphMeta *meta, bool phases) {
     SolveResult res;
     require(k >= 1, "k must be >= 1");
     c.prof_l0 = false;
@@ -750,7 +750,7 @@ SolveResult solve(Ctx &c, const DGraph &g0, u32 k, double imbalance, u64 seed, b
     u32 *cur = pa, *other = pb;
     for (size_t l = maps.size(); l-- > 0;) {
         double ta = now_ms();
-        project(c, maps[l], graphs[l].n, cur, other);
+        project(c, maps[l], graphs[l].n, cur, other, phases && l < Ctx::SPAN_LEVELS ? c.spans + 3 * l : nullptr);
         std::swap(cur, other);
         double tb = now_ms();
         res.ms[3] += tb - ta;
@@ -769,6 +769,15 @@ SolveResult solve(Ctx &c, const DGraph &g0, u32 k, double imbalance, u64 seed, b
     }
     copy_d2d(c, part, cur, 4ull * n0);
     c.sync();
+    // A projection runs while the refinement's set-up is queued, whose wall time
+    // so includes it.  The kernels' own clocks (100 MHz) tell the two apart: a
+    // wait per level took 12 us, events around the launches 18.
+    for (size_t l = 0; phases && l < maps.size() && l < Ctx::SPAN_LEVELS; ++l) {
+        const u64 *t = c.spans + 3 * l, end = std::max(t[1], t[2]);
+        const double ms = end > t[0] ? (double) (end - t[0]) * 1e-5 : 0.0;
+        res.ms[3] += ms;
+        res.ms[4] -= ms;
+    }
     res.cut = cut;
     res.maxw = maxw;
     res.levels = (u32) graphs.size();
