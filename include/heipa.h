@@ -234,15 +234,15 @@ double heipa_pool_clock(const heipa_pool *pool);
  * one cache that all workers share */
 int heipa_pool_set_option(heipa_pool *pool, int option, uint64_t value);
 /* Autotuner of the batched form (no counterpart in the reference: its launch shapes are fixed).  Runs
- * the sample jobs through the pool once per candidate setting of three options that change launch
- * shapes but never results -- HEIPA_OPT_GROUP_CAP in {64, 16, 8}, HEIPA_OPT_BLOCK_GROUP_CAP in
- * {16, 8, 4}, HEIPA_OPT_BLOCK_JET in {1024, 2048, 4096} -- one option at a time starting from the
- * current setting (each value other than the option's starting one runs once: 2 + 6 runs from the
- * defaults), takes a candidate when the sample runs at least 2% faster with it than the best so far,
- * and leaves the chosen setting on every worker (call while no job runs).  The sample's outputs are those of its
- * last run; a failed sample job ends the tuning with its status. */
+ * the sample jobs through the pool once per candidate setting of two options that change launch
+ * shapes but never results -- HEIPA_OPT_GROUP_CAP in {64, 16, 8}, HEIPA_OPT_BLOCK_JET in {1024, 2048,
+ * 4096} -- one option at a time starting from the current setting (each value other than the option's
+ * starting one runs once), takes a candidate when the sample runs at least 2% faster with it than the
+ * best so far, times the chosen and the starting setting once more (2 + 4 + 2 runs from the defaults)
+ * and leaves the faster of these two on every worker (call while no job runs).  The sample's outputs
+ * are those of its last run; a failed sample job ends the tuning with its status. */
 typedef struct {
-    uint32_t group_cap, block_group_cap, block_jet;  /* the chosen setting */
+    uint32_t group_cap, block_group_cap, block_jet;  /* the setting left (the second: as it was, without effect) */
     uint32_t runs;                                   /* sample runs, the untimed first one included */
     double ms_start, ms_best;                        /* sample wall time at the starting and the chosen setting */
 } heipa_tune;
@@ -311,7 +311,7 @@ int heipa_pool_hier_cache_stats(const heipa_pool *pool, uint64_t *entries, uint6
  * apply and row launches (default 64, i.e. the power of two at or above the level's average degree,
  * at most 64; a smaller value rounds down to a power of two, at least 4).  Results do not depend on it.
  * HEIPA_OPT_BLOCK_GROUP_CAP: accepted, without effect (it was the same cap of the former
- * single-workgroup form; a team's rows are 16 lanes wide).  heipa_pool_autotune picks both for a pool. */
+ * single-workgroup form; a team's rows are 16 lanes wide).  heipa_pool_autotune picks the former for a pool. */
 #define HEIPA_OPT_GROUP_CAP 12
 #define HEIPA_OPT_BLOCK_GROUP_CAP 13
 /* HEIPA_OPT_REGION_EDGES: the multi-launch Jet gives each sweep workgroup a region of the level's

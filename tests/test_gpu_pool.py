@@ -204,3 +204,20 @@ def test_pool_autotune_reports_a_failed_sample_job(ctx):
     finally:
         pool.close()
 
+
+
+def test_pool_autotune_leaves_dead_options(ctx):
+    """Options without effect are not searched: no sample run is spent on
+    HEIPA_OPT_BLOCK_GROUP_CAP, and it stays as it was set."""
+    reqs = workloads.batched(4)
+    dgs = [_dev(g) for g, _, _ in reqs]
+    pool = heipa.Pool(2, 256 << 20)
+    try:
+        pool.set_option(heipa.OPT_BLOCK_GROUP_CAP, 5)
+        t = pool.autotune([heipa.Pool.job(dg, imbalance=0.03, seed=1, **spec) for dg, (_, spec, _) in zip(dgs, reqs)])
+        assert t["block_group_cap"] == 5
+        assert t["runs"] == 8  # a warm-up, the start, two options of two further values, the choice and the start again
+        assert t["group_cap"] in (64, 16, 8) and t["block_jet"] in (1024, 2048, 4096)
+        assert 0 < t["ms_best"] <= t["ms_start"]
+    finally:
+        pool.close()
