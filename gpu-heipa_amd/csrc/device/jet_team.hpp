@@ -1135,8 +1135,10 @@ __global__ __launch_bounds__(TM, PER_CU == 2 ? 4 : 1) void jet_team_kernel(JetDe
     __syncthreads();
     if (failed && tid == 0) dg.ctl->failed = 1;
     if (rank == 0 && !failed) {
-        if (tid == 0) ctl->launches++;
-        __syncthreads();
-        if (tid < CW) ((u64 *) dg.ctl)[tid] = s_ctl[tid];
+        // all but `failed`, the last word's other half: a member that gave up
+        // on the last barrier has set it
+        static_assert(offsetof(JetCtl, launches) == 8 * (CW - 1) && offsetof(JetCtl, failed) == 8 * (CW - 1) + 4, "last word");
+        if (tid == 0) dg.ctl->launches = ctl->launches + 1;
+        if (tid < CW - 1) ((u64 *) dg.ctl)[tid] = s_ctl[tid];
     }
 }
