@@ -233,69 +233,69 @@ __global__ __launch_bounds__(CB) void row_block_kernel(DGraph g, const u32 *__re
     __shared__ u32 red[CB / WAVE];
     const u32 rows = *len_ptr;
     for (u32 row = blockIdx.x; row < rows; row += gridDim.x) {
-    const u32 c = list[row];
-    const u32 len = uboff[c + 1] - uboff[c];
-    // P is a power of two and a multiple of the block size, so every thread's
-    // slot in the dedupe loop below holds a sorted key or PAD
-    u32 P = CB;
-    while (P < len) P <<= 1;
-    // gather: walk the members' adjacency ranges in order
-    {
-        u32 base = 0;
-        for (u32 t = moff[c]; t < moff[c + 1]; ++t) {
-            const u32 u = mem[t];
-            const u32 b = g.xadj[u], d = g.xadj[u + 1] - b;
-            for (u32 x = threadIdx.x; x < d; x += CB) {
-                const u32 y = map[g.adj[b + x]];
-                skey[base + x] = y == c ? PAD : y;
-                sw[base + x] = UEW ? 1 : g.ew[b + x];
+        const u32 c = list[row];
+        const u32 len = uboff[c + 1] - uboff[c];
+        // P is a power of two and a multiple of the block size, so every thread's
+        // slot in the dedupe loop below holds a sorted key or PAD
+        u32 P = CB;
+        while (P < len) P <<= 1;
+        // gather: walk the members' adjacency ranges in order
+        {
+            u32 base = 0;
+            for (u32 t = moff[c]; t < moff[c + 1]; ++t) {
+                const u32 u = mem[t];
+                const u32 b = g.xadj[u], d = g.xadj[u + 1] - b;
+                for (u32 x = threadIdx.x; x < d; x += CB) {
+                    const u32 y = map[g.adj[b + x]];
+                    skey[base + x] = y == c ? PAD : y;
+                    sw[base + x] = UEW ? 1 : g.ew[b + x];
+                }
+                base += d;
             }
-            base += d;
+            for (u32 x = len + threadIdx.x; x < P; x += CB) {
+                skey[x] = PAD;
+                sw[x] = 0;
+            }
         }
-        for (u32 x = len + threadIdx.x; x < P; x += CB) {
-            skey[x] = PAD;
-            sw[x] = 0;
-        }
-    }
-    __syncthreads();
-    for (u32 k = 2; k <= P; k <<= 1) {
-        for (u32 jj = k >> 1; jj > 0; jj >>= 1) {
-            for (u32 i = threadIdx.x; i < P; i += CB) {
-                const u32 p = i ^ jj;
-                if (p > i) {
-                    const bool up = (i & k) == 0;
-                    const u32 a = skey[i], b = skey[p];
-                    if (up ? (a > b) : (a < b)) {
-                        skey[i] = b;
-                        skey[p] = a;
-                        const s32 t = sw[i];
-                        sw[i] = sw[p];
-                        sw[p] = t;
+        __syncthreads();
+        for (u32 k = 2; k <= P; k <<= 1) {
+            for (u32 jj = k >> 1; jj > 0; jj >>= 1) {
+                for (u32 i = threadIdx.x; i < P; i += CB) {
+                    const u32 p = i ^ jj;
+                    if (p > i) {
+                        const bool up = (i & k) == 0;
+                        const u32 a = skey[i], b = skey[p];
+                        if (up ? (a > b) : (a < b)) {
+                            skey[i] = b;
+                            skey[p] = a;
+                            const s32 t = sw[i];
+                            sw[i] = sw[p];
+                            sw[p] = t;
+                        }
                     }
                 }
+                __syncthreads();
             }
-            __syncthreads();
         }
-    }
-    // unique heads, ranks by block scan, run sums by the head thread
-    u32 carry = 0;
-    for (u32 b0 = 0; b0 < P; b0 += CB) {
-        const u32 i = b0 + threadIdx.x;
-        const u32 key = skey[i];
-        const bool head = key != PAD && (i == 0 || skey[i - 1] != key);
-        u32 tot;
-        const u32 rank = block_exclusive_scan<CB>(head ? 1u : 0u, red, tot);
-        if (head) {
-            s64 s = 0;
-            for (u32 x = i; x < P && skey[x] == key; ++x) s += sw[x];
-            if (s > INT32_MAX) *overflow = 1;
-            tkey[uboff[c] + carry + rank] = key;
-            tw[uboff[c] + carry + rank] = (s32) s;
+        // unique heads, ranks by block scan, run sums by the head thread
+        u32 carry = 0;
+        for (u32 b0 = 0; b0 < P; b0 += CB) {
+            const u32 i = b0 + threadIdx.x;
+            const u32 key = skey[i];
+            const bool head = key != PAD && (i == 0 || skey[i - 1] != key);
+            u32 tot;
+            const u32 rank = block_exclusive_scan<CB>(head ? 1u : 0u, red, tot);
+            if (head) {
+                s64 s = 0;
+                for (u32 x = i; x < P && skey[x] == key; ++x) s += sw[x];
+                if (s > INT32_MAX) *overflow = 1;
+                tkey[uboff[c] + carry + rank] = key;
+                tw[uboff[c] + carry + rank] = (s32) s;
+            }
+            carry += tot;
         }
-        carry += tot;
-    }
-    if (threadIdx.x == 0) cnt[c] = carry;
-    __syncthreads();  // the next row restages the LDS
+        if (threadIdx.x == 0) cnt[c] = carry;
+        __syncthreads();  // the next row restages the LDS
     }
 }
 

@@ -1707,24 +1707,24 @@ __device__ __forceinline__ bool resolve_body(const JD &d, bool strong, u32 stamp
     } else if (P2 <= NT) {
         sort_keys_one_per_thread(d.rlist, L, P2, skey);
     } else {
-    for (u32 i = threadIdx.x; i < P2; i += NT) skey[i] = i < L ? (u64) d.rlist[i] : ~0ull;
-    __syncthreads();
-    // bitonic sort, ascending
-    for (u32 kk = 2; kk <= P2; kk <<= 1) {
-        for (u32 j = kk >> 1; j > 0; j >>= 1) {
-            for (u32 i = threadIdx.x; i < P2; i += NT) {
-                const u32 p = i ^ j;
-                if (p > i) {
-                    const u64 a = skey[i], b = skey[p];
-                    if (((i & kk) == 0) ? (a > b) : (a < b)) {
-                        skey[i] = b;
-                        skey[p] = a;
+        for (u32 i = threadIdx.x; i < P2; i += NT) skey[i] = i < L ? (u64) d.rlist[i] : ~0ull;
+        __syncthreads();
+        // bitonic sort, ascending
+        for (u32 kk = 2; kk <= P2; kk <<= 1) {
+            for (u32 j = kk >> 1; j > 0; j >>= 1) {
+                for (u32 i = threadIdx.x; i < P2; i += NT) {
+                    const u32 p = i ^ j;
+                    if (p > i) {
+                        const u64 a = skey[i], b = skey[p];
+                        if (((i & kk) == 0) ? (a > b) : (a < b)) {
+                            skey[i] = b;
+                            skey[p] = a;
+                        }
                     }
                 }
+                __syncthreads();
             }
-            __syncthreads();
         }
-    }
     }
     // exclusive prefix of the weights in sorted order
     s64 carry = 0;
