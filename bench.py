@@ -10,8 +10,8 @@ the plain drop-in, with p50/p99 latency at equal cut:
     `default`) through the worker pool.  The K timed steps together process
     every graph exactly once (ceil(4096 / K) graphs per step); `value` is
     their undirected input edges / the time of the K steps.  Before the
-    warmup, the pool's autotuner picks the lane-group caps and the
-    edge bound of Jet's teams on a sample of 64 of the graphs (launch shapes
+    warmup, the pool's autotuner picks the lane-group cap and the
+    edge bound of Jet's one-XCD team on a sample of 64 of the graphs (launch shapes
     only: results do not change).  The plain path
     (one context, graphs one after another) is timed on the graphs of the
     first timed step beside it, and every one of those partitions must be

@@ -3094,12 +3094,17 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
     }
     h.big_resolve = c.max_lds >= 160 * 1024;
     // Team form on one XCD: levels whose iterations are chains of latency; on
-    // all XCDs: larger ones.  Measured, us per iteration (one XCD / all XCDs /
-    // multi-launch): RGG, k = 64, 8000 vertices 16.5 / 21.8 / 33, 16000 18.9 /
-    // 21.1 / 34, 30000 22.3 / 22.4 / 34, 60000 29.5 / 23.0 / 33, 500000 - / 37 /
-    // 45, 1000000 - / 47 / 50, 3000000 - / 130 / 135.  Skewed levels, k = 16:
-    // R-MAT of 400 vertices and 3200 edges 42 / 46 / 61, 1000 and 8000 55 / 48 /
-    // 68, 16000 and 256000 274 / 104 / 132, 1000000 and 12 million - / 1150 / 1840.
+    // all XCDs: larger ones.  Measured on whole refine calls of 13 to 26
+    // iterations, us per iteration with the level's set-up (one XCD / all XCDs /
+    // multi-launch): RGG of degree 12, k = 64, 3000 vertices 17.1 / 24.2 / 35.5,
+    // 16000 21.5 / 25.4 / 38.0, 30000 27.4 / 27.2 / 40.2, 60000 41.6 / 29.5 /
+    // 44.6, 500000 - / 47 / 58, 1000000 - / 64 / 75, 3000000 - / 142 / 164.
+    // Skewed levels, k = 16: R-MAT of 400 vertices and 5150 edges 33.4 / 42.8 /
+    // 61.2, 1000 and 12158 38.7 / 45.2 / 67.4, 3000 and 19482 52.7 / 43.4 / 71.2,
+    // 16000 and 425936 288 / 79 / 129, 1000000 and 16 million - / 693 / 954.
+    // With eight contexts at once the one-XCD form gains: 400 vertices 452 us a
+    // call against 634, 1000 vertices and 9580 edges 406 against 577, 3000 and
+    // 10174 616 against 566.
     {
         const size_t cgb = conn_group_bytes(k);
         h.ta.wgroups = (u32) std::min<size_t>(WAVE / ROW, std::max<size_t>(1, TEAM_CONN_LDS / (cgb * TW)));
@@ -3111,8 +3116,14 @@ JetResult jet_refine(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 *part, 
         const bool narrow = (!h.flat && n <= c.team_jet_max_n && (u64) g.m <= 16ull * n) ||
                             (n <= std::max(c.team_jet_max_n, c.block_jet_max_n) && (u64) g.m <= dense);
         const u32 want = std::min<u32>({WIDE_MAX, (u32) c.num_cus, std::max<u32>(div_up(n, 64), div_up(g.m, 512u))});
-        // two members per compute unit: where one would take a second sweep step
-        // (regular levels only: skewed ones have long resolve lists)
+        // Two members per compute unit: where one would take a second sweep step.
+        // The figures are at the kernel; the price is a resolve list of 2048
+        // instead of 8192 entries, the longer ones (levels far out of balance)
+        // leave the launch.  RGG of degree 6, k = 64, ms per refine with two / one
+        // / as launches: 140000 vertices, 300 of them moved to one block 6.67 /
+        // 7.06 / 8.54, 100000 moved 4.95 / 3.79 / 6.04; 300000 vertices 8.73 / 8.19
+        // / 10.6 and 8.44 / 6.81 / 9.75; 1000000 16.3 / 18.1 / 22.9 and 10.5 / 11.3 /
+        // 17.0.  Skewed levels keep one: theirs are long.
         const size_t all = team_lds_bytes(k, h.ta.wgroups, RESOLVE_CAP), half = team_lds_bytes(k, h.ta.wgroups, 2048);
         const bool twice = !h.flat && n > (u64) c.num_cus * TW * WAVE && 2 * (half + 2048) <= c.max_lds;
         const u32 members = twice ? std::min<u32>(WIDE_MAX, 2 * (u32) c.num_cus) : want;

@@ -11,9 +11,9 @@
 // 0.6 us whether 8 or 32 take part, and the level's state stays in that L2 (88
 // ns); over all XCDs a barrier takes 2.0 us.  What bounds both is the chain of
 // dependent loads and instructions of each phase, plus three barriers (LP) or
-// five (rebalancing) per iteration.  us per iteration: 15 against 33 at 3000
-// vertices, 23 against 33 at 60000, 37 against 45 at 500000 (RGG, k = 64), 104
-// against 132 at 16000 vertices of R-MAT.
+// five (rebalancing) per iteration.  us per iteration, set-up of the level
+// included: 17 against 36 at 3000 vertices, 30 against 45 at 60000, 47 against
+// 58 at 500000 (RGG, k = 64), 79 against 129 at 16000 vertices of R-MAT.
 //
 // The team itself (formation, barrier, hand-offs) is team.hpp.
 #pragma once
@@ -386,9 +386,10 @@ __host__ __device__ inline u32 wide_cap(u32 n, u32 members, u32 n_hubs) {
 // the member that made them (regions of cand and moves, counted in LDS): one
 // list for all would cost an update of one address per wave (15 ns each, 2048
 // waves).  Totals have a copy per XCD.  PER_CU 2: two members per compute unit,
-// 128 registers each (26 spilled), for levels whose sweep takes one member per
-// unit several steps: us per iteration with one / two, RGG, 300000 vertices
-// 31.6 / 29.4, 1000000 51.4 / 47.0, 1500000 48.7 / 41.4, 3000000 151 / 130.
+// 128 registers each (28 spilled), for levels whose sweep takes one member per
+// unit several steps: us per iteration with one / two, balanced RGG, k = 64, set-up
+// included: degree 12, 140000 vertices 33.5 / 31.8, 1000000 67.4 / 63.9; degree 6,
+// 300000 31.9 / 31.6, 1500000 63.1 / 57.7, 3000000 110 / 90.
 template<bool FLAT, bool MAP, bool WIDE, int PER_CU = 1>
 __global__ __launch_bounds__(TM, PER_CU == 2 ? 4 : 1) void jet_team_kernel(JetDevT<true, MAP> dg, TeamArgs ta) {
     extern __shared__ __align__(16) char smem[];

@@ -77,6 +77,8 @@ typedef struct {
     int64_t initial_cut;       /* cut of the initial partition on the coarsest graph */
     uint32_t levels;           /* number of graphs in the hierarchy */
     uint32_t jet_iterations;   /* Jet iterations over all levels */
+    /* wall time of the phases; ms_uncontraction is the projections', whose time on the device is taken from
+     * their own clocks (they overlap the set-up of the refinement that follows) */
     double ms_coarsening, ms_contraction, ms_initial, ms_uncontraction, ms_refinement;
 } heipa_solve_stats;
 
