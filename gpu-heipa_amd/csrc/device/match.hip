@@ -1088,7 +1088,7 @@ void pair_by_key(Ctx &c, K *keys, u32 *vals, u32 len, u32 bits, u32 *vcmap) {
     K *ktmp = bs.get<K>(len);
     u32 *vtmp = bs.get<u32>(len);
     const u64 tiles = div_up(len, RS_TILE);
-    if (c.n_xcc && c.block_jet_max_n && len <= PT_LIST && c.arena.spare(sizeof(PairTeam), 12ull * len + 1024 * tiles)) {
+    if (c.n_xcc && c.block_jet_max_n && len <= PT_LIST && c.arena.spare(sizeof(PairTeam), 12ull * len + 1100 * tiles)) {
         PairTeam *pt = bs.get<PairTeam>(1);
         fill<u32>(c, (u32 *) pt, sizeof(TeamHead) / 4 + 32, 0u);
         PairTeamArgs<K> a{pt, {{keys}, {ktmp}}, {{vals}, {vtmp}}, len, bits, c.xcc, std::min<u32>(TEAM_WANT, div_up(len, 256)),
@@ -1136,7 +1136,7 @@ u32 match(Ctx &c, const DGraph &g, const GraphMeta &meta, u32 seed, u32 *mapping
     u64 *pkeys[2] = {nullptr, nullptr};
     PairScratch *ps = nullptr;
     {
-        const u64 keep = 32ull * n + 1024ull * div_up(n, RS_TILE), ent = std::min(n, PT_LIST);
+        const u64 keep = 32ull * n + 1100ull * div_up(n, RS_TILE), ent = std::min(n, PT_LIST);
         const u64 pair = 16 * ent + sizeof(PairScratch);
         if (c.n_xcc && c.block_jet_max_n && c.arena.spare(sizeof(MatchTeam), keep))  // HEIPA_OPT_BLOCK_JET 0: one launch per step
             mt = bs.get<MatchTeam>(1);
