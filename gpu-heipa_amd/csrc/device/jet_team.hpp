@@ -25,6 +25,7 @@ constexpr u32 TILE = WAVE * TEAM_U;           // vertices of one sweep step of a
 constexpr u32 TEAM_BUF = 2048;                // list entries a workgroup collects (edge-balanced form)
 constexpr u32 ROW_DEG = 2 * ROW;              // largest degree of the register form of a rebuild
 constexpr u32 LONG_DEG = 128;                 // degree from which a rebuild takes a whole wave
+constexpr u32 ROW_FEW = 16;                   // wide vertices of a wave up to which 16 lanes update each one's row
 constexpr size_t TEAM_CONN_LDS = 64 * 1024;   // block counters of the others, per workgroup
 constexpr u32 TEAM_BW = 1024;                 // blocks whose weight changes a workgroup sums in LDS
 
@@ -1064,9 +1065,13 @@ __global__ __launch_bounds__(TM, PER_CU == 2 ? 4 : 1) void jet_team_kernel(JetDe
             if (FLAT && WIDE) off = wl * NWV + (gw + wl * 37) % NWV;
             if (d.W <= 2) {
                 // From the adjacencies, a lane, a row or a wave each by their
-                // length.  Counts kept by the moves (two updates of shared
-                // memory per edge of a moved vertex) made the apply step of a
-                // skewed level 50 us where most vertices move; walking the
+                // length; where a wave has few of them, a row takes also those
+                // that a lane would walk alone, four neighbours at a time: with
+                // lanes only, the rows took 12 of the 28 us of an iteration at 40
+                // to 75 vertices of degree 24 (3 of 19 us now; a limit of 8 or 32
+                // vertices: the same).  Counts kept by the moves (two updates of
+                // shared memory per edge of a moved vertex) made the apply step of
+                // a skewed level 50 us where most vertices move; walking the
                 // touched rows again is a gather per edge.
                 u32 *list = (u32 *) um + wid * TILE;
                 for (u64 t0 = 0; t0 < d.n; t0 += (u64) NWV * tile) {
@@ -1074,10 +1079,11 @@ __global__ __launch_bounds__(TM, PER_CU == 2 ? 4 : 1) void jet_team_kernel(JetDe
                     const u32 v = (u32) vv;
                     const bool flagged = wl < tile && vv < d.n && (d.rflag[v] & 3u) == 3u;
                     const u32 deg = flagged ? degree(d, v) : 0u;
-                    const bool mid = deg > ROW_THREAD_DEG && deg <= 2 * LONG_DEG;
+                    const u32 lane_deg = (u32) __popcll(__ballot(deg > 4 && deg <= ROW_THREAD_DEG)) <= ROW_FEW ? 4u : ROW_THREAD_DEG;
+                    const bool mid = deg > lane_deg && deg <= 2 * LONG_DEG;
                     const u64 bm = __ballot(mid);
                     if (mid) list[(u32) __popcll(bm & lanemask_lt())] = v;
-                    if (flagged && deg <= ROW_THREAD_DEG) row_thread(d, v, rmode);
+                    if (flagged && deg <= lane_deg) row_thread(d, v, rmode);
                     wave_sync();
                     const u32 nl = (u32) __popcll(bm);
                     for (u32 r0 = 0; r0 < nl; r0 += WAVE / ROW) {

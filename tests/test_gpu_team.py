@@ -287,11 +287,7 @@ ROWS = {
 }
 
 
-@pytest.mark.parametrize("form", ["one_xcd", "all_xcds"])
-@pytest.mark.parametrize("name", sorted(ROWS))
-def test_team_rows_many_blocks(ctx, name, form):
-    make, k = ROWS[name]
-    g = make()
+def _rows(ctx, name, g, k, form):
     part0 = _start(g, k, 0.8)
     lmax = math.ceil(1.03 * g.g_weight / k)
     cut0, maxw0 = orc.edge_cut(g, part0), int(block_weights(g, part0, k).max())
@@ -309,3 +305,18 @@ def test_team_rows_many_blocks(ctx, name, form):
     _compare(gtr, otr, name)
     assert (gcut, gmaxw) == (ocut, omaxw)
     assert np.array_equal(heipa.to_numpy_u32(pd), op)
+
+
+@pytest.mark.parametrize("form", ["one_xcd", "all_xcds"])
+@pytest.mark.parametrize("name", sorted(ROWS))
+def test_team_rows_many_blocks(ctx, name, form):
+    make, k = ROWS[name]
+    _rows(ctx, name, make(), k, form)
+
+
+@pytest.mark.parametrize("form", ["one_xcd", "all_xcds"])
+@pytest.mark.parametrize("deg", [4, 5, 32, 33])
+@pytest.mark.parametrize("n", [40, 700, 20000])
+def test_team_rows_few_blocks(ctx, n, deg, form):
+    """Every vertex wide, few or many of them to a wave: rows by a lane or by 16."""
+    _rows(ctx, f"n{n} deg{deg}", _regular(n, deg), 4, form)
